@@ -16,6 +16,7 @@
 
 #include "rr_device.hpp"
 #include "rr_internal.hpp"
+#include "window_flux.hpp"
 
 namespace rr {
 
@@ -136,15 +137,13 @@ __device__ double ma_quad_z(double z, double k, double u1, double u2) {
 }
 
 struct MaArgs {
-    const double* times; const int32_t* lcids; const int32_t* pbids; const int32_t* epids;
-    const int32_t* nsamples; const double* exptimes;
-    const double* k; const double* t0; const double* p; const double* a; const double* ldc;
+    WfData d;
+    const int32_t* pbids; const int32_t* epids; const double* exptimes;
+    const double* k; const double* t0; const double* ldc;
     const PvRec* rec;
     double* flux;
-    int npv, npt, nlc, npb, kcols, t0cols, ntiles;
+    int npv, npb, kcols, t0cols;
 };
-
-constexpr int kMaThreads = 256;
 
 // Orbit and contact window of each pv (the reference computes them for every pv).
 __global__ void __launch_bounds__(64) ma_orbit_kernel(int npv, const double* P, const double* A, const double* I,
@@ -170,50 +169,126 @@ __global__ void __launch_bounds__(64) ma_orbit_kernel(int npv, const double* P, 
     }
 }
 
-// ma_quadratic_nb.py:557-594
-__global__ void __launch_bounds__(kMaThreads) ma_flux_kernel(MaArgs f) {
-    const int bid = xcd_remap(blockIdx.x, gridDim.x);
-    const int pv = bid / f.ntiles;
-    const int it = (bid - pv * f.ntiles) * kMaThreads + threadIdx.x;
-    if (it >= f.npt) return;
-    const PvRec& r = f.rec[pv];
-    double* out = f.flux + (size_t)pv * f.npt + it;
-    if (!r.good) {
-        *out = INFINITY;
-        return;
+// Flux at separation z of a planet with 0 < k < 1 inside the disk (z < 1 - k) or
+// across its limb, away from the special separations: ma_quad_z's two general cases
+// written with the quantities they share.  With x1 = (k-z)^2 and x2 = (k+z)^2 and
+// D = 1 - x1 (inside) or 4 k z (limb), the squared complementary modulus is
+// |1 - x2| / D in both, the prefactor 2 / (9 pi sqrt D), and Bulirsch's start value
+// sqrt(n + 1) is (k+z) / |k-z| inside and 1 / |k-z| on the limb, so that the modulus,
+// its square root and the square root of n + 1 are not formed, and both cases run the
+// same iteration.  Iterations take one reciprocal and one square root each.
+__device__ __forceinline__ double ma_general(double z, double k, double u1, double u2, bool inside) {
+    const double inv_pi = 1.0 / kPi;
+    const double k2 = k * k, z2 = z * z;
+    const double dm = k - z, sp = k + z;
+    const double x1 = dm * dm, x2 = sp * sp, x3 = dm * sp;
+    const double D = inside ? 1.0 - x1 : 4.0 * k * z;
+    const double rD = f64_rcp(D);
+    const double m1 = fabs(1.0 - x2) * rD;
+    const double ratio = f64_div(sp, dm);                    // (k + z) / (k - z)
+    const double kc0 = f64_sqrt(m1);
+    // K and E by the polynomials of ma_ellk and ma_ellec, one logarithm for both
+    const double lm = log(m1);
+    const double kk = (1.38629436112 + m1 * (0.09666344259 + m1 * (0.03590092383 + m1 * (0.03742563713 + m1 * 0.01451196212)))) -
+                      (0.5 + m1 * (0.12498593597 + m1 * (0.06880248576 + m1 * (0.03328355346 + m1 * 0.00441787012)))) * lm;
+    const double ek = (1.0 + m1 * (0.44325141463 + m1 * (0.06260601220 + m1 * (0.04757383546 + m1 * 0.01736506451)))) -
+                      m1 * (0.24998368310 + m1 * (0.09200180037 + m1 * (0.04069697526 + m1 * 0.00526449639))) * lm;
+    // Pi (ma_ellpicb)
+    double p = inside ? fabs(ratio) : f64_rcp(fabs(dm));
+    double kc = kc0, e = kc0, m0 = 1.0, c = 1.0, dd = inside ? f64_rcp(p) : fabs(dm), pk = 0.0;
+    for (int it = 0; it < 1000; ++it) {
+        const double rp = it == 0 ? dd : f64_rcp(p);
+        const double fo = c;
+        c = fma(dd, rp, c);
+        const double g = e * rp;
+        dd = 2.0 * fma(fo, g, dd);
+        p = g + p;
+        const double mo = m0;
+        m0 = kc + m0;
+        if (fabs(mo - kc) > 1e-8 * mo) {
+            kc = 2.0 * f64_sqrt(e);
+            e = kc * m0;
+        } else {
+            pk = kHalfPi * f64_div(fma(c, m0, dd), m0 * (m0 + p));
+            break;
+        }
     }
-    const int ilc = f.nlc == 1 ? 0 : min(max(f.lcids[it], 0), f.nlc - 1);
-    const int iep = min(max(f.epids[ilc], 0), f.t0cols - 1);
-    const double t0v = f.t0[(size_t)pv * f.t0cols + iep];
-    const double p = r.p;
-    double tc;
-    {
-#pragma clang fp contract(off)
-        const double t = f.times[it];
-        const double epoch = floor((t - t0v + 0.5 * p) / p);
-        tc = t - (t0v + epoch * p);
+    const double A = inside ? 1.0 - 5.0 * z2 + k2 + x3 * x3 : (1.0 - x2) * (2.0 * x2 + x1 - 3.0) - 3.0 * x3 * (x2 - 2.0);
+    const double B = (inside ? 1.0 - x1 : D) * (z2 + 7.0 * k2 - 4.0);
+    double ld = 2.0 / 9.0 * inv_pi * f64_sqrt(rD) * (A * kk + B * ek - 3.0 * ratio * pk);
+    if (z < k) ld += 2.0 / 3.0;
+    double le, ed;
+    if (inside) {
+        le = k2;
+        ed = 0.5 * k2 * (k2 + 2.0 * z2);
+    } else {
+        const double kap1 = acos(fmin(f64_div(1.0 - k2 + z2, 2.0 * z), 1.0));
+        const double kap0 = acos(fmin(f64_div(k2 + z2 - 1.0, 2.0 * k * z), 1.0));
+        const double lune = f64_sqrt((1.0 - x1) * (x2 - 1.0));
+        le = (k2 * kap0 + kap1 - 0.5 * lune) * inv_pi;
+        ed = 0.5 * inv_pi * (kap1 + k2 * (k2 + 2.0 * z2) * kap0 - 0.25 * (1.0 + 5.0 * k2 + z2) * lune);
     }
-    if (!(r.bt1 - 0.025 <= tc && tc <= r.bt4 + 0.025)) {
-        *out = 1.0;
-        return;
-    }
-    const int ipb = min(max(f.pbids[ilc], 0), f.npb - 1);
-    const double k = f.k[(size_t)pv * f.kcols + (f.kcols == 1 ? 0 : ipb)];
-    const double u1 = f.ldc[(size_t)pv * 2 * f.npb + 2 * ipb], u2 = f.ldc[(size_t)pv * 2 * f.npb + 2 * ipb + 1];
-    if (isnan(u1) || isnan(u2)) {
-        *out = INFINITY;
-        return;
-    }
-    const int ns = f.nsamples[ilc];
-    const double ext = f.exptimes[ilc];
-    double acc = 0.0;
-    for (int is = 1; is <= ns; ++is) {
-        const double off = ext * ((is - 0.5) / ns - 0.5);
-        const double z = taylor_z<double>(tc + off, r.c);
-        acc += (z > 1.0 + k) ? 1.0 : ma_quad_z(z, k, u1, u2);
-    }
-    *out = acc / ns;
+    return 1.0 - f64_div((1.0 - u1 - 2.0 * u2) * le + (u1 + 2.0 * u2) * ld + u2 * ed, 1.0 - u1 / 3.0 - u2 / 6.0);
 }
+
+// ma_quadratic_nb.py:557-594 on the window kernel.
+struct MaModel {
+    using Real = double;
+    using Args = MaArgs;
+    static constexpr int kKinds = 2;    // 1 inside the disk (and the special cases), 2 on the limb
+    static constexpr int kGroup = 1;
+    struct Pv {
+        double c[10], lo, hi, p, inv_p;
+        bool good;
+    };
+    struct Item {
+        double ext, inv_ns, k, u1, u2;
+    };
+    static __device__ __forceinline__ Pv load(const MaArgs& f, int pv) {
+        const PvRec& r = f.rec[pv];
+        Pv o;
+#pragma unroll
+        for (int j = 0; j < 10; ++j) o.c[j] = r.c[j];
+        o.lo = r.bt1 - 0.025;
+        o.hi = r.bt4 + 0.025;
+        o.p = r.p;
+        o.inv_p = r.inv_p;
+        o.good = r.good != 0;
+        return o;
+    }
+    static __device__ __forceinline__ double fill(const Pv&) { return 1.0; }
+    static __device__ __forceinline__ double bad() { return INFINITY; }
+    static __device__ __forceinline__ WfWindow window(const MaArgs& f, const Pv& c, int pv, int ilc) {
+        return {f.t0[(size_t)pv * f.t0cols + min(max(f.epids[ilc], 0), f.t0cols - 1)], c.lo, c.hi};
+    }
+    static __device__ __forceinline__ Item item(const MaArgs& f, const Pv&, int pv, int ilc) {
+        const int ipb = min(max(f.pbids[ilc], 0), f.npb - 1);
+        const double* u = f.ldc + (size_t)pv * 2 * f.npb + 2 * ipb;
+        return {f.exptimes[ilc], 1.0 / f.d.nsamples[ilc], f.k[(size_t)pv * f.kcols + (f.kcols == 1 ? 0 : ipb)], u[0], u[1]};
+    }
+    static __device__ __forceinline__ int classify(const MaArgs&, const Pv& c, const Item& I, double t, double& v) {
+        if (isnan(I.u1) || isnan(I.u2)) {
+            v = INFINITY;
+            return 0;
+        }
+        const double z = taylor_z<double>(t, c.c);
+        v = z > 1.0 + I.k ? 1.0 : z;
+        if (z > 1.0 + I.k) return 0;
+        return z < 1.0 - I.k ? 1 : 2;
+    }
+    template <int G>
+    static __device__ __forceinline__ double heavy(const MaArgs&, const Pv&, const Item& I, double, double z, int kind,
+                                                   int, unsigned char*) {
+        const double k = I.k;
+        // a planet as large as the star, k = 0.5, the disk's centre or limb grazed by the
+        // planet's centre or edge, and anything not finite: the case analysis in full
+        const bool general = k > 0.0 && k < 1.0 && fabs(k - 0.5) >= 1e-4 && z > 0.0 &&
+                             fabs(z - k) >= 1e-4 * (z + k) && fabs(z - k) >= 1e-6 && fabs(k + z - 1.0) >= 1e-4;
+        return general ? ma_general(z, k, I.u1, I.u2, kind == 1) : ma_quad_z(z, k, I.u1, I.u2);
+    }
+    static __device__ __forceinline__ double finish(const Pv&, double acc, int ns, const Item&) { return acc / ns; }
+    static __device__ __forceinline__ void stage(const MaArgs&, const Pv&, int, unsigned char*) {}
+};
 
 }  // namespace rr
 
@@ -247,15 +322,11 @@ int ma_evaluate(const rr_lcdata* lc, const rr_params* pv, const double* ldc, voi
     int rc = check_launch("ma_orbit_kernel");
     if (rc) return rc;
     MaArgs f;
-    f.times = lc->times; f.lcids = lc->lcids; f.pbids = lc->pbids; f.epids = lc->epids;
-    f.nsamples = lc->nsamples; f.exptimes = lc->exptimes;
-    f.k = pv->k; f.t0 = pv->t0; f.p = pv->p; f.a = pv->a; f.ldc = ldc; f.rec = rec; f.flux = flux;
-    f.npv = npv; f.npt = npt; f.nlc = nlc; f.npb = npb; f.kcols = pv->kcols; f.t0cols = pv->t0cols;
-    f.ntiles = (npt + kMaThreads - 1) / kMaThreads;
-    const long long nb = (long long)f.ntiles * npv;
-    if (nb > 0x7fffffffLL) return set_error(RR_ERANGE, "ma_evaluate: grid too large");
-    hipLaunchKernelGGL(ma_flux_kernel, dim3((unsigned)nb), dim3(kMaThreads), 0, s, f);
-    return check_launch("ma_flux_kernel");
+    f.d = wf_data(lc, true);
+    f.pbids = lc->pbids; f.epids = lc->epids; f.exptimes = lc->exptimes;
+    f.k = pv->k; f.t0 = pv->t0; f.ldc = ldc; f.rec = rec; f.flux = flux;
+    f.npv = npv; f.npb = npb; f.kcols = pv->kcols; f.t0cols = pv->t0cols;
+    return wf_launch<MaModel>("ma_evaluate", f, npv, 0, s);
 }
 
 }  // extern "C"

@@ -23,6 +23,31 @@ __device__ __forceinline__ double d_sqrt(double x) { return sqrt(x); }
 // arguments here are squared distances and kite products, never denormal.
 __device__ __forceinline__ float d_sqrt(float x) { return __builtin_amdgcn_sqrtf(x); }
 
+// FP64 reciprocal, quotient and square root of ordinary magnitudes (no denormal or
+// overflow rescaling): the hardware's seed refined by Newton steps, to an ulp or so.
+// The compiler's forms add the scaling and fix-up steps that only extreme exponents
+// need, twice the instructions.
+__device__ __forceinline__ double f64_rcp(double x) {
+    double r = __builtin_amdgcn_rcp(x);
+    r = fma(fma(-x, r, 1.0), r, r);
+    return fma(fma(-x, r, 1.0), r, r);
+}
+__device__ __forceinline__ double f64_div(double a, double b) {
+    const double r = f64_rcp(b), q = a * r;
+    return fma(fma(-b, q, a), r, q);
+}
+// 0 for x <= 0
+__device__ __forceinline__ double f64_sqrt(double x) {
+    const double y = __builtin_amdgcn_rsq(x);
+    double g = x * y, h = 0.5 * y;
+    const double e = fma(-h, g, 0.5);
+    g = fma(g, e, g);
+    h = fma(h, e, h);
+    g = fma(fma(-g, g, x), h, g);
+    g = fma(fma(-g, g, x), h, g);
+    return x > 0.0 ? g : 0.0;
+}
+
 // atan2(y, x) for y >= 0 in FP32: octant reduction with one hardware reciprocal
 // and atan(t) = t P(t^2) on [0, 1], P of degree 7 fitted by Lawson's minimax
 // iteration (pytransit_amd/csrc/atan_poly.py).  Max error 1.4e-7 rad.

@@ -1,0 +1,73 @@
+"""The window kernel (window_flux.hpp) at the edges of its tiles, chunks and item
+arrays, for each model that runs on it, against the FP64 oracle.
+
+Every model is evaluated in FP64 with the oracle's formulas; the kernels differ from
+them in the order of a few roundings, so the bar is the suite's FP64 bar, 1e-9
+absolute on fluxes of order one.
+"""
+import numpy as np
+import pytest
+
+from pytransit_amd import QuadraticModel, workloads
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-9
+
+
+def layout(name, npt, rng):
+    """set_data arguments: times within a transit's reach, so tiles hold points inside
+    and outside the window."""
+    t = np.linspace(-0.17, 0.21, npt) if npt > 1 else np.array([0.004])
+    if name == 'one':
+        return dict(time=t, lcids=np.zeros(npt, int), pbids=np.array([0]), nsamples=np.array([5]),
+                    exptimes=np.array([0.02]), epids=np.array([0]))
+    if name == 'many samples':       # more samples than a chunk's item arrays hold
+        return dict(time=t, lcids=np.zeros(npt, int), pbids=np.array([0]), nsamples=np.array([1100]),
+                    exptimes=np.array([0.02]), epids=np.array([0]))
+    nlc = 4
+    lcids = (np.arange(npt) * nlc) // npt
+    lcids[:min(npt, nlc)] = np.minimum(lcids[:min(npt, nlc)], nlc - 1)
+    ns, ex = np.array([1, 10, 3, 7]), np.array([0.0, 0.02, 0.01, 0.015])
+    if name == 'uneven beyond':      # one light curve above the item arrays
+        ns = np.array([2, 1, 1030, 4])
+    if name == 'shuffled':           # light curves interleaved, times out of order
+        order = rng.permutation(npt)
+        t, lcids = t[order], lcids[rng.permutation(npt)]
+    lcids[:nlc] = np.arange(nlc) if name == 'shuffled' else lcids[:nlc]
+    return dict(time=t, lcids=lcids, pbids=np.array([0, 1, 0, 1]), nsamples=ns, exptimes=ex,
+                epids=np.array([0, 1, 1, 0]))
+
+
+CASES = [('one', 1, 3), ('one', 255, 3), ('one', 257, 3), ('one', 1500, 2), ('sorted', 600, 3), ('sorted', 1025, 2),
+         ('shuffled', 700, 3), ('many samples', 40, 2), ('uneven beyond', 90, 2),
+         ('one', 1027, 1030), ('sorted', 1100, 1030)]
+
+
+def population(npv, rng, pb):
+    wl = workloads.rr_small(npv=npv, npt=4, seed=int(rng.integers(1000)))
+    k = wl.k if pb == 1 else np.concatenate([wl.k, wl.k * 1.03], 1)
+    t0 = wl.t0 if pb == 1 else np.concatenate([wl.t0, wl.t0 + 0.01], 1)
+    return wl, k, t0
+
+
+def rows(npv):
+    return np.arange(npv) if npv < 20 else np.array([0, 1, npv // 2, npv - 2, npv - 1])
+
+
+@pytest.mark.parametrize('name,npt,npv', CASES)
+def test_mandel_agol(gpu, oracle, name, npt, npv):
+    rng = np.random.default_rng(npt + npv)
+    d = layout(name, npt, rng)
+    pb = int(d['pbids'].max()) + 1
+    wl, k, t0 = population(npv, rng, pb)
+    k[0], wl.i[0] = 0.5, 0.5 * np.pi       # the special radius ratio, a central transit
+    ldc = rng.uniform(0.1, 0.4, (npv, 2 * pb))
+    tm = QuadraticModel()
+    tm.set_data(**d)
+    f = np.atleast_2d(tm.evaluate(k, ldc, t0, wl.p, wl.a, wl.i)).reshape(npv, npt)
+    r = rows(npv)
+    ref = oracle.quadratic_model(d['time'], k[r], t0[r], wl.p[r], wl.a[r], wl.i[r], wl.e[r], wl.w[r], ldc[r],
+                                 d['lcids'], d['pbids'], d['epids'], d['nsamples'], d['exptimes'])
+    assert (ref < 1).any()
+    assert np.abs(f[r] - ref).max() <= TOL
