@@ -8,8 +8,15 @@
 // Kernels:
 //   ma_orbit_kernel   8 pv per 64-lane block: the Taylor orbit and contact window of
 //                     the RoadRunner path (taylor_z.py:23-102,298-328)
-//   ma_flux_kernel    one lane per (pv, time): epoch, window (contact times
-//                     +- 0.025 d), supersampling, analytic flux; flux [npv, npt]
+//   window_flux_kernel<MaModel>   epoch, window (contact times +- 0.025 d),
+//                     supersampling and analytic flux of a tile of times of one pv;
+//                     flux [npv, npt] (window_flux.hpp)
+//
+// 1000 pv x 10,007 t with 5 samples (80 MB written, 2 % of the points in transit): the
+// flux kernel takes 60 us against 430 us with one lane per (pv, time), the orbits 10 us.
+// The write alone is 12 us and the samples' FP64 arithmetic about as much again; the
+// rest is the latency of the workgroups that hold a window (about 10 us each, four
+// resident per CU).
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -20,120 +27,104 @@
 
 namespace rr {
 
-// Complete elliptic integral of the third kind by Bulirsch's algorithm (Bulirsch
-// 1965, Numer. Math. 7, 78-90, as used at ma_quadratic_nb.py:55-91): arguments
-// n and the modulus k; at most 1000 iterations, relative tolerance 1e-8.
-__device__ double ma_ellpicb(double n, double k) {
-    double kc = sqrt(1.0 - k * k);
-    double e = kc;
-    double p = sqrt(n + 1.0);
-    double m0 = 1.0, c = 1.0, d = 1.0 / p;
-    for (int it = 0; it < 1000; ++it) {
-        const double f = c;
-        c = d / p + c;
-        double g = e / p;
-        d = 2.0 * (f * g + d);
-        p = g + p;
-        g = m0;
-        m0 = kc + m0;
-        if (fabs(1.0 - kc / g) > 1e-8) {
-            kc = 2.0 * sqrt(e);
-            e = kc * m0;
-        } else {
-            return kHalfPi * (c * m0 + d) / (m0 * (m0 + p));
-        }
-    }
-    return 0.0;
-}
-
-// Complete elliptic integrals E(k) and K(k) by Hastings' polynomial approximations
-// (Hastings 1955, Approximations for Digital Computers; Abramowitz & Stegun
-// 17.3.34 and 17.3.36), the forms of ma_quadratic_nb.py:93-126.
-__device__ __forceinline__ double ma_ellec(double k) {
-    const double m1 = 1.0 - k * k;
-    const double e1 = 1.0 + m1 * (0.44325141463 + m1 * (0.0626060122 + m1 * (0.04757383546 + m1 * 0.01736506451)));
-    const double e2 = m1 * (0.2499836831 + m1 * (0.09200180037 + m1 * (0.04069697526 + m1 * 0.00526449639))) *
-                      log(1.0 / m1);
-    return e1 + e2;
-}
-
-__device__ __forceinline__ double ma_ellk(double k) {
-    const double m1 = 1.0 - k * k;
-    const double k1 = 1.38629436112 + m1 * (0.09666344259 + m1 * (0.03590092383 + m1 * (0.03742563713 + m1 * 0.01451196212)));
-    const double k2 = (0.5 + m1 * (0.12498593597 + m1 * (0.06880248576 + m1 * (0.03328355346 + m1 * 0.00441787012)))) *
-                      log(m1);
-    return k1 - k2;
-}
+// Hastings' coefficients of K (both polynomials in m1, the second with the logarithm)
+// and of E
+__constant__ const double kEllipticTable[19] = {
+    1.38629436112, 0.09666344259, 0.03590092383, 0.03742563713, 0.01451196212,
+    0.5, 0.12498593597, 0.06880248576, 0.03328355346, 0.00441787012,
+    1.0, 0.44325141463, 0.06260601220, 0.04757383546, 0.01736506451,
+    0.24998368310, 0.09200180037, 0.04069697526, 0.00526449639};
 
 // Flux of a star with quadratic limb darkening (u1, u2) occulted by a disk of
-// radius k at separation z; the case analysis of Mandel & Agol (2002) as in
+// radius k at separation z <= 1 + k; the case analysis of Mandel & Agol (2002) as in
 // ma_quadratic_nb.py:277-389 (uniform part le, linear part ld, quadratic part ed).
-__device__ double ma_quad_z(double z, double k, double u1, double u2) {
+// `inside` says z < 1 - k.
+//
+// The cases are written with the quantities they share, since a wave pays for every
+// case it holds.  With x1 = (k-z)^2, x2 = (k+z)^2 and D = 1 - x1 (inside) or 4 k z
+// (limb), the squared complementary modulus is |1 - x2| / D in both, the prefactor
+// 2 / (9 pi sqrt D), and the start value sqrt(n + 1) of Bulirsch's algorithm
+// (k+z) / |k-z| inside and 1 / |k-z| on the limb: neither the modulus nor n is formed.
+// K and E are Hastings' polynomials (Hastings 1955; Abramowitz & Stegun 17.3.34 and
+// 17.3.36, the forms of ma_quadratic_nb.py:93-126) on one logarithm; Pi is Bulirsch's
+// iteration (Bulirsch 1965, Numer. Math. 7, 78-90; ma_quadratic_nb.py:55-91, relative
+// tolerance 1e-8, at most 1000 steps), a reciprocal and a square root a step.
+__device__ __forceinline__ double ma_quad_z(double z, double k, double u1, double u2, bool inside) {
     const double inv_pi = 1.0 / kPi;
-    if (fabs(k - 0.5) < 1.0e-4) k = 0.5;
-    const double k2 = k * k;
-    const double omega = 1.0 - u1 / 3.0 - u2 / 6.0;
-    if (fabs(z - k) < 1e-6) z += 1e-6;
-    if (z > 1.0 + k || signbit(z)) return 1.0;
-    if (k >= 1.0 && z <= k - 1.0) return 0.0;
-    const double z2 = z * z;
-    const double x1 = (k - z) * (k - z);
-    const double x2 = (k + z) * (k + z);
-    const double x3 = k * k - z * z;
-    double kap0 = 0.0, kap1 = 0.0, le = 0.0;
-    if (z <= 1.0 - k) {
-        le = k2;
-    } else if (fabs(1.0 - k) <= z && z <= 1.0 + k) {
-        kap1 = acos(fmin((1.0 - k2 + z2) / (2.0 * z), 1.0));
-        kap0 = acos(fmin((k2 + z2 - 1.0) / (2.0 * k * z), 1.0));
-        le = k2 * kap0 + kap1;
-        le = (le - 0.5 * sqrt(fmax(4.0 * z2 - (1.0 + z2 - k2) * (1.0 + z2 - k2), 0.0))) * inv_pi;
+    if (fabs(k - 0.5) < 1.0e-4) {
+        k = 0.5;
+        inside = z < 0.5;
     }
-    const bool edge_at_origin = fabs(z - k) < 1.e-4 * (z + k);
-    const bool full_transit = k <= 1.0 && z < (1.0 - k);
-    double ld, ed;
-    if (edge_at_origin) {
-        if (k == 0.5) {
-            ld = 1.0 / 3.0 - 4.0 * inv_pi / 9.0;
-            ed = 3.0 / 32.0;
-        } else if (z > 0.5) {
-            const double q = 0.5 / k;
-            const double kk = ma_ellk(q), ek = ma_ellec(q);
-            ld = 1.0 / 3.0 + 16.0 * k / 9.0 * inv_pi * (2.0 * k2 - 1.0) * ek -
-                 (32.0 * k2 * k2 - 20.0 * k2 + 3.0) / 9.0 * inv_pi / k * kk;
-            ed = 1.0 / 2.0 * inv_pi *
-                 (kap1 + k2 * (k2 + 2.0 * z2) * kap0 - (1.0 + 5.0 * k2 + z2) / 4.0 * sqrt((1.0 - x1) * (x2 - 1.0)));
-        } else {
-            const double q = 2.0 * k;
-            const double kk = ma_ellk(q), ek = ma_ellec(q);
-            ld = 1.0 / 3.0 + 2.0 / 9.0 * inv_pi * (4.0 * (2.0 * k2 - 1.0) * ek + (1.0 - 4.0 * k2) * kk);
-            ed = k2 / 2.0 * (k2 + 2.0 * z2);
+    if (fabs(z - k) < 1e-6) {
+        z += 1e-6;
+        inside = inside && z < 1.0 - k;
+    }
+    if (z > 1.0 + k) return 1.0;
+    if (k >= 1.0 && z <= k - 1.0) return 0.0;
+    const double k2 = k * k, z2 = z * z;
+    const double dm = k - z, sp = k + z;
+    const double x1 = dm * dm, x2 = sp * sp, x3 = dm * sp;
+    const bool edge = fabs(dm) < 1.e-4 * sp;                 // the planet's edge at the disk's centre
+    const double D = inside ? 1.0 - x1 : 4.0 * k * z;
+    const double rD = f64_rcp(D);
+    const double qe = z > 0.5 ? 0.5 / k : 2.0 * k;           // the modulus of the edge case
+    const double m1 = edge ? 1.0 - qe * qe : fabs(1.0 - x2) * rD;
+    const double lm = f64_log(m1);
+    const ConstTable ct = const_table(kEllipticTable);
+    const double kk = table_poly<5>(ct, m1) - table_poly<5>(ct + 5, m1) * lm;
+    const double ek = table_poly<5>(ct + 10, m1) - m1 * table_poly<4>(ct + 15, m1) * lm;
+    double ld;
+    if (!edge) {
+        const double ratio = f64_div(sp, dm);
+        double kc = f64_sqrt(m1), p = inside ? fabs(ratio) : f64_rcp(fabs(dm));
+        double e = kc, m0 = 1.0, c = 1.0, d = inside ? f64_rcp(p) : fabs(dm), rp = d, pk = 0.0;
+        for (int it = 0; it < 1000; ++it) {
+            const double f = c;
+            c = fma(d, rp, c);
+            const double g = e * rp;
+            d = 2.0 * fma(f, g, d);
+            p = g + p;
+            const double mo = m0;
+            m0 = kc + m0;
+            if (!(fabs(mo - kc) > 1e-8 * mo)) {
+                pk = kHalfPi * f64_div(fma(c, m0, d), m0 * (m0 + p));
+                break;
+            }
+            kc = 2.0 * f64_sqrt(e);
+            e = kc * m0;
+            rp = f64_rcp(p);
         }
-    } else if (full_transit) {
-        const double q = sqrt((x2 - x1) / (1.0 - x1));
-        const double kk = ma_ellk(q), ek = ma_ellec(q);
-        const double n = x2 / x1 - 1.0;
-        const double pk = ma_ellpicb(n, q);
-        ld = 2.0 / 9.0 * inv_pi / sqrt(1.0 - x1) *
-             ((1.0 - 5.0 * z2 + k2 + x3 * x3) * kk + (1.0 - x1) * (z2 + 7.0 * k2 - 4.0) * ek - 3.0 * x3 / x1 * pk);
-        if (z < k) ld = ld + 2.0 / 3.0;
-        if (fabs(k + z - 1.0) < 1.e-4)
+        const double A = inside ? 1.0 - 5.0 * z2 + k2 + x3 * x3 : (1.0 - x2) * (2.0 * x2 + x1 - 3.0) - 3.0 * x3 * (x2 - 2.0);
+        ld = 2.0 / 9.0 * inv_pi * f64_sqrt(rD) * (A * kk + (inside ? 1.0 - x1 : D) * (z2 + 7.0 * k2 - 4.0) * ek - 3.0 * ratio * pk);
+        if (z < k) ld += 2.0 / 3.0;
+        if (inside && fabs(k + z - 1.0) < 1.e-4)
             ld = 2.0 / 3.0 * inv_pi * acos(1.0 - 2.0 * k) -
                  4.0 / 9.0 * inv_pi * sqrt(k * (1.0 - k)) * (3.0 + 2.0 * k - 8.0 * k2);
-        ed = k2 / 2.0 * (k2 + 2.0 * z2);
+    } else if (k == 0.5) {
+        ld = 1.0 / 3.0 - 4.0 * inv_pi / 9.0;
+    } else if (z > 0.5) {
+        ld = 1.0 / 3.0 + 16.0 * k / 9.0 * inv_pi * (2.0 * k2 - 1.0) * ek -
+             (32.0 * k2 * k2 - 20.0 * k2 + 3.0) / 9.0 * inv_pi / k * kk;
     } else {
-        const double q = sqrt((1.0 - (k - z) * (k - z)) / 4.0 / z / k);
-        const double kk = ma_ellk(q), ek = ma_ellec(q);
-        const double n = 1.0 / x1 - 1.0;
-        const double pk = ma_ellpicb(n, q);
-        ld = 1.0 / 9.0 * inv_pi / sqrt(k * z) *
-             (((1.0 - x2) * (2.0 * x2 + x1 - 3.0) - 3.0 * x3 * (x2 - 2.0)) * kk + 4.0 * k * z * (z2 + 7.0 * k2 - 4.0) * ek -
-              3.0 * x3 / x1 * pk);
-        if (z < k) ld = ld + 2.0 / 3.0;
-        ed = 1.0 / 2.0 * inv_pi *
-             (kap1 + k2 * (k2 + 2.0 * z2) * kap0 - (1.0 + 5.0 * k2 + z2) / 4.0 * sqrt((1.0 - x1) * (x2 - 1.0)));
+        ld = 1.0 / 3.0 + 2.0 / 9.0 * inv_pi * (4.0 * (2.0 * k2 - 1.0) * ek + (1.0 - 4.0 * k2) * kk);
     }
-    return 1.0 - ((1.0 - u1 - 2.0 * u2) * le + (u1 + 2.0 * u2) * ld + u2 * ed) / omega;
+    double le, ed = 0.5 * k2 * (k2 + 2.0 * z2);
+    if (z <= 1.0 - k) {
+        le = k2;
+        // first or last contact of the inner limb itself: the limb case's ed with no lune
+        if (!inside && !(edge && !(z > 0.5))) ed = 0.0 - 0.125 * inv_pi * (1.0 + 5.0 * k2 + z2) * sqrt((1.0 - x1) * (x2 - 1.0));
+    } else {
+        // cos kappa1 = (1 - k^2 + z^2) / 2z and cos kappa0 = (k^2 + z^2 - 1) / 2kz, whose
+        // sines are the lune term over 2z and 2kz: angles without the quotients
+        const double lune = f64_sqrt(fmax((1.0 - x1) * (x2 - 1.0), 0.0));
+        const double kap1 = f64_atan2_ypos(lune, 1.0 - k2 + z2);
+        const double kap0 = f64_atan2_ypos(lune, k2 + z2 - 1.0);
+        le = (k2 * kap0 + kap1 - 0.5 * lune) * inv_pi;
+        if (!(edge && !(z > 0.5)))
+            ed = 0.5 * inv_pi * (kap1 + k2 * (k2 + 2.0 * z2) * kap0 - 0.25 * (1.0 + 5.0 * k2 + z2) * lune);
+    }
+    if (edge && k == 0.5) ed = 3.0 / 32.0;
+    return 1.0 - f64_div((1.0 - u1 - 2.0 * u2) * le + (u1 + 2.0 * u2) * ld + u2 * ed, 1.0 - u1 / 3.0 - u2 / 6.0);
 }
 
 struct MaArgs {
@@ -169,74 +160,13 @@ __global__ void __launch_bounds__(64) ma_orbit_kernel(int npv, const double* P, 
     }
 }
 
-// Flux at separation z of a planet with 0 < k < 1 inside the disk (z < 1 - k) or
-// across its limb, away from the special separations: ma_quad_z's two general cases
-// written with the quantities they share.  With x1 = (k-z)^2 and x2 = (k+z)^2 and
-// D = 1 - x1 (inside) or 4 k z (limb), the squared complementary modulus is
-// |1 - x2| / D in both, the prefactor 2 / (9 pi sqrt D), and Bulirsch's start value
-// sqrt(n + 1) is (k+z) / |k-z| inside and 1 / |k-z| on the limb, so that the modulus,
-// its square root and the square root of n + 1 are not formed, and both cases run the
-// same iteration.  Iterations take one reciprocal and one square root each.
-__device__ __forceinline__ double ma_general(double z, double k, double u1, double u2, bool inside) {
-    const double inv_pi = 1.0 / kPi;
-    const double k2 = k * k, z2 = z * z;
-    const double dm = k - z, sp = k + z;
-    const double x1 = dm * dm, x2 = sp * sp, x3 = dm * sp;
-    const double D = inside ? 1.0 - x1 : 4.0 * k * z;
-    const double rD = f64_rcp(D);
-    const double m1 = fabs(1.0 - x2) * rD;
-    const double ratio = f64_div(sp, dm);                    // (k + z) / (k - z)
-    const double kc0 = f64_sqrt(m1);
-    // K and E by the polynomials of ma_ellk and ma_ellec, one logarithm for both
-    const double lm = log(m1);
-    const double kk = (1.38629436112 + m1 * (0.09666344259 + m1 * (0.03590092383 + m1 * (0.03742563713 + m1 * 0.01451196212)))) -
-                      (0.5 + m1 * (0.12498593597 + m1 * (0.06880248576 + m1 * (0.03328355346 + m1 * 0.00441787012)))) * lm;
-    const double ek = (1.0 + m1 * (0.44325141463 + m1 * (0.06260601220 + m1 * (0.04757383546 + m1 * 0.01736506451)))) -
-                      m1 * (0.24998368310 + m1 * (0.09200180037 + m1 * (0.04069697526 + m1 * 0.00526449639))) * lm;
-    // Pi (ma_ellpicb)
-    double p = inside ? fabs(ratio) : f64_rcp(fabs(dm));
-    double kc = kc0, e = kc0, m0 = 1.0, c = 1.0, dd = inside ? f64_rcp(p) : fabs(dm), pk = 0.0;
-    for (int it = 0; it < 1000; ++it) {
-        const double rp = it == 0 ? dd : f64_rcp(p);
-        const double fo = c;
-        c = fma(dd, rp, c);
-        const double g = e * rp;
-        dd = 2.0 * fma(fo, g, dd);
-        p = g + p;
-        const double mo = m0;
-        m0 = kc + m0;
-        if (fabs(mo - kc) > 1e-8 * mo) {
-            kc = 2.0 * f64_sqrt(e);
-            e = kc * m0;
-        } else {
-            pk = kHalfPi * f64_div(fma(c, m0, dd), m0 * (m0 + p));
-            break;
-        }
-    }
-    const double A = inside ? 1.0 - 5.0 * z2 + k2 + x3 * x3 : (1.0 - x2) * (2.0 * x2 + x1 - 3.0) - 3.0 * x3 * (x2 - 2.0);
-    const double B = (inside ? 1.0 - x1 : D) * (z2 + 7.0 * k2 - 4.0);
-    double ld = 2.0 / 9.0 * inv_pi * f64_sqrt(rD) * (A * kk + B * ek - 3.0 * ratio * pk);
-    if (z < k) ld += 2.0 / 3.0;
-    double le, ed;
-    if (inside) {
-        le = k2;
-        ed = 0.5 * k2 * (k2 + 2.0 * z2);
-    } else {
-        const double kap1 = acos(fmin(f64_div(1.0 - k2 + z2, 2.0 * z), 1.0));
-        const double kap0 = acos(fmin(f64_div(k2 + z2 - 1.0, 2.0 * k * z), 1.0));
-        const double lune = f64_sqrt((1.0 - x1) * (x2 - 1.0));
-        le = (k2 * kap0 + kap1 - 0.5 * lune) * inv_pi;
-        ed = 0.5 * inv_pi * (kap1 + k2 * (k2 + 2.0 * z2) * kap0 - 0.25 * (1.0 + 5.0 * k2 + z2) * lune);
-    }
-    return 1.0 - f64_div((1.0 - u1 - 2.0 * u2) * le + (u1 + 2.0 * u2) * ld + u2 * ed, 1.0 - u1 / 3.0 - u2 / 6.0);
-}
-
 // ma_quadratic_nb.py:557-594 on the window kernel.
 struct MaModel {
     using Real = double;
     using Args = MaArgs;
-    static constexpr int kKinds = 2;    // 1 inside the disk (and the special cases), 2 on the limb
+    static constexpr int kKinds = 2;    // 1 inside the disk, 2 on the limb
     static constexpr int kGroup = 1;
+    static constexpr int kBlocks = 4;   // workgroups per CU: 128 registers (3: 87, 4: 80, 5 with spills: 84 us)
     struct Pv {
         double c[10], lo, hi, p, inv_p;
         bool good;
@@ -276,15 +206,9 @@ struct MaModel {
         if (z > 1.0 + I.k) return 0;
         return z < 1.0 - I.k ? 1 : 2;
     }
-    template <int G>
     static __device__ __forceinline__ double heavy(const MaArgs&, const Pv&, const Item& I, double, double z, int kind,
                                                    int, unsigned char*) {
-        const double k = I.k;
-        // a planet as large as the star, k = 0.5, the disk's centre or limb grazed by the
-        // planet's centre or edge, and anything not finite: the case analysis in full
-        const bool general = k > 0.0 && k < 1.0 && fabs(k - 0.5) >= 1e-4 && z > 0.0 &&
-                             fabs(z - k) >= 1e-4 * (z + k) && fabs(z - k) >= 1e-6 && fabs(k + z - 1.0) >= 1e-4;
-        return general ? ma_general(z, k, I.u1, I.u2, kind == 1) : ma_quad_z(z, k, I.u1, I.u2);
+        return ma_quad_z(z, I.k, I.u1, I.u2, kind == 1);
     }
     static __device__ __forceinline__ double finish(const Pv&, double acc, int ns, const Item&) { return acc / ns; }
     static __device__ __forceinline__ void stage(const MaArgs&, const Pv&, int, unsigned char*) {}

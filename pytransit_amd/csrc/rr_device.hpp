@@ -33,10 +33,11 @@ __device__ __forceinline__ double f64_rcp(double x) {
     return fma(fma(-x, r, 1.0), r, r);
 }
 __device__ __forceinline__ double f64_div(double a, double b) {
-    const double r = f64_rcp(b), q = a * r;
+    double r = __builtin_amdgcn_rcp(b);
+    r = fma(fma(-b, r, 1.0), r, r);
+    const double q = a * r;
     return fma(fma(-b, q, a), r, q);
 }
-// 0 for x <= 0
 __device__ __forceinline__ double f64_sqrt(double x) {
     const double y = __builtin_amdgcn_rsq(x);
     double g = x * y, h = 0.5 * y;
@@ -44,8 +45,67 @@ __device__ __forceinline__ double f64_sqrt(double x) {
     g = fma(g, e, g);
     h = fma(h, e, h);
     g = fma(fma(-g, g, x), h, g);
-    g = fma(fma(-g, g, x), h, g);
-    return x > 0.0 ? g : 0.0;
+    return x == 0.0 ? x : g;
+}
+
+// Coefficient tables in constant memory, read inside loops through a pointer the
+// compiler cannot follow.  Written as literals, a loop's 64-bit constants are hoisted
+// out of it, two registers each, and a kernel with three such polynomials held 185
+// vector registers (2 waves per SIMD) for them; scalar loads from a hot cache line
+// leave it at half of that.
+typedef const double __attribute__((address_space(4)))* ConstTable;
+__device__ __forceinline__ ConstTable const_table(const double* t) {
+    ConstTable p = (ConstTable)t;
+    asm volatile("" : "+s"(p));
+    return p;
+}
+__constant__ const double kLogTable[8] = {
+    0.66666666666667606655, 0.39999999999325053235, 0.285714287554372115, 0.22222197590380998733,
+    0.18183604510887957373, 0.15313202419441696023, 0.14803194289933532812, 0.69314718055994530942};
+__constant__ const double kAtanTable[12] = {
+    -0.33333333333333120541, 0.19999999999940004658, -0.14285714279170125263, 0.11111110741399687907,
+    -0.090908967204580554133, 0.076920439540218640828, -0.066629381856421199259, 0.058467923393252907438,
+    -0.050347684883633600506, 0.037957984254848413375, -0.017798614429732888959, 0.0};
+// sum_j t[j] x^j over N coefficients
+template <int N>
+__device__ __forceinline__ double table_poly(ConstTable t, double x) {
+    double q = t[N - 1];
+#pragma unroll
+    for (int j = N - 2; j >= 0; --j) q = fma(q, x, t[j]);
+    return q;
+}
+
+// log(x) in FP64: x = m 2^e with m in [sqrt(1/2), sqrt 2), log m = 2 atanh(s) with
+// s = (m - 1) / (m + 1), atanh(s) / s an interpolating polynomial in s^2 at Chebyshev
+// nodes (relative error 1.5e-18).
+__device__ __forceinline__ double f64_log(double x) {
+    double m = __builtin_amdgcn_frexp_mant(x);
+    int e = __builtin_amdgcn_frexp_exp(x);
+    const bool low = m < 0.70710678118654752;
+    m = low ? m + m : m;
+    e -= low ? 1 : 0;
+    const double s = f64_div(m - 1.0, m + 1.0), u = s * s;
+    const ConstTable c = const_table(kLogTable);
+    const double q = table_poly<7>(c, u);
+    const double r = fma((double)e, c[7], fma(s * u, q, s + s));
+    return x > 0.0 ? r : (x == 0.0 ? -INFINITY : (double)NAN);
+}
+
+// atan2(y, x) in FP64 for y >= 0, not both 0: the quotient of the smaller by the larger
+// side, taken about tan(pi/4) above tan(pi/8), then atan(t) / t on |t| <= tan(pi/8) as
+// an interpolating polynomial in t^2 at Chebyshev nodes (relative error 1.4e-18).  One
+// division; libm's form handles signs, zeros and infinities that the kite never gives.
+__device__ __forceinline__ double f64_atan2_ypos(double y, double x) {
+    const double ax = fabs(x);
+    const bool steep = y > ax;
+    const double mx = steep ? y : ax, mn = steep ? ax : y;
+    const bool big = mn > 0.41421356237309504880 * mx;
+    const double t = f64_div(big ? mn - mx : mn, big ? mn + mx : mx), s = t * t;
+    const double q = table_poly<11>(const_table(kAtanTable), s);
+    double r = fma(t * s, q, t);
+    r = big ? r + 0.25 * kPi : r;
+    r = steep ? kHalfPi - r : r;
+    return x < 0.0 ? kPi - r : r;
 }
 
 // atan2(y, x) for y >= 0 in FP32: octant reduction with one hardware reciprocal

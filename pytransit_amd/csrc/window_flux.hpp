@@ -1,20 +1,24 @@
 // Light-curve kernel shared by the models whose flux is a constant outside a window
 // around the conjunction and an average over exposure samples inside it.
 //
-// One workgroup of 256 lanes takes a tile of 256 * P consecutive times of one pv.
-//   1. A tile of one sorted light curve whose first and last times lie on the same
-//      side of the window is filled with the constant (16-byte stores).
-//   2. Otherwise every lane classifies P times; the points in the window go to an
-//      LDS queue with their phase, the others are stored as the constant.
-//   3. The queue is worked through in chunks of up to 256 points and kWfCap (point,
+// One workgroup of 256 lanes takes up to kWfMaxSub sub-tiles of 256 * P consecutive
+// times of one pv.
+//   1. A sub-tile of one sorted light curve whose first and last times lie on the same
+//      side of the window is outside it.  In the others every lane classifies P times;
+//      the points in the window go to an LDS queue, the rest is stored as the constant.
+//   2. The queue is worked through in chunks of up to 256 points and kWfCap (point,
 //      sample) items, one item a lane: a first pass settles the cheap samples (planet
 //      off the disk, wholly inside it) and lists the others, which a second pass
 //      evaluates on full waves, M::kGroup lanes to a sample.
-//   4. A lane sums the samples of a point in order and stores the point.
+//   3. A lane sums the samples of a point in order and stores the point.
+//   4. The sub-tiles outside are filled with the constant (16-byte stores), last: loads
+//      after them would wait for them.
 // One lane per (pv, time), the form this replaces, ran the samples of a point in
 // series, paid every branch of the sample in any wave that held a window point, and
 // left the rest of the chip waiting for those waves: only 2-10 % of the times of a
-// survey light curve are in a window.
+// survey light curve are in a window.  A workgroup's entry (arguments, record, epoch,
+// boundary times: four dependent loads) is 2-3 us however few points it has, so it
+// takes several sub-tiles when that leaves enough workgroups.
 //
 // A model M gives
 //   Args                      kernel arguments, with a WfData member `d`
@@ -27,8 +31,8 @@
 //   classify(f, P, I, t, v)   the sample at time t from conjunction: 0 when v is its
 //                             value, 1 or 2 when a heavy evaluation has to follow,
 //                             with v the separation
-//   heavy<G>(f, P, I, t, z, kind, sub, sh)   that evaluation by G lanes, this one the
-//                             sub-th; every lane of the group returns the value
+//   heavy(f, P, I, t, z, kind, sub, sh)   that evaluation by kGroup lanes, this one the
+//                             sub-th; lane 0 of the group returns the value
 //   stage(f, P, pv, sh), shared_bytes(f)     block-wide tables in LDS
 #pragma once
 
@@ -41,7 +45,8 @@ struct WfData {
     const double* times;
     const int32_t* lcids;
     const int32_t* nsamples;
-    int npt, nlc, ntiles;
+    int npt, nlc;
+    int ntiles, nsub;  // workgroups per pv, sub-tiles of each
     int sorted;       // contiguous light curves, each sorted in time
     int one_window;   // with `sorted`: times sorted throughout, one window for all
     int uniform_ns;   // the common nsamples, or 0
@@ -82,41 +87,40 @@ __device__ __forceinline__ void block_fill(T* base, int n, T v) {
     for (int i = head + nv * kVec + tid; i < n; i += kWfThreads) base[i] = v;
 }
 
-// Dynamic LDS of a launch: the queue, the chunk's item values, lists and contexts.
+// Dynamic LDS of a launch: the queue, the chunk's phases, item values, lists and contexts.
+constexpr int kWfMaxSub = 8;
 template <class M>
-static inline size_t wf_lds_bytes(int P, int nlc, int uniform_ns, size_t shared) {
-    size_t b = (size_t)kWfThreads * P * (sizeof(double) + sizeof(uint16_t));
+static inline size_t wf_lds_bytes(int queue, bool multi, size_t shared) {
+    size_t b = (size_t)kWfThreads * sizeof(double) + (size_t)queue * sizeof(uint16_t);
     b += (size_t)kWfCap * (sizeof(typename M::Real) + sizeof(uint16_t));
-    if (nlc > 1) b += (size_t)kWfThreads * sizeof(typename M::Item);
-    if (uniform_ns == 0) b += (size_t)(kWfCap + kWfThreads) * sizeof(uint16_t);
+    if (multi) b += (size_t)kWfThreads * sizeof(typename M::Item) + (size_t)(kWfCap + kWfThreads) * sizeof(uint16_t);
     return (b + 15) / 16 * 16 + shared;
 }
 
-template <class M, int P>
-__global__ void __launch_bounds__(kWfThreads) window_flux_kernel(typename M::Args f) {
+template <class M, int P, bool kMulti>
+__global__ void __launch_bounds__(kWfThreads, M::kBlocks) window_flux_kernel(typename M::Args f) {
     using Real = typename M::Real;
     using Item = typename M::Item;
-    constexpr int kTileN = kWfThreads * P;
+    constexpr int kSub = kWfThreads * P;
     constexpr int kWaves = kWfThreads / 64;
     extern __shared__ __align__(16) unsigned char lds[];
     __shared__ int s_n, s_na, s_nb, s_sum[kWaves];
     const WfData& d = f.d;
-    const bool multi = d.nlc > 1;
-    double* s_tc = (double*)lds;                                   // [kTileN] phases of the queue
-    Item* s_ctx = (Item*)(s_tc + kTileN);                          // [kWfThreads] of several light curves
-    Real* s_val = (Real*)(s_ctx + (multi ? kWfThreads : 0));       // [kWfCap] item values
-    uint16_t* s_it = (uint16_t*)(s_val + kWfCap);                  // [kTileN] time index in the tile
-    uint16_t* s_list = s_it + kTileN;                              // [kWfCap] heavy items, kind 1 from the front, 2 from the back
-    uint16_t* s_map = s_list + kWfCap;                             // [kWfCap] item -> point (uneven nsamples)
+    double* s_tc = (double*)lds;                                   // [kWfThreads] phases of the chunk's points
+    Item* s_ctx = (Item*)(s_tc + kWfThreads);                      // [kWfThreads] of several light curves
+    Real* s_val = (Real*)(s_ctx + (kMulti ? kWfThreads : 0));      // [kWfCap] item values
+    uint16_t* s_it = (uint16_t*)(s_val + kWfCap);                  // [kSub * d.nsub] time index of the queued points
+    uint16_t* s_list = s_it + kSub * d.nsub;                       // [kWfCap] heavy items, kind 1 from the front, 2 from the back
+    uint16_t* s_map = s_list + kWfCap;                             // [kWfCap] item -> point (several light curves)
     uint16_t* s_beg = s_map + kWfCap;                              // [kWfThreads] point -> first item
-    const uintptr_t end = (uintptr_t)(d.uniform_ns > 0 ? s_map : s_beg + kWfThreads);
+    const uintptr_t end = (uintptr_t)(kMulti ? s_beg + kWfThreads : s_map);
     unsigned char* shared = (unsigned char*)((end + 15) & ~(uintptr_t)15);
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int bid = xcd_remap(blockIdx.x, gridDim.x);
     const int pv = bid / d.ntiles;
-    const int base = (bid - pv * d.ntiles) * kTileN;
-    const int cnt = min(kTileN, d.npt - base);
+    const int base = (bid - pv * d.ntiles) * kSub * d.nsub;
+    const int cnt = min(kSub * d.nsub, d.npt - base);
     const typename M::Pv c = M::load(f, pv);
     Real* out = (Real*)f.flux + (size_t)pv * d.npt + base;
     if (!c.good) {
@@ -124,68 +128,80 @@ __global__ void __launch_bounds__(kWfThreads) window_flux_kernel(typename M::Arg
         return;
     }
     const Real fill = M::fill(c);
-    auto lc_of = [&](int it) { return multi ? min(max(d.lcids[base + it], 0), d.nlc - 1) : 0; };
+    auto lc_of = [&](int it) { return kMulti ? min(max(d.lcids[base + it], 0), d.nlc - 1) : 0; };
+    // ---- sub-tiles outside the window, one a lane (every wave alike) ------------------
+    unsigned out_mask = 0u;
+    const WfWindow w0 = M::window(f, c, pv, 0);
     if (d.sorted) {
-        const int la = lc_of(0), lb = lc_of(cnt - 1);
-        if (la == lb || d.one_window) {
-            const WfWindow w = M::window(f, c, pv, la);
-            double ea, eb;
-            const double ta = wf_phase(d.times[base], w.t0, c.p, c.inv_p, ea);
-            const double tb = wf_phase(d.times[base + cnt - 1], w.t0, c.p, c.inv_p, eb);
-            const bool outside = ea == eb ? (tb < w.lo || ta > w.hi) : (eb == ea + 1.0 && ta > w.hi && tb < w.lo);
-            if (outside) {
-                block_fill<Real>(out, cnt, fill);
-                return;
+        const int i0 = lane * kSub, i1 = min(i0 + kSub, cnt) - 1;
+        bool outside = false;
+        if (lane < d.nsub && i0 < cnt) {
+            const double tf = d.times[base + i0], tl = d.times[base + i1];
+            const int la = lc_of(i0);
+            if (!kMulti || d.one_window || la == lc_of(i1)) {
+                const WfWindow w = kMulti ? M::window(f, c, pv, la) : w0;
+                double ea, eb;
+                const double ta = wf_phase(tf, w.t0, c.p, c.inv_p, ea);
+                const double tb = wf_phase(tl, w.t0, c.p, c.inv_p, eb);
+                outside = ea == eb ? (tb < w.lo || ta > w.hi) : (eb == ea + 1.0 && ta > w.hi && tb < w.lo);
             }
         }
+        out_mask = (unsigned)__ballot(outside);
+    }
+    const int nsub = (cnt + kSub - 1) / kSub;
+    if (out_mask == (1u << nsub) - 1u) {
+        block_fill<Real>(out, cnt, fill);
+        return;
     }
     if (tid == 0) s_n = 0;
     M::stage(f, c, pv, shared);
     __syncthreads();
     // ---- the points in the window into the queue --------------------------------------
-    WfWindow w = M::window(f, c, pv, 0);
-    double tv[P];
+    for (int j0 = 0; j0 < nsub; ++j0) {
+        if ((out_mask >> j0) & 1u) continue;
+        double tv[P];
 #pragma unroll
-    for (int j = 0; j < P; ++j) {
-        const int it = j * kWfThreads + tid;
-        tv[j] = it < cnt ? d.times[base + it] : 0.0;
-    }
-#pragma unroll
-    for (int j = 0; j < P; ++j) {
-        const int it = j * kWfThreads + tid;
-        bool inw = false;
-        double tc = 0.0;
-        if (it < cnt) {
-            if (multi) w = M::window(f, c, pv, lc_of(it));
-            double ep;
-            tc = wf_phase(tv[j], w.t0, c.p, c.inv_p, ep);
-            inw = w.lo <= tc && tc <= w.hi;
-            if (!inw) out[it] = fill;
+        for (int j = 0; j < P; ++j) {
+            const int it = j0 * kSub + j * kWfThreads + tid;
+            tv[j] = it < cnt ? d.times[base + it] : 0.0;
         }
-        const unsigned long long mk = __ballot(inw);
-        if (mk) {
-            int at = 0;
-            if (lane == 0) at = atomicAdd(&s_n, __popcll(mk));
-            at = __shfl(at, 0, 64) + __popcll(mk & ((1ull << lane) - 1ull));
-            if (inw) {
-                s_tc[at] = tc;
-                s_it[at] = (uint16_t)it;
+#pragma unroll
+        for (int j = 0; j < P; ++j) {
+            const int it = j0 * kSub + j * kWfThreads + tid;
+            bool inw = false;
+            if (it < cnt) {
+                const WfWindow w = kMulti ? M::window(f, c, pv, lc_of(it)) : w0;
+                double ep;
+                const double tc = wf_phase(tv[j], w.t0, c.p, c.inv_p, ep);
+                inw = w.lo <= tc && tc <= w.hi;
+                if (!inw) out[it] = fill;
+            }
+            const unsigned long long mk = __ballot(inw);
+            if (mk) {
+                int at = 0;
+                if (lane == 0) at = atomicAdd(&s_n, __popcll(mk));
+                at = __shfl(at, 0, 64) + __popcll(mk & ((1ull << lane) - 1ull));
+                if (inw) s_it[at] = (uint16_t)it;
             }
         }
     }
     __syncthreads();
     const int n = s_n;
-    const int uns = d.uniform_ns;
+    // the common nsamples, or 0
+    const int uns = d.uniform_ns > 0 ? d.uniform_ns : (kMulti ? 0 : max(d.nsamples[0], 1));
     const float inv_uns = uns > 0 ? 1.0f / (float)uns : 0.0f;
     Item ctx0;
-    if (!multi) ctx0 = M::item(f, c, pv, 0);
+    if (!kMulti) ctx0 = M::item(f, c, pv, 0);
     // ---- chunks of points -------------------------------------------------------------
-    int c0 = 0;
+    // c0: first point of the chunk; s0: its first sample, above 0 only for a point with
+    // more samples than the item arrays hold, which is a chunk of its own in several passes
+    int c0 = 0, s0 = 0;
+    Real carry = Real(0);
     while (c0 < n) {
-        int cn, tot;
+        int cn, tot, ns1 = uns;
         if (uns > 0) {
-            cn = min(min(kWfThreads, kWfCap / uns), n - c0);
-            tot = cn * uns;
+            cn = min(max(1, min(kWfThreads, kWfCap / uns)), n - c0);
+            tot = min(kWfCap, cn * (uns - s0));
         } else {
             // points whose samples fit the item arrays, by a block-wide prefix sum
             const int mine = c0 + tid < n ? max(0, min(d.nsamples[lc_of(s_it[c0 + tid])], kWfCap + 1)) : 0;
@@ -206,21 +222,39 @@ __global__ void __launch_bounds__(kWfThreads) window_flux_kernel(typename M::Arg
             }
             if (tid == cn - 1) s_sum[0] = run;
             __syncthreads();
-            tot = cn > 0 ? s_sum[0] : 0;
+            tot = s_sum[0];
+            if (cn == 0) {
+                ns1 = d.nsamples[lc_of(s_it[c0])];
+                cn = 1;
+                tot = min(kWfCap, ns1 - s0);
+                for (int i = tid; i < tot; i += kWfThreads) s_map[i] = 0;
+                if (tid == 0) s_beg[0] = 0;
+            }
         }
-        if (cn == 0) break;                     // more samples a point than the arrays hold: below
         if (tid == 0) s_na = s_nb = 0;
-        if (multi && tid < cn) s_ctx[tid] = M::item(f, c, pv, lc_of(s_it[c0 + tid]));
+        if (tid < cn) {
+            const int it = s_it[c0 + tid];
+            WfWindow w = w0;
+            if (kMulti) {
+                const int ilc = lc_of(it);
+                w = M::window(f, c, pv, ilc);
+                s_ctx[tid] = M::item(f, c, pv, ilc);
+            }
+            double ep;
+            s_tc[tid] = wf_phase(d.times[base + it], w.t0, c.p, c.inv_p, ep);
+        }
         __syncthreads();
-        auto point_of = [&](int i) { return uns > 0 ? (int)(((float)i + 0.5f) * inv_uns) : (int)s_map[i]; };
+        auto point_of = [&](int i) {
+            return uns > 0 ? (uns > kWfCap ? 0 : (int)(((float)i + 0.5f) * inv_uns)) : (int)s_map[i];
+        };
         auto first_of = [&](int q) { return uns > 0 ? q * uns : (int)s_beg[q]; };
         for (int b = 0; b < tot; b += kWfThreads) {
             const int i = b + tid;
             int kind = 0;
             if (i < tot) {
                 const int q = point_of(i);
-                const Item I = multi ? s_ctx[q] : ctx0;
-                const double t = s_tc[c0 + q] + I.ext * ((i - first_of(q) + 0.5) * I.inv_ns - 0.5);
+                const Item I = kMulti ? s_ctx[q] : ctx0;
+                const double t = s_tc[q] + I.ext * ((s0 + i - first_of(q) + 0.5) * I.inv_ns - 0.5);
                 kind = M::classify(f, c, I, t, s_val[i]);
             }
 #pragma unroll
@@ -237,56 +271,60 @@ __global__ void __launch_bounds__(kWfThreads) window_flux_kernel(typename M::Arg
         __syncthreads();
         constexpr int G = M::kGroup;
         const int na = s_na, nh = na + s_nb;
+#pragma unroll 1
         for (int j = tid / G; j < nh; j += kWfThreads / G) {
             const int kind = j < na ? 1 : 2;
             const int i = s_list[j < na ? j : kWfCap - 1 - (j - na)];
             const int q = point_of(i);
-            const Item I = multi ? s_ctx[q] : ctx0;
-            const double t = s_tc[c0 + q] + I.ext * ((i - first_of(q) + 0.5) * I.inv_ns - 0.5);
-            const Real v = M::template heavy<G>(f, c, I, t, s_val[i], kind, tid % G, shared);
+            const Item I = kMulti ? s_ctx[q] : ctx0;
+            const double t = s_tc[q] + I.ext * ((s0 + i - first_of(q) + 0.5) * I.inv_ns - 0.5);
+            const Real v = M::heavy(f, c, I, t, s_val[i], kind, tid % G, shared);
             if (tid % G == 0) s_val[i] = v;
         }
         __syncthreads();
+        const bool partial = cn == 1 && tot < ns1 - s0;
         if (tid < cn) {
             const int it = s_it[c0 + tid];
-            const int i0 = first_of(tid), ns = uns > 0 ? uns : d.nsamples[lc_of(it)];
-            Real acc = Real(0);
-            for (int k = 0; k < ns; ++k) acc += s_val[i0 + k];
-            out[it] = M::finish(c, acc, ns, multi ? s_ctx[tid] : ctx0);
+            const int ns = uns > 0 ? uns : d.nsamples[lc_of(it)];
+            const int i0 = first_of(tid), i1 = min(i0 + ns - s0, tot);
+            Real acc = carry;
+            for (int k = i0; k < i1; ++k) acc += s_val[k];
+            carry = partial ? acc : Real(0);
+            if (!partial) out[it] = M::finish(c, acc, ns, kMulti ? s_ctx[tid] : ctx0);
         }
         __syncthreads();
-        c0 += cn;
+        s0 = partial ? s0 + tot : 0;
+        c0 += partial ? 0 : cn;
     }
-    // points with more samples than kWfCap: one lane a point
-    for (int j = c0 + tid; j < n; j += kWfThreads) {
-        const int ilc = lc_of(s_it[j]);
-        const Item I = M::item(f, c, pv, ilc);
-        const int ns = d.nsamples[ilc];
-        Real acc = Real(0);
-        for (int k = 0; k < ns; ++k) {
-            const double t = s_tc[j] + I.ext * ((k + 0.5) * I.inv_ns - 0.5);
-            Real v;
-            const int kind = M::classify(f, c, I, t, v);
-            acc += kind == 0 ? v : M::template heavy<1>(f, c, I, t, v, kind, 0, shared);
-        }
-        out[s_it[j]] = M::finish(c, acc, ns, I);
-    }
+    for (int j0 = 0; j0 < nsub; ++j0)
+        if ((out_mask >> j0) & 1u) block_fill<Real>(out + j0 * kSub, min(kSub, cnt - j0 * kSub), fill);
 }
 
-// Launch over npv x npt.  Four times a lane; one time a lane (tiles of 256) when that
-// would leave CUs without a workgroup.
+// Launch over npv x npt: four times a lane and as many sub-tiles a workgroup as leave
+// kWfBlocks workgroups (the Mandel-Agol model at 1000 pv x 10,007 t, nss 5: 115, 80, 76
+// and 92 us with 2000, 3000, 5000 and 10,000 workgroups; at 2000 x 20,000, nss 1: 119
+// and 160 us with 6000 and 20,000); one time a lane where single sub-tiles of four
+// leave CUs short of work.
+constexpr int kWfBlocks = 4096;
 template <class M>
 static inline int wf_launch(const char* who, typename M::Args& f, int npv, size_t shared, hipStream_t s) {
     const int npt = f.d.npt;
-    const long long tiles4 = (npt + 4 * kWfThreads - 1) / (4 * kWfThreads);
-    const int P = tiles4 * npv < 2048 ? 1 : 4;
-    const long long ntiles = P == 4 ? tiles4 : (npt + kWfThreads - 1) / kWfThreads;
+    const long long sub4 = ((long long)npt + 4 * kWfThreads - 1) / (4 * kWfThreads);
+    const int P = sub4 * npv < 2048 ? 1 : 4;
+    const long long nsubs = P == 4 ? sub4 : ((long long)npt + kWfThreads - 1) / kWfThreads;
+    int per = 1;
+    while (per < kWfMaxSub && (nsubs + 2 * per - 1) / (2 * per) * npv >= kWfBlocks) per *= 2;
+    const long long ntiles = (nsubs + per - 1) / per;
     if (ntiles * npv > 0x7fffffffLL) return set_error(RR_ERANGE, "%s: grid too large", who);
     f.d.ntiles = (int)ntiles;
-    const size_t lds = wf_lds_bytes<M>(P, f.d.nlc, f.d.uniform_ns, shared);
+    f.d.nsub = per;
+    const bool multi = f.d.nlc > 1;
+    const size_t lds = wf_lds_bytes<M>(kWfThreads * P * per, multi, shared);
     const dim3 grid((unsigned)(ntiles * npv)), block(kWfThreads);
-    if (P == 4) hipLaunchKernelGGL((window_flux_kernel<M, 4>), grid, block, lds, s, f);
-    else hipLaunchKernelGGL((window_flux_kernel<M, 1>), grid, block, lds, s, f);
+    if (multi && P == 4) hipLaunchKernelGGL((window_flux_kernel<M, 4, true>), grid, block, lds, s, f);
+    else if (multi) hipLaunchKernelGGL((window_flux_kernel<M, 1, true>), grid, block, lds, s, f);
+    else if (P == 4) hipLaunchKernelGGL((window_flux_kernel<M, 4, false>), grid, block, lds, s, f);
+    else hipLaunchKernelGGL((window_flux_kernel<M, 1, false>), grid, block, lds, s, f);
     return check_launch(who);
 }
 
@@ -299,7 +337,7 @@ static inline WfData wf_data(const rr_lcdata* lc, bool shared_epochs) {
     d.nsamples = lc->nsamples;
     d.npt = lc->npt;
     d.nlc = lc->nlc;
-    d.ntiles = 0;
+    d.ntiles = d.nsub = 1;
     d.sorted = (lc->sorted & RR_SORTED_RUNS) != 0;
     const int one = RR_SORTED_RUNS | RR_SORTED_TIMES | RR_ONE_WINDOW;
     d.one_window = shared_epochs && (lc->sorted & one) == one;

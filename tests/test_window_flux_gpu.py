@@ -41,7 +41,9 @@ def layout(name, npt, rng):
 
 CASES = [('one', 1, 3), ('one', 255, 3), ('one', 257, 3), ('one', 1500, 2), ('sorted', 600, 3), ('sorted', 1025, 2),
          ('shuffled', 700, 3), ('many samples', 40, 2), ('uneven beyond', 90, 2),
-         ('one', 1027, 1030), ('sorted', 1100, 1030)]
+         ('one', 1027, 1030), ('sorted', 1100, 1030),
+         # several sub-tiles a workgroup
+         ('one', 9001, 1030), ('sorted', 9001, 1030), ('shuffled', 9001, 1030)]
 
 
 def population(npv, rng, pb):
