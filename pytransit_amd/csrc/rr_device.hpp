@@ -188,6 +188,16 @@ __device__ __forceinline__ void ccia_kite3(T r1, T r2, T b, T& area, T& kap0, T&
     area = T(NAN); kap0 = T(NAN);
 }
 
+// Lens area of the unit disk and a disk of radius k at separation z, |1 - k| < z < 1 + k,
+// in FP64: the kite form above with the arctangent and square root of f64_*.
+__device__ __forceinline__ double lens_area_f64(double k, double z) {
+    const double hi = fmax(1.0, k), lo = fmin(1.0, k);
+    const double x = fmax(hi, z), c = fmin(lo, z), y = fmax(lo, fmin(hi, z));
+    const double sq = f64_sqrt((x + (y + c)) * (c - (x - y)) * (c + (x - y)) * (x + (y - c)));   // 2 akite
+    const double zz = z * z, kk = (k - 1.0) * (k + 1.0);
+    return f64_atan2_ypos(sq, zz - kk) + k * k * f64_atan2_ypos(sq, zz + kk) - 0.5 * sq;
+}
+
 template <typename T>
 __device__ __forceinline__ void ccia_kite(T r1, T r2, T b, T& area, T& kap0) {
     T akite;

@@ -8,7 +8,7 @@ absolute on fluxes of order one.
 import numpy as np
 import pytest
 
-from pytransit_amd import QuadraticModel, workloads
+from pytransit_amd import EclipseModel, QuadraticModel, workloads
 
 pytestmark = pytest.mark.gpu
 
@@ -73,3 +73,26 @@ def test_mandel_agol(gpu, oracle, name, npt, npv):
                                  d['lcids'], d['pbids'], d['epids'], d['nsamples'], d['exptimes'])
     assert (ref < 1).any()
     assert np.abs(f[r] - ref).max() <= TOL
+
+
+@pytest.mark.parametrize('name,npt,npv', CASES)
+def test_eclipse(gpu, name, npt, npv):
+    from oracle import ec_oracle as eo
+    rng = np.random.default_rng(npt + 2 * npv)
+    d = layout(name, npt, rng)
+    d['time'] = d['time'] + 1.01            # around p / 2
+    pb = int(d['pbids'].max()) + 1
+    wl, k, t0 = population(npv, rng, pb)
+    k = k[:, 0].copy()
+    k[0] = 0.4
+    p = rng.uniform(1.9, 2.1, npv)
+    rstar = rng.uniform(0.8, 1.2, npv)
+    em = EclipseModel()
+    em.set_data(**d)
+    f = np.atleast_2d(em.evaluate(k, t0, p, wl.a, wl.i, rstar=rstar)).reshape(npv, npt)
+    for j in rows(npv):
+        # the model takes passband indices where the kernel takes epoch indices
+        ref = eo.eclipse_model(d['time'], k[j:j + 1], t0[j:j + 1], p[j:j + 1], wl.a[j:j + 1], wl.i[j:j + 1],
+                               wl.e[j:j + 1], wl.w[j:j + 1], rstar[j], d['pbids'].size, d['lcids'], d['pbids'],
+                               d['nsamples'], d['exptimes'])
+        assert np.abs(f[j] - ref[0]).max() <= TOL
