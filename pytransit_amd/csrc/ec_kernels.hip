@@ -22,9 +22,9 @@
 //                     with two libm arctangents each
 //   es_flux_kernel    one lane per (pv, time): the mean lens area, fanned out over the
 //                     passbands of the spectroscopy model
-//   op_flux_kernel    one block per (pv, 256 times): the pv's ellipse scanlines in
-//                     LDS, then per lane the supersampled flux with the scanline
-//                     ellipse-disk area; the per-pv state comes from rr_setup
+//   window_flux_kernel<OblateFlux>   the oblate planet's flux: the pv's ellipse
+//                     scanlines in LDS, shared by the lanes that evaluate a sample; the
+//                     per-pv state comes from rr_setup
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -234,81 +234,114 @@ struct EclipseFlux {
 
 // ---- Oblate planet ---------------------------------------------------------------
 
-constexpr int kOpThreads = 256;
 constexpr int kOpMaxLines = 2048;
 
 struct OpArgs {
-    const double* times; const int32_t* lcids; const int32_t* pbids; const int32_t* epids;
-    const int32_t* nsamples; const double* exptimes;
+    WfData d;
+    const int32_t* pbids; const int32_t* epids; const double* exptimes;
     const double* k; const double* t0; const double* fl; const double* alpha;
     const PvRec* rec; const double* istar; const double* ldm;
     double* flux;
-    int npv, npt, nlc, npb, kcols, t0cols, ng, nlines, ntiles;
-    double dg;
+    int npb, kcols, t0cols, ng, nlines;
+    double dg, inv_dg;
 };
 
-// Area of the ellipse with rows (ys, xl, xr) about its centre (cx, cy) inside the
-// unit disk; ecintersection.py:137-207, the three branches by the centre's x.  The
-// rows are ordered and a row with no chord has xl = NaN.
-__device__ double op_ellipse_area(double cx, double cy, double z, double k, double fl, const double* ys,
-                                  const double* xl, const double* xr, int ny) {
-    if (z <= 1.0 - k) return kPi * k * (1.0 - fl) * k;
-    if (z >= 1.0 + k) return 0.0;
-    const double dy = ys[1] - ys[0];
-    double acc = 0.0;
-    if (cx < -k) {
-        for (int j = 0; j < ny; ++j) {
-            const double x0 = xl[j], x1 = xr[j];
-            if (isfinite(x0)) {
-                const double v = ys[j] + cy;
-                const double xs = -sqrt(1.0 - v * v) - cx;   // NaN off the disk: no branch taken
-                if (xs <= x0) acc += x1 - x0;
-                else if (xs <= x1) acc += x1 - xs;
-            }
-        }
-    } else if (cx > k) {
-        for (int j = 0; j < ny; ++j) {
-            const double x0 = xl[j], x1 = xr[j];
-            if (isfinite(x0)) {
-                const double v = ys[j] + cy;
-                const double xs = sqrt(1.0 - v * v) - cx;
-                if (xs >= x1) acc += x1 - x0;
-                else if (xs >= x0) acc += xs - x0;
-            }
-        }
-    } else {
-        for (int j = 0; j < ny; ++j) {
-            const double x0 = xl[j], x1 = xr[j];
-            if (isfinite(x0)) {
-                const double v = ys[j] + cy;
-                if (fabs(v) <= 1.0) {
-                    const double xs = sqrt(1.0 - v * v);
-                    const double a1 = -xs - cx, a2 = xs - cx;
-                    const double hi = fmin(a2, x1);
-                    if (a1 <= x0) acc += hi - x0;
-                    else if (a1 > x0) acc += hi - a1;
-                }
-            }
-        }
+// opmodel_full.py:95-131 on the window kernel.  The planet's ellipse is a table of
+// scanlines (create_ellipse, ecintersection.py:93-134, at k[:, 0]) in LDS; a sample
+// whose planet crosses the limb sums the part of every scanline on the stellar disk
+// (ecintersection.py:137-207, the three branches by the centre's x).  Eight lanes
+// share a sample's scanlines: with one lane a sample the 100 square roots in a row
+// ran on the few lanes of a wave that held one (400 pv x 10,000 t, 5 samples, 100
+// lines: 744 us a call, now 81; floor 5 us of writes and 2 us of FP64).
+struct OblateFlux {
+    using Real = double;
+    using Args = OpArgs;
+    static constexpr int kKinds = 1;
+    static constexpr int kGroup = 8;    // 400 pv x 10,000 t, nss 5: 8 lanes 81, 16 lanes 90, 32 lanes 109 us
+    static constexpr int kBlocks = 4;
+    struct Pv {
+        double c[10], bt1, bt4, p, inv_p, fl;
+        bool good;
+    };
+    struct Item {
+        double ext, inv_ns, k, inv_1pk, ist;
+        const double* row;
+    };
+    static __device__ __forceinline__ Pv load(const OpArgs& f, int pv) {
+        const PvRec& r = f.rec[pv];
+        Pv o;
+#pragma unroll
+        for (int j = 0; j < 10; ++j) o.c[j] = r.c[j];
+        o.bt1 = r.bt1;
+        o.bt4 = r.bt4;
+        o.p = r.p;
+        o.inv_p = r.inv_p;
+        o.fl = f.fl[pv];
+        o.good = r.good && r.ldok;
+        return o;
     }
-    return acc * dy;
-}
-
-__global__ void __launch_bounds__(kOpThreads) op_flux_kernel(OpArgs f) {
-    __shared__ double s_y[kOpMaxLines], s_xl[kOpMaxLines], s_xr[kOpMaxLines];
-    const int bid = xcd_remap(blockIdx.x, gridDim.x);
-    const int pv = bid / f.ntiles;
-    const int it = (bid - pv * f.ntiles) * kOpThreads + threadIdx.x;
-    const PvRec& r = f.rec[pv];
-    const bool ok = r.good && r.ldok;
-    // the pv's ellipse scanlines (create_ellipse, ecintersection.py:93-134) at k[:, 0]
-    if (ok) {
+    static __device__ __forceinline__ double fill(const Pv&) { return 1.0; }
+    static __device__ __forceinline__ double bad() { return NAN; }
+    static __device__ __forceinline__ WfWindow window(const OpArgs& f, const Pv& c, int pv, int ilc) {
+        const double margin = 0.0015 + f.exptimes[ilc];
+        return {f.t0[(size_t)pv * f.t0cols + min(max(f.epids[ilc], 0), f.t0cols - 1)], c.bt1 - margin, c.bt4 + margin};
+    }
+    static __device__ __forceinline__ Item item(const OpArgs& f, const Pv&, int pv, int ilc) {
+        const int ipb = min(max(f.pbids[ilc], 0), f.npb - 1);
+        const double k = f.k[(size_t)pv * f.kcols + (f.kcols == 1 ? 0 : ipb)];
+        const size_t j = (size_t)pv * f.npb + ipb;
+        return {f.exptimes[ilc], 1.0 / f.d.nsamples[ilc], k, 1.0 / (1.0 + k), f.istar[j], f.ldm + j * f.ng};
+    }
+    static __device__ __forceinline__ double centre(const double* c, double t) {
+        return (((c[4] * t + c[3]) * t + c[2]) * t + c[1]) * t + c[0];
+    }
+    static __device__ __forceinline__ double flux_of(const OpArgs& f, const Item& I, double z, double area) {
+        return (I.ist - interp_ld_r(z * I.inv_1pk, f.dg, f.inv_dg, I.row, f.ng) * area) / I.ist;
+    }
+    static __device__ __forceinline__ int classify(const OpArgs& f, const Pv& c, const Item& I, double t, double& v) {
+        const double z = taylor_z<double>(t, c.c);
+        v = z;
+        const bool in = z <= 1.0 - I.k;
+        if (!in && !(z >= 1.0 + I.k)) return 1;
+        v = flux_of(f, I, z, in ? kPi * I.k * (1.0 - c.fl) * I.k : 0.0);
+        return 0;
+    }
+    static __device__ __forceinline__ double heavy(const OpArgs& f, const Pv& c, const Item& I, double t, double z, int,
+                                                   int sub, unsigned char* sh) {
+        const double* ys = (const double*)sh;
+        const double* xl = ys + f.nlines;
+        const double* xr = xl + f.nlines;
+        const double cx = centre(c.c, t), cy = centre(c.c + 5, t), k = I.k;
+        const bool west = cx < -k, east = cx > k;
+        double acc = 0.0;
+        for (int j = sub; j < f.nlines; j += kGroup) {
+            const double x0 = xl[j], x1 = xr[j], v = ys[j] + cy;
+            const double h2 = 1.0 - v * v;
+            // a row without a chord or off the disk adds nothing
+            if (isfinite(x0) && h2 >= 0.0) {
+                const double half = f64_sqrt(h2);
+                const double left = east ? x0 : fmax(x0, -half - cx);
+                const double right = west ? x1 : fmin(x1, half - cx);
+                const double w = right - left;
+                acc += west || east ? fmax(w, 0.0) : w;
+            }
+        }
+#pragma unroll
+        for (int o = kGroup / 2; o > 0; o >>= 1) acc += __shfl_xor(acc, o, kGroup);
+        return flux_of(f, I, z, acc * (ys[1] - ys[0]));
+    }
+    static __device__ __forceinline__ double finish(const Pv&, double acc, int ns, const Item&) { return acc / ns; }
+    static size_t shared_bytes(int nlines) { return 3 * (size_t)nlines * sizeof(double); }
+    static __device__ __forceinline__ void stage(const OpArgs& f, const Pv& c, int pv, unsigned char* sh) {
+        double* ys = (double*)sh;
+        double* s_xl = ys + f.nlines;
+        double* s_xr = s_xl + f.nlines;
         const double k0 = f.k[(size_t)pv * f.kcols];
-        const double fl = f.fl[pv], al = f.alpha[pv];
+        const double al = f.alpha[pv];
         const double ca = cos(al), sa = sin(al);
-        const double b = 1.0 - fl, b2 = b * b, ca2 = ca * ca, sa2 = sa * sa;
+        const double b = 1.0 - c.fl, b2 = b * b, ca2 = ca * ca, sa2 = sa * sa;
         const double dy = 2.0 / (f.nlines + 1);
-        for (int j = threadIdx.x; j < f.nlines; j += kOpThreads) {
+        for (int j = threadIdx.x; j < f.nlines; j += kWfThreads) {
             const double y = (double)(j + 1) * dy - 1.0;
             const double y2 = y * y;
             double d = b2 * ca2 + ca2 * ca2 * (-y2) - 2.0 * ca2 * sa2 * y2 - sa2 * sa2 * y2 + sa2;
@@ -320,53 +353,12 @@ __global__ void __launch_bounds__(kOpThreads) op_flux_kernel(OpArgs f) {
                 xl = (-d + u) / v;
                 xr = (d + u) / v;
             }
-            s_y[j] = k0 * y;
+            ys[j] = k0 * y;
             s_xl[j] = k0 * xl;
             s_xr[j] = k0 * xr;
         }
     }
-    __syncthreads();
-    if (it >= f.npt) return;
-    double* out = f.flux + (size_t)pv * f.npt + it;
-    if (!ok) {
-        *out = NAN;
-        return;
-    }
-    const int ilc = f.nlc == 1 ? 0 : min(max(f.lcids[it], 0), f.nlc - 1);
-    const int ipb = min(max(f.pbids[ilc], 0), f.npb - 1);
-    const int iep = min(max(f.epids[ilc], 0), f.t0cols - 1);
-    const double t0v = f.t0[(size_t)pv * f.t0cols + iep];
-    const double p = r.p;
-    double tc;
-    {
-#pragma clang fp contract(off)
-        const double t = f.times[it];
-        const double epoch = floor((t - t0v + 0.5 * p) / p);
-        tc = t - (t0v + epoch * p);
-    }
-    const double ext = f.exptimes[ilc];
-    const double margin = 0.0015 + ext;
-    if (!(r.bt1 - margin <= tc && tc <= r.bt4 + margin)) {
-        *out = 1.0;
-        return;
-    }
-    const int ns = f.nsamples[ilc];
-    const double k = f.k[(size_t)pv * f.kcols + (f.kcols == 1 ? 0 : ipb)];
-    const double ist = f.istar[(size_t)pv * f.npb + ipb];
-    const double* lrow = f.ldm + ((size_t)pv * f.npb + ipb) * f.ng;
-    const double fl = f.fl[pv];
-    double acc = 0.0;
-    for (int is = 1; is <= ns; ++is) {
-        const double tt = tc + ext * ((is - 0.5) / ns - 0.5);
-        const double cx = (((r.c[4] * tt + r.c[3]) * tt + r.c[2]) * tt + r.c[1]) * tt + r.c[0];
-        const double cy = (((r.c[9] * tt + r.c[8]) * tt + r.c[7]) * tt + r.c[6]) * tt + r.c[5];
-        const double z = sqrt(cx * cx + cy * cy);
-        const double ip = interp_ld(z / (1.0 + k), f.dg, lrow, f.ng);
-        const double ap = op_ellipse_area(cx, cy, z, k, fl, s_y, s_xl, s_xr, f.nlines);
-        acc += (ist - ip * ap) / ist;
-    }
-    *out = acc / ns;
-}
+};
 
 }  // namespace rr
 
@@ -447,24 +439,20 @@ int op_evaluate(const rr_table* tab, const rr_lcdata* lc, const rr_params* pv, c
     if (!flux) return set_error(RR_EINVAL, "op_evaluate: null flux");
     // the workspace layout of rr_workspace_bytes: PvRec[npv] | istar[npv, npb] | ldm64[npv, npb, ng]
     char* ws = (char*)workspace;
+    if (!lc->times || !lc->nsamples || !lc->exptimes || (lc->nlc > 1 && !lc->lcids))
+        return set_error(RR_EINVAL, "op_evaluate: null light-curve array");
     OpArgs f;
     f.rec = (const PvRec*)ws;
     ws += align_up((size_t)npv * sizeof(PvRec), 256);
     f.istar = (const double*)ws;
     ws += align_up((size_t)npv * npb * sizeof(double), 256);
     f.ldm = (const double*)ws;
-    f.times = lc->times; f.lcids = lc->lcids; f.pbids = lc->pbids; f.epids = lc->epids;
-    f.nsamples = lc->nsamples; f.exptimes = lc->exptimes;
+    f.d = wf_data(lc, true);
+    f.pbids = lc->pbids; f.epids = lc->epids; f.exptimes = lc->exptimes;
     f.k = pv->k; f.t0 = pv->t0; f.fl = fl; f.alpha = alpha; f.flux = flux;
-    f.npv = npv; f.npt = npt; f.nlc = lc->nlc; f.npb = npb; f.kcols = pv->kcols; f.t0cols = pv->t0cols;
-    f.ng = tab->ng; f.nlines = nlines; f.dg = tab->dg;
-    f.ntiles = (npt + kOpThreads - 1) / kOpThreads;
-    const long long nb = (long long)f.ntiles * npv;
-    if (nb > 0x7fffffffLL) return set_error(RR_ERANGE, "op_evaluate: grid too large");
-    if (!lc->times || !lc->nsamples || !lc->exptimes || (lc->nlc > 1 && !lc->lcids))
-        return set_error(RR_EINVAL, "op_evaluate: null light-curve array");
-    hipLaunchKernelGGL(op_flux_kernel, dim3((unsigned)nb), dim3(kOpThreads), 0, (hipStream_t)stream, f);
-    return check_launch("op_flux_kernel");
+    f.npb = npb; f.kcols = pv->kcols; f.t0cols = pv->t0cols;
+    f.ng = tab->ng; f.nlines = nlines; f.dg = tab->dg; f.inv_dg = 1.0 / tab->dg;
+    return wf_launch<OblateFlux>("op_evaluate", f, npv, OblateFlux::shared_bytes(nlines), (hipStream_t)stream);
 }
 
 }  // extern "C"

@@ -215,6 +215,16 @@ __device__ __forceinline__ double interp_ld(double g, double dg, const double* _
     return (1.0 - a) * row[i] + a * row[i + 1];
 }
 
+// interp_ld with g / dg as g * (1 / dg)
+__device__ __forceinline__ double interp_ld_r(double g, double dg, double inv_dg, const double* __restrict__ row, int ng) {
+    if (g < 0.0) return NAN;
+    if (g > 1.0) return 0.0;
+    int i = (int)floor(g * inv_dg);
+    i = i > ng - 2 ? ng - 2 : (i < 0 ? 0 : i);
+    const double a = (g - i * dg) * inv_dg;
+    return (1.0 - a) * row[i] + a * row[i + 1];
+}
+
 // FP32 form: g / dg by a multiply with 1/dg.  The lerp is continuous across
 // knots, so a knot assigned to the neighbouring interval changes the value by
 // rounding only.

@@ -1034,16 +1034,6 @@ struct RecipF64 {
     double inv_1pk, inv_ist, inv_dg, inv_ns;
 };
 
-// interp_ld with g / dg as g * (1 / dg)
-__device__ __forceinline__ double interp_ld_r(double g, double dg, double inv_dg, const double* __restrict__ row, int ng) {
-    if (g < 0.0) return NAN;
-    if (g > 1.0) return 0.0;
-    int i = (int)floor(g * inv_dg);
-    i = i > ng - 2 ? ng - 2 : (i < 0 ? 0 : i);
-    const double a = (g - i * dg) * inv_dg;
-    return (1.0 - a) * row[i] + a * row[i + 1];
-}
-
 __device__ __forceinline__ double sample_f64_pass1(const double* cc, double dg, int ng, const PointCtx& c,
                                                    const RecipF64& rc, const double* lrow, double tc, int is,
                                                    double& z, bool& part) {

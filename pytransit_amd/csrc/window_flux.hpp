@@ -154,7 +154,6 @@ __global__ void __launch_bounds__(kWfThreads, M::kBlocks) window_flux_kernel(typ
         return;
     }
     if (tid == 0) s_n = 0;
-    M::stage(f, c, pv, shared);
     __syncthreads();
     // ---- the points in the window into the queue --------------------------------------
     for (int j0 = 0; j0 < nsub; ++j0) {
@@ -192,6 +191,7 @@ __global__ void __launch_bounds__(kWfThreads, M::kBlocks) window_flux_kernel(typ
     const float inv_uns = uns > 0 ? 1.0f / (float)uns : 0.0f;
     Item ctx0;
     if (!kMulti) ctx0 = M::item(f, c, pv, 0);
+    if (n > 0) M::stage(f, c, pv, shared);   // read after the chunk's first barrier
     // ---- chunks of points -------------------------------------------------------------
     // c0: first point of the chunk; s0: its first sample, above 0 only for a point with
     // more samples than the item arrays hold, which is a chunk of its own in several passes

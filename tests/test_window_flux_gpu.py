@@ -8,7 +8,7 @@ absolute on fluxes of order one.
 import numpy as np
 import pytest
 
-from pytransit_amd import EclipseModel, QuadraticModel, workloads
+from pytransit_amd import EclipseModel, OblatePlanetModel, QuadraticModel, workloads
 
 pytestmark = pytest.mark.gpu
 
@@ -96,3 +96,27 @@ def test_eclipse(gpu, name, npt, npv):
                                wl.e[j:j + 1], wl.w[j:j + 1], rstar[j], d['pbids'].size, d['lcids'], d['pbids'],
                                d['nsamples'], d['exptimes'])
         assert np.abs(f[j] - ref[0]).max() <= TOL
+
+
+@pytest.mark.parametrize('name,npt,npv', CASES)
+def test_oblate(gpu, oracle, name, npt, npv):
+    from oracle import ec_oracle as eo
+    nlines = 3 if npt == 9001 else 20
+    rng = np.random.default_rng(npt + 3 * npv)
+    d = layout(name, npt, rng)
+    pb = int(d['pbids'].max()) + 1
+    wl, k, t0 = population(npv, rng, pb)
+    f, alpha = rng.uniform(0.0, 0.4, npv), rng.uniform(-1.5, 1.5, npv)
+    ldc = rng.uniform(0.1, 0.4, (npv, pb, 2))
+    m = OblatePlanetModel('quadratic', nlines=nlines)
+    m.set_data(**d)
+    got = np.atleast_2d(m.evaluate(k, f, alpha, ldc, t0, wl.p, wl.a, wl.i)).reshape(npv, npt)
+    ze, zm = oracle.create_z_grid(0.7, 20, 20)
+    dk, dg, wt = oracle.weights_3d(256, 0.005, 0.5, ze, 100)
+    r = rows(npv)
+    ldp, istar = oracle.evaluate_ld('quadratic', oracle.mu_nodes(zm), ldc[r])[:2]
+    ref = eo.opmodel(d['time'], k[r], f[r], alpha[r], t0[r], wl.p[r], wl.a[r], wl.i[r], wl.e[r], wl.w[r],
+                     d['pbids'].size, pb, 2, nlines, d['lcids'], d['pbids'], d['epids'], d['nsamples'], d['exptimes'],
+                     ldp, istar, wt, dk, 0.005, 0.5, dg, ze)
+    assert (ref < 1).any()
+    assert np.abs(got[r] - ref).max() <= TOL
