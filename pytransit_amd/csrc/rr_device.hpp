@@ -188,14 +188,59 @@ __device__ __forceinline__ void ccia_kite3(T r1, T r2, T b, T& area, T& kap0, T&
     area = T(NAN); kap0 = T(NAN);
 }
 
-// Lens area of the unit disk and a disk of radius k at separation z, |1 - k| < z < 1 + k,
-// in FP64: the kite form above with the arctangent and square root of f64_*.
+// Lens area of the unit disk and a disk of radius k at separation z, |1 - k| < z < 1 + k:
+// the kite form above, in FP64 with the arctangent and square root of f64_*.  Products
+// and sums are fused where written, so every kernel that calls it rounds alike.
 __device__ __forceinline__ double lens_area_f64(double k, double z) {
+#pragma clang fp contract(off)
     const double hi = fmax(1.0, k), lo = fmin(1.0, k);
     const double x = fmax(hi, z), c = fmin(lo, z), y = fmax(lo, fmin(hi, z));
     const double sq = f64_sqrt((x + (y + c)) * (c - (x - y)) * (c + (x - y)) * (x + (y - c)));   // 2 akite
-    const double zz = z * z, kk = (k - 1.0) * (k + 1.0);
-    return f64_atan2_ypos(sq, zz - kk) + k * k * f64_atan2_ypos(sq, zz + kk) - 0.5 * sq;
+    const double kk = (k - 1.0) * (k + 1.0);
+    const double k1 = f64_atan2_ypos(sq, fma(z, z, -kk)), k0 = f64_atan2_ypos(sq, fma(z, z, kk));
+    return fma(-0.5, sq, fma(k * k, k0, k1));
+}
+__device__ __forceinline__ float lens_area_f32(float k, float z) {
+#pragma clang fp contract(off)
+    const float hi = d_max(1.0f, k), lo = d_min(1.0f, k);
+    const float x = d_max(hi, z), c = d_min(lo, z), y = d_max(lo, d_min(hi, z));
+    const float sq = d_sqrt((x + (y + c)) * (c - (x - y)) * (c + (x - y)) * (x + (y - c)));
+    const float kk = (k - 1.0f) * (k + 1.0f);
+    const float k1 = atan2_ypos_f(sq, fmaf(z, z, -kk)), k0 = atan2_ypos_f(sq, fmaf(z, z, kk));
+    return fmaf(-0.5f, sq, fmaf(k * k, k0, k1));
+}
+
+// ---- One exposure sample, rounded alike in every kernel that evaluates it -------------
+
+// Time of sample `is` (0-based) of an exposure centred at tc.
+__device__ __forceinline__ double sample_time(double tc, double ext, double inv_ns, int is) {
+#pragma clang fp contract(off)
+    return fma(ext, fma(is + 0.5, inv_ns, -0.5), tc);
+}
+
+// Separation from the Taylor coefficients, Horner's rule in fused steps.
+__device__ __forceinline__ double sample_z(double t, const double* c) {
+#pragma clang fp contract(off)
+    const double x = fma(fma(fma(fma(c[4], t, c[3]), t, c[2]), t, c[1]), t, c[0]);
+    const double y = fma(fma(fma(fma(c[9], t, c[8]), t, c[7]), t, c[6]), t, c[5]);
+    return f64_sqrt(fma(x, x, y * y));
+}
+__device__ __forceinline__ float sample_z(float t, const float* c) {
+#pragma clang fp contract(off)
+    const float x = fmaf(fmaf(fmaf(fmaf(c[4], t, c[3]), t, c[2]), t, c[1]), t, c[0]);
+    const float y = fmaf(fmaf(fmaf(fmaf(c[9], t, c[8]), t, c[7]), t, c[6]), t, c[5]);
+    return d_sqrt(fmaf(x, x, y * y));
+}
+
+// Mean limb darkening at g = z / (1 + k) <= 1, from the reciprocals of 1 + k and dg.
+template <typename T>
+__device__ __forceinline__ T sample_mean(T z, T inv_1pk, T inv_dg, const T* __restrict__ row, int ng) {
+#pragma clang fp contract(off)
+    const T x = z * inv_1pk * inv_dg;
+    int i = (int)x;
+    i = i > ng - 2 ? ng - 2 : (i < 0 ? 0 : i);
+    const T a = x - (T)i, l0 = row[i], l1 = row[i + 1];
+    return a * l1 + (T(1) - a) * l0;
 }
 
 template <typename T>

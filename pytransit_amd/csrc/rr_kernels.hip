@@ -33,6 +33,7 @@
 
 #include "rr_device.hpp"
 #include "rr_internal.hpp"
+#include "window_flux.hpp"
 
 namespace rr {
 
@@ -996,20 +997,6 @@ __device__ __forceinline__ PointCtx point_ctx0(const FluxArgs& f, const PvRec& r
     return c;
 }
 
-// Contribution of sample `is` (0-based) of a point at phase tc: FP64 gives the
-// reference's (istar - I*A)/istar, FP32 gives the depth I*A (the flux is
-// 1 - mean(depth)/istar).
-__device__ __forceinline__ double sample_f64(const double* cc, double dg, int ng, const PointCtx& c,
-                                             const double* lrow, double tc, int is) {
-    const double off = c.ext * ((is + 1 - 0.5) / c.ns - 0.5);
-    const double z = taylor_z<double>(tc + off, cc);
-    if (!(z < 1.0 + c.kk)) return 1.0;  // ccia gives 0 and interp 0 for z >= 1+k: (ist - 0)/ist
-    const double ip = interp_ld(z / (1.0 + c.kk), dg, lrow, ng);
-    double ap, kap;
-    ccia_kite<double>(1.0, c.kk, z, ap, kap);
-    return (c.ist - ip * ap) / c.ist;
-}
-
 __device__ __forceinline__ float sample_f32(const float* cf, float kf, float inv_dg, float tcf, float extf,
                                             float inv_ns, const float* lrow, int ng, int is) {
     const float zlim = 1.0f + kf;
@@ -1022,12 +1009,12 @@ __device__ __forceinline__ float sample_f32(const float* cf, float kf, float inv
     return ip * ap;
 }
 
-// sample_f64 in two passes for the item loop with a queue of partial overlaps:
-// returns the sample's 1 - I*A/istar unless the planet straddles the limb,
+// One FP64 sample in two passes for the item loop with a queue of partial overlaps:
+// pass 1 returns the sample's 1 - I*A/istar unless the planet straddles the limb,
 // |1 - k| < z < 1 + k, where it returns I and sets `part`; sample_f64_finish then
-// completes it.  The divisions of sample_f64 (by ns, 1 + k, dg and istar) are
-// products with the light curve's reciprocals (RecipF64): each changes a result
-// by an ulp or so, and they were the long-latency links of the sample's chain.
+// completes it.  The divisions of model_full.py:93-98 (by ns, 1 + k, dg and istar) are
+// products with the light curve's reciprocals (RecipF64): each changes a result by an
+// ulp or so, and they were the long-latency links of the sample's chain.
 // Reciprocals of one light curve's per-sample divisors, for the FP64 item loop: the
 // divisions become products (a change of the last bit at most).
 struct RecipF64 {
@@ -1171,6 +1158,125 @@ __device__ __forceinline__ bool window_edges(const double* times, int tbase, int
     }
     return true;
 }
+
+// ---- Samples with their own light curve's constants -------------------------------------
+// Used by the general path of flux_body and by the window kernel of several light
+// curves: the same functions, so a request gives the same bits alone and in a batch.
+template <typename Real>
+struct RrItem {
+    double ext, inv_ns;
+    Real k, inv_1pk;
+    double ist;
+    const Real* row;     // the passband's limb-darkening means
+};
+
+template <typename Real>
+__device__ __forceinline__ RrItem<Real> rr_item(double ext, int ns, double k, double ist, const Real* row) {
+    const Real kr = (Real)k;
+    return {ext, 1.0 / ns, kr, Real(1) / (Real(1) + kr), ist, row};
+}
+
+// A sample's value (FP64: (istar - I A) / istar as model_full.py:97; FP32: the depth I A)
+// from its limb-darkening mean and lens area.
+template <typename Real>
+__device__ __forceinline__ Real rr_value(const RrItem<Real>& I, Real mean, Real area) {
+#pragma clang fp contract(off)
+    if constexpr (std::is_same<Real, float>::value) return mean * area;
+    else return fma(-mean, area, I.ist) / I.ist;
+}
+
+// The sample at time t from conjunction: true, with v = z, when the planet crosses the
+// limb, else its value.
+template <typename Real>
+__device__ __forceinline__ bool rr_light(const RrItem<Real>& I, const Real* c, Real inv_dg, int ng, double t, Real& v) {
+    const Real z = sample_z((Real)t, c);
+    v = z;
+    if (!(z < Real(1) + I.k)) {
+        v = std::is_same<Real, float>::value ? Real(0) : Real(1);
+    } else if (d_abs(Real(1) - I.k) < z) {
+        return true;
+    } else {    // inside the disk, or a planet larger than the star covering it
+        const Real r = d_min(Real(1), I.k);
+        v = rr_value<Real>(I, sample_mean<Real>(z, I.inv_1pk, inv_dg, I.row, ng), pi_of<Real>() * (r * r));
+    }
+    return false;
+}
+template <typename Real>
+__device__ __forceinline__ Real rr_limb(const RrItem<Real>& I, Real inv_dg, int ng, Real z) {
+    const Real mean = sample_mean<Real>(z, I.inv_1pk, inv_dg, I.row, ng);
+    if constexpr (std::is_same<Real, float>::value) return rr_value<Real>(I, mean, lens_area_f32(I.k, z));
+    else return rr_value<Real>(I, mean, lens_area_f64(I.k, z));
+}
+// The point's flux from the sum over its ns samples.
+template <typename Real>
+__device__ __forceinline__ Real rr_point(const RrItem<Real>& I, Real acc, int ns) {
+    if constexpr (std::is_same<Real, float>::value) return fmaf(-acc, (float)(I.inv_ns / I.ist), 1.0f);
+    else return acc / ns;
+}
+
+// The window kernel's model for several light curves with their own exposures,
+// passbands and epochs.
+template <bool kMixed>
+struct RrWindowArgs {
+    WfData d;
+    const int32_t* pbids; const int32_t* epids; const double* exptimes;
+    const double* k; const double* t0; const double* istar;
+    const void* ldm;
+    const PvRec* rec;
+    void* flux;
+    int npb, kcols, t0cols, ng;
+    double inv_dg;
+};
+
+template <bool kMixed>
+struct RrWindow {
+    using Real = typename std::conditional<kMixed, float, double>::type;
+    using Args = RrWindowArgs<kMixed>;
+    using Item = RrItem<Real>;
+    static constexpr int kKinds = 1;
+    static constexpr int kGroup = 1;
+    static constexpr int kBlocks = kMixed ? 6 : 5;
+    struct Pv {
+        Real c[10];
+        double bt1, bt4, p, inv_p;
+        bool good;
+    };
+    static __device__ __forceinline__ Pv load(const Args& f, int pv) {
+        const PvRec& r = f.rec[pv];
+        Pv o;
+#pragma unroll
+        for (int j = 0; j < 10; ++j) o.c[j] = (Real)r.c[j];
+        o.bt1 = r.bt1;
+        o.bt4 = r.bt4;
+        o.p = r.p;
+        o.inv_p = r.inv_p;
+        o.good = r.good && r.ldok;
+        return o;
+    }
+    static __device__ __forceinline__ Real fill(const Pv&) { return Real(1); }
+    static __device__ __forceinline__ Real bad() { return Real(NAN); }
+    static __device__ __forceinline__ WfWindow window(const Args& f, const Pv& c, int pv, int ilc) {
+        const double margin = 0.003 + f.exptimes[ilc];
+        return {f.t0[(size_t)pv * f.t0cols + min(max(f.epids[ilc], 0), f.t0cols - 1)], c.bt1 - margin, c.bt4 + margin};
+    }
+    static __device__ __forceinline__ Item item(const Args& f, const Pv&, int pv, int ilc) {
+        const int ipb = min(max(f.pbids[ilc], 0), f.npb - 1);
+        const size_t j = (size_t)pv * f.npb + ipb;
+        return rr_item<Real>(f.exptimes[ilc], f.d.nsamples[ilc], f.k[(size_t)pv * f.kcols + (f.kcols == 1 ? 0 : ipb)],
+                             f.istar[j], (const Real*)f.ldm + j * f.ng);
+    }
+    static __device__ __forceinline__ int classify(const Args& f, const Pv& c, const Item& I, double t, Real& v) {
+        return rr_light<Real>(I, c.c, (Real)f.inv_dg, f.ng, t, v) ? 1 : 0;
+    }
+    static __device__ __forceinline__ Real heavy(const Args& f, const Pv&, const Item& I, double, Real z, int, int,
+                                                 unsigned char*) {
+        return rr_limb<Real>(I, (Real)f.inv_dg, f.ng, z);
+    }
+    static __device__ __forceinline__ Real finish(const Pv&, Real acc, int ns, const Item& I) {
+        return rr_point<Real>(I, acc, ns);
+    }
+    static __device__ __forceinline__ void stage(const Args&, const Pv&, int, unsigned char*) {}
+};
 
 template <bool kMixed, bool kFast>
 __device__ __forceinline__ void flux_body(const FluxArgs& f, int pv, int tile) {
@@ -1613,22 +1719,19 @@ __device__ __forceinline__ void flux_body(const FluxArgs& f, int pv, int tile) {
         double ep;
         const double tc = phase_of(f.times[it], c.t0v, p, inv_p, ep);
         const size_t row = ((size_t)pv * f.npb + c.ipb) * f.ng;
-        if (kMixed) {
-            float cf[10];
+        const Real* lrow = f.row_lds ? s_row : (kMixed ? (const Real*)f.ldm32 : (const Real*)f.ldm64) + row;
+        const RrItem<Real> I = rr_item<Real>(c.ext, c.ns, c.kk, c.ist, lrow);
+        Real cr[10];
 #pragma unroll
-            for (int k = 0; k < 10; ++k) cf[k] = (float)r.c[k];
-            const float inv_ns = 1.0f / (float)c.ns;
-            const float* lrow = f.row_lds ? (const float*)s_row : f.ldm32 + row;
-            float depth = 0.0f;
-            for (int is = 0; is < c.ns; ++is)
-                depth += sample_f32(cf, (float)c.kk, inv_dg, (float)tc, (float)c.ext, inv_ns, lrow, f.ng, is);
-            out[it] = Real(1.0f - depth * ((float)(1.0 / c.ist) * inv_ns));
-        } else {
-            const double* lrow = f.row_lds ? (const double*)s_row : f.ldm64 + row;
-            double acc = 0.0;
-            for (int is = 0; is < c.ns; ++is) acc += sample_f64(r.c, f.dg, f.ng, c, lrow, tc, is);
-            out[it] = Real(acc / c.ns);
+        for (int k = 0; k < 10; ++k) cr[k] = (Real)r.c[k];
+        Real acc = Real(0);
+        for (int is = 0; is < c.ns; ++is) {
+            Real v;
+            if (rr_light<Real>(I, cr, (Real)(1.0 / f.dg), f.ng, sample_time(tc, I.ext, I.inv_ns, is), v))
+                v = rr_limb<Real>(I, (Real)(1.0 / f.dg), f.ng, v);
+            acc += v;
         }
+        out[it] = rr_point<Real>(I, acc, c.ns);
     }
     fill_deferred();
 }
@@ -1710,6 +1813,19 @@ struct BatchDesc {
 };
 
 static_assert(sizeof(SetupBatch) <= 4096 && sizeof(FluxBatch) <= 4096, "kernel arguments above 4 KB");
+
+template <bool kMixed>
+static int rr_window_flux(const rr_lcdata* lc, const rr_params* pv, const FluxArgs& fa, hipStream_t s) {
+    RrWindowArgs<kMixed> f;
+    f.d = wf_data(lc, true);
+    f.pbids = lc->pbids; f.epids = lc->epids; f.exptimes = lc->exptimes;
+    f.k = pv->k; f.t0 = pv->t0; f.istar = fa.istar;
+    f.ldm = kMixed ? (const void*)fa.ldm32 : (const void*)fa.ldm64;
+    f.rec = fa.rec; f.flux = fa.flux;
+    f.npb = fa.npb; f.kcols = pv->kcols; f.t0cols = pv->t0cols; f.ng = fa.ng;
+    f.inv_dg = 1.0 / fa.dg;
+    return wf_launch<RrWindow<kMixed>, true>("rr_flux", f, pv->npv, 0, s);
+}
 
 }  // namespace rr
 
@@ -1984,6 +2100,12 @@ int rr_flux(int precision, const rr_table* tab, const rr_lcdata* lc, const rr_pa
     int rc = prepare_flux("rr_flux", precision, tab, lc, pv, workspace, workspace_bytes, flux, fa, nblocks, lds, fast);
     if (rc || nblocks == 0) return rc;
     hipStream_t s = (hipStream_t)stream;
+    // several light curves whose samples the tile kernel's item loops do not take (FP64,
+    // or uneven nsamples): the window kernel
+    if (lc->nlc > 1 && (precision == RR_FP64 || fa.uniform_ns == 0)) {
+        if (precision == RR_FP64) return rr_window_flux<false>(lc, pv, fa, s);
+        return rr_window_flux<true>(lc, pv, fa, s);
+    }
     const dim3 grid((unsigned)nblocks), block(kThreads);
     if (precision == RR_MIXED) {
         if (fast) hipLaunchKernelGGL((rr_flux_kernel<true, true>), grid, block, lds, s, fa);

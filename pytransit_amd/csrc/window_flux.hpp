@@ -254,7 +254,7 @@ __global__ void __launch_bounds__(kWfThreads, M::kBlocks) window_flux_kernel(typ
             if (i < tot) {
                 const int q = point_of(i);
                 const Item I = kMulti ? s_ctx[q] : ctx0;
-                const double t = s_tc[q] + I.ext * ((s0 + i - first_of(q) + 0.5) * I.inv_ns - 0.5);
+                const double t = sample_time(s_tc[q], I.ext, I.inv_ns, s0 + i - first_of(q));
                 kind = M::classify(f, c, I, t, s_val[i]);
             }
 #pragma unroll
@@ -277,7 +277,7 @@ __global__ void __launch_bounds__(kWfThreads, M::kBlocks) window_flux_kernel(typ
             const int i = s_list[j < na ? j : kWfCap - 1 - (j - na)];
             const int q = point_of(i);
             const Item I = kMulti ? s_ctx[q] : ctx0;
-            const double t = s_tc[q] + I.ext * ((s0 + i - first_of(q) + 0.5) * I.inv_ns - 0.5);
+            const double t = sample_time(s_tc[q], I.ext, I.inv_ns, s0 + i - first_of(q));
             const Real v = M::heavy(f, c, I, t, s_val[i], kind, tid % G, shared);
             if (tid % G == 0) s_val[i] = v;
         }
@@ -306,7 +306,7 @@ __global__ void __launch_bounds__(kWfThreads, M::kBlocks) window_flux_kernel(typ
 // and 160 us with 6000 and 20,000); one time a lane where single sub-tiles of four
 // leave CUs short of work.
 constexpr int kWfBlocks = 4096;
-template <class M>
+template <class M, bool kMultiOnly = false>
 static inline int wf_launch(const char* who, typename M::Args& f, int npv, size_t shared, hipStream_t s) {
     const int npt = f.d.npt;
     const long long sub4 = ((long long)npt + 4 * kWfThreads - 1) / (4 * kWfThreads);
@@ -318,13 +318,16 @@ static inline int wf_launch(const char* who, typename M::Args& f, int npv, size_
     if (ntiles * npv > 0x7fffffffLL) return set_error(RR_ERANGE, "%s: grid too large", who);
     f.d.ntiles = (int)ntiles;
     f.d.nsub = per;
-    const bool multi = f.d.nlc > 1;
+    const bool multi = kMultiOnly || f.d.nlc > 1;
     const size_t lds = wf_lds_bytes<M>(kWfThreads * P * per, multi, shared);
     const dim3 grid((unsigned)(ntiles * npv)), block(kWfThreads);
-    if (multi && P == 4) hipLaunchKernelGGL((window_flux_kernel<M, 4, true>), grid, block, lds, s, f);
-    else if (multi) hipLaunchKernelGGL((window_flux_kernel<M, 1, true>), grid, block, lds, s, f);
-    else if (P == 4) hipLaunchKernelGGL((window_flux_kernel<M, 4, false>), grid, block, lds, s, f);
-    else hipLaunchKernelGGL((window_flux_kernel<M, 1, false>), grid, block, lds, s, f);
+    if (multi || kMultiOnly) {
+        if (P == 4) hipLaunchKernelGGL((window_flux_kernel<M, 4, true>), grid, block, lds, s, f);
+        else hipLaunchKernelGGL((window_flux_kernel<M, 1, true>), grid, block, lds, s, f);
+    } else if constexpr (!kMultiOnly) {
+        if (P == 4) hipLaunchKernelGGL((window_flux_kernel<M, 4, false>), grid, block, lds, s, f);
+        else hipLaunchKernelGGL((window_flux_kernel<M, 1, false>), grid, block, lds, s, f);
+    }
     return check_launch(who);
 }
 

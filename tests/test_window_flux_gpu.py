@@ -3,12 +3,13 @@ arrays, for each model that runs on it, against the FP64 oracle.
 
 Every model is evaluated in FP64 with the oracle's formulas; the kernels differ from
 them in the order of a few roundings, so the bar is the suite's FP64 bar, 1e-9
-absolute on fluxes of order one.
+absolute on fluxes of order one; the mixed-precision RoadRunner path has its own bar,
+1 ppm.
 """
 import numpy as np
 import pytest
 
-from pytransit_amd import EclipseModel, OblatePlanetModel, QuadraticModel, workloads
+from pytransit_amd import EclipseModel, OblatePlanetModel, QuadraticModel, RoadRunnerModel, workloads
 
 pytestmark = pytest.mark.gpu
 
@@ -120,3 +121,29 @@ def test_oblate(gpu, oracle, name, npt, npv):
                      ldp, istar, wt, dk, 0.005, 0.5, dg, ze)
     assert (ref < 1).any()
     assert np.abs(got[r] - ref).max() <= TOL
+
+
+@pytest.mark.parametrize('precision', ['fp64', 'mixed'])
+@pytest.mark.parametrize('name,npt,npv', [c for c in CASES if c[0] not in ('one', 'many samples')])
+def test_roadrunner_light_curves(gpu, oracle, name, npt, npv, precision):
+    rng = np.random.default_rng(npt + 5 * npv)
+    d = layout(name, npt, rng)
+    pb = int(d['pbids'].max()) + 1
+    wl, k, t0 = population(npv, rng, pb)
+    k[0] = (0.3, 0.31)
+    if npv > 2:
+        wl.a[1] = np.nan                   # an invalid vector, and a passband without a radius
+        k[2, 1] = np.nan
+    ldc = rng.uniform(0.1, 0.4, (npv, pb, 2))
+    om, tm = oracle.OracleRR('quadratic'), RoadRunnerModel('quadratic', precision=precision)
+    for m in (om, tm):
+        m.set_data(d['time'], d['lcids'], d['pbids'], d['nsamples'], d['exptimes'], d['epids'])
+    f = np.atleast_2d(tm.evaluate(k, ldc, t0, wl.p, wl.a, wl.i)).reshape(npv, npt)
+    r = rows(npv)
+    ref = om.evaluate(np.nan_to_num(k[r], nan=0.1), ldc[r], t0[r], wl.p[r], wl.a[r], wl.i[r], wl.e[r], wl.w[r]).reshape(r.size, npt)
+    seen = np.isfinite(k[r]).all(1)        # the reference leaves a NaN radius undefined
+    assert np.array_equal(np.isnan(f[r][seen]), np.isnan(ref[seen])) and np.isnan(ref).any() == (npv > 2)
+    assert np.nanmin(ref[seen]) < 1
+    assert np.nanmax(np.abs(f[r] - ref)[seen]) <= (TOL if precision == 'fp64' else 1e-6)
+    if npv > 2:
+        assert (f[2][d['pbids'][d['lcids']] == 1] == 1).all()
