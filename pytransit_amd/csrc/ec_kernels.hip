@@ -15,14 +15,14 @@
 //                     conjunction phase (orbits/orbits_py.py:544-555), the 7 Kepler
 //                     solves of the Taylor stencil about it (orbits/taylor_z.py:
 //                     106-185), the light travel time and the contact window
-//   window_flux_kernel<EclipseFlux>   the planet disk area left visible by the star
+//   ec_flux_kernel    the planet disk area left visible by the star
 //                     over a tile of times of one pv (window_flux.hpp).  1000 pv x
 //                     20,001 t with 5 samples (160 MB written, 23 us): 45 us against
 //                     147 us with one lane per (pv, time), whose samples ran in series
 //                     with two libm arctangents each
 //   es_flux_kernel    one lane per (pv, time): the mean lens area, fanned out over the
 //                     passbands of the spectroscopy model
-//   window_flux_kernel<OblateFlux>   the oblate planet's flux: the pv's ellipse
+//   op_flux_kernel    the oblate planet's flux: the pv's ellipse
 //                     scanlines in LDS, shared by the lanes that evaluate a sample; the
 //                     per-pv state comes from rr_setup
 #include <hip/hip_runtime.h>
@@ -232,6 +232,11 @@ struct EclipseFlux {
     static __device__ __forceinline__ void stage(const EclArgs&, const Pv&, int, unsigned char*) {}
 };
 
+template <int P, bool kMulti>
+__global__ void __launch_bounds__(kWfThreads, EclipseFlux::kBlocks) ec_flux_kernel(EclArgs f) {
+    window_flux_body<EclipseFlux, P, kMulti>(f);
+}
+
 // ---- Oblate planet ---------------------------------------------------------------
 
 constexpr int kOpMaxLines = 2048;
@@ -360,6 +365,11 @@ struct OblateFlux {
     }
 };
 
+template <int P, bool kMulti>
+__global__ void __launch_bounds__(kWfThreads, OblateFlux::kBlocks) op_flux_kernel(OpArgs f) {
+    window_flux_body<OblateFlux, P, kMulti>(f);
+}
+
 }  // namespace rr
 
 using namespace rr;
@@ -400,7 +410,9 @@ static int ec_common(const char* who, const rr_lcdata* lc, const rr_params* pv, 
         f.d = wf_data(lc, pv->t0cols == 1);
         f.epids = lc->epids; f.exptimes = lc->exptimes; f.t0 = pv->t0; f.rec = rec; f.flux = flux;
         f.t0cols = pv->t0cols;
-        return wf_launch<EclipseFlux>(who, f, npv, 0, s);
+        return wf_launch<EclipseFlux>(who,
+                                      {ec_flux_kernel<4, false>, ec_flux_kernel<1, false>, ec_flux_kernel<4, true>, ec_flux_kernel<1, true>},
+                                      f, npv, 0, s);
     }
     EcArgs f;
     f.times = lc->times; f.nsamples = lc->nsamples;
@@ -452,7 +464,9 @@ int op_evaluate(const rr_table* tab, const rr_lcdata* lc, const rr_params* pv, c
     f.k = pv->k; f.t0 = pv->t0; f.fl = fl; f.alpha = alpha; f.flux = flux;
     f.npb = npb; f.kcols = pv->kcols; f.t0cols = pv->t0cols;
     f.ng = tab->ng; f.nlines = nlines; f.dg = tab->dg; f.inv_dg = 1.0 / tab->dg;
-    return wf_launch<OblateFlux>("op_evaluate", f, npv, OblateFlux::shared_bytes(nlines), (hipStream_t)stream);
+    return wf_launch<OblateFlux>("op_evaluate",
+                                 {op_flux_kernel<4, false>, op_flux_kernel<1, false>, op_flux_kernel<4, true>, op_flux_kernel<1, true>},
+                                 f, npv, OblateFlux::shared_bytes(nlines), (hipStream_t)stream);
 }
 
 }  // extern "C"

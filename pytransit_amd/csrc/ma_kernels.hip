@@ -8,7 +8,7 @@
 // Kernels:
 //   ma_orbit_kernel   8 pv per 64-lane block: the Taylor orbit and contact window of
 //                     the RoadRunner path (taylor_z.py:23-102,298-328)
-//   window_flux_kernel<MaModel>   epoch, window (contact times +- 0.025 d),
+//   ma_flux_kernel    epoch, window (contact times +- 0.025 d),
 //                     supersampling and analytic flux of a tile of times of one pv;
 //                     flux [npv, npt] (window_flux.hpp)
 //
@@ -214,6 +214,11 @@ struct MaModel {
     static __device__ __forceinline__ void stage(const MaArgs&, const Pv&, int, unsigned char*) {}
 };
 
+template <int P, bool kMulti>
+__global__ void __launch_bounds__(kWfThreads, MaModel::kBlocks) ma_flux_kernel(MaArgs f) {
+    window_flux_body<MaModel, P, kMulti>(f);
+}
+
 }  // namespace rr
 
 using namespace rr;
@@ -250,7 +255,9 @@ int ma_evaluate(const rr_lcdata* lc, const rr_params* pv, const double* ldc, voi
     f.pbids = lc->pbids; f.epids = lc->epids; f.exptimes = lc->exptimes;
     f.k = pv->k; f.t0 = pv->t0; f.ldc = ldc; f.rec = rec; f.flux = flux;
     f.npv = npv; f.npb = npb; f.kcols = pv->kcols; f.t0cols = pv->t0cols;
-    return wf_launch<MaModel>("ma_evaluate", f, npv, 0, s);
+    return wf_launch<MaModel>("ma_evaluate",
+                              {ma_flux_kernel<4, false>, ma_flux_kernel<1, false>, ma_flux_kernel<4, true>, ma_flux_kernel<1, true>},
+                              f, npv, 0, s);
 }
 
 }  // extern "C"

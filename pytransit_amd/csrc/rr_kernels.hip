@@ -1278,6 +1278,11 @@ struct RrWindow {
     static __device__ __forceinline__ void stage(const Args&, const Pv&, int, unsigned char*) {}
 };
 
+template <bool kMixed, int P>
+__global__ void __launch_bounds__(kWfThreads, RrWindow<kMixed>::kBlocks) rr_window_flux_kernel(RrWindowArgs<kMixed> f) {
+    window_flux_body<RrWindow<kMixed>, P, true>(f);
+}
+
 template <bool kMixed, bool kFast>
 __device__ __forceinline__ void flux_body(const FluxArgs& f, int pv, int tile) {
     using Real = typename std::conditional<kMixed, float, double>::type;
@@ -1824,7 +1829,8 @@ static int rr_window_flux(const rr_lcdata* lc, const rr_params* pv, const FluxAr
     f.rec = fa.rec; f.flux = fa.flux;
     f.npb = fa.npb; f.kcols = pv->kcols; f.t0cols = pv->t0cols; f.ng = fa.ng;
     f.inv_dg = 1.0 / fa.dg;
-    return wf_launch<RrWindow<kMixed>, true>("rr_flux", f, pv->npv, 0, s);
+    return wf_launch<RrWindow<kMixed>>("rr_flux", {nullptr, nullptr, rr_window_flux_kernel<kMixed, 4>,
+                                                  rr_window_flux_kernel<kMixed, 1>}, f, pv->npv, 0, s);
 }
 
 }  // namespace rr

@@ -1,4 +1,4 @@
-// Light-curve kernel shared by the models whose flux is a constant outside a window
+// Light-curve kernel body shared by the models whose flux is a constant outside a window
 // around the conjunction and an average over exposure samples inside it.
 //
 // One workgroup of 256 lanes takes up to kWfMaxSub sub-tiles of 256 * P consecutive
@@ -98,7 +98,7 @@ static inline size_t wf_lds_bytes(int queue, bool multi, size_t shared) {
 }
 
 template <class M, int P, bool kMulti>
-__global__ void __launch_bounds__(kWfThreads, M::kBlocks) window_flux_kernel(typename M::Args f) {
+__device__ __forceinline__ void window_flux_body(const typename M::Args& f) {
     using Real = typename M::Real;
     using Item = typename M::Item;
     constexpr int kSub = kWfThreads * P;
@@ -306,8 +306,15 @@ __global__ void __launch_bounds__(kWfThreads, M::kBlocks) window_flux_kernel(typ
 // and 160 us with 6000 and 20,000); one time a lane where single sub-tiles of four
 // leave CUs short of work.
 constexpr int kWfBlocks = 4096;
-template <class M, bool kMultiOnly = false>
-static inline int wf_launch(const char* who, typename M::Args& f, int npv, size_t shared, hipStream_t s) {
+template <class M>
+struct WfKernels {
+    typedef void (*Fn)(typename M::Args);
+    Fn one4, one1;     // one light curve: four times a lane, one time a lane
+    Fn multi4, multi1; // several
+};
+template <class M>
+static inline int wf_launch(const char* who, const WfKernels<M>& kn, typename M::Args& f, int npv, size_t shared,
+                            hipStream_t s) {
     const int npt = f.d.npt;
     const long long sub4 = ((long long)npt + 4 * kWfThreads - 1) / (4 * kWfThreads);
     const int P = sub4 * npv < 2048 ? 1 : 4;
@@ -318,16 +325,11 @@ static inline int wf_launch(const char* who, typename M::Args& f, int npv, size_
     if (ntiles * npv > 0x7fffffffLL) return set_error(RR_ERANGE, "%s: grid too large", who);
     f.d.ntiles = (int)ntiles;
     f.d.nsub = per;
-    const bool multi = kMultiOnly || f.d.nlc > 1;
+    const bool multi = f.d.nlc > 1;
     const size_t lds = wf_lds_bytes<M>(kWfThreads * P * per, multi, shared);
     const dim3 grid((unsigned)(ntiles * npv)), block(kWfThreads);
-    if (multi || kMultiOnly) {
-        if (P == 4) hipLaunchKernelGGL((window_flux_kernel<M, 4, true>), grid, block, lds, s, f);
-        else hipLaunchKernelGGL((window_flux_kernel<M, 1, true>), grid, block, lds, s, f);
-    } else if constexpr (!kMultiOnly) {
-        if (P == 4) hipLaunchKernelGGL((window_flux_kernel<M, 4, false>), grid, block, lds, s, f);
-        else hipLaunchKernelGGL((window_flux_kernel<M, 1, false>), grid, block, lds, s, f);
-    }
+    const auto fn = multi ? (P == 4 ? kn.multi4 : kn.multi1) : (P == 4 ? kn.one4 : kn.one1);
+    hipLaunchKernelGGL(fn, grid, block, lds, s, f);
     return check_launch(who);
 }
 
