@@ -249,6 +249,24 @@ int rr_lnlike(int precision, const rr_table* tab, const rr_lcdata* lc, const rr_
               const rr_ld* ld, const double* obs, const double* sigma, double* lnl, double* grad,
               void* stream);
 
+/* A per-parameter-vector input read in place: element i is ptr[i * stride] (stride 0:
+ * one value for every pv), or `value` for every pv where ptr is NULL. */
+typedef struct rr_vec {
+    const double* ptr;
+    int64_t stride;
+    double value;
+} rr_vec;
+
+/* rr_lnlike with the inputs read where they are: par[7] = (k, t0, p, a, i, e, w),
+ * ldc[2] = (c0, c1), sigma.  t0 with several epochs has t0cols consecutive columns at
+ * ptr + i * stride.  The setup runs in its own kernel and a light curve is split over
+ * several workgroups when npv is small, with the state in between in the caller's
+ * workspace; with RR_SORTED_RUNS times outside the transit window are not read per pv. */
+size_t rr_lnlike_workspace_bytes(int npv, int npt, int ng);
+int rr_lnlike_vec(int precision, const rr_table* tab, const rr_lcdata* lc, int npv, int t0cols,
+                  const rr_vec* par, int law, const rr_vec* ldc, const double* obs, const rr_vec* sigma,
+                  void* workspace, size_t workspace_bytes, double* lnl, double* grad, void* stream);
+
 /* Mandel & Agol (2002) quadratic limb-darkening model: flux [npv, npt] (FP64) for
  * ldc [npv, 2*npb] = (u1, u2) per passband, k [npv, 1|npb], t0 [npv, nep], with the
  * Taylor orbit and contact window of the RoadRunner path widened by 0.025 d and

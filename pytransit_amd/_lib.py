@@ -54,6 +54,10 @@ class RRParams(ctypes.Structure):
                 ('e', c_void_p), ('w', c_void_p)]
 
 
+class RRVec(ctypes.Structure):
+    _fields_ = [('ptr', c_void_p), ('stride', ctypes.c_int64), ('value', c_double)]
+
+
 class RRRequest(ctypes.Structure):
     _fields_ = [('lc', RRLcData), ('pv', RRParams), ('ld', RRLd), ('workspace', c_void_p),
                 ('workspace_bytes', c_size_t), ('flux', c_void_p)]
@@ -86,6 +90,10 @@ _SIGNATURES = {
     'ts_workspace_bytes': (c_size_t, [c_int, c_int, c_int, c_int, c_int]),
     'rr_lnlike': (c_int, [c_int, POINTER(RRTable), POINTER(RRLcData), POINTER(RRParams), POINTER(RRLd), c_void_p,
                           c_void_p, c_void_p, c_void_p, c_void_p]),
+    'rr_lnlike_workspace_bytes': (c_size_t, [c_int, c_int, c_int]),
+    'rr_lnlike_vec': (c_int, [c_int, POINTER(RRTable), POINTER(RRLcData), c_int, c_int, POINTER(RRVec), c_int,
+                              POINTER(RRVec), c_void_p, POINTER(RRVec), c_void_p, c_size_t, c_void_p, c_void_p,
+                              c_void_p]),
     'ts_evaluate': (c_int, [c_int, POINTER(RRTable), POINTER(RRLcData), POINTER(RRParams), POINTER(RRLd),
                             c_void_p, c_size_t, c_void_p, c_void_p]),
     'rr_max_batch': (c_int, []),

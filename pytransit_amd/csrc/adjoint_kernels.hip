@@ -15,6 +15,19 @@
 // chord), dA/dk = 2 k kappa0.  Points outside the window have m = 1 and zero
 // gradient.  FP64 epoch reduction and accumulation; per-sample arithmetic in
 // Real (float for RR_MIXED, double for RR_FP64).
+//
+// Kernels (rr_lnlike_vec):
+//   rr_lnlike_setup_kernel   orbits of 8 pvs a block, a pv's limb-darkening rows a block,
+//                            and each tile's sum of (o - 1)^2
+//   rr_lnlike_kernel         (pv, range of times) a block: window test of tiles, queue of
+//                            the points in the window, samples, block sums
+//   rr_lnlike_reduce_kernel  the blocks' sums of a pv, where a light curve is split
+// One block per pv did all of it before: the setup idled three of its four waves for
+// 10-15 us, every pv read every time, a population of 250 left the chip two thirds
+// empty and the gradient was computed whether asked for or not.  250 pv x 18,000 t over
+// 24 d, nss 5, FP64, value only: 50 -> 11 + 13 + 4 us; 2048 pv x 10,000 t, 22 % in the
+// window, nss 5, mixed, with the gradient: 125 -> 16 + 74 us, VALU-bound (about 150
+// instructions a sample at 128 registers).
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -25,21 +38,60 @@
 
 namespace rr {
 
+// A per-pv input: element i at p[i * stride] (stride 0: one value for every pv), or the
+// value v where there is no array.  The callers' strided columns and plain numbers are
+// read as they are, without a copy or an upload for each.
+struct LnlVec {
+    const double* p;
+    long long stride;
+    double v;
+    __device__ __forceinline__ double at(int i, int off = 0) const { return p ? p[i * stride + off] : v; }
+};
+
+// Per-pv state between the setup and the main kernel.
+struct alignas(16) LnlRec {
+    double c[10], dc[10];          // orbit coefficients and their period derivatives
+    double lo, hi;                 // the window
+    double k, t0, p, inv_p, inv_a, tan_i;
+    double ist, dist0, dist1;      // disk integral and its coefficient derivatives
+    int32_t orbit_ok, ld_ok;
+};
+static_assert(sizeof(LnlRec) == 256, "LnlRec must be 256 bytes");
+
 struct LnlArgs {
-    const double* times; const double* obs; const double* sigma;
+    const double* times; const double* obs;
     const int32_t* nsamples; const double* exptimes; const int32_t* epids;
-    const double* k; const double* t0; const double* p; const double* a; const double* inc;
-    const double* e; const double* w;
-    int law, nldc; const double* ldc;
+    LnlVec k, t0, p, a, inc, e, w, sigma, c0, c1;
     const double* W; const double* mu;
     double* lnl; double* grad;
-    int npv, npt, kcols, t0cols, nk, ng, nz;
+    LnlRec* rec; void* rows; double* tsum; double* part;
+    int law, npv, npt, t0cols, nk, ng, nz;
+    int sorted;        // times non-decreasing: tiles outside the window are skipped
+    int ntile, per, nsplit;   // tiles of the light curve, tiles per block, blocks per pv
     double kmin, kmax, dk, dg;
 };
 
 constexpr int kLnlThreads = 256;
+constexpr int kLnlTile = 256;     // times of a tile
 constexpr int kLnlMaxNg = 512;
 constexpr int kLnlMaxNz = 1024;
+constexpr int kLnlQueue = 5 * kLnlTile;
+
+// A pv's limb-darkening rows: L and, for the gradient, dL/dk, dL/dc0 and dL/dc1.
+// FP64: per interval of g each row's value at the left knot and its rise to the right
+// one.  FP32: per knot the rows' values (one 16-byte read), then, for the gradient, the
+// g slope of each interval from the FP64 means: the difference of two rounded values
+// would lose ~1e-5 of the slope, which the t0, p, a and i gradients carry through the
+// chain rule.
+template <typename Real, bool kGrad>
+__host__ __device__ inline int lnl_rows_count(int ng) {
+    if (sizeof(Real) == 4) return kGrad ? 5 * ng : ng;
+    return (ng - 1) * (kGrad ? 8 : 2);
+}
+template <typename Real, bool kGrad>
+__host__ __device__ inline size_t lnl_rows_bytes(int ng) {
+    return ((size_t)lnl_rows_count<Real, kGrad>(ng) * sizeof(Real) + 15) / 16 * 16;
+}
 
 // Position at stencil time t and its derivative with respect to the period:
 // dM/dp = -2 pi t / p^2 (t0 = 0) and df/dM = (1 + e cos f)^2 / (1 - e^2)^(3/2).
@@ -85,6 +137,13 @@ __device__ __forceinline__ Real dhorner5(const Real* c, Real t) {
     return ((Real(4) * c[4] * t + Real(3) * c[3]) * t + Real(2) * c[2]) * t + c[1];
 }
 
+// a times the hardware's reciprocal of a divisor: the bits of the FP32 quotient without
+// its exponent scaling, and never fused into a following sum.
+__device__ __forceinline__ float f32_quotient(float a, float rcp) {
+#pragma clang fp contract(off)
+    return a * rcp;
+}
+
 // Lens area of the unit disk and a disk of radius k < 1 at separation z, in the
 // lens case |z - 1| < k, from u = z - 1 given to full FP32 precision.  With the
 // kite area written as akite = z sin kappa1 (Heron), the kite form
@@ -96,7 +155,8 @@ __device__ __forceinline__ Real dhorner5(const Real* c, Real t) {
 // it.  The kite's square root is ((1 + z)^2 - k^2)(k^2 - u^2), the sorted-sides
 // product of common.py:5-33,52-73 regrouped, and z^2 - 1 = u (2 + u).  Returns A,
 // kappa0 and akite.
-__device__ __forceinline__ void lens_seg_f32(float k, float z, float u, float& area, float& kap0, float& akite) {
+__device__ __forceinline__ void lens_seg_f32(float k, float z, float inv_z, float u, float& area, float& kap0,
+                                             float& akite) {
     const float zp1 = 1.0f + z;
     const float sq = __builtin_amdgcn_sqrtf((zp1 * zp1 - k * k) * ((k - u) * (k + u)));  // 2 akite
     const float zm = u * (2.0f + u);                                                     // z^2 - 1
@@ -110,58 +170,125 @@ __device__ __forceinline__ void lens_seg_f32(float k, float z, float u, float& a
         sr = fmaf(sr, x2, 1.0f / 5040.0f);
         sr = fmaf(sr, x2, -1.0f / 120.0f);
         sr = fmaf(sr, x2, 1.0f / 6.0f);
-        area = k * k * kap0 + kap1 * x2 * sr - u * akite / z;
+        area = d_fma(k * k, kap0, kap1 * x2 * sr) - f32_quotient(u * akite, inv_z);
     } else {
         area = kap1 + k * k * kap0 - akite;
     }
 }
 
-template <typename Real>
-__global__ void __launch_bounds__(kLnlThreads) rr_lnlike_kernel(LnlArgs s) {
-    __shared__ double s_x[7], s_y[7], s_dx[7], s_dy[7], s_c[10], s_dc[10], s_win[2];
-    __shared__ double s_l[kLnlMaxNz], s_d0[kLnlMaxNz], s_d1[kLnlMaxNz];
-    __shared__ Real s_L[kLnlMaxNg], s_Lk[kLnlMaxNg], s_Lc0[kLnlMaxNg], s_Lc1[kLnlMaxNg], s_dL[kLnlMaxNg];
-    __shared__ double s_L64[kLnlMaxNg];
-    __shared__ double s_red[kLnlThreads / 64][8];
-    __shared__ double s_ist, s_dist0, s_dist1;
-    __shared__ int s_ok;
+// ---- per-pv setup ---------------------------------------------------------------------
 
-    constexpr bool kMixed = std::is_same<Real, float>::value;
-    const int pv = blockIdx.x;
-    const int tid = threadIdx.x;
-    const double a = s.a[pv], e = s.e[pv], p = s.p[pv], inc = s.inc[pv], w = s.w[pv];
-    const double kk = s.k[(size_t)pv * s.kcols];
-    const double* c = s.ldc + (size_t)pv * s.nldc;
-    const bool in_table = s.kmin <= kk && kk <= s.kmax;
-    // ---- prologue: orbit, window, limb-darkening rows ----------------------------
-    if (tid < 7) {
-        double x, y, dx, dy;
-        kepler_xy_dp((tid - 3) * 2e-2, p, a, cos(inc), e, w, x, y, dx, dy);
-        s_x[tid] = x; s_y[tid] = y; s_dx[tid] = dx; s_dy[tid] = dy;
-    }
-    for (int iz = tid; iz < s.nz; iz += kLnlThreads) {
-        const double mu = s.mu[iz];
-        s_l[iz] = ld_law(s.law, mu, c, s.nldc);
-        s_d0[iz] = dld_dc(s.law, mu, c, 0);
-        s_d1[iz] = dld_dc(s.law, mu, c, 1);
+constexpr int kLnlOrbitLds = kOrbitGroup * (4 * 8 + 20 + 2);   // doubles
+
+// Orbit, its period derivative and the window of a pv by a group of 8 lanes (sub: the
+// group, j: its lane); every thread of the block calls it (barriers).
+template <bool kGrad>
+__device__ __forceinline__ void lnl_orbit(const LnlArgs& s, int pv, bool active, int sub, int j, LnlRec* rec, double* sm) {
+    double* s_x = sm + sub * 32;       // x, y, dx, dy at the seven stencil times
+    double* s_c = sm + kOrbitGroup * 32 + sub * 20;
+    double* s_w = sm + kOrbitGroup * 52 + sub * 2;
+    const int q = active ? pv : 0;
+    const double p = s.p.at(q), a = s.a.at(q), inc = s.inc.at(q), e = s.e.at(q), w = s.w.at(q), k = s.k.at(q);
+    const bool valid = active && !(isnan(a) || a <= 1.0 || e < 0.0);
+    if (valid && j < 7) {
+        if (kGrad) kepler_xy_dp((j - 3) * 2e-2, p, a, cos(inc), e, w, s_x[j], s_x[8 + j], s_x[16 + j], s_x[24 + j]);
+        else kepler_xy((j - 3) * 2e-2, p, a, cos(inc), e, w, s_x[j], s_x[8 + j]);
     }
     __syncthreads();
-    if (tid == 0) {
-        taylor_from_stencil(s_x, s_y, s_c);
-        taylor_from_stencil(s_dx, s_dy, s_dc);
-        double ist;
-        if (!ld_integral(s.law, c, ist)) {
-            double sum = 0.0;
-            for (int m = 1; m < 200; ++m) sum += ld_trapz_segment(s.law, c, s.nldc, m);
-            ist = 2.0 * kPi * sum;
+    if (valid && j < (kGrad ? 2 : 1)) taylor_from_stencil(s_x + 16 * j, s_x + 16 * j + 8, s_c + 10 * j);
+    __syncthreads();
+    if (valid && j < 2) s_w[j] = find_contact_point(k, j == 0 ? 1 : 4, s_c);
+    __syncthreads();
+    if (!active) return;
+    if (valid)
+        for (int m = j; m < (kGrad ? 20 : 10); m += 8) rec->c[m] = s_c[m];   // c, then dc
+    if (j == 0) {
+        const double ext = s.exptimes[0];
+        // the light curve's epoch column, clamped as the evaluate path does
+        const int ep = min(max(s.epids[0], 0), s.t0cols - 1);
+        rec->lo = valid ? s_w[0] - (0.003 + ext) : 0.0;
+        rec->hi = valid ? s_w[1] + (0.003 + ext) : 0.0;
+        rec->k = k;
+        rec->t0 = s.t0.at(q, ep);
+        rec->p = p;
+        rec->inv_p = 1.0 / p;
+        rec->inv_a = 1.0 / a;
+        rec->tan_i = tan(inc);
+        rec->orbit_ok = valid ? 1 : 0;
+    }
+}
+
+// The limb-darkening intervals of a pv by NT threads: the profile and its coefficient
+// derivatives at the mu nodes in LDS, the table's two rows of k contracted with them
+// (lanes over g), then the intervals.  `sm`: lnl_ld_lds doubles.
+template <bool kGrad> __host__ __device__ inline int lnl_ld_lds(int nz, int ng) { return (kGrad ? 3 : 1) * nz + (kGrad ? 4 : 1) * ng; }
+
+// The rows' means at every g: V neighbouring g a lane, eight mu nodes' loads together.
+template <bool kGrad, int V, int NT>
+__device__ __forceinline__ void lnl_contract(const LnlArgs& s, int ik, double ak, const double* s_l, double* s_m) {
+    typedef double vec __attribute__((ext_vector_type(V)));
+    constexpr int kP = kGrad ? 3 : 1;
+    constexpr int kB = 8;
+    const int nz = s.nz, ng = s.ng;
+    for (int iv = threadIdx.x; iv < ng / V; iv += NT) {
+        const double* w0 = s.W + (size_t)ik * nz * ng + V * iv;
+        const double* w1 = w0 + (size_t)nz * ng;
+        double a0[kP][V], a1[kP][V];
+#pragma unroll
+        for (int m = 0; m < kP; ++m)
+#pragma unroll
+            for (int e = 0; e < V; ++e) a0[m][e] = a1[m][e] = 0.0;
+        for (int iz0 = 0; iz0 < nz; iz0 += kB) {
+            vec u0[kB], u1[kB];
+#pragma unroll
+            for (int u = 0; u < kB; ++u) {
+                const size_t o = (size_t)min(iz0 + u, nz - 1) * ng;
+                u0[u] = *(const vec*)(w0 + o);
+                u1[u] = *(const vec*)(w1 + o);
+            }
+#pragma unroll
+            for (int u = 0; u < kB; ++u) {
+                if (iz0 + u < nz) {
+#pragma unroll
+                    for (int m = 0; m < kP; ++m)
+#pragma unroll
+                        for (int e = 0; e < V; ++e) {
+                            a0[m][e] += u0[u][e] * s_l[m * nz + iz0 + u];
+                            a1[m][e] += u1[u][e] * s_l[m * nz + iz0 + u];
+                        }
+                }
+            }
         }
-        s_ist = ist;
-        s_dist0 = distar_dc(s.law, c, 0);
-        s_dist1 = distar_dc(s.law, c, 1);
-        s_ok = !(isnan(a) || a <= 1.0 || e < 0.0 || isnan(s_l[0])) && in_table;
+#pragma unroll
+        for (int e = 0; e < V; ++e) {
+            const int ig = V * iv + e;
+            s_m[ig] = (1.0 - ak) * a0[0][e] + ak * a1[0][e];
+            if constexpr (kGrad) {
+                s_m[ng + ig] = (a1[0][e] - a0[0][e]) / s.dk;
+                s_m[2 * ng + ig] = (1.0 - ak) * a0[1][e] + ak * a1[1][e];
+                s_m[3 * ng + ig] = (1.0 - ak) * a0[2][e] + ak * a1[2][e];
+            }
+        }
     }
-    __syncthreads();
-    if (tid < 2) s_win[tid] = find_contact_point(kk, tid == 0 ? 1 : 4, s_c);
+}
+
+template <typename Real, bool kGrad, int NT>
+__device__ __forceinline__ void lnl_rows(const LnlArgs& s, int pv, LnlRec* rec, Real* rows, double* sm) {
+    constexpr int kP = kGrad ? 3 : 1;
+    const int tid = threadIdx.x, nz = s.nz, ng = s.ng;
+    double* s_l = sm;                  // [kP][nz]
+    double* s_m = sm + kP * nz;        // [kGrad ? 4 : 1][ng]
+    const double c[2] = {s.c0.at(pv), s.c1.at(pv)};
+    const double kk = s.k.at(pv);
+    for (int iz = tid; iz < nz; iz += NT) {
+        const double mu = s.mu[iz];
+        s_l[iz] = ld_law(s.law, mu, c, 2);
+        if (kGrad) {
+            s_l[nz + iz] = dld_dc(s.law, mu, c, 0);
+            s_l[2 * nz + iz] = dld_dc(s.law, mu, c, 1);
+        }
+    }
+    const bool in_table = s.kmin <= kk && kk <= s.kmax;
     int ik = 0;
     double ak = 0.0;
     if (in_table) {
@@ -169,191 +296,428 @@ __global__ void __launch_bounds__(kLnlThreads) rr_lnlike_kernel(LnlArgs s) {
         ik = ik > s.nk - 2 ? s.nk - 2 : ik;
         ak = (kk - s.kmin - ik * s.dk) / s.dk;
     }
-    for (int ig = tid; ig < s.ng; ig += kLnlThreads) {
-        double a0 = 0, a1 = 0, b0 = 0, b1 = 0, c0 = 0, c1 = 0;
-        const double* w0 = s.W + (size_t)ik * s.nz * s.ng + ig;
-        const double* w1 = w0 + (size_t)s.nz * s.ng;
-        for (int iz = 0; iz < s.nz; ++iz) {
-            const double u0 = w0[(size_t)iz * s.ng], u1 = w1[(size_t)iz * s.ng];
-            a0 += u0 * s_l[iz]; a1 += u1 * s_l[iz];
-            b0 += u0 * s_d0[iz]; b1 += u1 * s_d0[iz];
-            c0 += u0 * s_d1[iz]; c1 += u1 * s_d1[iz];
-        }
-        const double L = (1.0 - ak) * a0 + ak * a1;
-        s_L64[ig] = L;
-        s_L[ig] = (Real)L;
-        s_Lk[ig] = (Real)((a1 - a0) / s.dk);
-        s_Lc0[ig] = (Real)((1.0 - ak) * b0 + ak * b1);
-        s_Lc1[ig] = (Real)((1.0 - ak) * c0 + ak * c1);
-    }
-    __syncthreads();
-    // the g slope of each interval from the FP64 means: the difference of two
-    // rounded FP32 values would lose ~1e-5 of the slope, which the t0, p, a and i
-    // gradients carry through the chain rule
-    for (int ig = tid; ig < s.ng - 1; ig += kLnlThreads) s_dL[ig] = (Real)((s_L64[ig + 1] - s_L64[ig]) / s.dg);
-    __syncthreads();
-    if (!s_ok) {
-        if (tid == 0) {
-            s.lnl[pv] = NAN;
-            if (s.grad)
-                for (int j = 0; j < 7; ++j) s.grad[(size_t)pv * 7 + j] = NAN;
-        }
-        return;
-    }
-
-    // ---- main loop over times ----------------------------------------------------
-    const int ns = s.nsamples[0];
-    const double ext = s.exptimes[0];
-    // the light curve's epoch column, clamped as the evaluate path does
-    const int ep = min(max(s.epids[0], 0), s.t0cols - 1);
-    const double t0v = s.t0[(size_t)pv * s.t0cols + ep];
-    const double lo = s_win[0] - (0.003 + ext), hi = s_win[1] + (0.003 + ext);
-    const double inv_p = 1.0 / p;
-    Real cx[5], cy[5], dcx[5], dcy[5];
-#pragma unroll
-    for (int i = 0; i < 5; ++i) {
-        cx[i] = (Real)s_c[i]; cy[i] = (Real)s_c[5 + i];
-        dcx[i] = (Real)s_dc[i]; dcy[i] = (Real)s_dc[5 + i];
-    }
-    const Real kr = (Real)kk, zlim = Real(1) + kr, inv1pk = Real(1) / zlim;
-    const Real dg = (Real)s.dg, inv_dg = (Real)(1.0 / s.dg);
-    const double g_scale = 1.0 / ((1.0 + kk) * s.dg);   // g / dg = z g_scale
-    const Real tan_i = (Real)tan(inc), inv_a = (Real)(1.0 / a);
-    const Real pik2 = (Real)(kPi * kk * kk), dpik2 = (Real)(2.0 * kPi * kk);
-    const double scale = 1.0 / (ns * s_ist);
-    const Real rscale = (Real)scale;
-    // per-sample and per-point divisors as reciprocals (off the samples' chains)
-    const double inv_ns = 1.0 / ns, scale_ist = scale / s_ist;
-    double chi = 0.0, g[7] = {0, 0, 0, 0, 0, 0, 0};
-    for (int it = tid; it < s.npt; it += kLnlThreads) {
-        const double t = s.times[it];
-        const double om1 = s.obs[it] - 1.0;
-        double epoch;
-        double tc;
-        {
-#pragma clang fp contract(off)
-            const double u = t - t0v + 0.5 * p;
-            double ep = floor(u * inv_p);
-            const double rr = u - ep * p;
-            ep += (rr < 0.0) ? -1.0 : ((rr >= p) ? 1.0 : 0.0);
-            epoch = ep;
-            tc = t - (t0v + ep * p);
-        }
-        if (!(lo <= tc && tc <= hi)) {
-            chi += om1 * om1;
-            continue;
-        }
-        Real D = 0, dDk = 0, dDt0 = 0, dDp = 0, dDa = 0, dDi = 0, dDc0 = 0, dDc1 = 0;
-        const Real ep = (Real)epoch;
-        for (int is = 1; is <= ns; ++is) {
-            const double taud = tc + ext * ((is - 0.5) * inv_ns - 0.5);
-            const Real tau = (Real)taud;
-            Real x, y, z, u;
-            if constexpr (kMixed) {
-                // the constant and linear terms of the position in FP64: the phase
-                // resolves ~1e-9 d that an FP32 time would drop, ~1e-7 of the
-                // position at sky speeds of ~40 stellar radii per day.  z - 1 is
-                // formed from the FP64 squared distance, so the lens area below
-                // does not see the rounding of z.
-                const Real t2 = tau * tau;
-                const double xd = s_c[0] + s_c[1] * taud + (double)(((cx[4] * tau + cx[3]) * tau + cx[2]) * t2);
-                const double yd = s_c[5] + s_c[6] * taud + (double)(((cy[4] * tau + cy[3]) * tau + cy[2]) * t2);
-                const double s2 = xd * xd + yd * yd;
-                x = (Real)xd;
-                y = (Real)yd;
-                z = d_sqrt((Real)s2);
-                u = (Real)(s2 - 1.0) / (Real(1) + z);
-            } else {
-                x = horner5(cx, tau);
-                y = horner5(cy, tau);
-                z = sqrt(x * x + y * y);
-                u = z - Real(1);
-            }
-            if (!(z < zlim)) continue;
-            const Real vx = dhorner5(cx, tau), vy = dhorner5(cy, tau);
-            const Real px = horner5(dcx, tau), py = horner5(dcy, tau);
-            // limb darkening and its slopes at g = z/(1+k)
-            // the grazing parameter in units of the g step: in the mixed form from
-            // 1 + u in FP64, so the lerp position keeps the precision of u
-            Real gg, gx;
-            if constexpr (kMixed) {
-                const double gxd = (1.0 + (double)u) * g_scale;
-                gx = (Real)gxd;
-                gg = (Real)(gxd * s.dg);
-            } else {
-                gg = z * inv1pk;
-                gx = gg * inv_dg;
-            }
-            Real Ii = 0, dIdg = 0, Ik = 0, Ic0 = 0, Ic1 = 0;
-            if (gg <= Real(1)) {
-                int i = (int)floor(gx);
-                i = i > s.ng - 2 ? s.ng - 2 : (i < 0 ? 0 : i);
-                const Real al = gx - (Real)i;
-                Ii = s_L[i] + al * (s_L[i + 1] - s_L[i]);
-                dIdg = s_dL[i];
-                Ik = s_Lk[i] + al * (s_Lk[i + 1] - s_Lk[i]);
-                Ic0 = s_Lc0[i] + al * (s_Lc0[i + 1] - s_Lc0[i]);
-                Ic1 = s_Lc1[i] + al * (s_Lc1[i + 1] - s_Lc1[i]);
-            }
-            const Real inv_z = Real(1) / z;
-            // area and its slopes
-            Real A, dAdz, dAdk;
-            if (z <= Real(1) - kr) {
-                A = pik2; dAdz = 0; dAdk = dpik2;
-            } else {
-                Real kap, akite;
-                if constexpr (kMixed) {
-                    if (kk < 1.0) lens_seg_f32(kr, z, u, A, kap, akite);
-                    else ccia_kite3<Real>(Real(1), kr, z, A, kap, akite);
-                } else {
-                    ccia_kite3<Real>(Real(1), kr, z, A, kap, akite);
-                }
-                dAdz = Real(-2) * akite * inv_z;   // minus the chord of the lens
-                dAdk = Real(2) * kr * kap;
-            }
-            // z derivatives
-            const Real dz_t0 = -(x * vx + y * vy) * inv_z;
-            const Real dz_p = (x * (px - ep * vx) + y * (py - ep * vy)) * inv_z;
-            const Real dz_a = z * inv_a;
-            const Real dz_i = -(y * y) * tan_i * inv_z;
-            const Real G = dIdg * inv1pk * A + Ii * dAdz;
-            D += Ii * A;
-            dDk += (Ik - dIdg * z * inv1pk * inv1pk) * A + Ii * dAdk;
-            dDt0 += G * dz_t0;
-            dDp += G * dz_p;
-            dDa += G * dz_a;
-            dDi += G * dz_i;
-            dDc0 += Ic0 * A;
-            dDc1 += Ic1 * A;
-        }
-        const double r = om1 + (double)(D * rscale);     // o - m, with m = 1 - D/(ns istar)
-        chi += r * r;
-        const double rs = -r * scale;                     // r * dm/dD
-        g[0] += rs * (double)dDk;
-        g[1] += rs * (double)dDt0;
-        g[2] += rs * (double)dDp;
-        g[3] += rs * (double)dDa;
-        g[4] += rs * (double)dDi;
-        g[5] += rs * (double)dDc0 + r * (double)D * scale_ist * s_dist0;
-        g[6] += rs * (double)dDc1 + r * (double)D * scale_ist * s_dist1;
-    }
-    // ---- block reduction ----------------------------------------------------------
-    double v[8] = {chi, g[0], g[1], g[2], g[3], g[4], g[5], g[6]};
-#pragma unroll
-    for (int j = 0; j < 8; ++j) v[j] = wave_sum(v[j]);
-    if ((tid & 63) == 0)
-        for (int j = 0; j < 8; ++j) s_red[tid >> 6][j] = v[j];
     __syncthreads();
     if (tid == 0) {
-        double tot[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-        for (int wv = 0; wv < kLnlThreads / 64; ++wv)
-            for (int j = 0; j < 8; ++j) tot[j] += s_red[wv][j];
-        const double sig = s.sigma[pv];
-        const double is2 = 1.0 / (sig * sig);
-        s.lnl[pv] = s.npt * (-log(sig) - 0.5 * log(2.0 * kPi)) - 0.5 * tot[0] * is2;
-        if (s.grad)
-            for (int j = 0; j < 7; ++j) s.grad[(size_t)pv * 7 + j] = tot[1 + j] * is2;
+        double ist = NAN;
+        ld_integral(s.law, c, ist);    // analytic for both laws
+        rec->ist = ist;
+        rec->dist0 = distar_dc(s.law, c, 0);
+        rec->dist1 = distar_dc(s.law, c, 1);
+        rec->ld_ok = (in_table && !isnan(s_l[0])) ? 1 : 0;
     }
+    // two neighbouring g a lane (16-byte loads) where the table's rows allow it
+    if (ng % 2 == 0 && ((uintptr_t)s.W & 15) == 0) lnl_contract<kGrad, 2, NT>(s, ik, ak, s_l, s_m);
+    else lnl_contract<kGrad, 1, NT>(s, ik, ak, s_l, s_m);
+    __syncthreads();
+    constexpr int kR = kGrad ? 4 : 1;
+    if constexpr (std::is_same<Real, float>::value) {
+        for (int i = tid; i < kR * ng; i += NT) rows[i] = (float)s_m[(i % kR) * ng + i / kR];
+        if (kGrad)
+            for (int ig = tid; ig < ng - 1; ig += NT) rows[kR * ng + ig] = (float)((s_m[ig + 1] - s_m[ig]) / s.dg);
+    } else {
+        for (int i = tid; i < (ng - 1) * 2 * kR; i += NT) {
+            const int ig = i / (2 * kR), m = i - ig * 2 * kR, r = (m >> 1) * ng + ig;
+            rows[i] = (m & 1) ? s_m[r + 1] - s_m[r] : s_m[r];
+        }
+    }
+}
+
+// Blocks of 64: the orbits of 8 pvs, then one per pv for its limb-darkening intervals,
+// then one per tile of times for its sum of (o - 1)^2 (a tile outside a pv's window
+// adds that to the pv's chi^2 without being read again).
+template <typename Real, bool kGrad>
+__global__ void __launch_bounds__(64) rr_lnlike_setup_kernel(LnlArgs s) {
+    extern __shared__ __align__(16) unsigned char lds[];
+    double* sm = (double*)lds;
+    const int nob = (s.npv + kOrbitGroup - 1) / kOrbitGroup;
+    const int b = blockIdx.x;
+    if (b < nob) {
+        const int sub = threadIdx.x / kOrbitGroup, pv = b * kOrbitGroup + sub;
+        lnl_orbit<kGrad>(s, pv, pv < s.npv, sub, threadIdx.x % kOrbitGroup, s.rec + pv, sm);
+    } else if (b < nob + s.npv) {
+        const int pv = b - nob;
+        lnl_rows<Real, kGrad, 64>(s, pv, s.rec + pv, (Real*)((char*)s.rows + pv * lnl_rows_bytes<Real, kGrad>(s.ng)), sm);
+    } else {
+        const int t = b - nob - s.npv;
+        double v = 0.0;
+#pragma unroll
+        for (int j = 0; j < kLnlTile / 64; ++j) {
+            const int it = t * kLnlTile + j * 64 + threadIdx.x;
+            const double om1 = it < s.npt ? s.obs[it] - 1.0 : 0.0;
+            v += om1 * om1;
+        }
+        v = wave_sum(v);
+        if (threadIdx.x == 0) s.tsum[t] = v;
+    }
+}
+
+// ---- samples --------------------------------------------------------------------------
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+// A pv's constants of the sample loop in the working precision.
+template <typename Real>
+struct LnlPv {
+    Real cx[5], cy[5], dcx[5], dcy[5];
+    double c0, c1, c5, c6;         // constant and linear terms of the position in FP64
+    double g_scale, dg;            // g / dg = z g_scale
+    Real k, zlim, inv1pk, inv_dg, tan_i, inv_a, pik2, dpik2;
+};
+
+// Sums over a point's samples: I A and its derivatives by k, t0, p, a, i, c0, c1.
+template <typename Real, bool kGrad>
+struct LnlSums {
+    Real v[kGrad ? 8 : 1];
+};
+
+template <typename Real, bool kGrad>
+__device__ __forceinline__ void lnl_sample(const LnlPv<Real>& v, const Real* rows, int ng, double taud, Real ep,
+                                           LnlSums<Real, kGrad>& d) {
+    constexpr bool kMixed = std::is_same<Real, float>::value;
+    const Real tau = (Real)taud;
+    Real x, y, z, u, inv_z;
+    if constexpr (kMixed) {
+        // the constant and linear terms of the position in FP64: the phase resolves
+        // ~1e-9 d that an FP32 time would drop, ~1e-7 of the position at sky speeds of
+        // ~40 stellar radii per day.  z - 1 is formed from the FP64 squared distance,
+        // so the lens area below does not see the rounding of z.
+        const Real t2 = tau * tau;
+        const double xd = v.c0 + v.c1 * taud + (double)(((v.cx[4] * tau + v.cx[3]) * tau + v.cx[2]) * t2);
+        const double yd = v.c5 + v.c6 * taud + (double)(((v.cy[4] * tau + v.cy[3]) * tau + v.cy[2]) * t2);
+        const double s2 = xd * xd + yd * yd;
+        x = (Real)xd;
+        y = (Real)yd;
+        z = d_sqrt((Real)s2);
+        if (!(z < v.zlim)) return;
+        u = f32_quotient((Real)(s2 - 1.0), __builtin_amdgcn_rcpf(Real(1) + z));
+        inv_z = __builtin_amdgcn_rcpf(z);
+    } else {
+        x = horner5(v.cx, tau);
+        y = horner5(v.cy, tau);
+        f64_sqrt_rsqrt(x * x + y * y, z, inv_z);
+        if (!(z < v.zlim)) return;
+        u = z - Real(1);
+    }
+    // limb darkening and its slopes at g = z/(1+k), in units of the g step: in the mixed
+    // form from 1 + u in FP64, so the lerp position keeps the precision of u
+    Real gx;
+    if constexpr (kMixed) {
+        const double gxd = (1.0 + (double)u) * v.g_scale;
+        gx = (Real)gxd;
+        if (!((Real)(gxd * v.dg) <= Real(1))) return;   // g > 1: the mean and its slopes are 0
+    } else {
+        gx = z * v.inv1pk * v.inv_dg;
+    }
+    int i = (int)gx;
+    i = i > ng - 2 ? ng - 2 : (i < 0 ? 0 : i);
+    const Real al = gx - (Real)i;
+    Real Ii, dIdg = 0, Ik = 0, Ic0 = 0, Ic1 = 0;
+    if constexpr (kMixed && kGrad) {
+        const f32x4 l = *(const f32x4*)(rows + 4 * i), r = *(const f32x4*)(rows + 4 * i + 4);
+        Ii = l[0] + al * (r[0] - l[0]);
+        dIdg = rows[4 * ng + i];
+        Ik = l[1] + al * (r[1] - l[1]);
+        Ic0 = l[2] + al * (r[2] - l[2]);
+        Ic1 = l[3] + al * (r[3] - l[3]);
+    } else if constexpr (kMixed) {
+        Ii = rows[i] + al * (rows[i + 1] - rows[i]);
+    } else {
+        const Real* r = rows + i * (kGrad ? 8 : 2);
+        Ii = r[0] + al * r[1];
+        if constexpr (kGrad) {
+            dIdg = r[1] * v.inv_dg;
+            Ik = r[2] + al * r[3];
+            Ic0 = r[4] + al * r[5];
+            Ic1 = r[6] + al * r[7];
+        }
+    }
+    // area and its slopes
+    Real A, dAdz = 0, dAdk;
+    if (z <= Real(1) - v.k) {
+        A = v.pik2;
+        dAdk = v.dpik2;
+    } else {
+        Real kap, akite;
+        if constexpr (kMixed) {
+            if (v.k < Real(1)) lens_seg_f32(v.k, z, inv_z, u, A, kap, akite);
+            else ccia_kite3<Real>(Real(1), v.k, z, A, kap, akite);
+        } else if (fabs(1.0 - v.k) < z) {
+            A = lens_f64(v.k, z, kap, akite);
+        } else {
+            A = kPi;
+            kap = akite = 0.0;
+        }
+        dAdz = Real(-2) * akite * inv_z;   // minus the chord of the lens
+        dAdk = Real(2) * v.k * kap;
+    }
+    d.v[0] += Ii * A;
+    if constexpr (kGrad) {
+        const Real vx = dhorner5(v.cx, tau), vy = dhorner5(v.cy, tau);
+        const Real px = horner5(v.dcx, tau), py = horner5(v.dcy, tau);
+        const Real dz_t0 = -(x * vx + y * vy) * inv_z;
+        const Real dz_p = (x * (px - ep * vx) + y * (py - ep * vy)) * inv_z;
+        const Real dz_a = z * v.inv_a;
+        const Real dz_i = -(y * y) * v.tan_i * inv_z;
+        const Real G = d_fma(dIdg * v.inv1pk, A, Ii * dAdz);
+        d.v[1] += d_fma(Ik - dIdg * z * v.inv1pk * v.inv1pk, A, Ii * dAdk);
+        d.v[2] += G * dz_t0;
+        d.v[3] += G * dz_p;
+        d.v[4] += G * dz_a;
+        d.v[5] += G * dz_i;
+        d.v[6] += Ic0 * A;
+        d.v[7] += Ic1 * A;
+    }
+}
+
+// lnL (value 0) and its gradient (1-7) of a pv from the sums over its times.
+__device__ __forceinline__ void lnl_store(const LnlArgs& s, int pv, int j, double tot, bool ok) {
+    const double sig = s.sigma.at(pv);
+    const double is2 = 1.0 / (sig * sig);
+    if (j == 0) s.lnl[pv] = s.npt * (-log(sig) - 0.5 * log(2.0 * kPi)) - 0.5 * tot * is2;
+    else s.grad[(size_t)pv * 7 + j - 1] = ok ? tot * is2 : (double)NAN;
+}
+
+// ---- main kernel ----------------------------------------------------------------------
+//
+// One block per (pv, range of tiles).  A lane of each wave tests one of 64 tiles
+// against the window; tiles outside add their sum of (o - 1)^2, the others are
+// classified point by point and the points in the window queued, so that the samples
+// run on full waves.  The last points, fewer than the block, take several lanes each.
+// kFused computes the pv's setup in the block itself (no workspace, one block per pv).
+template <typename Real, bool kGrad, bool kFused>
+__global__ void __launch_bounds__(kLnlThreads) rr_lnlike_kernel(LnlArgs s) {
+    extern __shared__ __align__(16) unsigned char lds[];
+    __shared__ LnlRec s_rec;
+    __shared__ double s_red[kLnlThreads / 64][8];
+    __shared__ int s_cnt[4][kLnlThreads / 64];
+    Real* s_rows = (Real*)lds;
+    int* s_q = (int*)(lds + lnl_rows_bytes<Real, kGrad>(s.ng));
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int pv = blockIdx.x / s.nsplit, part = blockIdx.x - pv * s.nsplit;
+    if (kFused) {
+        double* sm = (double*)(s_q + kLnlQueue);
+        lnl_orbit<kGrad>(s, pv, tid < kOrbitGroup, 0, tid % kOrbitGroup, &s_rec, sm);
+        lnl_rows<Real, kGrad, kLnlThreads>(s, pv, &s_rec, s_rows, sm + kLnlOrbitLds);
+    } else {
+        const int4* rows = (const int4*)((const char*)s.rows + pv * lnl_rows_bytes<Real, kGrad>(s.ng));
+        for (int i = tid; i < (int)(lnl_rows_bytes<Real, kGrad>(s.ng) / 16); i += kLnlThreads) ((int4*)s_rows)[i] = rows[i];
+    }
+    __syncthreads();
+    const LnlRec& r = kFused ? s_rec : s.rec[pv];
+    const bool ok = r.orbit_ok && r.ld_ok;
+    double chi = 0.0, g[7] = {0, 0, 0, 0, 0, 0, 0};
+    if (ok) {
+        const int ns = s.nsamples[0];
+        const double ext = s.exptimes[0], inv_ns = 1.0 / ns;
+        const double t0 = r.t0, p = r.p, inv_p = r.inv_p, lo = r.lo, hi = r.hi;
+        const double scale = 1.0 / (ns * r.ist), scale_ist = scale / r.ist;
+        LnlPv<Real> v;
+#pragma unroll
+        for (int i = 0; i < 5; ++i) {
+            v.cx[i] = (Real)r.c[i];
+            v.cy[i] = (Real)r.c[5 + i];
+            v.dcx[i] = kGrad ? (Real)r.dc[i] : Real(0);
+            v.dcy[i] = kGrad ? (Real)r.dc[5 + i] : Real(0);
+        }
+        v.c0 = r.c[0]; v.c1 = r.c[1]; v.c5 = r.c[5]; v.c6 = r.c[6];
+        v.k = (Real)r.k;
+        v.zlim = Real(1) + v.k;
+        v.inv1pk = Real(1) / v.zlim;
+        v.inv_dg = (Real)(1.0 / s.dg);
+        v.g_scale = 1.0 / ((1.0 + r.k) * s.dg);
+        v.dg = s.dg;
+        v.tan_i = (Real)r.tan_i;
+        v.inv_a = (Real)r.inv_a;
+        v.pik2 = (Real)(kPi * r.k * r.k);
+        v.dpik2 = (Real)(2.0 * kPi * r.k);
+        // point `it` by G lanes of a wave, this one the sub-th
+        auto point = [&](int it, int G, int sub) {
+            const double om1 = s.obs[it] - 1.0;
+            double epoch;
+            const double tc = epoch_phase(s.times[it], t0, p, inv_p, epoch);
+            LnlSums<Real, kGrad> d = {};
+            const Real ep = (Real)epoch;
+            if (G == 1) {
+#pragma unroll 1
+                for (int is = 0; is < ns; ++is)
+                    lnl_sample<Real, kGrad>(v, s_rows, s.ng, tc + ext * ((is + 0.5) * inv_ns - 0.5), ep, d);
+            } else {
+                // a sample a lane, summed in sample order as by one lane
+#pragma unroll 1
+                for (int i0 = 0; i0 < ns; i0 += G) {
+                    LnlSums<Real, kGrad> one = {};
+                    if (i0 + sub < ns)
+                        lnl_sample<Real, kGrad>(v, s_rows, s.ng, tc + ext * ((i0 + sub + 0.5) * inv_ns - 0.5), ep, one);
+                    for (int q = 0; q < G; ++q)
+#pragma unroll
+                        for (int m = 0; m < (kGrad ? 8 : 1); ++m) d.v[m] += __shfl(one.v[m], (lane & ~(G - 1)) + q, 64);
+                }
+            }
+            if (sub != 0) return;
+            const double D = (double)d.v[0];
+            const double res = om1 + (double)(d.v[0] * (Real)scale);  // o - m, with m = 1 - D/(ns istar)
+            chi += res * res;
+            if constexpr (kGrad) {
+                const double rs = -res * scale;                       // r * dm/dD
+#pragma unroll
+                for (int m = 0; m < 7; ++m) g[m] += rs * (double)d.v[m + 1];
+                g[5] += res * D * scale_ist * r.dist0;
+                g[6] += res * D * scale_ist * r.dist1;
+            }
+        };
+        const int tb = part * s.per, te = min(tb + s.per, s.ntile);
+        int n = 0;
+        for (int g0 = tb; g0 < te; g0 += 64) {
+            // tiles outside the window, one a lane (every wave alike)
+            const int tile = g0 + lane;
+            bool inside = tile < te;
+            if (inside && s.sorted) {
+                double ea, eb;
+                const double ta = epoch_phase(s.times[tile * kLnlTile], t0, p, inv_p, ea);
+                const double tl = epoch_phase(s.times[tile * kLnlTile + min(kLnlTile, s.npt - tile * kLnlTile) - 1], t0, p, inv_p, eb);
+                if (ea == eb ? (tl < lo || ta > hi) : (eb == ea + 1.0 && ta > hi && tl < lo)) {
+                    inside = false;
+                    if (tid < 64) chi += s.tsum[tile];
+                }
+            }
+            unsigned long long mask = __ballot(inside);
+            while (mask) {
+                // four tiles at a time, their loads in flight together
+                int tl[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    tl[j] = mask ? g0 + __ffsll((long long)mask) - 1 : -1;
+                    mask &= mask - 1;
+                }
+                double tv[4], ov[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const int it = tl[j] * kLnlTile + tid;
+                    const bool in = tl[j] >= 0 && tid < s.npt - tl[j] * kLnlTile;
+                    tv[j] = in ? s.times[it] : 0.0;
+                    ov[j] = in ? s.obs[it] : 1.0;
+                }
+                unsigned long long mk[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    bool inw = false;
+                    if (tl[j] >= 0 && tid < s.npt - tl[j] * kLnlTile) {
+                        double epoch;
+                        const double tc = epoch_phase(tv[j], t0, p, inv_p, epoch);
+                        inw = lo <= tc && tc <= hi;
+                        if (!inw) chi += (ov[j] - 1.0) * (ov[j] - 1.0);
+                    }
+                    mk[j] = __ballot(inw);
+                    if (lane == 0) s_cnt[j][tid >> 6] = __popcll(mk[j]);
+                }
+                __syncthreads();
+                // queue slots in time order: the sums do not depend on the schedule
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    int at = n;
+                    for (int wv = 0; wv < kLnlThreads / 64; ++wv) {
+                        at += wv < (tid >> 6) ? s_cnt[j][wv] : 0;
+                        n += s_cnt[j][wv];
+                    }
+                    if ((mk[j] >> lane) & 1ull) s_q[at + __popcll(mk[j] & ((1ull << lane) - 1ull))] = tl[j] * kLnlTile + tid;
+                }
+                __syncthreads();
+                for (; n >= kLnlThreads; n -= kLnlThreads) point(s_q[n - kLnlThreads + tid], 1, 0);
+            }
+        }
+        if (n > 0) {
+            int G = 1;
+            while (G < 16 && 2 * G * n <= kLnlThreads && 2 * G <= ns) G *= 2;
+            if (tid / G < n) point(s_q[tid / G], G, tid % G);
+        }
+    } else {
+        chi = NAN;
+    }
+    // ---- block reduction ----------------------------------------------------------
+    double t[8] = {chi, g[0], g[1], g[2], g[3], g[4], g[5], g[6]};
+#pragma unroll
+    for (int j = 0; j < (kGrad ? 8 : 1); ++j) {
+        t[j] = wave_sum(t[j]);
+        if (lane == 0) s_red[tid >> 6][j] = t[j];
+    }
+    __syncthreads();
+    if (tid < (kGrad ? 8 : 1)) {
+        double tot = 0.0;
+        for (int wv = 0; wv < kLnlThreads / 64; ++wv) tot += s_red[wv][tid];
+        if (s.nsplit > 1) s.part[((size_t)pv * s.nsplit + part) * 8 + tid] = tot;
+        else lnl_store(s, pv, tid, tot, ok);
+    }
+}
+
+// Sums the blocks' parts of a pv in order; one lane per (pv, value).
+__global__ void __launch_bounds__(256) rr_lnlike_reduce_kernel(LnlArgs s) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    const int pv = i >> 3, j = i & 7;
+    if (pv >= s.npv || (j > 0 && !s.grad)) return;
+    double tot = 0.0;
+    for (int q = 0; q < s.nsplit; ++q) tot += s.part[((size_t)pv * s.nsplit + q) * 8 + j];
+    lnl_store(s, pv, j, tot, s.rec[pv].orbit_ok && s.rec[pv].ld_ok);
+}
+
+template <typename Real, bool kGrad>
+static int lnl_launch(LnlArgs& s, bool fused, hipStream_t st) {
+    const size_t rows = lnl_rows_bytes<Real, kGrad>(s.ng) + kLnlQueue * sizeof(int);
+    const size_t ld = sizeof(double) * (size_t)lnl_ld_lds<kGrad>(s.nz, s.ng), orb = sizeof(double) * kLnlOrbitLds;
+    if (fused) {
+        hipLaunchKernelGGL((rr_lnlike_kernel<Real, kGrad, true>), dim3(s.npv), dim3(kLnlThreads), rows + orb + ld, st, s);
+        return check_launch("rr_lnlike_kernel");
+    }
+    const int nob = (s.npv + kOrbitGroup - 1) / kOrbitGroup;
+    const long long nb = (long long)nob + s.npv + (s.sorted ? s.ntile : 0);
+    if (nb > 0x7fffffffLL || (long long)s.npv * s.nsplit > 0x7fffffffLL)
+        return set_error(RR_ERANGE, "rr_lnlike: grid too large");
+    hipLaunchKernelGGL((rr_lnlike_setup_kernel<Real, kGrad>), dim3((unsigned)nb), dim3(64), ld > orb ? ld : orb, st, s);
+    int rc = check_launch("rr_lnlike_setup_kernel");
+    if (rc) return rc;
+    hipLaunchKernelGGL((rr_lnlike_kernel<Real, kGrad, false>), dim3((unsigned)(s.npv * s.nsplit)), dim3(kLnlThreads),
+                       rows, st, s);
+    rc = check_launch("rr_lnlike_kernel");
+    if (rc || s.nsplit == 1) return rc;
+    hipLaunchKernelGGL(rr_lnlike_reduce_kernel, dim3((s.npv * 8 + 255) / 256), dim3(256), 0, st, s);
+    return check_launch("rr_lnlike_reduce_kernel");
+}
+
+static int lnl_dispatch(int precision, LnlArgs& s, bool fused, hipStream_t st) {
+    if (precision == RR_MIXED) return s.grad ? lnl_launch<float, true>(s, fused, st) : lnl_launch<float, false>(s, fused, st);
+    return s.grad ? lnl_launch<double, true>(s, fused, st) : lnl_launch<double, false>(s, fused, st);
+}
+
+// Checks shared by the two entries; fills the light curve's and table's arguments.
+static int lnl_prepare(const char* who, int precision, const rr_table* tab, const rr_lcdata* lc, int npv, int t0cols,
+                       int law, const double* obs, double* lnl, double* grad, LnlArgs& s) {
+    if (precision != RR_FP64 && precision != RR_MIXED) return set_error(RR_EINVAL, "%s: bad precision", who);
+    if (lc->nlc != 1) return set_error(RR_EINVAL, "%s: one light curve only (nlc = %d)", who, lc->nlc);
+    if (law != RR_LD_QUADRATIC && law != RR_LD_POWER_2)
+        return set_error(RR_EINVAL, "%s: the quadratic and power-2 laws are supported", who);
+    if (tab->ng < 2 || tab->ng > kLnlMaxNg || tab->nz < 1 || tab->nz > kLnlMaxNz || !tab->weights || !tab->mu)
+        return set_error(RR_EINVAL, "%s: bad weight table (ng <= %d, nz <= %d)", who, kLnlMaxNg, kLnlMaxNz);
+    if (npv < 0 || lc->npt < 0 || t0cols < 1) return set_error(RR_EINVAL, "%s: bad sizes", who);
+    if (npv == 0) return RR_OK;
+    if (!lc->times || !lc->nsamples || !lc->exptimes || !lc->epids || !obs || !lnl)
+        return set_error(RR_EINVAL, "%s: null array", who);
+    s.times = lc->times; s.obs = obs; s.nsamples = lc->nsamples; s.exptimes = lc->exptimes; s.epids = lc->epids;
+    s.W = tab->weights; s.mu = tab->mu; s.lnl = lnl; s.grad = grad;
+    s.rec = nullptr; s.rows = nullptr; s.tsum = nullptr; s.part = nullptr;
+    s.law = law; s.npv = npv; s.npt = lc->npt; s.t0cols = t0cols; s.nk = tab->nk; s.ng = tab->ng; s.nz = tab->nz;
+    s.sorted = 0;
+    s.ntile = (int)(((long long)lc->npt + kLnlTile - 1) / kLnlTile);
+    s.per = s.ntile;
+    s.nsplit = 1;
+    s.kmin = tab->kmin; s.kmax = tab->kmax; s.dk = tab->dk; s.dg = tab->dg;
+    return RR_OK;
+}
+
+// Blocks per pv: enough for four on each of 256 CUs, of at least four tiles each.
+static int lnl_split(int npv, int npt) {
+    const int ntile = (int)(((long long)npt + kLnlTile - 1) / kLnlTile);
+    int n = (1024 + npv - 1) / (npv > 0 ? npv : 1);
+    n = n < ntile / 4 ? n : ntile / 4;
+    return n < 1 ? 1 : n;
 }
 
 }  // namespace rr
@@ -371,27 +735,53 @@ int rr_lnlike(int precision, const rr_table* tab, const rr_lcdata* lc, const rr_
     if (ld->law != RR_LD_QUADRATIC && ld->law != RR_LD_POWER_2)
         return set_error(RR_EINVAL, "rr_lnlike: the quadratic and power-2 laws are supported");
     if (ld->nldc < 2 || !ld->ldc) return set_error(RR_EINVAL, "rr_lnlike: two limb-darkening coefficients needed");
-    if (tab->ng < 2 || tab->ng > kLnlMaxNg || tab->nz < 1 || tab->nz > kLnlMaxNz || !tab->weights || !tab->mu)
-        return set_error(RR_EINVAL, "rr_lnlike: bad weight table (ng <= %d, nz <= %d)", kLnlMaxNg, kLnlMaxNz);
-    const int npv = pv->npv, npt = lc->npt;
-    if (npv < 0 || npt < 0 || pv->t0cols < 1) return set_error(RR_EINVAL, "rr_lnlike: bad sizes");
-    if (npv == 0) return RR_OK;
-    if (!lc->times || !lc->nsamples || !lc->exptimes || !lc->epids || !obs || !sigma || !lnl)
-        return set_error(RR_EINVAL, "rr_lnlike: null array");
+    LnlArgs s;
+    int rc = lnl_prepare("rr_lnlike", precision, tab, lc, pv->npv, pv->t0cols, ld->law, obs, lnl, grad, s);
+    if (rc || pv->npv == 0) return rc;
+    if (!sigma) return set_error(RR_EINVAL, "rr_lnlike: null array");
     if (!pv->k || !pv->t0 || !pv->p || !pv->a || !pv->inc || !pv->e || !pv->w)
         return set_error(RR_EINVAL, "rr_lnlike: null parameter array");
+    auto vec = [](const double* p, long long stride) { return LnlVec{p, stride, 0.0}; };
+    s.k = vec(pv->k, 1); s.t0 = vec(pv->t0, pv->t0cols); s.p = vec(pv->p, 1); s.a = vec(pv->a, 1);
+    s.inc = vec(pv->inc, 1); s.e = vec(pv->e, 1); s.w = vec(pv->w, 1); s.sigma = vec(sigma, 1);
+    s.c0 = vec(ld->ldc, ld->nldc); s.c1 = vec(ld->ldc + 1, ld->nldc);
+    return lnl_dispatch(precision, s, true, (hipStream_t)stream);
+}
+
+size_t rr_lnlike_workspace_bytes(int npv, int npt, int ng) {
+    if (npv < 0 || npt < 0 || ng < 2) return 0;
+    const size_t ntile = ((size_t)npt + kLnlTile - 1) / kLnlTile;
+    size_t b = align_up((size_t)npv * sizeof(LnlRec), 256);
+    b += align_up((size_t)npv * lnl_rows_bytes<double, true>(ng), 256);
+    b += align_up(ntile * sizeof(double), 256);
+    return b + align_up((size_t)npv * lnl_split(npv, npt) * 8 * sizeof(double), 256);
+}
+
+int rr_lnlike_vec(int precision, const rr_table* tab, const rr_lcdata* lc, int npv, int t0cols, const rr_vec* par,
+                  int law, const rr_vec* ldc, const double* obs, const rr_vec* sigma, void* workspace,
+                  size_t workspace_bytes, double* lnl, double* grad, void* stream) {
+    if (!tab || !lc || !par || !ldc || !sigma) return set_error(RR_EINVAL, "rr_lnlike_vec: null descriptor");
     LnlArgs s;
-    s.times = lc->times; s.obs = obs; s.sigma = sigma; s.nsamples = lc->nsamples; s.exptimes = lc->exptimes;
-    s.epids = lc->epids;
-    s.k = pv->k; s.t0 = pv->t0; s.p = pv->p; s.a = pv->a; s.inc = pv->inc; s.e = pv->e; s.w = pv->w;
-    s.law = ld->law; s.nldc = ld->nldc; s.ldc = ld->ldc;
-    s.W = tab->weights; s.mu = tab->mu; s.lnl = lnl; s.grad = grad;
-    s.npv = npv; s.npt = npt; s.kcols = pv->kcols; s.t0cols = pv->t0cols; s.nk = tab->nk; s.ng = tab->ng;
-    s.nz = tab->nz; s.kmin = tab->kmin; s.kmax = tab->kmax; s.dk = tab->dk; s.dg = tab->dg;
-    hipStream_t st = (hipStream_t)stream;
-    if (precision == RR_MIXED) hipLaunchKernelGGL(rr_lnlike_kernel<float>, dim3(npv), dim3(kLnlThreads), 0, st, s);
-    else hipLaunchKernelGGL(rr_lnlike_kernel<double>, dim3(npv), dim3(kLnlThreads), 0, st, s);
-    return check_launch("rr_lnlike_kernel");
+    int rc = lnl_prepare("rr_lnlike_vec", precision, tab, lc, npv, t0cols, law, obs, lnl, grad, s);
+    if (rc || npv == 0) return rc;
+    const size_t need = rr_lnlike_workspace_bytes(npv, lc->npt, tab->ng);
+    if (!workspace || workspace_bytes < need)
+        return set_error(RR_EINVAL, "rr_lnlike_vec: workspace of %zu bytes needed, got %zu", need, workspace_bytes);
+    auto vec = [](const rr_vec& v) { return LnlVec{v.ptr, (long long)v.stride, v.value}; };
+    s.k = vec(par[0]); s.t0 = vec(par[1]); s.p = vec(par[2]); s.a = vec(par[3]); s.inc = vec(par[4]);
+    s.e = vec(par[5]); s.w = vec(par[6]); s.c0 = vec(ldc[0]); s.c1 = vec(ldc[1]); s.sigma = vec(*sigma);
+    s.sorted = (lc->sorted & RR_SORTED_RUNS) != 0;
+    s.nsplit = lnl_split(npv, lc->npt);
+    s.per = (s.ntile + s.nsplit - 1) / s.nsplit;
+    char* ws = (char*)workspace;
+    s.rec = (LnlRec*)ws;
+    ws += align_up((size_t)npv * sizeof(LnlRec), 256);
+    s.rows = ws;
+    ws += align_up((size_t)npv * lnl_rows_bytes<double, true>(tab->ng), 256);
+    s.tsum = (double*)ws;
+    ws += align_up((size_t)s.ntile * sizeof(double), 256);
+    s.part = (double*)ws;
+    return lnl_dispatch(precision, s, false, (hipStream_t)stream);
 }
 
 }  // extern "C"

@@ -75,6 +75,18 @@ __device__ __forceinline__ double table_poly(ConstTable t, double x) {
     return q;
 }
 
+// sqrt(x) and 1 / sqrt(x) together, x > 0.
+__device__ __forceinline__ void f64_sqrt_rsqrt(double x, double& s, double& r) {
+    const double y = __builtin_amdgcn_rsq(x);
+    double g = x * y, h = 0.5 * y;
+    const double e = fma(-h, g, 0.5);
+    g = fma(g, e, g);
+    h = fma(h, e, h);
+    s = fma(fma(-g, g, x), h, g);
+    r = h + h;
+    r = fma(fma(-s, r, 1.0), r, r);
+}
+
 // log(x) in FP64: x = m 2^e with m in [sqrt(1/2), sqrt 2), log m = 2 atanh(s) with
 // s = (m - 1) / (m + 1), atanh(s) / s an interpolating polynomial in s^2 at Chebyshev
 // nodes (relative error 1.5e-18).
@@ -132,6 +144,8 @@ __device__ __forceinline__ float atan2_ypos_f(float y, float x) {
 // atan2 with y >= 0 (the kite angles): libm in FP64, the polynomial in FP32.
 __device__ __forceinline__ double d_atan2_ypos(double y, double x) { return atan2(y, x); }
 __device__ __forceinline__ float d_atan2_ypos(float y, float x) { return atan2_ypos_f(y, x); }
+__device__ __forceinline__ double d_fma(double a, double b, double c) { return fma(a, b, c); }
+__device__ __forceinline__ float d_fma(float a, float b, float c) { return fmaf(a, b, c); }
 __device__ __forceinline__ double d_abs(double x) { return fabs(x); }
 __device__ __forceinline__ float d_abs(float x) { return fabsf(x); }
 __device__ __forceinline__ double d_max(double a, double b) { return fmax(a, b); }
@@ -191,14 +205,20 @@ __device__ __forceinline__ void ccia_kite3(T r1, T r2, T b, T& area, T& kap0, T&
 // Lens area of the unit disk and a disk of radius k at separation z, |1 - k| < z < 1 + k:
 // the kite form above, in FP64 with the arctangent and square root of f64_*.  Products
 // and sums are fused where written, so every kernel that calls it rounds alike.
-__device__ __forceinline__ double lens_area_f64(double k, double z) {
+__device__ __forceinline__ double lens_f64(double k, double z, double& kap0, double& akite) {
 #pragma clang fp contract(off)
     const double hi = fmax(1.0, k), lo = fmin(1.0, k);
     const double x = fmax(hi, z), c = fmin(lo, z), y = fmax(lo, fmin(hi, z));
-    const double sq = f64_sqrt((x + (y + c)) * (c - (x - y)) * (c + (x - y)) * (x + (y - c)));   // 2 akite
+    const double sq = f64_sqrt((x + (y + c)) * (c - (x - y)) * (c + (x - y)) * (x + (y - c)));
     const double kk = (k - 1.0) * (k + 1.0);
-    const double k1 = f64_atan2_ypos(sq, fma(z, z, -kk)), k0 = f64_atan2_ypos(sq, fma(z, z, kk));
-    return fma(-0.5, sq, fma(k * k, k0, k1));
+    const double k1 = f64_atan2_ypos(sq, fma(z, z, -kk));
+    kap0 = f64_atan2_ypos(sq, fma(z, z, kk));
+    akite = 0.5 * sq;
+    return fma(-0.5, sq, fma(k * k, kap0, k1));
+}
+__device__ __forceinline__ double lens_area_f64(double k, double z) {
+    double kap0, akite;
+    return lens_f64(k, z, kap0, akite);
 }
 __device__ __forceinline__ float lens_area_f32(float k, float z) {
 #pragma clang fp contract(off)
@@ -404,25 +424,19 @@ __device__ __forceinline__ double find_contact_point(double k, int point, const 
 
 // ---- Epoch reduction (model_full.py:88-89) -------------------------------------------
 
-// Exact form: floor((t - t0 + p/2) / p) with an IEEE division, then
-// tc = t - (t0 + epoch*p), with no contraction so each step rounds as in numpy.
-__device__ __forceinline__ double phase_exact(double t, double t0, double p) {
-#pragma clang fp contract(off)
-    const double epoch = floor((t - t0 + 0.5 * p) / p);
-    return t - (t0 + epoch * p);
-}
-
-// Division-free form for the mixed path: epoch from a multiply by 1/p, then one
-// correction step so that r = (t - t0 + p/2) - epoch*p lies in [0, p).  It can
-// differ from phase_exact only where the quotient is within rounding of an
-// integer, i.e. at tc = +-p/2, far outside any transit window.
-__device__ __forceinline__ double phase_fast(double t, double t0, double p, double inv_p) {
+// Division-free form of epoch = floor((t - t0 + p/2) / p), tc = t - (t0 + epoch*p): the
+// epoch from a multiply by 1/p, then one correction step so that
+// r = (t - t0 + p/2) - epoch*p lies in [0, p), with no contraction so each step rounds
+// as in numpy.  It can differ from the division only where the quotient is within
+// rounding of an integer, i.e. at tc = +-p/2, far outside any transit window.
+__device__ __forceinline__ double epoch_phase(double t, double t0, double p, double inv_p, double& epoch) {
 #pragma clang fp contract(off)
     const double u = t - t0 + 0.5 * p;
-    double epoch = floor(u * inv_p);
-    const double r = u - epoch * p;
-    epoch += (r < 0.0) ? -1.0 : ((r >= p) ? 1.0 : 0.0);
-    return t - (t0 + epoch * p);
+    double ep = floor(u * inv_p);
+    const double r = u - ep * p;
+    ep += (r < 0.0) ? -1.0 : ((r >= p) ? 1.0 : 0.0);
+    epoch = ep;
+    return t - (t0 + ep * p);
 }
 
 // ---- Limb-darkening laws; models/numba/ldmodels.py:22-139 -----------------------------

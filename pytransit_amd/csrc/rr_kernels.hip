@@ -884,17 +884,6 @@ constexpr int kPartQ = 2 * kThreads;                  // queued partial-overlap 
 constexpr int kCtxWords = 5;  // per-point context of a multi-light-curve chunk (FP32)
 
 
-// Epoch and phase of time t (the division-free form of model_full.py:88-89).
-__device__ __forceinline__ double phase_of(double t, double t0, double p, double inv_p, double& epoch) {
-#pragma clang fp contract(off)
-    const double u = t - t0 + 0.5 * p;
-    double ep = floor(u * inv_p);
-    const double r = u - ep * p;
-    ep += (r < 0.0) ? -1.0 : ((r >= p) ? 1.0 : 0.0);
-    epoch = ep;
-    return t - (t0 + ep * p);
-}
-
 // t0 + epoch * p, the subtrahend of model_full.py:89, rounded as the reference does.
 __device__ __forceinline__ double epoch_base(double t0, double epoch, double p) {
 #pragma clang fp contract(off)
@@ -1312,8 +1301,8 @@ __device__ __forceinline__ void flux_body(const FluxArgs& f, int pv, int tile) {
     const PointCtx ctx0 = point_ctx0(f, r);
     const double p = r.p, inv_p = r.inv_p;
     double ea0, eb0;
-    const double tca0 = phase_of(t_first, ctx0.t0v, p, inv_p, ea0);
-    const double tcb0 = phase_of(t_last, ctx0.t0v, p, inv_p, eb0);
+    const double tca0 = epoch_phase(t_first, ctx0.t0v, p, inv_p, ea0);
+    const double tcb0 = epoch_phase(t_last, ctx0.t0v, p, inv_p, eb0);
     const bool one_ctx = kFast && (f.nlc == 1 || f.one_window);
     const bool skip = (!rec_ok) | (one_ctx & tile_outside(tca0, tcb0, ea0, eb0, ctx0));  // no short circuit
     if (skip) {
@@ -1376,8 +1365,8 @@ __device__ __forceinline__ void flux_body(const FluxArgs& f, int pv, int tile) {
                 double ea = ea0, eb = eb0;
                 if (!one_ctx) {
                     c = point_ctx(f, r, pv, la);
-                    const double tca = phase_of(t_first, c.t0v, p, inv_p, ea);
-                    const double tcb = phase_of(t_last, c.t0v, p, inv_p, eb);
+                    const double tca = epoch_phase(t_first, c.t0v, p, inv_p, ea);
+                    const double tcb = epoch_phase(t_last, c.t0v, p, inv_p, eb);
                     if (tile_outside(tca, tcb, ea, eb, c)) {
                         wave_fill<Real>(out, tbase, last + 1 - tbase, Real(1), wl);
                         return;
@@ -1427,8 +1416,8 @@ __device__ __forceinline__ void flux_body(const FluxArgs& f, int pv, int tile) {
                 all_out = false;
                 if (one_lc) {
                     double ef, el;
-                    const double tcf = phase_of(tf[m], c.t0v, p, inv_p, ef);
-                    const double tcl = phase_of(tl[m], c.t0v, p, inv_p, el);
+                    const double tcf = epoch_phase(tf[m], c.t0v, p, inv_p, ef);
+                    const double tcl = epoch_phase(tl[m], c.t0v, p, inv_p, el);
                     all_out = (ef == el) ? (tcl < c.lo || tcf > c.hi)
                                          : ((el == ef + 1.0) ? (tcf > c.hi && tcl < c.lo) : false);
                     // the epoch is monotone in t: equal at both ends, equal throughout
@@ -1459,7 +1448,7 @@ __device__ __forceinline__ void flux_body(const FluxArgs& f, int pv, int tile) {
                     } else {
                         if (!one_lc) cc = ctx_of(min(max(f.lcids[it], 0), f.nlc - 1));
                         double ep;
-                        tc = phase_of(tv[j], cc.t0v, p, inv_p, ep);
+                        tc = epoch_phase(tv[j], cc.t0v, p, inv_p, ep);
                     }
                     inw = (cc.lo <= tc) && (tc <= cc.hi);
                     if (!inw) out[it] = Real(1);
@@ -1480,7 +1469,7 @@ __device__ __forceinline__ void flux_body(const FluxArgs& f, int pv, int tile) {
                     const int ilc = f.nlc == 1 ? 0 : min(max(f.lcids[it], 0), f.nlc - 1);
                     const PointCtx c = point_ctx(f, r, pv, ilc);
                     double ep;
-                    const double tc = phase_of(tv[j], c.t0v, p, inv_p, ep);
+                    const double tc = epoch_phase(tv[j], c.t0v, p, inv_p, ep);
                     inw = (c.lo <= tc) && (tc <= c.hi);
                     if (!inw) out[it] = Real(1);
                 }
@@ -1544,7 +1533,7 @@ __device__ __forceinline__ void flux_body(const FluxArgs& f, int pv, int tile) {
             if (wl < cp && wl < n - (c0 + cp)) tnext = f.times[tbase + s_q[c0 + cp + wl]];
             if (wl < cn) {
                 double ep;
-                const double tc = phase_of(tcur, c.t0v, p, inv_p, ep);
+                const double tc = epoch_phase(tcur, c.t0v, p, inv_p, ep);
                 if (kMixed) s_tcf[wl] = (float)tc;
                 else s_tc[wl] = tc;
             }
@@ -1657,7 +1646,7 @@ __device__ __forceinline__ void flux_body(const FluxArgs& f, int pv, int tile) {
                 const int ilc = min(max(f.lcids[it], 0), f.nlc - 1);
                 const PointCtx c = ctx_of(ilc);
                 double ep;
-                s_ptc[wl] = (float)phase_of(f.times[it], c.t0v, p, inv_p, ep);
+                s_ptc[wl] = (float)epoch_phase(f.times[it], c.t0v, p, inv_p, ep);
                 s_pk[wl] = (float)c.kk;
                 s_pext[wl] = (float)c.ext;
                 s_pist[wl] = (float)(1.0 / c.ist);
@@ -1722,7 +1711,7 @@ __device__ __forceinline__ void flux_body(const FluxArgs& f, int pv, int tile) {
         const int ilc = f.nlc == 1 ? 0 : min(max(f.lcids[it], 0), f.nlc - 1);
         const PointCtx c = ctx_of(ilc);
         double ep;
-        const double tc = phase_of(f.times[it], c.t0v, p, inv_p, ep);
+        const double tc = epoch_phase(f.times[it], c.t0v, p, inv_p, ep);
         const size_t row = ((size_t)pv * f.npb + c.ipb) * f.ng;
         const Real* lrow = f.row_lds ? s_row : (kMixed ? (const Real*)f.ldm32 : (const Real*)f.ldm64) + row;
         const RrItem<Real> I = rr_item<Real>(c.ext, c.ns, c.kk, c.ist, lrow);

@@ -59,17 +59,6 @@ struct WfWindow {
 constexpr int kWfThreads = 256;
 constexpr int kWfCap = 1024;    // (point, sample) items of a chunk
 
-// Time from the nearest conjunction after the division-free epoch reduction.
-__device__ __forceinline__ double wf_phase(double t, double t0, double p, double inv_p, double& epoch) {
-#pragma clang fp contract(off)
-    const double u = t - t0 + 0.5 * p;
-    double ep = floor(u * inv_p);
-    const double r = u - ep * p;
-    ep += (r < 0.0) ? -1.0 : ((r >= p) ? 1.0 : 0.0);
-    epoch = ep;
-    return t - (t0 + ep * p);
-}
-
 // base[0 .. n) = v by the block: 16-byte vectors from the first aligned element on.
 template <typename T>
 __device__ __forceinline__ void block_fill(T* base, int n, T v) {
@@ -141,8 +130,8 @@ __device__ __forceinline__ void window_flux_body(const typename M::Args& f) {
             if (!kMulti || d.one_window || la == lc_of(i1)) {
                 const WfWindow w = kMulti ? M::window(f, c, pv, la) : w0;
                 double ea, eb;
-                const double ta = wf_phase(tf, w.t0, c.p, c.inv_p, ea);
-                const double tb = wf_phase(tl, w.t0, c.p, c.inv_p, eb);
+                const double ta = epoch_phase(tf, w.t0, c.p, c.inv_p, ea);
+                const double tb = epoch_phase(tl, w.t0, c.p, c.inv_p, eb);
                 outside = ea == eb ? (tb < w.lo || ta > w.hi) : (eb == ea + 1.0 && ta > w.hi && tb < w.lo);
             }
         }
@@ -171,7 +160,7 @@ __device__ __forceinline__ void window_flux_body(const typename M::Args& f) {
             if (it < cnt) {
                 const WfWindow w = kMulti ? M::window(f, c, pv, lc_of(it)) : w0;
                 double ep;
-                const double tc = wf_phase(tv[j], w.t0, c.p, c.inv_p, ep);
+                const double tc = epoch_phase(tv[j], w.t0, c.p, c.inv_p, ep);
                 inw = w.lo <= tc && tc <= w.hi;
                 if (!inw) out[it] = fill;
             }
@@ -241,7 +230,7 @@ __device__ __forceinline__ void window_flux_body(const typename M::Args& f) {
                 s_ctx[tid] = M::item(f, c, pv, ilc);
             }
             double ep;
-            s_tc[tid] = wf_phase(d.times[base + it], w.t0, c.p, c.inv_p, ep);
+            s_tc[tid] = epoch_phase(d.times[base + it], w.t0, c.p, c.inv_p, ep);
         }
         __syncthreads();
         auto point_of = [&](int i) {

@@ -30,7 +30,7 @@ from numpy import isscalar, linspace, ndarray, pi, sqrt, zeros
 from scipy.integrate import trapezoid
 
 from . import _lib
-from ._lib import LD_LAW_IDS, RRLcData, RRLd, RRParams, RRTable, check, ptr, stream_handle
+from ._lib import LD_LAW_IDS, RRLcData, RRLd, RRParams, RRTable, RRVec, check, ptr, stream_handle
 from .ldmodel import LDModel
 from .transitmodel import TransitModel
 
@@ -44,6 +44,22 @@ def _as_dev(x, device, dtype=torch.float64) -> torch.Tensor:
     if isinstance(x, torch.Tensor):
         return x.to(device=device, dtype=dtype).contiguous()
     return torch.as_tensor(np.ascontiguousarray(np.asarray(x, dtype=np.float64)), device=device).to(dtype)
+
+
+def _vec_in_place(x, npv, device):
+    """The RRVec of one value per pv that can be read where it is: a number, or a
+    float64 tensor on ``device`` with one value or one per pv (any stride).  None for
+    everything else."""
+    if isinstance(x, (int, float)):
+        return RRVec(0, 0, float(x))
+    if not (isinstance(x, torch.Tensor) and x.dtype == torch.float64 and x.device == device):
+        return None
+    n = x.numel()
+    if n == 1:
+        return RRVec(x.data_ptr(), 0, 0.0)
+    if n == npv and (x.dim() == 1 or (x.dim() == 2 and x.shape[1] == 1)):
+        return RRVec(x.data_ptr(), x.stride(0), 0.0)
+    return None
 
 
 def _shape_of(x):
@@ -385,32 +401,50 @@ class RoadRunnerModel(TransitModel):
             raise ValueError('lnlike supports one light curve')
         if self.ldname not in ('quadratic', 'power-2'):
             raise ValueError("lnlike supports the 'quadratic' and 'power-2' laws")
-        npv, k, t0, (p, a, inc, e, w) = self._params(k, t0, p, a, i, e, w, device)
-        if k.shape[1] != 1:
-            raise ValueError('lnlike needs one radius ratio per parameter vector')
-        if self.epids.max() >= t0.shape[1]:
-            raise ValueError(f"t0 has {t0.shape[1]} columns but the epoch indices go up to {self.epids.max()}")
-        ld, _keep = self._ld_descriptor(ldc, npv, 1, device)
+        npv = 1 if isscalar(p) else _size_of(p)
+        vecs = [_vec_in_place(x, npv, device) for x in (k, t0, p, a, i, e, w)]
+        keep = [k, t0, p, a, i, e, w]
+        t0cols = 1
+        if any(v is None for v in vecs):
+            # other shapes, host arrays or types: contiguous device copies
+            npv, k, t0, (p, a, inc, e, w) = self._params(k, t0, p, a, i, e, w, device)
+            if k.shape[1] != 1:
+                raise ValueError('lnlike needs one radius ratio per parameter vector')
+            t0cols = t0.shape[1]
+            keep = [k, t0, p, a, inc, e, w]
+            vecs = [RRVec(ptr(x), x.stride(0), 0.0) for x in keep]
+        if self.epids.max() >= t0cols:
+            raise ValueError(f"t0 has {t0cols} columns but the epoch indices go up to {self.epids.max()}")
+        if (isinstance(ldc, torch.Tensor) and ldc.device == device and ldc.dtype == torch.float64 and ldc.dim() == 3
+                and ldc.shape[0] in (1, npv) and ldc.shape[1] == 1 and ldc.shape[2] >= 2):
+            c, cs, cc = ldc, (ldc.stride(0) if ldc.shape[0] > 1 else 0), ldc.stride(2)
+        else:
+            ld, _keep = self._ld_descriptor(ldc, npv, 1, device)
+            c, cs, cc = _keep[0], ld.nldc, 1
         obs = _as_dev(obs, device).reshape(-1)
         if obs.numel() != self.npt:
             raise ValueError(f'obs has {obs.numel()} values, the data have {self.npt} times')
-        sig = _as_dev(sigma, device).reshape(-1)
-        if sig.numel() not in (1, npv):
-            raise ValueError('sigma must be a scalar or one value per parameter vector')
-        sig = sig.expand(npv).contiguous()
+        sv = _vec_in_place(sigma, npv, device)
+        if sv is None:
+            sigma = _as_dev(sigma, device).reshape(-1)
+            if sigma.numel() not in (1, npv):
+                raise ValueError('sigma must be a scalar or one value per parameter vector')
+            sv = RRVec(ptr(sigma), 1 if sigma.numel() > 1 else 0, 0.0)
         tab, _k = self._table(device)
         d = self._device_data(device)
-        lc = RRLcData(npt=self.npt, nlc=1, npb=1, nep=t0.shape[1], sorted=int(d['sorted']),
+        lc = RRLcData(npt=self.npt, nlc=1, npb=1, nep=t0cols, sorted=int(d['sorted']),
                       uniform_nsamples=d['uniform_ns'], times=ptr(d['times']), lcids=ptr(d['lcids']),
                       pbids=ptr(d['pbids']), epids=ptr(d['epids']), nsamples=ptr(d['nsamples']),
                       exptimes=ptr(d['exptimes']))
-        prm = RRParams(npv=npv, kcols=1, t0cols=t0.shape[1], pad_=0, k=ptr(k), t0=ptr(t0), p=ptr(p), a=ptr(a),
-                       inc=ptr(inc), e=ptr(e), w=ptr(w))
         lnl = torch.empty(npv, dtype=torch.float64, device=device)
         g = torch.empty((npv, 7), dtype=torch.float64, device=device) if grad else None
+        nbytes = lib.rr_lnlike_workspace_bytes(npv, self.npt, self.ng)
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=device)
         byref = _lib.ctypes.byref
-        check(lib.rr_lnlike(_PRECISIONS[self.precision], byref(tab), byref(lc), byref(prm), byref(ld), ptr(obs),
-                            ptr(sig), ptr(lnl), ptr(g), stream_handle(device)))
+        law = LD_LAW_IDS[self.ldname][0]
+        cv = (RRVec * 2)(RRVec(c.data_ptr(), cs, 0.0), RRVec(c.data_ptr() + 8 * cc, cs, 0.0))
+        check(lib.rr_lnlike_vec(_PRECISIONS[self.precision], byref(tab), byref(lc), npv, t0cols, (RRVec * 7)(*vecs), law,
+                                cv, ptr(obs), byref(sv), ptr(ws), nbytes, ptr(lnl), ptr(g), stream_handle(device)))
         return lnl, g
 
 
