@@ -9,11 +9,12 @@
 //   k^2/k_mean^2 (z <= 1 - k_max) or extrapolated linearly in k otherwise.
 //
 // Kernels:
-//   ts_setup_kernel    one 64-lane workgroup per pv (orbit on lanes 0-6, disk integrals)
+//   ts_setup_kernel    8 pvs a 64-lane workgroup (orbit, mean and maximum k, window)
 //   ts_weights_kernel  up to 16 (pv, g) rows per workgroup: the 2-D weight rows at
 //                      k_mean, the lens areas that need arccos evaluated from a
 //                      list on full waves, written transposed W2T[pv][z][g] (FP64
-//                      and FP32, g padded to 16)
+//                      and FP32, g padded to 16); the launch's last workgroups take
+//                      the disk integrals
 //   ts_ldm_tab_mfma_kernel  FP32 MFMA contraction ldm = ldp . W2T for tabulated FP64
 //                      profiles: one 8-wave workgroup per pv, W2T in LDS, each row
 //                      read as 128-byte pieces (16-byte loads, a permuted z order)
@@ -21,12 +22,13 @@
 //                      the shapes the first does not take
 //   ts_ldm_mfma64_kernel the FP64 contraction on v_mfma_f64_16x16x4f64 (W2T in LDS
 //                      when it fits in 128 KB), else ts_ldm_f64_kernel on the VALU
-//   ts_flux_kernel     one lane per time, a workgroup per (pv, 256 times): the FP64
-//                      geometry once per (time, sample), then the passband fan-out
-//                      over chunks of 64 (FP32) or 32 (FP64) LD rows staged in LDS
+//   ts_flux_rows_aligned_kernel, ts_flux_rows_kernel  one sample, whole rows of a pv a
+//                      workgroup
+//   ts_flux_table_kernel  up to 32 samples, any row length: a tile of times of a pv a
+//                      workgroup, its geometry in LDS
+//   ts_flux_kernel     the rest (more samples, very fine g grids)
 //
-// Flux layout [npv, npb, npt]; for one passband row 256 lanes write 1 KB (FP32)
-// contiguously.
+// Flux layout [npv, npb, npt].
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -57,40 +59,43 @@ struct TsArgs {
     const double* W; const double* ze; const double* mu;
     TsRec* rec; double* istar; double* w2_64; float* w2_32; double* ldm64; float* ldm32;
     int npv, npb, npt, nk, ng, ngp, nz, nzp, use_table;
+    int row_split;       // workgroups of a pv in the row forms, each a range of passbands
+    int ldm_split;       // workgroups of a pv in the contraction, each every ldm_split-th group of row tiles
     double kmin, kmax_tab, dk, dg;
 };
 
 constexpr int kTsGroup = 8;
 
 // ---- per-pv setup; model_trspec.py:36-68 ----------------------------------------------
-constexpr int kTsKChunk = 512;   // radius ratios of a pv staged in LDS at a time
-
 __global__ void __launch_bounds__(64) ts_setup_kernel(TsArgs s) {
     __shared__ double s_x[8][8], s_y[8][8], s_c[8][10], s_w[8][2], s_km[8];
-    __shared__ double s_kb[kTsGroup][kTsKChunk];
     const int sub = threadIdx.x / kTsGroup, j = threadIdx.x % kTsGroup;
     const int pv = blockIdx.x * kTsGroup + sub;
     const bool inrange = pv < s.npv;
     const int q = inrange ? pv : 0;
     const double a = s.a[q], e = s.e[q];
     const bool valid = inrange && !(isnan(a) || a <= 1.0 || e < 0.0);
-    // mean as numba's left-to-right sum, and the max, of the pv's row of radius
-    // ratios: the row is loaded into LDS by the pv's 8 lanes (all loads in flight
-    // at once), then summed in order by one lane
+    // the mean and the maximum of the pv's row of radius ratios: each of its 8 lanes
+    // takes every eighth value, eight loads in flight, and the lanes' sums meet by
+    // shuffles (one lane summing 512 values in order took 8 us; the sums agree to
+    // rounding)
     double sum = 0.0, kmx = -INFINITY;
     const double* kr = s.k + (size_t)q * s.npb;
-    for (int c0 = 0; c0 < s.npb; c0 += kTsKChunk) {
-        const int cn = min(kTsKChunk, s.npb - c0);
-        if (inrange)
-            for (int i = j; i < cn; i += kTsGroup) s_kb[sub][i] = kr[c0 + i];
-        __syncthreads();
-        if (inrange && j == 0)
-#pragma unroll 8
-            for (int i = 0; i < cn; ++i) {
-                sum += s_kb[sub][i];
-                kmx = fmax(kmx, s_kb[sub][i]);
-            }
-        __syncthreads();
+    for (int c0 = j; c0 < s.npb; c0 += 8 * kTsGroup) {
+        double v[8];
+#pragma unroll
+        for (int m = 0; m < 8; ++m) v[m] = kr[min(c0 + m * kTsGroup, s.npb - 1)];
+#pragma unroll
+        for (int m = 0; m < 8; ++m) {
+            const bool in = c0 + m * kTsGroup < s.npb;
+            sum += in ? v[m] : 0.0;
+            kmx = in ? fmax(kmx, v[m]) : kmx;
+        }
+    }
+#pragma unroll
+    for (int o = kTsGroup / 2; o > 0; o >>= 1) {
+        sum += __shfl_xor(sum, o, 64);
+        kmx = fmax(kmx, __shfl_xor(kmx, o, 64));
     }
     if (inrange && j == 0) {
         s_km[sub] = sum / s.npb;
@@ -136,9 +141,8 @@ __global__ void __launch_bounds__(64) ts_setup_kernel(TsArgs s) {
     }
 }
 
-// Disk integrals per (pv, pb): given, analytic, or the 200-node trapezoid.
-__global__ void __launch_bounds__(256) ts_istar_kernel(TsArgs s) {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
+// Disk integral of (pv, passband) j: given, analytic, or the 200-node trapezoid.
+__device__ __forceinline__ void ts_istar(const TsArgs& s, int j) {
     if (j >= s.npv * s.npb) return;
     double is;
     if (s.law == RR_LD_TABULATED) {
@@ -182,6 +186,12 @@ __global__ void __launch_bounds__(256) ts_weights_kernel(TsArgs s) {
     __shared__ double s_sum[kTwMaxRows];
     const int R = ts_weight_rows(s.nz), nz = s.nz;
     const int nchunk = (s.ngp + R - 1) / R;
+    // the launch's last blocks take the disk integrals
+    const int wb = s.npv * nchunk;
+    if ((int)blockIdx.x >= wb) {
+        ts_istar(s, (blockIdx.x - wb) * blockDim.x + threadIdx.x);
+        return;
+    }
     const int pv = blockIdx.x / nchunk;
     const int g0 = (blockIdx.x - pv * nchunk) * R;
     const int nr = min(R, s.ngp - g0);
@@ -278,45 +288,52 @@ __device__ __forceinline__ double ts_profile(const TsArgs& s, int pv, int pb, in
 // A rows are passbands, B columns are g.  W2T of the pv sits in LDS with a padded
 // row stride so the 16 lanes reading one k hit distinct banks.
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
-constexpr int kMfmaK = 128;   // k per register-resident A fragment
+
+// LDS row stride of W2T: a 16-byte multiple, 4 mod 8 floats, so that the four z rows of
+// an MFMA step are in distinct banks.
+__host__ __device__ inline int ts_tab_ldb(int ngp) { return ngp + ((4 - ngp % 8) + 8) % 8; }
 
 template <bool kTab>
 __global__ void __launch_bounds__(256) ts_ldm_mfma_kernel(TsArgs s) {
-    extern __shared__ float lds_b[];  // [nzp][ngp + 1]
-    const int pv = blockIdx.x;
-    const int ldb = s.ngp + 1;
-    for (int i = threadIdx.x; i < s.nzp * s.ngp; i += blockDim.x) {
-        const int iz = i / s.ngp, ig = i - iz * s.ngp;
-        lds_b[iz * ldb + ig] = s.w2_32[(size_t)pv * s.nzp * s.ngp + i];
+    extern __shared__ float lds_b[];  // [nzp][ldb]
+    const int pv = blockIdx.x / s.ldm_split, part = blockIdx.x - pv * s.ldm_split;
+    const int ldb = ts_tab_ldb(s.ngp);
+    const f32x4_t* w2 = (const f32x4_t*)(s.w2_32 + (size_t)pv * s.nzp * s.ngp);
+#pragma unroll 4
+    for (int i = threadIdx.x; i < s.nzp * s.ngp / 4; i += 256) {
+        const int iz = 4 * i / s.ngp;
+        *(f32x4_t*)(lds_b + iz * ldb + 4 * i - iz * s.ngp) = w2[i];
     }
     __syncthreads();
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int li = lane & 15, lk = lane >> 4;
     const int nrt = (s.npb + 15) / 16, nct = s.ngp / 16;
-    for (int rt = wave; rt < nrt; rt += 4) {
+    for (int rt = part * 4 + wave; rt < nrt; rt += 4 * s.ldm_split) {
         const int pb = rt * 16 + li;
         const bool row_ok = pb < s.npb;
         for (int ct0 = 0; ct0 < nct; ct0 += 8) {
             f32x4_t acc[8];
 #pragma unroll
             for (int c = 0; c < 8; ++c) acc[c] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-            for (int k0 = 0; k0 < s.nzp; k0 += kMfmaK) {
-                float afrag[kMfmaK / 4];
+            // four steps' profile values at a time, their loads in flight together
+            constexpr int kU = 4;
+            for (int k0 = 0; k0 < s.nzp; k0 += 4 * kU) {
+                float a[kU];
 #pragma unroll
-                for (int st = 0; st < kMfmaK / 4; ++st) {
-                    const int iz = k0 + st * 4 + lk;
-                    afrag[st] = (row_ok && iz < s.nz) ? (float)ts_profile<kTab>(s, pv, pb, iz) : 0.0f;
+                for (int u = 0; u < kU; ++u) {
+                    const int iz = k0 + 4 * u + lk;
+                    a[u] = (row_ok && iz < s.nz) ? (float)ts_profile<kTab>(s, pv, pb, iz) : 0.0f;
                 }
 #pragma unroll
-                for (int st = 0; st < kMfmaK / 4; ++st) {
-                    const int iz = k0 + st * 4 + lk;
-                    if (k0 + st * 4 >= s.nzp) break;
+                for (int u = 0; u < kU; ++u) {
+                    if (k0 + 4 * u >= s.nzp) break;
+                    const int iz = k0 + 4 * u + lk;
 #pragma unroll
                     for (int c = 0; c < 8; ++c) {
                         const int ct = ct0 + c;
                         if (ct < nct) {
                             const float b = lds_b[iz * ldb + ct * 16 + li];
-                            acc[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(afrag[st], b, acc[c], 0, 0, 0);
+                            acc[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u], b, acc[c], 0, 0, 0);
                         }
                     }
                 }
@@ -350,24 +367,27 @@ constexpr int kTabMfmaThreads = 512;
 constexpr int kTabMfmaMaxJ = 8;    // z groups of 16: nz <= 128
 constexpr int kTabMfmaMaxCt = 8;   // g tiles of 16: ngp <= 128
 
-__host__ __device__ inline int ts_tab_ldb(int ngp) { return ngp + ((4 - ngp % 8) + 8) % 8; }
-
 template <int NCT>
 __global__ void __launch_bounds__(kTabMfmaThreads) ts_ldm_tab_mfma_kernel(TsArgs s) {
     extern __shared__ float lds_t[];  // [nz16][ldb]
-    const int pv = blockIdx.x;
+    const int pv = blockIdx.x / s.ldm_split, part = blockIdx.x - pv * s.ldm_split;
     const int ldb = ts_tab_ldb(s.ngp);
     const int nj = (s.nz + 15) / 16, nz16 = nj * 16;
-    for (int i = threadIdx.x; i < nz16 * s.ngp; i += blockDim.x) {
-        const int iz = i / s.ngp, ig = i - iz * s.ngp;
-        lds_t[iz * ldb + ig] = iz < s.nzp ? s.w2_32[(size_t)pv * s.nzp * s.ngp + i] : 0.0f;
+    // (ngp a multiple of 16 and ldb of 4: 16-byte pieces of one row)
+    const f32x4_t* w2 = (const f32x4_t*)(s.w2_32 + (size_t)pv * s.nzp * s.ngp);
+#pragma unroll 4
+    for (int i = threadIdx.x; i < nz16 * s.ngp / 4; i += kTabMfmaThreads) {
+        const int iz = 4 * i / s.ngp;
+        const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+        const f32x4_t v = iz < s.nzp ? w2[i] : zero;
+        *(f32x4_t*)(lds_t + iz * ldb + 4 * i - iz * s.ngp) = v;
     }
     __syncthreads();
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int li = lane & 15, lk = lane >> 4;
     const int nrt = (s.npb + 15) / 16;
     constexpr int kWaves = kTabMfmaThreads / 64;
-    for (int rt = wave; rt < nrt; rt += kWaves) {
+    for (int rt = part * kWaves + wave; rt < nrt; rt += kWaves * s.ldm_split) {
         const int pb = rt * 16 + li;
         const bool row_ok = pb < s.npb;
         const double* arow = s.ldp_in + ((size_t)pv * s.npb + (row_ok ? pb : 0)) * s.nz;
@@ -430,33 +450,49 @@ constexpr size_t kMfma64MaxLds = 128 * 1024;
 template <bool kTab>
 __global__ void __launch_bounds__(kMfma64Threads) ts_ldm_mfma64_kernel(TsArgs s) {
     extern __shared__ double lds_b64[];  // [nzp][ngp + 1]
-    const int pv = blockIdx.x;
+    const int pv = blockIdx.x / s.ldm_split, part = blockIdx.x - pv * s.ldm_split;
     const int ldb = s.ngp + 1;
-    for (int i = threadIdx.x; i < s.nzp * s.ngp; i += blockDim.x) {
-        const int iz = i / s.ngp, ig = i - iz * s.ngp;
-        lds_b64[iz * ldb + ig] = s.w2_64[(size_t)pv * s.nzp * s.ngp + i];
+    // (ngp a multiple of 16: pairs of one row, several loads in flight)
+    const f64x2_t* w2 = (const f64x2_t*)(s.w2_64 + (size_t)pv * s.nzp * s.ngp);
+#pragma unroll 4
+    for (int i = threadIdx.x; i < s.nzp * s.ngp / 2; i += kMfma64Threads) {
+        const f64x2_t v = w2[i];
+        const int iz = 2 * i / s.ngp, o = iz * ldb + 2 * i - iz * s.ngp;
+        lds_b64[o] = v.x;
+        lds_b64[o + 1] = v.y;
     }
     __syncthreads();
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int li = lane & 15, lk = lane >> 4;
     const int nrt = (s.npb + 15) / 16, nct = s.ngp / 16;
     constexpr int kWaves = kMfma64Threads / 64;
-    for (int rt = wave; rt < nrt; rt += kWaves) {
+    for (int rt = part * kWaves + wave; rt < nrt; rt += kWaves * s.ldm_split) {
         const int pb = rt * 16 + li;
         const bool row_ok = pb < s.npb;
         for (int ct0 = 0; ct0 < nct; ct0 += 8) {
             f64x4_t acc[8];
 #pragma unroll
             for (int c = 0; c < 8; ++c) acc[c] = (f64x4_t){0.0, 0.0, 0.0, 0.0};
-            for (int k0 = 0; k0 < s.nzp; k0 += 4) {
-                const int iz = k0 + lk;
-                const double a = (row_ok && iz < s.nz) ? ts_profile<kTab>(s, pv, pb, iz) : 0.0;
+            // four steps' profile values at a time, their loads in flight together
+            constexpr int kU = 4;
+            for (int k0 = 0; k0 < s.nzp; k0 += 4 * kU) {
+                double a[kU];
 #pragma unroll
-                for (int c = 0; c < 8; ++c) {
-                    const int ct = ct0 + c;
-                    if (ct < nct) {
-                        const double b = lds_b64[iz * ldb + ct * 16 + li];
-                        acc[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, acc[c], 0, 0, 0);
+                for (int u = 0; u < kU; ++u) {
+                    const int iz = k0 + 4 * u + lk;
+                    a[u] = (row_ok && iz < s.nz) ? ts_profile<kTab>(s, pv, pb, iz) : 0.0;
+                }
+#pragma unroll
+                for (int u = 0; u < kU; ++u) {
+                    if (k0 + 4 * u >= s.nzp) break;
+                    const int iz = k0 + 4 * u + lk;
+#pragma unroll
+                    for (int c = 0; c < 8; ++c) {
+                        const int ct = ct0 + c;
+                        if (ct < nct) {
+                            const double b = lds_b64[iz * ldb + ct * 16 + li];
+                            acc[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[u], b, acc[c], 0, 0, 0);
+                        }
                     }
                 }
             }
@@ -507,9 +543,8 @@ __global__ void __launch_bounds__(256) ts_ldm_f32_kernel(TsArgs s) {
 // ---- flux --------------------------------------------------------------------------
 constexpr int kTsThreads = 256;
 
-// Passbands per LDS chunk: 64 (FP32) / 32 (FP64) with one accumulator per lane,
-// half that when a lane keeps one accumulator per passband of the chunk.
-constexpr int ts_pb_chunk(bool mixed, bool cached) { return cached ? (mixed ? 64 : 32) : (mixed ? 32 : 16); }
+// Passbands per LDS chunk where a lane keeps one accumulator per passband.
+constexpr int ts_pb_chunk(bool mixed) { return mixed ? 32 : 16; }
 
 // Geometry of one (time, sample): the lens at k_mean in FP64 (model_trspec.py:79-84)
 // and the lerp position in g; shared by every passband.
@@ -522,25 +557,31 @@ struct TsGeo {
     bool gz;          // g > 1: the limb-darkening mean is 0
 };
 
+// inv_1pk, inv_dg and inv_ns: the reciprocals of 1 + k_mean, dg and nsamples.
 template <typename Real>
-__device__ __forceinline__ TsGeo<Real> ts_geometry(const TsRec& r, double tc, double ext, int ns, int is,
-                                                   double dg, int ng) {
+__device__ __forceinline__ TsGeo<Real> ts_geometry(const TsRec& r, double tc, double ext, double inv_ns, int is,
+                                                   double inv_1pk, double inv_dg, int ng) {
     TsGeo<Real> o;
     const double km = r.kmean;
-    const double off = ext * ((is + 1 - 0.5) / ns - 0.5);
-    const double z = taylor_z<double>(tc + off, r.c);
+    const double z = sample_z(sample_time(tc, ext, inv_ns, is), r.c);
     double ap0, kap;
-    ccia_kite<double>(1.0, km, z, ap0, kap);
+    if (fabs(1.0 - km) < z && z < 1.0 + km) {
+        double akite;
+        ap0 = lens_f64(km, z, kap, akite);
+    } else {
+        ccia_kite<double>(1.0, km, z, ap0, kap);     // off the disk, inside it, NaN
+    }
     o.inside = z <= 1.0 - r.kmax;
-    const double g = z / (1.0 + km);
+    const double g = z * inv_1pk;
     // lerp position (common.py:225-233, index clamped to ng-2)
     o.gz = g > 1.0;
     o.ig = 0;
     double al = 0.0;
     if (!o.gz) {
-        int ig = (int)floor(g / dg);
+        const double x = g * inv_dg;
+        const int ig = (int)x;
         o.ig = ig > ng - 2 ? ng - 2 : (ig < 0 ? 0 : ig);
-        al = (g - o.ig * dg) / dg;
+        al = x - o.ig;
     }
     o.ra = (Real)al;
     o.rb = (Real)(1.0 - al);
@@ -549,13 +590,7 @@ __device__ __forceinline__ TsGeo<Real> ts_geometry(const TsRec& r, double tc, do
     return o;
 }
 
-// With nsamples <= kTsGeoRegs the geometry of a lane's samples stays in registers,
-// the passbands are the outer loop and a lane owns 16 bytes of consecutive times
-// (4 FP32 or 2 FP64), so a wave stores 1 KB of one passband row per instruction.  Otherwise a lane
-// owns one time, the samples are the outer loop over a chunk of PC accumulators
-// and the geometry is recomputed per chunk.
-constexpr int kTsGeoRegs = 2;
-// times per lane of the cached form: one 16-byte store per passband row
+// times per lane of the row forms: one 16-byte store per passband row
 template <typename Real> constexpr int ts_tpl() { return 16 / (int)sizeof(Real); }
 
 template <typename Real>
@@ -607,6 +642,14 @@ template <typename Real> constexpr int ts_row_max_npt() { return kTsRowThreads *
 
 __host__ __device__ inline size_t ts_rows_lds(int ng, size_t real) { return ((size_t)kTsRowLd * ng + 3 * kTsRowPc) * real; }
 
+// A workgroup's pv and passband range, row_split to a pv.
+__device__ __forceinline__ void ts_row_range(const TsArgs& s, int bid, int& pv, int& qa, int& qb) {
+    pv = bid / s.row_split;
+    const int part = bid - pv * s.row_split, per = (s.npb + s.row_split - 1) / s.row_split;
+    qa = min(part * per, s.npb);
+    qb = min(qa + per, s.npb);
+}
+
 template <typename Real>
 __global__ void __launch_bounds__(kTsRowThreads) ts_flux_rows_kernel(TsArgs s, Real* flux) {
     constexpr int TPL = ts_tpl<Real>();
@@ -617,7 +660,8 @@ __global__ void __launch_bounds__(kTsRowThreads) ts_flux_rows_kernel(TsArgs s, R
     Real* s_kd = s_afac + kTsRowPc;
     Real* s_iist = s_kd + kTsRowPc;
 
-    const int pv = xcd_remap(blockIdx.x, gridDim.x);
+    int pv, qa, qb;      // this workgroup's pv and passbands
+    ts_row_range(s, xcd_remap(blockIdx.x, gridDim.x), pv, qa, qb);
     const int npt = s.npt, nv = npt / TPL;
     const TsRec& r = s.rec[pv];
     Real* out = flux + (size_t)pv * s.npb * npt;
@@ -628,11 +672,13 @@ __global__ void __launch_bounds__(kTsRowThreads) ts_flux_rows_kernel(TsArgs s, R
         vone[j] = Real(1);
     }
     if (!r.good) {
-        for (size_t i = threadIdx.x; i < (size_t)s.npb * nv; i += kTsRowThreads) ts_store(out + i * TPL, vnan, TPL, true);
+        for (size_t i = (size_t)qa * nv + threadIdx.x; i < (size_t)qb * nv; i += kTsRowThreads)
+            ts_store(out + i * TPL, vnan, TPL, true);
         return;
     }
     // the geometry of the thread's times, once, as row coefficients
     const double ext = s.exptimes[0];
+    const double inv_1pk = 1.0 / (1.0 + r.kmean), inv_dg = 1.0 / s.dg;
     int off[NV][TPL];
     Real rb[NV][TPL], ra[NV][TPL], c1[NV][TPL], c2[NV][TPL], c3[NV][TPL];
     bool use[NV][TPL];   // in the window with g <= 1
@@ -659,7 +705,7 @@ __global__ void __launch_bounds__(kTsRowThreads) ts_flux_rows_kernel(TsArgs s, R
                     tc = t - (t0v + ep * r.p);
                 }
                 if ((r.bt1 <= tc) && (tc <= r.bt4)) {
-                    const TsGeo<Real> g = ts_geometry<Real>(r, tc, ext, 1, 0, s.dg, s.ng);
+                    const TsGeo<Real> g = ts_geometry<Real>(r, tc, ext, 1.0, 0, inv_1pk, inv_dg, s.ng);
                     any = true;
                     if (!g.gz) {
                         use[u][j] = true;
@@ -675,8 +721,8 @@ __global__ void __launch_bounds__(kTsRowThreads) ts_flux_rows_kernel(TsArgs s, R
         }
         act[u] = __ballot(any) != 0ull;
     }
-    for (int pb0 = 0; pb0 < s.npb; pb0 += kTsRowPc) {
-        const int npc = min(kTsRowPc, s.npb - pb0);
+    for (int pb0 = qa; pb0 < qb; pb0 += kTsRowPc) {
+        const int npc = min(kTsRowPc, qb - pb0);
         __syncthreads();  // the previous chunk's rows are no longer read
         for (int i = threadIdx.x; i < kTsRowPc * s.ng; i += kTsRowThreads) {
             const int q = i / s.ng, g = i - q * s.ng;   // coalesced global reads along g
@@ -763,12 +809,13 @@ __global__ void __launch_bounds__(kTsRowThreads) ts_flux_rows_aligned_kernel(TsA
     Real* t_a0 = t_rb + npt;
     Real* t_dk = t_a0 + npt;
 
-    const int pv = xcd_remap(blockIdx.x, gridDim.x);
+    int pv, qa, qb;      // this workgroup's pv and passbands
+    ts_row_range(s, xcd_remap(blockIdx.x, gridDim.x), pv, qa, qb);
     const TsRec& r = s.rec[pv];
     float* out = flux + (size_t)pv * s.npb * npt;
     if (!r.good) {
         const f32x4_t vnan = {NAN, NAN, NAN, NAN};
-        for (size_t i = threadIdx.x; i < (size_t)s.npb * nv; i += kTsRowThreads)
+        for (size_t i = (size_t)qa * nv + threadIdx.x; i < (size_t)qb * nv; i += kTsRowThreads)
             __builtin_nontemporal_store(vnan, (f32x4_t*)(out + i * TPL));
         return;
     }
@@ -778,7 +825,7 @@ __global__ void __launch_bounds__(kTsRowThreads) ts_flux_rows_aligned_kernel(TsA
     float st[kTsStageRegs];
     double kq = 0.0, isq = 1.0;
     auto stage_load = [&](int pb0) {
-        const int npc = min(kTsRowPc, s.npb - pb0);
+        const int npc = min(kTsRowPc, qb - pb0);
 #pragma unroll
         for (int m = 0; m < kTsStageRegs; ++m) {
             const int i = threadIdx.x + m * kTsRowThreads;
@@ -791,7 +838,7 @@ __global__ void __launch_bounds__(kTsRowThreads) ts_flux_rows_aligned_kernel(TsA
         }
     };
     auto stage_store = [&](int pb0) {
-        const int npc = min(kTsRowPc, s.npb - pb0);
+        const int npc = min(kTsRowPc, qb - pb0);
 #pragma unroll
         for (int m = 0; m < kTsStageRegs; ++m) {
             const int i = threadIdx.x + m * kTsRowThreads;
@@ -805,6 +852,7 @@ __global__ void __launch_bounds__(kTsRowThreads) ts_flux_rows_aligned_kernel(TsA
         }
     };
     const double ext = s.exptimes[0];
+    const double inv_1pk = 1.0 / (1.0 + r.kmean), inv_dg = 1.0 / s.dg;
     const double t0v = s.t0[pv];
     for (int t = threadIdx.x; t < npt; t += kTsRowThreads) {
         double tc;
@@ -820,7 +868,7 @@ __global__ void __launch_bounds__(kTsRowThreads) ts_flux_rows_aligned_kernel(TsA
         int pk = 0;
         Real ra = Real(0), rb = Real(0), a0 = Real(0), dk = Real(0);
         if ((r.bt1 <= tc) && (tc <= r.bt4)) {
-            const TsGeo<Real> g = ts_geometry<Real>(r, tc, ext, 1, 0, s.dg, s.ng);
+            const TsGeo<Real> g = ts_geometry<Real>(r, tc, ext, 1.0, 0, inv_1pk, inv_dg, s.ng);
             if (!g.gz) {
                 pk = ((g.ig * kTsRowLd) << 2) | (g.inside ? 2 : 0) | 1;
                 ra = g.ra;
@@ -835,16 +883,16 @@ __global__ void __launch_bounds__(kTsRowThreads) ts_flux_rows_aligned_kernel(TsA
         t_a0[t] = a0;
         t_dk[t] = dk;
     }
-    stage_load(0);
+    stage_load(qa);
     // rows P apart start equally far past a 128-byte boundary
     const int gl = npt & -npt;   // lowest set bit of npt
     const int P = kTsLine / (gl < kTsLine ? gl : kTsLine);
-    for (int pb0 = 0; pb0 < s.npb; pb0 += kTsRowPc) {
-        const int npc = min(kTsRowPc, s.npb - pb0);
+    for (int pb0 = qa; pb0 < qb; pb0 += kTsRowPc) {
+        const int npc = min(kTsRowPc, qb - pb0);
         __syncthreads();  // the previous chunk's rows are no longer read (and the table is written)
         stage_store(pb0);
         __syncthreads();
-        if (pb0 + kTsRowPc < s.npb) stage_load(pb0 + kTsRowPc);
+        if (pb0 + kTsRowPc < qb) stage_load(pb0 + kTsRowPc);
         for (int q0 = pb0; q0 < pb0 + min(P, npc); ++q0) {
             // this class's head, and each slot's coefficients from the table
             const int mis = (int)(((uintptr_t)(out + (size_t)q0 * npt) >> 2) & (kTsLine - 1));
@@ -918,11 +966,183 @@ __global__ void __launch_bounds__(kTsRowThreads) ts_flux_rows_aligned_kernel(TsA
     }
 }
 
-template <bool kMixed, bool kCached>
+// ---- any number of samples up to kTsTabSamples: geometry in LDS --------------------------
+//
+// A workgroup of 4 waves takes a tile of T = 64, 128 or 256 times of one pv and a range
+// of passbands.  The geometry of every (time, sample) of the tile goes to LDS once, and
+// the passbands' LD rows pass through LDS in chunks; a wave takes 64 times, one a lane
+// (so its stores are contiguous), and every (4 / (T / 64))-th passband of a chunk.  The
+// form that recomputed the geometry for each chunk of 16 passbands spent most of its
+// time on FP64 arctangents: 100 pv x 203 passbands x 1,237 t, 3 samples, FP64: 172 -> 65
+// us (201 MB written: 29 us at the rate of a fill, 45 as rows of odd length).
+constexpr int kTsTabSamples = 32;
+// passbands of a chunk (FP64: 32 takes 105, 16 takes 100 us at the size above)
+template <typename Real> constexpr int ts_tab_pc() { return sizeof(Real) == 4 ? 32 : 16; }
+constexpr int kTsTabQ = 4;        // passbands a lane takes together
+// LDS stride of one g, a 16-byte multiple off a multiple of all banks
+template <typename Real> constexpr int ts_tab_ld() { return ts_tab_pc<Real>() + 16 / (int)sizeof(Real); }
+
+template <typename Real> struct TsTab { static constexpr int kBytes = 3 * (int)sizeof(Real) + 4; };
+
+// Times of a tile: as many as keep the geometry within 40 KB.
+template <typename Real>
+__host__ __device__ inline int ts_tab_times(int ns) {
+    int t = 256;
+    while (t > 64 && t * ns * TsTab<Real>::kBytes > 40 * 1024) t /= 2;
+    return t;
+}
+template <typename Real>
+__host__ inline size_t ts_tab_lds(int ns, int ng) {
+    const size_t geo = (size_t)ts_tab_times<Real>(ns) * ns * TsTab<Real>::kBytes;
+    return (geo + 15) / 16 * 16 + ((size_t)ts_tab_ld<Real>() * ng + 3 * ts_tab_pc<Real>()) * sizeof(Real);
+}
+
+template <typename Real>
+__global__ void __launch_bounds__(kTsThreads) ts_flux_table_kernel(TsArgs s, Real* flux, int ntiles, int nsplit, int ns) {
+    extern __shared__ __align__(16) unsigned char lds[];
+    __shared__ unsigned s_act;
+    const int T = ts_tab_times<Real>(ns), n = T * ns;
+    Real* t_ra = (Real*)lds;                    // [ns][T]
+    Real* t_a0 = t_ra + n;
+    Real* t_dk = t_a0 + n;
+    int* t_pk = (int*)(t_dk + n);               // interval << 3 | in the window << 2 | inside << 1 | g <= 1
+    constexpr int kLd = ts_tab_ld<Real>(), kPc = ts_tab_pc<Real>();
+    Real* s_l = (Real*)(((uintptr_t)(t_pk + n) + 15) & ~(uintptr_t)15);   // [ng][kLd]
+    Real* s_afac = s_l + (size_t)kLd * s.ng;
+    Real* s_kd = s_afac + kPc;
+    Real* s_f = s_kd + kPc;
+
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int bid = xcd_remap(blockIdx.x, gridDim.x);
+    const int split = bid % nsplit, tile = (bid / nsplit) % ntiles, pv = bid / nsplit / ntiles;
+    const int per = (s.npb + nsplit - 1) / nsplit;
+    const int q0 = split * per, q1 = min(q0 + per, s.npb);
+    const TsRec& r = s.rec[pv];
+    const int nt = min(T, s.npt - tile * T);    // the tile's times
+    Real* out = flux + (size_t)pv * s.npb * s.npt + (size_t)tile * T;
+    auto fill = [&](Real v) {
+        for (int q = q0 + wave; q < q1; q += 4)
+            for (int t = lane; t < nt; t += 64) out[(size_t)q * s.npt + t] = v;
+    };
+    if (!r.good) {
+        fill(Real(NAN));
+        return;
+    }
+    if (tid == 0) s_act = 0u;
+    __syncthreads();
+    // geometry: item i is sample i / T of the tile's time i % T (T is a power of two)
+    const double ext = s.exptimes[0], t0v = s.t0[pv], p = r.p, inv_p = r.inv_p, inv_ns = 1.0 / ns;
+    const double inv_1pk = 1.0 / (1.0 + r.kmean), inv_dg = 1.0 / s.dg;
+    for (int i = tid; i < n; i += kTsThreads) {
+        const int t = i & (T - 1), is = i / T, jt = tile * T + t;
+        int pk = 0;
+        Real ra = Real(0), a0 = Real(0), dk = Real(0);
+        if (jt < s.npt) {
+            double ep;
+            const double tc = epoch_phase(s.times[jt], t0v, p, inv_p, ep);
+            if (r.bt1 <= tc && tc <= r.bt4) {
+                const TsGeo<Real> g = ts_geometry<Real>(r, tc, ext, inv_ns, is, inv_1pk, inv_dg, s.ng);
+                pk = (g.ig << 3) | 4 | (g.inside ? 2 : 0) | (g.gz ? 0 : 1);
+                ra = g.ra;
+                a0 = g.ap0;
+                dk = g.dadk;
+                if (is == 0) atomicOr(&s_act, 1u << (t >> 6));
+            }
+        }
+        t_pk[i] = pk;
+        t_ra[i] = ra;
+        t_a0[i] = a0;
+        t_dk[i] = dk;
+    }
+    __syncthreads();
+    const unsigned act = s_act;                 // bit j: times 64 j .. 64 j + 63 hold a point in the window
+    if (!act) {
+        fill(Real(1));
+        return;
+    }
+    const double km = r.kmean;
+    // a wave stages every fourth row of a chunk, loaded (the first 128 g of each) one
+    // chunk ahead
+    constexpr int kRows = kPc / 4;
+    const Real* ldm = sizeof(Real) == 4 ? (const Real*)s.ldm32 : (const Real*)s.ldm64;
+    Real st[kRows][2];
+    auto stage_load = [&](int pb0) {
+#pragma unroll
+        for (int m = 0; m < kRows; ++m) {
+            const int q = pb0 + wave + 4 * m;
+            const Real* src = ldm + ((size_t)pv * s.npb + q) * s.ng;
+            st[m][0] = q < q1 && lane < s.ng ? src[lane] : Real(0);
+            st[m][1] = q < q1 && lane + 64 < s.ng ? src[lane + 64] : Real(0);
+        }
+    };
+    stage_load(q0);
+    for (int pb0 = q0; pb0 < q1; pb0 += kPc) {
+        const int npc = min(kPc, q1 - pb0);
+        __syncthreads();  // the previous chunk's rows are no longer read
+#pragma unroll
+        for (int m = 0; m < kRows; ++m) {
+            const int q = wave + 4 * m;
+            if (lane < s.ng) s_l[lane * kLd + q] = st[m][0];
+            if (lane + 64 < s.ng) s_l[(lane + 64) * kLd + q] = st[m][1];
+            for (int g = lane + 128; g < s.ng; g += 64)
+                s_l[g * kLd + q] = q < npc ? ldm[((size_t)pv * s.npb + pb0 + q) * s.ng + g] : Real(0);
+        }
+        if (pb0 + kPc < q1) stage_load(pb0 + kPc);
+        if (tid < kPc) {
+            const size_t j = (size_t)pv * s.npb + pb0 + min(tid, npc - 1);
+            const double kq = s.k[j];
+            s_afac[tid] = (Real)(kq * kq / (km * km));
+            s_kd[tid] = (Real)(kq - km);
+            s_f[tid] = (Real)(inv_ns / s.istar[j]);
+        }
+        __syncthreads();
+        for (int q = wave * kTsTabQ; q < npc; q += 4 * kTsTabQ) {
+            Real afac[kTsTabQ], kd[kTsTabQ], f[kTsTabQ];
+#pragma unroll
+            for (int j = 0; j < kTsTabQ; ++j) {
+                afac[j] = s_afac[q + j];
+                kd[j] = s_kd[q + j];
+                f[j] = s_f[q + j];
+            }
+            Real* o = out + (size_t)(pb0 + q) * s.npt;
+            for (int t0 = 0; t0 < nt; t0 += 64) {
+                const int t = t0 + lane;
+                Real v[kTsTabQ];
+#pragma unroll
+                for (int j = 0; j < kTsTabQ; ++j) v[j] = Real(1);
+                if ((act >> (t0 >> 6)) & 1u) {
+                    Real acc[kTsTabQ];
+#pragma unroll
+                    for (int j = 0; j < kTsTabQ; ++j) acc[j] = Real(0);
+                    for (int is = 0; is < ns; ++is) {
+                        const int i = is * T + t, pk = t_pk[i];
+                        const Real ra = t_ra[i], rb = Real(1) - ra, a0 = t_a0[i], dk = t_dk[i];
+                        const Real* l = s_l + (pk >> 3) * kLd + q;
+#pragma unroll
+                        for (int j = 0; j < kTsTabQ; ++j) {
+                            const Real ip = rb * l[j] + ra * l[kLd + j];
+                            const Real area = (pk & 2) ? a0 * afac[j] : a0 + kd[j] * dk;
+                            acc[j] += (pk & 1) ? ip * area : Real(0);
+                        }
+                    }
+                    const bool inw = (t_pk[t] & 4) != 0;
+#pragma unroll
+                    for (int j = 0; j < kTsTabQ; ++j) v[j] = inw ? Real(1) - acc[j] * f[j] : Real(1);
+                }
+#pragma unroll
+                for (int j = 0; j < kTsTabQ; ++j)
+                    if (t < nt && q + j < npc) o[(size_t)j * s.npt + t] = v[j];
+            }
+        }
+    }
+}
+
+// ---- any number of samples, any g grid: the geometry recomputed for each chunk of
+// passbands, one accumulator a passband and lane ------------------------------------------
+template <bool kMixed>
 __global__ void __launch_bounds__(kTsThreads) ts_flux_kernel(TsArgs s, void* flux, int ntiles) {
     using Real = typename std::conditional<kMixed, float, double>::type;
-    constexpr int PC = ts_pb_chunk(kMixed, kCached);
-    constexpr int TPL = kCached ? ts_tpl<Real>() : 1;
+    constexpr int PC = ts_pb_chunk(kMixed);
     extern __shared__ __align__(16) unsigned char lds[];
     Real* s_ldm = (Real*)lds;                       // [PC][ng]
     Real* s_afac = s_ldm + (size_t)PC * s.ng;       // k^2 / k_mean^2
@@ -933,64 +1153,35 @@ __global__ void __launch_bounds__(kTsThreads) ts_flux_kernel(TsArgs s, void* flu
     const int bid = xcd_remap(blockIdx.x, gridDim.x);
     const int tile = bid % ntiles;
     const int pv = bid / ntiles;
-    const int t0l = (tile * kTsThreads + (int)threadIdx.x) * TPL;  // first time of the lane
-    const int nt = max(0, min(TPL, s.npt - t0l));                   // its valid times
+    const int it = tile * kTsThreads + (int)threadIdx.x;
+    const bool in = it < s.npt;
     const TsRec& r = s.rec[pv];
-    Real* out = (Real*)flux + (size_t)pv * s.npb * s.npt;
-    // whole-vector stores need every row start 16-B aligned
-    const bool vec = TPL > 1 && (s.npt % TPL) == 0 && (((uintptr_t)out) % 16) == 0;
-    Real ones[TPL], v[TPL];
-#pragma unroll
-    for (int j = 0; j < TPL; ++j) ones[j] = Real(1);
+    Real* out = (Real*)flux + (size_t)pv * s.npb * s.npt + it;
     if (!r.good) {
-#pragma unroll
-        for (int j = 0; j < TPL; ++j) v[j] = Real(NAN);
-        if (nt > 0)
-            for (int q = 0; q < s.npb; ++q) ts_store(out + (size_t)q * s.npt + t0l, v, nt, vec);
+        if (in)
+            for (int q = 0; q < s.npb; ++q) out[(size_t)q * s.npt] = Real(NAN);
         return;
     }
-    double tc[TPL];
-    bool inw[TPL];
-    bool any = false;
-#pragma unroll
-    for (int j = 0; j < TPL; ++j) {
-        tc[j] = 0.0;
-        inw[j] = false;
-        if (j < nt) {
-#pragma clang fp contract(off)
-            const double t = s.times[t0l + j];
-            const double t0v = s.t0[pv];
-            const double epoch = floor((t - t0v + 0.5 * r.p) * r.inv_p);
-            const double u = t - t0v + 0.5 * r.p;
-            const double rem = u - epoch * r.p;
-            const double ep = epoch + ((rem < 0.0) ? -1.0 : ((rem >= r.p) ? 1.0 : 0.0));
-            tc[j] = t - (t0v + ep * r.p);
-            inw[j] = (r.bt1 <= tc[j]) && (tc[j] <= r.bt4);
-            any = any || inw[j];
-        }
+    double tc = 0.0;
+    bool inw = false;
+    if (in) {
+        double ep;
+        tc = epoch_phase(s.times[it], s.t0[pv], r.p, r.inv_p, ep);
+        inw = (r.bt1 <= tc) && (tc <= r.bt4);
     }
     if (threadIdx.x == 0) s_any = 0;
     __syncthreads();
-    if (any) s_any = 1;
+    if (inw) s_any = 1;
     __syncthreads();
     if (!s_any) {
-        if (nt > 0)
-            for (int q = 0; q < s.npb; ++q) ts_store(out + (size_t)q * s.npt + t0l, ones, nt, vec);
+        if (in)
+            for (int q = 0; q < s.npb; ++q) out[(size_t)q * s.npt] = Real(1);
         return;
     }
     const int ns = s.nsamples[0];
     const double ext = s.exptimes[0];
     const Real inv_ns = Real(1) / Real(ns);
-    const double km = r.kmean;
-    TsGeo<Real> geo[TPL][kCached ? kTsGeoRegs : 1];
-    if (kCached) {
-#pragma unroll
-        for (int j = 0; j < TPL; ++j)
-#pragma unroll
-            for (int is = 0; is < kTsGeoRegs; ++is)
-                if (inw[j] && is < ns) geo[j][is] = ts_geometry<Real>(r, tc[j], ext, ns, is, s.dg, s.ng);
-    }
-
+    const double km = r.kmean, inv_1pk = 1.0 / (1.0 + km), inv_dg = 1.0 / s.dg;
     for (int pb0 = 0; pb0 < s.npb; pb0 += PC) {
         const int npc = min(PC, s.npb - pb0);
         __syncthreads();  // the previous chunk's rows are no longer read
@@ -1006,46 +1197,25 @@ __global__ void __launch_bounds__(kTsThreads) ts_flux_kernel(TsArgs s, void* flu
             s_iist[q] = (Real)(1.0 / s.istar[(size_t)pv * s.npb + pb0 + q]);
         }
         __syncthreads();
-        if (nt == 0) continue;
-        Real* o = out + (size_t)pb0 * s.npt + t0l;
-        // depth of passband q for one sample; the flux is 1 - mean(depth) / istar
-        auto depth = [&](const TsGeo<Real>& g, int q) {
-            const Real* l = s_ldm + (size_t)q * s.ng;
-            const Real ip = g.gz ? Real(0) : (g.rb * l[g.ig] + g.ra * l[g.ig + 1]);
-            const Real area = g.inside ? g.ap0 * s_afac[q] : g.ap0 + s_kd[q] * g.dadk;
-            return ip * area;
-        };
-        if (kCached) {
-#pragma unroll 2
-            for (int q = 0; q < npc; ++q) {
-                const Real f = s_iist[q] * inv_ns;
+        if (!in) continue;
+        Real acc[PC];
 #pragma unroll
-                for (int j = 0; j < TPL; ++j) {
-                    Real acc = Real(0);
-                    if (inw[j]) {
-                        acc = depth(geo[j][0], q);
-                        if (ns > 1) acc += depth(geo[j][kTsGeoRegs - 1], q);
+        for (int q = 0; q < PC; ++q) acc[q] = Real(0);
+        if (inw) {
+            for (int is = 0; is < ns; ++is) {
+                const TsGeo<Real> g = ts_geometry<Real>(r, tc, ext, 1.0 / ns, is, inv_1pk, inv_dg, s.ng);
+#pragma unroll
+                for (int q = 0; q < PC; ++q)
+                    if (q < npc) {
+                        const Real* l = s_ldm + (size_t)q * s.ng;
+                        const Real ip = g.gz ? Real(0) : (g.rb * l[g.ig] + g.ra * l[g.ig + 1]);
+                        acc[q] += ip * (g.inside ? g.ap0 * s_afac[q] : g.ap0 + s_kd[q] * g.dadk);
                     }
-                    v[j] = inw[j] ? Real(1) - acc * f : Real(1);
-                }
-                ts_store(o + (size_t)q * s.npt, v, nt, vec);
             }
-        } else {
-            Real acc[PC];
-#pragma unroll
-            for (int q = 0; q < PC; ++q) acc[q] = Real(0);
-            if (inw[0]) {
-                for (int is = 0; is < ns; ++is) {
-                    const TsGeo<Real> g = ts_geometry<Real>(r, tc[0], ext, ns, is, s.dg, s.ng);
-#pragma unroll
-                    for (int q = 0; q < PC; ++q)
-                        if (q < npc) acc[q] += depth(g, q);
-                }
-            }
-#pragma unroll
-            for (int q = 0; q < PC; ++q)
-                if (q < npc) o[(size_t)q * s.npt] = inw[0] ? Real(1) - acc[q] * (s_iist[q] * inv_ns) : Real(1);
         }
+#pragma unroll
+        for (int q = 0; q < PC; ++q)
+            if (q < npc) out[(size_t)(pb0 + q) * s.npt] = inw ? Real(1) - acc[q] * (s_iist[q] * inv_ns) : Real(1);
     }
 }
 
@@ -1116,6 +1286,7 @@ int ts_evaluate(int precision, const rr_table* tab, const rr_lcdata* lc, const r
     a.ngp = (tab->ng + 15) / 16 * 16; a.nzp = (tab->nz + 3) / 4 * 4;
     a.use_table = tab->weights != nullptr && tab->nk >= 2;
     a.kmin = tab->kmin; a.kmax_tab = tab->kmax; a.dk = tab->dk; a.dg = tab->dg;
+    a.ldm_split = a.row_split = 1;
     hipStream_t st = (hipStream_t)stream;
     const bool tab_ld = ld->law == RR_LD_TABULATED;
     // the weight kernel lists (g, z) pairs of a workgroup as 16-bit indices
@@ -1124,20 +1295,27 @@ int ts_evaluate(int precision, const rr_table* tab, const rr_lcdata* lc, const r
     hipLaunchKernelGGL(ts_setup_kernel, dim3((npv + kTsGroup - 1) / kTsGroup), dim3(64), 0, st, a);
     int rc = check_launch("ts_setup_kernel");
     if (rc) return rc;
-    hipLaunchKernelGGL(ts_istar_kernel, dim3((npv * npb + 255) / 256), dim3(256), 0, st, a);
-    if ((rc = check_launch("ts_istar_kernel"))) return rc;
     const int wrows = ts_weight_rows(a.nz);
-    const long long nw = (long long)npv * ((a.ngp + wrows - 1) / wrows);
+    const long long nw = (long long)npv * ((a.ngp + wrows - 1) / wrows) + ((long long)npv * npb + 255) / 256;
+    if (nw > 0x7fffffffLL) return set_error(RR_ERANGE, "ts_evaluate: grid too large");
     hipLaunchKernelGGL(ts_weights_kernel, dim3((unsigned)nw), dim3(256), ts_weights_lds(a.nz), st, a);
     if ((rc = check_launch("ts_weights_kernel"))) return rc;
     // tabulated FP64 profiles with nz a multiple of 4 (16-byte aligned rows), nz <= 128
     // and ngp <= 128: the row-contiguous kernel
     const int nct = a.ngp / 16;
+    // few pvs: the row tiles of a pv over several workgroups (of 8 waves, the generic
+    // FP32 form 4), one round of row tiles a wave at the least
+    const int nrt = (npb + 15) / 16;
+    auto ldm_split = [&](int waves) {
+        const int most = (nrt + waves - 1) / waves, want = (512 + npv - 1) / npv;
+        return want < 1 ? 1 : (want < most ? want : most);
+    };
     const bool tab_rows = mixed && tab_ld && a.nz % 4 == 0 && a.nz <= 16 * kTabMfmaMaxJ && nct <= kTabMfmaMaxCt &&
                           ((uintptr_t)ld->ldp & 15) == 0;
     if (tab_rows) {
         const size_t lds = (size_t)((a.nz + 15) / 16 * 16) * ts_tab_ldb(a.ngp) * sizeof(float);
-        const dim3 g(npv), b(kTabMfmaThreads);
+        a.ldm_split = ldm_split(kTabMfmaThreads / 64);
+        const dim3 g((unsigned)npv * a.ldm_split), b(kTabMfmaThreads);
         switch (nct) {
             case 1: hipLaunchKernelGGL(ts_ldm_tab_mfma_kernel<1>, g, b, lds, st, a); break;
             case 2: hipLaunchKernelGGL(ts_ldm_tab_mfma_kernel<2>, g, b, lds, st, a); break;
@@ -1150,10 +1328,12 @@ int ts_evaluate(int precision, const rr_table* tab, const rr_lcdata* lc, const r
         }
         if ((rc = check_launch("ts_ldm_tab_mfma_kernel"))) return rc;
     } else if (mixed) {
-        const size_t lds = (size_t)a.nzp * (a.ngp + 1) * sizeof(float);
+        const size_t lds = (size_t)a.nzp * ts_tab_ldb(a.ngp) * sizeof(float);
         if (lds <= 160 * 1024) {
-            if (tab_ld) hipLaunchKernelGGL(ts_ldm_mfma_kernel<true>, dim3(npv), dim3(256), lds, st, a);
-            else hipLaunchKernelGGL(ts_ldm_mfma_kernel<false>, dim3(npv), dim3(256), lds, st, a);
+            a.ldm_split = ldm_split(4);
+            const dim3 g((unsigned)npv * a.ldm_split);
+            if (tab_ld) hipLaunchKernelGGL(ts_ldm_mfma_kernel<true>, g, dim3(256), lds, st, a);
+            else hipLaunchKernelGGL(ts_ldm_mfma_kernel<false>, g, dim3(256), lds, st, a);
             if ((rc = check_launch("ts_ldm_mfma_kernel"))) return rc;
         } else {
             const long long n = (long long)npv * npb * a.ng;
@@ -1165,8 +1345,10 @@ int ts_evaluate(int precision, const rr_table* tab, const rr_lcdata* lc, const r
     } else {
         const size_t lds = (size_t)a.nzp * (a.ngp + 1) * sizeof(double);
         if (lds <= kMfma64MaxLds) {
-            if (tab_ld) hipLaunchKernelGGL(ts_ldm_mfma64_kernel<true>, dim3(npv), dim3(kMfma64Threads), lds, st, a);
-            else hipLaunchKernelGGL(ts_ldm_mfma64_kernel<false>, dim3(npv), dim3(kMfma64Threads), lds, st, a);
+            a.ldm_split = ldm_split(kMfma64Threads / 64);
+            const dim3 g((unsigned)npv * a.ldm_split);
+            if (tab_ld) hipLaunchKernelGGL(ts_ldm_mfma64_kernel<true>, g, dim3(kMfma64Threads), lds, st, a);
+            else hipLaunchKernelGGL(ts_ldm_mfma64_kernel<false>, g, dim3(kMfma64Threads), lds, st, a);
             if ((rc = check_launch("ts_ldm_mfma64_kernel"))) return rc;
         } else {
             const long long n = (long long)npv * npb * a.ng;
@@ -1176,44 +1358,59 @@ int ts_evaluate(int precision, const rr_table* tab, const rr_lcdata* lc, const r
             if ((rc = check_launch("ts_ldm_f64_kernel"))) return rc;
         }
     }
-    // nsamples[0] as given by the host (0: unknown) selects the register-cached form
-    const bool cached = lc->uniform_nsamples >= 1 && lc->uniform_nsamples <= kTsGeoRegs;
-    const int per_tile = kTsThreads * (cached ? (mixed ? ts_tpl<float>() : ts_tpl<double>()) : 1);
-    const int ntiles = (npt + per_tile - 1) / per_tile;
-    const long long nb = (long long)npv * ntiles;
-    if (nb > 0x7fffffffLL) return set_error(RR_ERANGE, "ts_evaluate: grid too large");
-    const dim3 grid((unsigned)nb), block(kTsThreads);
+    const dim3 block(kTsThreads);
+    // nsamples[0] as given by the host (0: unknown)
     const int uns = lc->uniform_nsamples;
-    // one sample, rows of whole 16-byte vectors: the row form
-    if (uns == 1 && ((uintptr_t)flux % 16) == 0) {
+    // one sample, rows of whole 16-byte vectors: the row form, where it gives every CU a
+    // workgroup.  A pv's passbands go to several workgroups (1024 in all) if each keeps
+    // 64 rows and 320,000 values to pay for its geometry: 300 pv x 512 x 5,000 mixed 798
+    // -> 724 us with 4; 500 x 200 x 1,236 would go from 221 to 245.  With fewer
+    // workgroups than CUs the tiles below are faster (8 x 200 x 1,236: 95 -> 39 us, 128:
+    // 104 -> 72 us; at 256 125 against 130).
+    const int want = (1024 + npv - 1) / npv, min_rows = 320000 / npt > 64 ? 320000 / npt : 64, most_rows = npb / min_rows;
+    a.row_split = want < most_rows ? want : (most_rows > 1 ? most_rows : 1);
+    if (uns == 1 && ((uintptr_t)flux % 16) == 0 && (long long)npv * a.row_split >= 256) {
         if (mixed && npt % 4 == 0 && npt <= ts_row_max_npt<float>() && kTsRowPc * a.ng <= kTsStageRegs * kTsRowThreads &&
             ts_rows_aligned_lds(a.ng, npt) <= kTsRowsAlignedMaxLds) {
-            hipLaunchKernelGGL(ts_flux_rows_aligned_kernel, dim3((unsigned)npv), dim3(kTsRowThreads),
+            hipLaunchKernelGGL(ts_flux_rows_aligned_kernel, dim3((unsigned)npv * a.row_split), dim3(kTsRowThreads),
                                ts_rows_aligned_lds(a.ng, npt), st, a, (float*)flux);
             return check_launch("ts_flux_rows_aligned_kernel");
         }
         if (mixed && npt % 4 == 0 && npt <= ts_row_max_npt<float>() && ts_rows_lds(a.ng, 4) <= 64 * 1024) {
-            hipLaunchKernelGGL(ts_flux_rows_kernel<float>, dim3((unsigned)npv), dim3(kTsRowThreads),
+            hipLaunchKernelGGL(ts_flux_rows_kernel<float>, dim3((unsigned)npv * a.row_split), dim3(kTsRowThreads),
                                ts_rows_lds(a.ng, 4), st, a, (float*)flux);
             return check_launch("ts_flux_rows_kernel");
         }
         if (!mixed && npt % 2 == 0 && npt <= ts_row_max_npt<double>() && ts_rows_lds(a.ng, 8) <= 64 * 1024) {
-            hipLaunchKernelGGL(ts_flux_rows_kernel<double>, dim3((unsigned)npv), dim3(kTsRowThreads),
+            hipLaunchKernelGGL(ts_flux_rows_kernel<double>, dim3((unsigned)npv * a.row_split), dim3(kTsRowThreads),
                                ts_rows_lds(a.ng, 8), st, a, (double*)flux);
             return check_launch("ts_flux_rows_kernel");
         }
     }
-    if (mixed) {
-        const int PC = ts_pb_chunk(true, cached);
-        const size_t lds = ((size_t)PC * a.ng + 3 * PC) * sizeof(float);
-        if (cached) hipLaunchKernelGGL((ts_flux_kernel<true, true>), grid, block, lds, st, a, flux, ntiles);
-        else hipLaunchKernelGGL((ts_flux_kernel<true, false>), grid, block, lds, st, a, flux, ntiles);
-    } else {
-        const int PC = ts_pb_chunk(false, cached);
-        const size_t lds = ((size_t)PC * a.ng + 3 * PC) * sizeof(double);
-        if (cached) hipLaunchKernelGGL((ts_flux_kernel<false, true>), grid, block, lds, st, a, flux, ntiles);
-        else hipLaunchKernelGGL((ts_flux_kernel<false, false>), grid, block, lds, st, a, flux, ntiles);
+    if (uns >= 1 && uns <= kTsTabSamples) {
+        const size_t lds = mixed ? ts_tab_lds<float>(uns, a.ng) : ts_tab_lds<double>(uns, a.ng);
+        const int T = mixed ? ts_tab_times<float>(uns) : ts_tab_times<double>(uns);
+        if (lds <= 160 * 1024) {
+            // passbands split over workgroups where the tiles alone leave CUs without one
+            const int nt = (npt + T - 1) / T;
+            const long long tiles = (long long)npv * nt;
+            const int pc = mixed ? ts_tab_pc<float>() : ts_tab_pc<double>(), most = (npb + pc - 1) / pc;
+            const int nsplit = (int)(tiles >= 1024 ? 1 : (1024 + tiles - 1) / tiles < most ? (1024 + tiles - 1) / tiles : most);
+            if (tiles * nsplit > 0x7fffffffLL) return set_error(RR_ERANGE, "ts_evaluate: grid too large");
+            const dim3 g((unsigned)(tiles * nsplit));
+            if (mixed) hipLaunchKernelGGL(ts_flux_table_kernel<float>, g, block, lds, st, a, (float*)flux, nt, nsplit, uns);
+            else hipLaunchKernelGGL(ts_flux_table_kernel<double>, g, block, lds, st, a, (double*)flux, nt, nsplit, uns);
+            return check_launch("ts_flux_table_kernel");
+        }
     }
+    const int ntiles = (npt + kTsThreads - 1) / kTsThreads;
+    const long long nb = (long long)npv * ntiles;
+    if (nb > 0x7fffffffLL) return set_error(RR_ERANGE, "ts_evaluate: grid too large");
+    const int PC = ts_pb_chunk(mixed);
+    const size_t lds = ((size_t)PC * a.ng + 3 * PC) * (mixed ? sizeof(float) : sizeof(double));
+    const dim3 grid((unsigned)nb);
+    if (mixed) hipLaunchKernelGGL(ts_flux_kernel<true>, grid, block, lds, st, a, flux, ntiles);
+    else hipLaunchKernelGGL(ts_flux_kernel<false>, grid, block, lds, st, a, flux, ntiles);
     return check_launch("ts_flux_kernel");
 }
 

@@ -1,0 +1,35 @@
+"""TSModel at the edges of its tiles, passband chunks, splits and sample counts, against
+the FP64 oracle's tsmodel_serial.  Bars: the suite's, 1e-9 absolute in FP64 and 1 ppm
+mixed."""
+import numpy as np
+import pytest
+
+from pytransit_amd import TabulatedLDModel, TSModel, workloads
+
+pytestmark = pytest.mark.gpu
+
+
+# npv, npb, npt, nss: a single time; one lane and one passband past a tile or chunk;
+# short tiles (many samples); the form without a table (33 samples); rows of odd length
+# with few pvs; workgroups that share a pv's rows
+@pytest.mark.parametrize('npv,npb,npt,nss', [
+    (1, 1, 1, 1), (2, 3, 63, 2), (3, 17, 65, 3), (2, 33, 257, 1), (1, 70, 300, 10), (2, 5, 130, 32), (2, 5, 70, 33),
+    (4, 32, 1236, 1), (4, 31, 1237, 1), (260, 130, 5000, 1), (3, 200, 514, 2)])
+@pytest.mark.parametrize('precision', ['fp64', 'mixed'])
+def test_ts_sizes(gpu, oracle, npv, npb, npt, nss, precision):
+    wl = workloads.ts_many_pb(npv=npv, npt=npt, npb=npb, seed=npv + npt, mu=TSModel('quadratic', nzin=24, nzlimb=24).mu)
+    if npt == 1:
+        wl.times = np.array([0.003])
+    if npv > 3:
+        wl.a[1] = 0.5                       # an invalid vector
+    ext = 0.01 if nss > 1 else 0.0
+    tm = TSModel(TabulatedLDModel(wl.ldp, wl.istar), nzin=24, nzlimb=24, precision=precision)
+    tm.set_data(wl.times, nsamples=nss, exptimes=ext)
+    f = tm.evaluate(wl.k, None, wl.t0, wl.p, wl.a, wl.i)
+    assert f.shape == (npv, npb, npt)
+    r = np.arange(npv) if npv < 5 else np.array([0, 1, npv - 1])
+    ze, _ = oracle.create_z_grid(0.7, 24, 24)
+    ref = oracle.tsmodel_serial(wl.times, wl.k[r], wl.t0[r], wl.p[r], wl.a[r], wl.i[r], wl.e[r], wl.w[r], nss, ext,
+                                wl.ldp[r], wl.istar[r], None, 0, 0, 0, 100, 0, ze)
+    assert np.array_equal(np.isnan(f[r]), np.isnan(ref)) and np.nanmin(ref) < 1
+    assert np.nanmax(np.abs(f[r] - ref)) <= (1e-9 if precision == 'fp64' else 1e-6)
