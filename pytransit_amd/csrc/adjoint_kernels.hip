@@ -370,9 +370,31 @@ struct LnlSums {
     Real v[kGrad ? 8 : 1];
 };
 
+// A sample's terms of these sums as the factors of their products, so that a sum takes
+// the same fused steps whichever lane evaluated the sample: I, A, then the k derivative,
+// G = dI/dz A + I dA/dz, dz by t0, p, a and i, and dI by c0 and c1.
+template <typename Real, bool kGrad>
+struct LnlTerm {
+    static constexpr int kN = kGrad ? 10 : 2;
+    Real f[kN];
+};
+
+template <typename Real, bool kGrad>
+__device__ __forceinline__ void lnl_add(LnlSums<Real, kGrad>& d, const LnlTerm<Real, kGrad>& t) {
+    d.v[0] = d_fma(t.f[0], t.f[1], d.v[0]);
+    if constexpr (kGrad) {
+        d.v[1] += t.f[2];
+#pragma unroll
+        for (int m = 0; m < 4; ++m) d.v[2 + m] = d_fma(t.f[3], t.f[4 + m], d.v[2 + m]);
+        d.v[6] = d_fma(t.f[8], t.f[1], d.v[6]);
+        d.v[7] = d_fma(t.f[9], t.f[1], d.v[7]);
+    }
+}
+
+// One sample; `d` keeps its zeros where the planet is off the disk.
 template <typename Real, bool kGrad>
 __device__ __forceinline__ void lnl_sample(const LnlPv<Real>& v, const Real* rows, int ng, double taud, Real ep,
-                                           LnlSums<Real, kGrad>& d) {
+                                           LnlTerm<Real, kGrad>& d) {
     constexpr bool kMixed = std::is_same<Real, float>::value;
     const Real tau = (Real)taud;
     Real x, y, z, u, inv_z;
@@ -450,22 +472,19 @@ __device__ __forceinline__ void lnl_sample(const LnlPv<Real>& v, const Real* row
         dAdz = Real(-2) * akite * inv_z;   // minus the chord of the lens
         dAdk = Real(2) * v.k * kap;
     }
-    d.v[0] += Ii * A;
+    d.f[0] = Ii;
+    d.f[1] = A;
     if constexpr (kGrad) {
         const Real vx = dhorner5(v.cx, tau), vy = dhorner5(v.cy, tau);
         const Real px = horner5(v.dcx, tau), py = horner5(v.dcy, tau);
-        const Real dz_t0 = -(x * vx + y * vy) * inv_z;
-        const Real dz_p = (x * (px - ep * vx) + y * (py - ep * vy)) * inv_z;
-        const Real dz_a = z * v.inv_a;
-        const Real dz_i = -(y * y) * v.tan_i * inv_z;
-        const Real G = d_fma(dIdg * v.inv1pk, A, Ii * dAdz);
-        d.v[1] += d_fma(Ik - dIdg * z * v.inv1pk * v.inv1pk, A, Ii * dAdk);
-        d.v[2] += G * dz_t0;
-        d.v[3] += G * dz_p;
-        d.v[4] += G * dz_a;
-        d.v[5] += G * dz_i;
-        d.v[6] += Ic0 * A;
-        d.v[7] += Ic1 * A;
+        d.f[2] = d_fma(Ik - dIdg * z * v.inv1pk * v.inv1pk, A, Ii * dAdk);
+        d.f[3] = d_fma(dIdg * v.inv1pk, A, Ii * dAdz);
+        d.f[4] = -(x * vx + y * vy) * inv_z;
+        d.f[5] = (x * (px - ep * vx) + y * (py - ep * vy)) * inv_z;
+        d.f[6] = z * v.inv_a;
+        d.f[7] = -(y * y) * v.tan_i * inv_z;
+        d.f[8] = Ic0;
+        d.f[9] = Ic1;
     }
 }
 
@@ -539,18 +558,25 @@ __global__ void __launch_bounds__(kLnlThreads) rr_lnlike_kernel(LnlArgs s) {
             const Real ep = (Real)epoch;
             if (G == 1) {
 #pragma unroll 1
-                for (int is = 0; is < ns; ++is)
-                    lnl_sample<Real, kGrad>(v, s_rows, s.ng, tc + ext * ((is + 0.5) * inv_ns - 0.5), ep, d);
+                for (int is = 0; is < ns; ++is) {
+                    LnlTerm<Real, kGrad> one = {};
+                    lnl_sample<Real, kGrad>(v, s_rows, s.ng, tc + ext * ((is + 0.5) * inv_ns - 0.5), ep, one);
+                    lnl_add(d, one);
+                }
             } else {
                 // a sample a lane, summed in sample order as by one lane
 #pragma unroll 1
                 for (int i0 = 0; i0 < ns; i0 += G) {
-                    LnlSums<Real, kGrad> one = {};
+                    LnlTerm<Real, kGrad> one = {};
                     if (i0 + sub < ns)
                         lnl_sample<Real, kGrad>(v, s_rows, s.ng, tc + ext * ((i0 + sub + 0.5) * inv_ns - 0.5), ep, one);
-                    for (int q = 0; q < G; ++q)
+                    for (int q = 0; q < G; ++q) {
+                        LnlTerm<Real, kGrad> of;
 #pragma unroll
-                        for (int m = 0; m < (kGrad ? 8 : 1); ++m) d.v[m] += __shfl(one.v[m], (lane & ~(G - 1)) + q, 64);
+                        for (int m = 0; m < LnlTerm<Real, kGrad>::kN; ++m)
+                            of.f[m] = __shfl(one.f[m], (lane & ~(G - 1)) + q, 64);
+                        lnl_add(d, of);
+                    }
                 }
             }
             if (sub != 0) return;
