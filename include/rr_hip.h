@@ -197,6 +197,19 @@ int rr_max_batch(void);
 int rr_evaluate_batch(int precision, const rr_table* tab, int nreq, const rr_request* reqs,
                       void* stream);
 
+/* Up to rr_max_batch() blocks of host memory to device memory: their bytes are
+ * copied one behind the other (each rounded up to 16) into `staging` (pinned host
+ * memory that the device can read, of staging_bytes) before the call returns, and
+ * from there to their destinations by one kernel on `stream`.  `staging` must not
+ * be written again before that kernel has ended.  Destinations and `staging` are
+ * 16-byte aligned, and a destination has room for its bytes rounded up to 16. */
+typedef struct rr_piece {
+    const void* src;   /* host */
+    void* dst;         /* device */
+    size_t bytes;
+} rr_piece;
+int rr_upload(int n, const rr_piece* pieces, void* staging, size_t staging_bytes, void* stream);
+
 /* The batch of rr_evaluate_batch split into a plan on the host and a launch that
  * reads the plan from device memory, so the launch can be captured in a HIP graph
  * once and replayed for every later batch whose shape it covers.  rr_batch_plan

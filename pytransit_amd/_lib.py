@@ -63,6 +63,10 @@ class RRRequest(ctypes.Structure):
                 ('workspace_bytes', c_size_t), ('flux', c_void_p)]
 
 
+class RRPiece(ctypes.Structure):
+    _fields_ = [('src', c_void_p), ('dst', c_void_p), ('bytes', c_size_t)]
+
+
 class RRBatchShape(ctypes.Structure):
     _fields_ = [('setup_blocks', c_int32), ('setup_multi', c_int32), ('setup_lds', c_int32),
                 ('flux_blocks', c_int32 * 2), ('flux_lds', c_int32 * 2)]
@@ -96,6 +100,7 @@ _SIGNATURES = {
                               c_void_p]),
     'ts_evaluate': (c_int, [c_int, POINTER(RRTable), POINTER(RRLcData), POINTER(RRParams), POINTER(RRLd),
                             c_void_p, c_size_t, c_void_p, c_void_p]),
+    'rr_upload': (c_int, [c_int, POINTER(RRPiece), c_void_p, c_size_t, c_void_p]),
     'rr_max_batch': (c_int, []),
     'ma_workspace_bytes': (c_size_t, [c_int]),
     'ma_evaluate': (c_int, [POINTER(RRLcData), POINTER(RRParams), c_void_p, c_void_p, c_size_t, c_void_p, c_void_p]),
@@ -117,6 +122,7 @@ _SIGNATURES = {
 RR_NOALLOC_SCRATCH_BYTES = 32 << 20
 
 _lib = None
+_gpu_seen = False      # a GPU was visible at an earlier load()
 
 
 class RRError(RuntimeError):
@@ -137,9 +143,11 @@ def load(require_gpu: bool = True):
     Raises RuntimeError if the built library is missing, if it would bind a second
     HIP runtime next to torch's, or (``require_gpu``) if no GPU is visible.
     """
-    global _lib
-    if require_gpu and not torch.cuda.is_available():
-        raise RuntimeError('pytransit_amd needs a ROCm GPU; torch.cuda.is_available() is False')
+    global _lib, _gpu_seen
+    if require_gpu and not _gpu_seen:
+        if not torch.cuda.is_available():
+            raise RuntimeError('pytransit_amd needs a ROCm GPU; torch.cuda.is_available() is False')
+        _gpu_seen = True
     if _lib is not None:
         return _lib
     if not os.path.exists(LIB_PATH):
@@ -182,8 +190,13 @@ def ptr(t) -> int:
     return 0 if t is None else t.data_ptr()
 
 
+_raw_stream = getattr(torch._C, '_cuda_getCurrentRawStream', None)
+
+
 def stream_handle(device) -> int:
     """hipStream_t of torch's current stream on ``device``."""
+    if _raw_stream is not None and device.index is not None:
+        return _raw_stream(device.index)     # without building a Stream object (5 us)
     return torch.cuda.current_stream(device).cuda_stream
 
 

@@ -13,16 +13,22 @@ __all__ = ['RRLogLikelihood', 'rr_lnlike']
 class RRLogLikelihood(torch.autograd.Function):
     @staticmethod
     def forward(ctx, theta, model, obs, sigma, e=0.0, w=0.0):
-        th = theta.detach().to(torch.float64)
-        k, t0, p, a, i = th[:, 0], th[:, 1], th[:, 2], th[:, 3], th[:, 4]
-        ldc = th[:, 5:7].reshape(-1, 1, 2)
-        lnl, g = model._lnlike_device(k, ldc, t0, p, a, i, obs, sigma, e, w, grad=True)
+        th = theta.detach()
+        if th.dtype is not torch.float64 or th.device != model.device:
+            th = th.to(device=model.device, dtype=torch.float64)
+        if th.dim() == 2 and th.shape[1] >= 7:
+            lnl, g = model._lnlike_device(None, th[:, None, 5:7], None, None, None, None, obs, sigma, e, w, theta=th)
+        else:
+            k, t0, p, a, i = (th[:, j] for j in range(5))
+            lnl, g = model._lnlike_device(k, th[:, 5:7].reshape(-1, 1, 2), t0, p, a, i, obs, sigma, e, w)
         ctx.save_for_backward(g)
-        return lnl.to(theta.dtype)
+        return lnl if lnl.dtype is theta.dtype else lnl.to(theta.dtype)
 
     @staticmethod
     def backward(ctx, gout):
         (g,) = ctx.saved_tensors
+        if gout.dtype is g.dtype:
+            return gout[:, None] * g, None, None, None, None, None
         return (gout.to(g.dtype)[:, None] * g).to(gout.dtype), None, None, None, None, None
 
 

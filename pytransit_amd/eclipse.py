@@ -29,8 +29,8 @@ import torch
 from numpy import ndarray
 
 from . import _lib
-from ._lib import RRLcData, RRParams, check, ptr, stream_handle
-from .rrmodel import _as_dev
+from ._lib import RRParams, check, ptr, stream_handle
+from .rrmodel import _as_dev, _max_id, _per_pv
 from .transitmodel import TransitModel
 
 __all__ = ['EclipseModel', 'EclipseSpectroscopyModel']
@@ -49,7 +49,7 @@ class _EclipseBase(TransitModel):
         return self._device
 
     def _workspace(self, nbytes):
-        key = (str(self.device), stream_handle(self.device))
+        key = (self.device, stream_handle(self.device))
         ws = self._ws.get(key)
         if ws is None or ws.numel() < nbytes:
             ws = torch.empty(max(nbytes, 256), dtype=torch.uint8, device=self.device)
@@ -57,10 +57,7 @@ class _EclipseBase(TransitModel):
         return ws
 
     def _vec(self, name, x, npv, default=None):
-        x = _as_dev(default if x is None else x, self.device).reshape(-1)
-        if x.numel() not in (1, npv):
-            raise ValueError(f"{name} has {x.numel()} values, expected 1 or npv={npv}")
-        return x.expand(npv).contiguous() if x.numel() != npv else x
+        return _per_pv(name, default if x is None else x, npv, self.device)
 
 
 class EclipseModel(_EclipseBase):
@@ -91,19 +88,14 @@ class EclipseModel(_EclipseBase):
         npv = k.numel()
         t0 = _as_dev(t0, dev).reshape(npv, -1).contiguous()
         # new_eclipse_model.py:70 passes pbids where the kernel takes epoch indices
-        if self.pbids.max() >= t0.shape[1]:
+        if _max_id(self.pbids) >= t0.shape[1]:
             raise ValueError(f"t0 has {t0.shape[1]} columns but the passband indices (the eclipse model's epoch "
                              f"indices) go up to {self.pbids.max()}")
         p, a, inc = (self._vec(n, x, npv) for n, x in (('p', p), ('a', a), ('i', i)))
         e, w = self._vec('e', e, npv, 0.0), self._vec('w', w, npv, 0.0)
         rs = self._vec('rstar', rstar, npv)
-        d = self._device_data(dev)
-        lc = RRLcData(npt=self.npt, nlc=self.nlc, npb=self.npb, nep=t0.shape[1], sorted=int(d['sorted']),
-                      uniform_nsamples=d['uniform_ns'], times=ptr(d['times']), lcids=ptr(d['lcids']),
-                      pbids=ptr(d['pbids']), epids=ptr(d['pbids']), nsamples=ptr(d['nsamples']),
-                      exptimes=ptr(d['exptimes']))
-        prm = RRParams(npv=npv, kcols=1, t0cols=t0.shape[1], pad_=0, k=ptr(k), t0=ptr(t0), p=ptr(p), a=ptr(a),
-                       inc=ptr(inc), e=ptr(e), w=ptr(w))
+        lc = self._lc_descriptor(dev, self.npb, t0.shape[1], 'pbids')
+        prm = RRParams(npv, 1, t0.shape[1], 0, ptr(k), ptr(t0), ptr(p), ptr(a), ptr(inc), ptr(e), ptr(w))
         ws = self._workspace(int(lib.ec_workspace_bytes(npv)))
         flux = torch.empty((npv, self.npt), dtype=torch.float64, device=dev)
         byref = _lib.ctypes.byref
@@ -147,13 +139,8 @@ class EclipseSpectroscopyModel(_EclipseBase):
         t0 = self._vec('t0', t0, npv)
         p, a, inc, e, w, rs = (self._vec(n, x, npv) for n, x in
                                (('p', p), ('a', a), ('i', i), ('e', e), ('w', w), ('rstar', rstar)))
-        d = self._device_data(dev)
-        lc = RRLcData(npt=self.npt, nlc=self.nlc, npb=self.npb, nep=1, sorted=int(d['sorted']),
-                      uniform_nsamples=d['uniform_ns'], times=ptr(d['times']), lcids=ptr(d['lcids']),
-                      pbids=ptr(d['pbids']), epids=ptr(d['epids']), nsamples=ptr(d['nsamples']),
-                      exptimes=ptr(d['exptimes']))
-        prm = RRParams(npv=npv, kcols=1, t0cols=1, pad_=0, k=ptr(k), t0=ptr(t0), p=ptr(p), a=ptr(a), inc=ptr(inc),
-                       e=ptr(e), w=ptr(w))
+        lc = self._lc_descriptor(dev, self.npb, 1)
+        prm = RRParams(npv, 1, 1, 0, ptr(k), ptr(t0), ptr(p), ptr(a), ptr(inc), ptr(e), ptr(w))
         ws = self._workspace(int(lib.ec_workspace_bytes(npv)))
         flux = torch.empty((npv, npb, self.npt), dtype=torch.float64, device=dev)
         byref = _lib.ctypes.byref

@@ -21,7 +21,7 @@ from numpy import ndarray
 
 from . import _lib
 from ._lib import check, ptr, stream_handle
-from .rrmodel import RoadRunnerModel, _as_dev
+from .rrmodel import RoadRunnerModel, _per_pv
 
 __all__ = ['OblatePlanetModel']
 
@@ -56,13 +56,7 @@ class OblatePlanetModel(RoadRunnerModel):
         lib = _lib.load()
         dev = self.device
         npv, tab, lc, prm, ld, _keep = self._descriptors(k, ldc, t0, p, a, i, e, w)
-        fl = _as_dev(f, dev).reshape(-1)
-        al = _as_dev(alpha, dev).reshape(-1)
-        for name, x in (('f', fl), ('alpha', al)):
-            if x.numel() not in (1, npv):
-                raise ValueError(f"{name} has {x.numel()} values, expected 1 or npv={npv}")
-        fl = fl.expand(npv).contiguous()
-        al = al.expand(npv).contiguous()
+        fl, al = _per_pv('f', f, npv, dev), _per_pv('alpha', alpha, npv, dev)
         nbytes = lib.rr_workspace_bytes(npv, self.npt, self.npb, self.ng, self.nlc)
         ws = self._workspace(dev, nbytes)
         flux = torch.empty((npv, self.npt), dtype=torch.float64, device=dev)

@@ -16,8 +16,8 @@ import torch
 from numpy import isscalar, ndarray
 
 from . import _lib
-from ._lib import RRLcData, RRParams, check, ptr, stream_handle
-from .rrmodel import _as_dev
+from ._lib import RRParams, check, ptr, stream_handle
+from .rrmodel import _as_dev, _max_id, _per_pv
 from .transitmodel import TransitModel
 
 __all__ = ['QuadraticModel']
@@ -72,36 +72,27 @@ class QuadraticModel(TransitModel):
             ldc = ldc.reshape(npv, -1) if ldc.dim() == 3 else torch.atleast_2d(ldc)
         if ldc.shape[1] != 2 * self.npb:
             raise ValueError("The quadratic model needs two limb darkening coefficients per passband")
-        if self.epids.max() != t0.shape[1] - 1:
+        if _max_id(self.epids) != t0.shape[1] - 1:
             raise ValueError("The number of transit centers must equal to the number of individual epoch IDs.")
         if k.shape[1] not in (1, self.npb):
             raise ValueError('Radius ratios should be given either as an [npv, 1] or [npv, npb] array.')
-        prm = []
-        for name, x, dflt in (('p', p, None), ('a', a, None), ('i', i, None), ('e', e, 0.0), ('w', w, 0.0)):
-            x = _as_dev(dflt if x is None else x, device).reshape(-1)
-            if x.numel() not in (1, npv):
-                raise ValueError(f"{name} has {x.numel()} values, expected 1 or npv={npv}")
-            prm.append(x.expand(npv).contiguous() if x.numel() != npv else x)
-        p, a, inc, e, w = prm
+        p, a, inc, e, w = (_per_pv(name, 0.0 if x is None and name in 'ew' else x, npv, device)
+                           for name, x in (('p', p), ('a', a), ('i', i), ('e', e), ('w', w)))
         k = k.expand(npv, k.shape[1]).contiguous()
         t0 = t0.expand(npv, t0.shape[1]).contiguous()
         ldc = ldc.expand(npv, ldc.shape[1]).contiguous()
-        d = self._device_data(device)
-        lc = RRLcData(npt=self.npt, nlc=self.nlc, npb=self.npb, nep=t0.shape[1], sorted=int(d['sorted']),
-                      uniform_nsamples=d['uniform_ns'], times=ptr(d['times']), lcids=ptr(d['lcids']),
-                      pbids=ptr(d['pbids']), epids=ptr(d['epids']), nsamples=ptr(d['nsamples']),
-                      exptimes=ptr(d['exptimes']))
-        pv = RRParams(npv=npv, kcols=k.shape[1], t0cols=t0.shape[1], pad_=0, k=ptr(k), t0=ptr(t0), p=ptr(p),
-                      a=ptr(a), inc=ptr(inc), e=ptr(e), w=ptr(w))
+        lc = self._lc_descriptor(device, self.npb, t0.shape[1])
+        pv = RRParams(npv, k.shape[1], t0.shape[1], 0, ptr(k), ptr(t0), ptr(p), ptr(a), ptr(inc), ptr(e), ptr(w))
         nbytes = max(int(lib.ma_workspace_bytes(npv)), 256)
-        key = (str(device), stream_handle(device))
+        stream = stream_handle(device)
+        key = (device, stream)
         ws = self._ws.get(key)
         if ws is None or ws.numel() < nbytes:
             ws = torch.empty(nbytes, dtype=torch.uint8, device=device)
             self._ws[key] = ws
         flux = torch.empty((npv, self.npt), dtype=torch.float64, device=device)
         check(lib.ma_evaluate(_lib.ctypes.byref(lc), _lib.ctypes.byref(pv), ptr(ldc), ptr(ws),
-                              ws.numel(), ptr(flux), stream_handle(device)))
+                              ws.numel(), ptr(flux), stream))
         return flux
 
     def __call__(self, *args, **kwargs):

@@ -30,7 +30,7 @@ from numpy import isscalar, linspace, ndarray, pi, sqrt, zeros
 from scipy.integrate import trapezoid
 
 from . import _lib
-from ._lib import LD_LAW_IDS, RRLcData, RRLd, RRParams, RRTable, RRVec, check, ptr, stream_handle
+from ._lib import LD_LAW_IDS, RRLd, RRParams, RRTable, RRVec, check, ptr, stream_handle
 from .ldmodel import LDModel
 from .transitmodel import TransitModel
 
@@ -42,8 +42,31 @@ _PRECISIONS = {'fp64': _lib.RR_FP64, 'mixed': _lib.RR_MIXED}
 def _as_dev(x, device, dtype=torch.float64) -> torch.Tensor:
     """Contiguous device tensor of ``dtype`` (no copy if ``x`` already is one)."""
     if isinstance(x, torch.Tensor):
+        if x.dtype is dtype and x.device == device and x.is_contiguous():
+            return x
         return x.to(device=device, dtype=dtype).contiguous()
+    if isinstance(x, (int, float)):
+        return torch.full((1,), float(x), dtype=dtype, device=device)   # a fill, no upload to wait for
     return torch.as_tensor(np.ascontiguousarray(np.asarray(x, dtype=np.float64)), device=device).to(dtype)
+
+
+def _max_id(ids) -> int:
+    """Largest of an index array (one light curve: without numpy's 3 us reduction)."""
+    return ids[0] if ids.size == 1 else ids.max()
+
+
+def _per_pv(name, x, npv, device) -> torch.Tensor:
+    """One float64 value per pv, contiguous on ``device``."""
+    if isinstance(x, (int, float)):
+        return torch.full((npv,), float(x), dtype=torch.float64, device=device)
+    x = _as_dev(x, device)
+    if x.dim() != 1:
+        x = x.reshape(-1)
+    if x.numel() == npv:
+        return x
+    if x.numel() != 1:
+        raise ValueError(f"{name} has {x.numel()} values, expected 1 or npv={npv}")
+    return x.expand(npv).contiguous()
 
 
 def _vec_in_place(x, npv, device):
@@ -165,8 +188,7 @@ class RoadRunnerModel(TransitModel):
     def _table(self, device):
         """Device-resident z grid, mu nodes and weight table (FP64 and FP32 copies, in
         the device layout [nk, nz, ng]); returns (RRTable, keep-alive dict)."""
-        key = str(device)
-        t = self._tables.get(key)
+        t = self._tables.get(device)
         if t is None:
             lib = _lib.load()
             ze = torch.as_tensor(self.ze, device=device)
@@ -184,7 +206,7 @@ class RoadRunnerModel(TransitModel):
                           kmax=float(self.klims[1]), dk=self.dk, dg=self.dg, weights=ptr(W), weights32=ptr(W32),
                           ze=ptr(ze), mu=ptr(mu))
             t = (tab, dict(ze=ze, mu=mu, W=W, W32=W32))
-            self._tables[key] = t
+            self._tables[device] = t
         return t
 
     @property
@@ -209,7 +231,7 @@ class RoadRunnerModel(TransitModel):
         the other is still reading.  A buffer is allocated on, and only ever used
         by, its own stream, so the caching allocator can reuse a replaced buffer's
         memory only after that stream's earlier kernels."""
-        key = (str(device), stream_handle(device))
+        key = (device, stream_handle(device))
         ws = self._ws.get(key)
         if ws is None or ws.numel() < nbytes:
             ws = torch.empty(max(nbytes, 256), dtype=torch.uint8, device=device)
@@ -243,6 +265,9 @@ class RoadRunnerModel(TransitModel):
         if self.ldname is not None:
             law, ncoef = LD_LAW_IDS[self.ldname]
             shp = _ldc3_shape(_shape_of(ldc))
+            if len(shp) == 3 and shp[0] == npv and shp[1] == npb and shp[2] >= ncoef:
+                c3 = _as_dev(ldc, device)
+                return RRLd(law, shp[2], ptr(c3), 0, 0), (c3,)
             if shp[2] < ncoef:
                 raise ValueError(f"The '{self.ldname}' law needs {ncoef} coefficients per passband, got {shp[2]}")
             c3 = _as_dev(ldc, device).reshape(shp)
@@ -293,20 +318,16 @@ class RoadRunnerModel(TransitModel):
         t0s = _shape_of(t0)
         k = _as_dev(k, device)
         t0 = _as_dev(t0, device)
-        # Q4 (defined): a 1-D k or t0 of length npv > 1 is one value per pv.
-        k = k.reshape(npv, 1) if (len(ks) == 1 and npv > 1 and ks[0] == npv) else torch.atleast_2d(k)
-        t0 = t0.reshape(npv, 1) if (len(t0s) == 1 and npv > 1 and t0s[0] == npv) else torch.atleast_2d(t0)
-        if k.shape[0] not in (1, npv) or t0.shape[0] not in (1, npv):
-            raise ValueError(f"k and t0 need 1 or npv={npv} rows, got {tuple(k.shape)} and {tuple(t0.shape)}")
-        k = k.expand(npv, k.shape[1]).contiguous()
-        t0 = t0.expand(npv, t0.shape[1]).contiguous()
-        out = []
-        for name, x in (('p', p), ('a', a), ('i', i), ('e', e), ('w', w)):
-            x = _as_dev(x, device).reshape(-1)
-            if x.numel() not in (1, npv):
-                raise ValueError(f"{name} has {x.numel()} values, expected 1 or npv={npv}")
-            out.append(x.expand(npv).contiguous() if x.numel() != npv else x)
-        return npv, k, t0, out
+        if not (len(ks) == len(t0s) == 2 and ks[0] == t0s[0] == npv):
+            # Q4 (defined): a 1-D k or t0 of length npv > 1 is one value per pv.
+            k = k.reshape(npv, 1) if (len(ks) == 1 and npv > 1 and ks[0] == npv) else torch.atleast_2d(k)
+            t0 = t0.reshape(npv, 1) if (len(t0s) == 1 and npv > 1 and t0s[0] == npv) else torch.atleast_2d(t0)
+            if k.shape[0] not in (1, npv) or t0.shape[0] not in (1, npv):
+                raise ValueError(f"k and t0 need 1 or npv={npv} rows, got {tuple(k.shape)} and {tuple(t0.shape)}")
+            k = k.expand(npv, k.shape[1]).contiguous()
+            t0 = t0.expand(npv, t0.shape[1]).contiguous()
+        return npv, k, t0, [_per_pv(name, x, npv, device)
+                            for name, x in (('p', p), ('a', a), ('i', i), ('e', e), ('w', w))]
 
     def evaluate(self, k: Union[float, ndarray], ldc: Union[ndarray, List],
                  t0: Union[float, ndarray], p: Union[float, ndarray], a: Union[float, ndarray],
@@ -332,19 +353,14 @@ class RoadRunnerModel(TransitModel):
         npb = self.npb
         if k.shape[1] > 1 and k.shape[1] != npb:
             raise ValueError('Radius ratios should be given either as an [npv, 1] or [npv, npb] array.')
-        if self.epids.max() >= t0.shape[1]:
+        if _max_id(self.epids) >= t0.shape[1]:
             raise ValueError(f"t0 has {t0.shape[1]} columns but the epoch indices go up to {self.epids.max()}")
         if not isscalar(ldc) and not isinstance(ldc, torch.Tensor):
             ldc = np.atleast_1d(ldc)
         ld, _ld_keep = self._ld_descriptor(ldc, npv, npb, device)
         tab, _keep = self._table(device)
-        d = self._device_data(device)
-        lc = RRLcData(npt=self.npt, nlc=self.nlc, npb=npb, nep=t0.shape[1], sorted=int(d['sorted']),
-                      uniform_nsamples=d['uniform_ns'], times=ptr(d['times']),
-                      lcids=ptr(d['lcids']), pbids=ptr(d['pbids']), epids=ptr(d['epids']),
-                      nsamples=ptr(d['nsamples']), exptimes=ptr(d['exptimes']))
-        prm = RRParams(npv=npv, kcols=k.shape[1], t0cols=t0.shape[1], pad_=0, k=ptr(k), t0=ptr(t0), p=ptr(p),
-                       a=ptr(a), inc=ptr(inc), e=ptr(e), w=ptr(w))
+        lc = self._lc_descriptor(device, npb, t0.shape[1])
+        prm = RRParams(npv, k.shape[1], t0.shape[1], 0, ptr(k), ptr(t0), ptr(p), ptr(a), ptr(inc), ptr(e), ptr(w))
         return npv, tab, lc, prm, ld, (k, t0, p, a, inc, e, w, _ld_keep, _keep)
 
     def _evaluate_device(self, k, ldc, t0, p, a, i, e, w, flux_events=None):
@@ -358,8 +374,7 @@ class RoadRunnerModel(TransitModel):
         prec = _PRECISIONS[self.precision]
         dtype = torch.float64 if prec == _lib.RR_FP64 else torch.float32
         flux = torch.empty((npv, self.npt), dtype=dtype, device=device)
-        nbytes = lib.rr_workspace_bytes(npv, self.npt, npb, self.ng, self.nlc)
-        ws = self._workspace(device, nbytes)
+        ws = self._workspace(device, lib.rr_workspace_bytes(npv, self.npt, npb, self.ng, self.nlc))
         stream = stream_handle(device)
         byref = _lib.ctypes.byref
         check(lib.rr_setup(prec, byref(tab), byref(lc), byref(prm), byref(ld), ptr(ws), ws.numel(), stream))
@@ -392,7 +407,9 @@ class RoadRunnerModel(TransitModel):
             return (lnl.cpu().numpy(), g.cpu().numpy()) if grad else lnl.cpu().numpy()
         return (lnl, g) if grad else lnl
 
-    def _lnlike_device(self, k, ldc, t0, p, a, i, obs, sigma, e=0.0, w=0.0, grad=True):
+    def _lnlike_device(self, k, ldc, t0, p, a, i, obs, sigma, e=0.0, w=0.0, grad=True, theta=None):
+        """lnL and its gradient on the device; ``theta`` [npv, 5 or more] (float64 on the
+        device) gives k, t0, p, a and i as columns instead of the five arguments."""
         lib = _lib.load()
         device = self.device
         if self.time is None:
@@ -401,11 +418,18 @@ class RoadRunnerModel(TransitModel):
             raise ValueError('lnlike supports one light curve')
         if self.ldname not in ('quadratic', 'power-2'):
             raise ValueError("lnlike supports the 'quadratic' and 'power-2' laws")
-        npv = 1 if isscalar(p) else _size_of(p)
-        vecs = [_vec_in_place(x, npv, device) for x in (k, t0, p, a, i, e, w)]
+        if theta is not None:
+            # columns of one tensor
+            npv, base, rs, cs = theta.shape[0], theta.data_ptr(), theta.stride(0), 8 * theta.stride(1)
+            vecs = [RRVec(base + cs * j, rs, 0.0) for j in range(5)]
+            vecs += [_vec_in_place(x, npv, device) for x in (e, w)]
+            k, t0, p, a, i = (theta[:, j] for j in range(5)) if None in vecs else (None,) * 5
+        else:
+            npv = 1 if isscalar(p) else _size_of(p)
+            vecs = [_vec_in_place(x, npv, device) for x in (k, t0, p, a, i, e, w)]
         keep = [k, t0, p, a, i, e, w]
         t0cols = 1
-        if any(v is None for v in vecs):
+        if None in vecs:
             # other shapes, host arrays or types: contiguous device copies
             npv, k, t0, (p, a, inc, e, w) = self._params(k, t0, p, a, i, e, w, device)
             if k.shape[1] != 1:
@@ -413,7 +437,7 @@ class RoadRunnerModel(TransitModel):
             t0cols = t0.shape[1]
             keep = [k, t0, p, a, inc, e, w]
             vecs = [RRVec(ptr(x), x.stride(0), 0.0) for x in keep]
-        if self.epids.max() >= t0cols:
+        if _max_id(self.epids) >= t0cols:
             raise ValueError(f"t0 has {t0cols} columns but the epoch indices go up to {self.epids.max()}")
         if (isinstance(ldc, torch.Tensor) and ldc.device == device and ldc.dtype == torch.float64 and ldc.dim() == 3
                 and ldc.shape[0] in (1, npv) and ldc.shape[1] == 1 and ldc.shape[2] >= 2):
@@ -431,11 +455,7 @@ class RoadRunnerModel(TransitModel):
                 raise ValueError('sigma must be a scalar or one value per parameter vector')
             sv = RRVec(ptr(sigma), 1 if sigma.numel() > 1 else 0, 0.0)
         tab, _k = self._table(device)
-        d = self._device_data(device)
-        lc = RRLcData(npt=self.npt, nlc=1, npb=1, nep=t0cols, sorted=int(d['sorted']),
-                      uniform_nsamples=d['uniform_ns'], times=ptr(d['times']), lcids=ptr(d['lcids']),
-                      pbids=ptr(d['pbids']), epids=ptr(d['epids']), nsamples=ptr(d['nsamples']),
-                      exptimes=ptr(d['exptimes']))
+        lc = self._lc_descriptor(device, 1, t0cols)
         lnl = torch.empty(npv, dtype=torch.float64, device=device)
         g = torch.empty((npv, 7), dtype=torch.float64, device=device) if grad else None
         nbytes = lib.rr_lnlike_workspace_bytes(npv, self.npt, self.ng)

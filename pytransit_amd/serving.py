@@ -35,6 +35,7 @@ This module adds one for many independent fits sharing a GPU:
 A batch evaluates each request with the same kernels and arithmetic as
 ``RoadRunnerModel.evaluate`` on its own, so results do not depend on the mix.
 """
+import math
 import time
 from collections import OrderedDict, deque
 from typing import Callable, List, Optional
@@ -43,7 +44,7 @@ import numpy as np
 import torch
 
 from . import _lib
-from ._lib import LD_LAW_IDS, RRBatchShape, RRLcData, RRLd, RRParams, RRRequest, check
+from ._lib import LD_LAW_IDS, RRBatchShape, RRLcData, RRLd, RRParams, RRPiece, RRRequest, check
 from .rrmodel import _PRECISIONS, RoadRunnerModel
 from .transitmodel import TransitModel, layout_flags
 
@@ -159,18 +160,29 @@ class Request:
         if t0.shape[1] <= dataset.max_epid:
             raise ValueError(f't0 has {t0.shape[1]} columns but the epoch indices go up to {dataset.max_epid}')
         c = np.asarray(ldc, np.float64)
-        c = c.reshape((1,) * (3 - c.ndim) + c.shape)
+        if c.ndim != 3:
+            c = c.reshape((1,) * (3 - c.ndim) + c.shape)
         if c.shape[0] not in (1, npv) or c.shape[1] not in (1, dataset.npb) or c.shape[2] < ncoef:
             raise ValueError(f"ldc of shape {c.shape} does not fit npv={npv}, npb={dataset.npb} and the "
                              f"'{ld}' law ({ncoef} coefficients)")
-        c = np.ascontiguousarray(np.broadcast_to(c, (npv, dataset.npb, c.shape[2])))
-        vec = [np.ascontiguousarray(np.broadcast_to(np.asarray(x, np.float64).reshape(-1), (npv,)))
-               for x in (p, a, i, e, w)]
         self.npv, self.law, self.nldc = npv, law, c.shape[2]
         self.kcols, self.t0cols = k.shape[1], t0.shape[1]
-        self.host = OrderedDict(k=np.ascontiguousarray(k), t0=np.ascontiguousarray(t0), p=vec[0], a=vec[1],
-                                inc=vec[2], e=vec[3], w=vec[4], ldc=c)
-        self.params = _Layout([(n, v.nbytes) for n, v in self.host.items()])
+        # one buffer in the device's layout, so that a launch uploads one block per request
+        shapes = dict(k=k.shape, t0=t0.shape, p=(npv,), a=(npv,), inc=(npv,), e=(npv,), w=(npv,),
+                      ldc=(npv, dataset.npb, c.shape[2]))
+        self.params = _Layout([(n, 8 * math.prod(s)) for n, s in shapes.items()])
+        self.block = np.empty(self.params.nbytes // 8, np.float64)
+        self.host = OrderedDict()
+        for (n, s), x in zip(shapes.items(), (k, t0, p, a, i, e, w, c)):
+            o = self.params.off[n] // 8
+            self.host[n] = v = self.block[o:o + math.prod(s)]
+            if len(s) > 1:
+                self.host[n] = v = v.reshape(s)
+            elif not isinstance(x, (int, float)):
+                x = np.asarray(x, np.float64)
+                if x.ndim != 1:
+                    x = x.reshape(-1)
+            v[...] = x
         self.ws_bytes = 0
         self.flux_bytes = 0
         self.offset: Optional[int] = None        # params + workspace block
@@ -428,6 +440,7 @@ class _HipExecutor:
         self.model = RoadRunnerModel('quadratic', precision=precision, device=self.device, **table_kw)
         self.table, self._table_keep = self.model._table(self.device)
         self.arena = torch.empty(server._arena.capacity, dtype=torch.uint8, device=self.device)
+        self.arena_out = self.arena.view(torch.float32 if precision == 'mixed' else torch.float64)
         self.base = self.arena.data_ptr()
         self.streams = [torch.cuda.Stream(self.device) for _ in range(slots)]
         self.upload_stream = torch.cuda.Stream(self.device)
@@ -483,32 +496,30 @@ class _HipExecutor:
     def launch(self, slot: int, reqs: List[Request]):
         stream, staging = self.streams[slot], self.staging[slot]
         lib = self.lib
-        soff = 0
         descs = (RRRequest * len(reqs))()
-        waited = set()
+        pieces = (RRPiece * len(reqs))()
+        dptrs = {}      # dataset -> addresses of its arrays, once its upload is waited for
+        out = self.arena_out
         for j, r in enumerate(reqs):
             ds = r.dataset
-            if id(ds) not in waited:
+            dptr = dptrs.get(id(ds))
+            if dptr is None:
                 stream.wait_event(ds.ready)
-                waited.add(id(ds))
-            base = r.offset
-            for name, arr in r.host.items():
-                soff = self._h2d(stream, staging, soff, base + r.params.off[name], arr)
-            ptrs = {n: self.base + base + o for n, o in r.params.off.items()}
-            dptr = {n: self.base + ds.offset + o for n, o in ds.layout.off.items()}
-            r.flux = self.arena[r.flux_offset:r.flux_offset + r.flux_bytes].view(
-                torch.float32 if self.server.precision == 'mixed' else torch.float64).view(r.npv, ds.npt)
-            d = descs[j]
-            d.lc = RRLcData(npt=ds.npt, nlc=ds.nlc, npb=ds.npb, nep=r.t0cols, sorted=int(ds.sorted),
-                            uniform_nsamples=ds.uniform_ns, times=dptr['times'], lcids=dptr['lcids'],
-                            pbids=dptr['pbids'], epids=dptr['epids'], nsamples=dptr['nsamples'],
-                            exptimes=dptr['exptimes'])
-            d.pv = RRParams(npv=r.npv, kcols=r.kcols, t0cols=r.t0cols, pad_=0, k=ptrs['k'], t0=ptrs['t0'],
-                            p=ptrs['p'], a=ptrs['a'], inc=ptrs['inc'], e=ptrs['e'], w=ptrs['w'])
-            d.ld = RRLd(law=r.law, nldc=r.nldc, ldc=ptrs['ldc'], ldp=0, istar=0)
-            d.workspace = self.base + base + r.params.nbytes
-            d.workspace_bytes = r.ws_bytes
-            d.flux = self.base + r.flux_offset
+                off = ds.layout.off
+                dptr = dptrs[id(ds)] = [self.base + ds.offset + off[n] for n in
+                                        ('times', 'lcids', 'pbids', 'epids', 'nsamples', 'exptimes')]
+            base = self.base + r.offset
+            pieces[j] = RRPiece(r.block.ctypes.data, base, r.params.nbytes)
+            o = r.params.off
+            f0 = r.flux_offset // out.element_size()
+            r.flux = out[f0:f0 + r.points].view(r.npv, ds.npt)
+            descs[j] = RRRequest(
+                RRLcData(ds.npt, ds.nlc, ds.npb, r.t0cols, int(ds.sorted), ds.uniform_ns, *dptr),
+                RRParams(r.npv, r.kcols, r.t0cols, 0, base + o['k'], base + o['t0'], base + o['p'], base + o['a'],
+                         base + o['inc'], base + o['e'], base + o['w']),
+                RRLd(r.law, r.nldc, base + o['ldc'], 0, 0),
+                base + r.params.nbytes, r.ws_bytes, self.base + r.flux_offset)
+        check(lib.rr_upload(len(reqs), pieces, staging.data_ptr(), self.staging_bytes, stream.cuda_stream))
         if self.graphs:
             self._replay(slot, stream, reqs, descs)
         else:

@@ -12,6 +12,8 @@ import numpy as np
 import torch
 from numpy import asarray, atleast_1d, float64, integer, issubdtype, ndarray, ones, unique, zeros
 
+from ._lib import RRLcData, ptr
+
 
 def runs_sorted(time: ndarray, lcids: ndarray) -> bool:
     """True if the light curves are contiguous (lcids non-decreasing) and each is
@@ -128,8 +130,7 @@ class TransitModel:
 
     def _device_data(self, device: torch.device):
         """Device copies of the light-curve arrays (uploaded once per set_data)."""
-        key = str(device)
-        d = self._dev_data.get(key)
+        d = self._dev_data.get(device)
         if d is None:
             if self.time is None:
                 raise ValueError('set_data() must be called before evaluate()')
@@ -146,8 +147,21 @@ class TransitModel:
                 nsamples=torch.as_tensor(nsamples.astype(np.int32), device=device),
                 exptimes=torch.as_tensor(self._per_lc(self.exptimes, np.float64), device=device),
             )
-            self._dev_data[key] = d
+            self._dev_data[device] = d
         return d
+
+    def _lc_descriptor(self, device, npb: int, nep: int, epids: str = 'epids', uniform_ns=None) -> RRLcData:
+        """The C-ABI view of the device copies; ``epids`` names the array passed as
+        epoch indices.  Only the pointers and flags of a set_data are laid out once
+        (12 us of ctypes each call): the sizes are the call's."""
+        d = self._device_data(device)
+        a = d.get('c')
+        if a is None:
+            a = d['c'] = ((int(d['sorted']), d['uniform_ns'], ptr(d['times']), ptr(d['lcids']), ptr(d['pbids'])),
+                          {x: ptr(d[x]) for x in ('epids', 'pbids')}, (ptr(d['nsamples']), ptr(d['exptimes'])))
+        (srt, uns, *arrays), ids, tail = a
+        return RRLcData(self.npt, self.nlc, npb, nep, srt, uns if uniform_ns is None else uniform_ns, *arrays,
+                        ids[epids], *tail)
 
     def __call__(self, *nargs, **kwargs):
         raise NotImplementedError

@@ -18,9 +18,9 @@ import torch
 from numpy import ndarray
 
 from . import _lib
-from ._lib import LD_LAW_IDS, RRLcData, RRLd, RRParams, RRTable, check, ptr, stream_handle
+from ._lib import LD_LAW_IDS, RRLd, RRParams, RRTable, check, ptr, stream_handle
 from .ldmodel import LDModel
-from .rrmodel import RoadRunnerModel, _PRECISIONS, _as_dev, _shape_of
+from .rrmodel import RoadRunnerModel, _PRECISIONS, _as_dev, _per_pv, _shape_of
 
 __all__ = ['TransmissionSpectroscopyModel', 'TSModel']
 
@@ -51,13 +51,8 @@ class TransmissionSpectroscopyModel(RoadRunnerModel):
         if npv > 1 and len(ldc_shape) != 3 and not isinstance(self.ldmodel, LDModel):
             raise ValueError("The limb darkening parameters (ldp) should be given as a 3D array with shape "
                              "[npv, npb, nldp] when evaluating the model for a set of parameters (npv > 1).")
-        prm_t = []
-        for name, x in (('t0', t0), ('p', p), ('a', a), ('i', i), ('e', e), ('w', w)):
-            x = _as_dev(x, device).reshape(-1)
-            if x.numel() not in (1, npv):
-                raise ValueError(f"{name} has {x.numel()} values, expected 1 or npv={npv}")
-            prm_t.append(x.expand(npv).contiguous() if x.numel() != npv else x)
-        t0, p, a, inc, e, w = prm_t
+        t0, p, a, inc, e, w = (_per_pv(name, x, npv, device) for name, x in
+                               (('t0', t0), ('p', p), ('a', a), ('i', i), ('e', e), ('w', w)))
         self.npb = npb
 
         keep = []
@@ -103,13 +98,8 @@ class TransmissionSpectroscopyModel(RoadRunnerModel):
         if not self.interpolate:
             tab = RRTable(nk=tab.nk, ng=tab.ng, nz=tab.nz, pad_=0, kmin=tab.kmin, kmax=tab.kmax, dk=tab.dk, dg=tab.dg,
                           weights=0, weights32=0, ze=tab.ze, mu=tab.mu)
-        d = self._device_data(device)
-        lc = RRLcData(npt=self.npt, nlc=self.nlc, npb=npb, nep=1, sorted=int(d['sorted']),
-                      uniform_nsamples=int(self._per_lc(self.nsamples, np.int64)[0]), times=ptr(d['times']),
-                      lcids=ptr(d['lcids']), pbids=ptr(d['pbids']), epids=ptr(d['epids']),
-                      nsamples=ptr(d['nsamples']), exptimes=ptr(d['exptimes']))
-        prm = RRParams(npv=npv, kcols=npb, t0cols=1, pad_=0, k=ptr(k), t0=ptr(t0), p=ptr(p), a=ptr(a), inc=ptr(inc),
-                       e=ptr(e), w=ptr(w))
+        lc = self._lc_descriptor(device, npb, 1, uniform_ns=int(self._per_lc(self.nsamples, np.int64)[0]))
+        prm = RRParams(npv, npb, 1, 0, ptr(k), ptr(t0), ptr(p), ptr(a), ptr(inc), ptr(e), ptr(w))
         prec = _PRECISIONS[self.precision]
         dtype = torch.float64 if prec == _lib.RR_FP64 else torch.float32
         flux = torch.empty((npv, npb, self.npt), dtype=dtype, device=device)
