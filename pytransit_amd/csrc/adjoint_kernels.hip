@@ -197,7 +197,10 @@ __device__ __forceinline__ void lnl_orbit(const LnlArgs& s, int pv, bool active,
     __syncthreads();
     if (valid && j < (kGrad ? 2 : 1)) taylor_from_stencil(s_x + 16 * j, s_x + 16 * j + 8, s_c + 10 * j);
     __syncthreads();
-    if (valid && j < 2) s_w[j] = find_contact_point(k, j == 0 ? 1 : 4, s_c);
+    if (valid) {
+        const double tc = find_contact_point(k, j < 4 ? 1 : 4, s_c);
+        if ((j & 3) == 0) s_w[j >> 2] = tc;
+    }
     __syncthreads();
     if (!active) return;
     if (valid)

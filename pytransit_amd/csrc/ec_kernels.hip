@@ -53,11 +53,13 @@ constexpr double kDaySec = 86400.0;
 // Time from mid-transit to mid-eclipse: the mean-anomaly difference between the
 // two conjunctions (true anomalies pi/2 - w and 3pi/2 - w); orbits_py.py:544-555.
 __device__ __forceinline__ double eclipse_phase(double p, double e, double w) {
-    const double se = sqrt(1.0 - e * e);
-    const double etr = atan2(se * sin(kHalfPi - w), e + cos(kHalfPi - w));
-    const double eec = atan2(se * sin(kHalfPi + kPi - w), e + cos(kHalfPi + kPi - w));
-    const double mtr = etr - e * sin(etr);
-    const double mec = eec - e * sin(eec);
+    // eccentric anomalies from sin(pi/2 - w) = cos w and so on; their sines from the
+    // atan2's arguments, whose squares sum to (1 +- e sin w)^2
+    double sw, cw;
+    sincos(w, &sw, &cw);
+    const double q = sqrt(1.0 - e * e) * cw;
+    const double mtr = atan2(q, e + sw) - e * (q / (1.0 + e * sw));
+    const double mec = atan2(-q, e - sw) - e * (-q / (1.0 - e * sw));
     const double ph = (mec - mtr) * p / kTwoPi;
     return ph > 0.0 ? ph : p + ph;
 }
@@ -91,7 +93,10 @@ __global__ void __launch_bounds__(64) ec_orbit_kernel(int npv, const double* P, 
     __syncthreads();
     if (valid && j == 0) taylor_from_stencil(s_x[sub], s_y[sub], s_c[sub]);
     __syncthreads();
-    if (valid && j < 2) s_w[sub][j] = contact_bisect(k, j == 0 ? 1 : 4, s_c[sub], fabs(s_c[sub][1]));
+    if (valid) {
+        const double tc = contact_bisect(k, j < 4 ? 1 : 4, s_c[sub], fabs(s_c[sub][1]));
+        if ((j & 3) == 0) s_w[sub][j >> 2] = tc;
+    }
     __syncthreads();
     if (!inrange) return;
     EcRec* r = rec + pv;

@@ -341,13 +341,39 @@ __device__ __forceinline__ double ta_newton(double t, double p, double e, double
     return atan2(sta, cta);
 }
 
-// Sky-plane position at time t (t0 = 0) for the finite-difference stencil; taylor_z.py:54-76.
+// Sky-plane position at time t (t0 = 0) for the finite-difference stencil;
+// taylor_z.py:54-76 with the orbits_py.py steps of ta_newton.  The setup kernels are
+// bound by this serial chain, so the angles stay sines and cosines: the true anomaly's
+// come from the eccentric anomaly's, the position's from the addition formulas, and
+// sin m of the offset from its atan2's arguments, (e + sin w)^2 + (1 - e^2) cos^2 w =
+// (1 + e sin w)^2.  That leaves one atan2 and, for each Newton step, one sincos of
+// what were two atan2, a fmod and eleven sines and cosines (orbits
+// and contacts of 1,000 pvs 9 -> 6.3 us transiting, 13 -> 8.2 us eclipsing).
 __device__ __forceinline__ void kepler_xy(double t, double p, double a, double ci, double e, double w,
                                           double& x, double& y) {
-    const double f = ta_newton(t, p, e, w);
-    const double r = a * (1.0 - e * e) / (1.0 + e * cos(f));
-    x = -r * cos(w + f);
-    y = -r * sin(w + f) * ci;
+    double sw, cw;
+    sincos(w, &sw, &cw);
+    const double q = 1.0 - e * e, sq = sqrt(q);
+    const double off = atan2(sq * cw, e + sw) - e * (sq * cw / (1.0 + e * sw));
+    double ma = kTwoPi * (t - (0.0 - off * p / kTwoPi)) / p;
+    // py_mod; less than a turn from transit its fmod is the identity
+    if (fabs(ma) < kTwoPi) ma = ma < 0.0 ? ma + kTwoPi : ma;
+    else ma = py_mod(ma, kTwoPi);
+    double ea = ma, err = 0.05, se, ce;
+    sincos(ea, &se, &ce);
+    int k = 0;
+    while (fabs(err) > 1e-8 && k < 1000) {
+        err = ea - e * se - ma;
+        const double step = err / (1.0 - e * ce);
+        ea = ea - step;
+        ++k;
+        if (step != 0.0) sincos(ea, &se, &ce);
+    }
+    const double den = 1.0 / (1.0 - e * ce);
+    const double sta = sq * se * den, cta = (ce - e) * den;
+    const double r = a * q / (1.0 + e * cta);
+    x = -r * (cw * cta - sw * sta);
+    y = -r * (sw * cta + cw * sta) * ci;
 }
 
 // Taylor coefficients from the seven stencil positions x[0..6], y[0..6] at
@@ -380,11 +406,12 @@ __device__ __forceinline__ T taylor_z(T t, const T* c) {
     return d_sqrt(px * px + py * py);
 }
 
-// z_taylor_s(t, t0=0, p=1): Taylor z with a unit-period phase wrap; taylor_z.py:198-226.
-__device__ __forceinline__ double taylor_z_wrapped(double t, const double* c) {
-    const double epoch = floor((t - 0.0 + 0.5 * 1.0) / 1.0);
-    const double tt = t - (0.0 + epoch * 1.0);
-    return taylor_z(tt, c);
+// `v` of lane q of the caller's quad (four neighbouring lanes, all active).
+template <int q>
+__device__ __forceinline__ double quad_lane(double v) {
+    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), 0x55 * q, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), 0x55 * q, 0xf, 0xf, false);
+    return __hiloint2double(hi, lo);
 }
 
 // Contact time by bisection, tol 1e-6 d and at most 100 steps; taylor_z.py:298-328.
@@ -393,25 +420,49 @@ __device__ __forceinline__ double taylor_z_wrapped(double t, const double* c) {
 // sky-plane x velocity (positive at a transit).  The eclipse path passes |vx|:
 // behind the star the planet moves in -x, and v = vx would put first contact after
 // mid-eclipse.
+// Called by the four lanes of a quad with the same arguments.  A step is a chain of
+// some 25 dependent FP64 operations, so two steps share one: the lanes evaluate the
+// next midpoint and both that can follow it, and the brackets taken are the
+// bisection's own.  The sign of z - zt is taken from z^2 - zt^2, without the root.
 __device__ __forceinline__ double contact_bisect(double k, int point, const double* c, double v) {
-    const double s = (point == 1 || point == 2 || point == 12) ? -1.0 : 1.0;
-    const double zt = (point == 1 || point == 4) ? 1.0 + k : ((point == 2 || point == 3) ? 1.0 - k : 1.0);
+    const double s = point == 1 ? -1.0 : 1.0;
+    const double zt = 1.0 + k, zt2 = zt * fabs(zt);
+    const int lane = threadIdx.x & 3;
+    auto above = [&](double t) {
+        const double tt = t - floor(t + 0.5);   // z_taylor_s with p = 1; taylor_z.py:198-226
+        const double x = (((c[4] * tt + c[3]) * tt + c[2]) * tt + c[1]) * tt + c[0];
+        const double y = (((c[9] * tt + c[8]) * tt + c[7]) * tt + c[6]) * tt + c[5];
+        return x * x + y * y - zt2;
+    };
     double t0 = 0.0;
     double t2 = s * 2.0 / v;
     double t1 = 0.5 * t2;
-    double z0 = taylor_z_wrapped(t0, c) - zt;
-    double z1 = taylor_z_wrapped(t1, c) - zt;
+    double d0 = above(lane == 0 ? t0 : t1);
+    double d1 = quad_lane<1>(d0);
+    d0 = quad_lane<0>(d0);
     int i = 0;
     while (fabs(t2 - t0) > 1e-6 && i < 100) {
-        if (z0 * z1 < 0.0) {
+        if (d0 * d1 < 0.0) {
             t2 = t1;
-            t1 = 0.5 * (t0 + t1);
-            z1 = taylor_z_wrapped(t1, c) - zt;
         } else {
             t0 = t1;
-            t1 = 0.5 * (t1 + t2);
-            z0 = z1;
-            z1 = taylor_z_wrapped(t1, c) - zt;
+            d0 = d1;
+        }
+        t1 = 0.5 * (t0 + t2);
+        ++i;
+        const double tl = 0.5 * (t0 + t1), tr = 0.5 * (t1 + t2);
+        const double d = above(lane == 1 ? tl : (lane == 2 ? tr : t1));
+        d1 = quad_lane<0>(d);
+        if (!(fabs(t2 - t0) > 1e-6 && i < 100)) break;
+        if (d0 * d1 < 0.0) {
+            t2 = t1;
+            t1 = tl;
+            d1 = quad_lane<1>(d);
+        } else {
+            t0 = t1;
+            t1 = tr;
+            d0 = d1;
+            d1 = quad_lane<2>(d);
         }
         ++i;
     }
@@ -561,7 +612,7 @@ __device__ __forceinline__ double ld_trapz_segment(int law, const double* c, int
 }
 
 // ---- Orbit for 8 parameter vectors per 64-lane block: lane j (0..6) of a group of 8
-// solves Kepler at t = (j-3)*dt, lane 0 forms the stencils, lanes 0 and 1 find
+// solves Kepler at t = (j-3)*dt, lane 0 forms the stencils, lanes 0-3 and 4-7 find
 // the first and fourth contacts.  Writes coefficients[10] and the window.
 constexpr int kOrbitGroup = 8;
 
@@ -584,7 +635,10 @@ __device__ __forceinline__ void orbit_group(int pv, bool valid, double p, double
     __syncthreads();
     if (valid && j == 0) taylor_from_stencil(s_x, s_y, s_c);
     __syncthreads();
-    if (valid && j < 2) s_w[j] = find_contact_point(kw, j == 0 ? 1 : 4, s_c);
+    if (valid) {
+        const double tc = find_contact_point(kw, j < 4 ? 1 : 4, s_c);
+        if ((j & 3) == 0) s_w[j >> 2] = tc;
+    }
     __syncthreads();
     if (valid) {
         out_c[j] = s_c[j];

@@ -130,7 +130,10 @@ __global__ void __launch_bounds__(64) ts_setup_kernel(TsArgs s) {
     __syncthreads();
     if (valid && j == 0) taylor_from_stencil(s_x[sub], s_y[sub], s_c[sub]);
     __syncthreads();
-    if (valid && j < 2) s_w[sub][j] = find_contact_point(s_km[sub], j == 0 ? 1 : 4, s_c[sub]);
+    if (valid) {
+        const double tc = find_contact_point(s_km[sub], j < 4 ? 1 : 4, s_c[sub]);
+        if ((j & 3) == 0) s_w[sub][j >> 2] = tc;
+    }
     __syncthreads();
     if (valid) {
         TsRec* r = s.rec + q;
