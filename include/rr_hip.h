@@ -65,8 +65,13 @@ typedef struct rr_table {
 /* Limb darkening of one evaluate() call.  law >= 0: a named law (RR_LD_*) with
  * coefficients ldc[npv, npb, nldc], evaluated on the device at tab->mu.
  * law == RR_LD_TABULATED: profiles ldp[npv, npb, nz] and integrals istar[npv, npb]
- * given by the caller (the LDModel protocol, ldmodel.py:21-39). */
+ * given by the caller (the LDModel protocol, ldmodel.py:21-39).
+ * law == RR_LD_BASIS + a named law that is linear in its coefficients (rr_ld_basis_count
+ * > 0): the same law, with ldp the basis table that rr_ld_basis_table made from the
+ * call's weight table and law (RoadRunner entries: rr_setup, rr_evaluate, rr_request,
+ * op_evaluate). */
 #define RR_LD_TABULATED (-1)
+#define RR_LD_BASIS 0x100
 typedef struct rr_ld {
     int32_t law;
     int32_t nldc;
@@ -136,6 +141,16 @@ int rr_z_grid(double zcut, int nin, int nedge, double* ze, double* zm, double* m
  * Replaces calculate_weights_3d (common.py:188-223), called at rrmodel.py:173. */
 int rr_weights_3d(int nk, double kmin, double kmax, const double* ze, int nz, int ng,
                   double* W, float* W32, double* dk_out, double* dg_out, void* stream);
+
+/* Number of basis functions of a law linear in its coefficients, of a fixed number of
+ * them (every named law but general and the power laws); 0 for the others. */
+int rr_ld_basis_count(int law);
+
+/* A law's basis functions contracted with a weight table: out[nk, nb, ng], then the
+ * nb disk integrals of the basis; nb = rr_ld_basis_count(law).  A limb-darkening mean
+ * is then nb products, not nz, at each (k, g).  The values depend on the table and the
+ * law alone.  Device memory of (nk ng + 1) nb doubles. */
+int rr_ld_basis_table(int law, const rr_table* tab, double* out, void* stream);
 
 /* Limb-darkening profiles ldp[npv, npb, nmu] at mu[nmu] and disk integrals
  * istar[npv, npb] for a named law; ldc is [npv, npb, nldc].  Laws without an

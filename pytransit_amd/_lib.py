@@ -29,6 +29,7 @@ LD_LAW_IDS = {
 
 
 RR_LD_TABULATED = -1
+RR_LD_BASIS = 0x100     # + law: with the law's basis table (rr_ld_basis_table)
 
 
 class RRTable(ctypes.Structure):
@@ -100,6 +101,8 @@ _SIGNATURES = {
                               c_void_p]),
     'ts_evaluate': (c_int, [c_int, POINTER(RRTable), POINTER(RRLcData), POINTER(RRParams), POINTER(RRLd),
                             c_void_p, c_size_t, c_void_p, c_void_p]),
+    'rr_ld_basis_count': (c_int, [c_int]),
+    'rr_ld_basis_table': (c_int, [c_int, POINTER(RRTable), c_void_p, c_void_p]),
     'rr_upload': (c_int, [c_int, POINTER(RRPiece), c_void_p, c_size_t, c_void_p]),
     'rr_max_batch': (c_int, []),
     'ma_workspace_bytes': (c_size_t, [c_int]),

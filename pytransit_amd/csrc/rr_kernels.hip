@@ -89,6 +89,38 @@ __global__ void __launch_bounds__(256) weights_3d_kernel(int nk, double kmin, do
 }
 
 // ------------------------------------------------------------------------------------
+// A law's basis means for every (k, g) of the weight table: out[ik][b][ig], lanes over
+// g, then the basis' disk integrals by the last block.  Once per table and law.
+// ------------------------------------------------------------------------------------
+__global__ void __launch_bounds__(64) ld_basis_table_kernel(int law, int nb, int nk, int nz, int ng,
+                                                            const double* __restrict__ W,
+                                                            const double* __restrict__ mu, double* __restrict__ out) {
+    __shared__ double s_y[kTrapzNodes];
+    const int per = (ng + 63) / 64;
+    if (blockIdx.x == (unsigned)(nk * per)) {
+        for (int b = 0; b < nb; ++b) {
+            const double t = ld_basis_trapz_wave(law, b, s_y);
+            if (threadIdx.x == 0) out[(size_t)nk * nb * ng + b] = t;
+        }
+        return;
+    }
+    const int ik = blockIdx.x / per, ig = (blockIdx.x - ik * per) * 64 + threadIdx.x;
+    if (ig >= ng) return;
+    double m[kMaxBasis];
+#pragma unroll
+    for (int b = 0; b < kMaxBasis; ++b) m[b] = 0.0;
+    for (int iz = 0; iz < nz; ++iz) {
+        const double w = W[((size_t)ik * nz + iz) * ng + ig], x = mu[iz];
+#pragma unroll
+        for (int b = 0; b < kMaxBasis; ++b)
+            if (b < nb) m[b] += w * ld_basis(law, b, x);
+    }
+#pragma unroll
+    for (int b = 0; b < kMaxBasis; ++b)
+        if (b < nb) out[((size_t)ik * nb + b) * ng + ig] = m[b];
+}
+
+// ------------------------------------------------------------------------------------
 // Limb-darkening profiles for the rr_ld_profiles entry point (one lane per value;
 // lane iz == 0 also computes the disk integral).
 // ------------------------------------------------------------------------------------
@@ -670,6 +702,75 @@ __device__ __forceinline__ void ld_basis_role(const SetupArgs& s, int pv, int pb
     }
 }
 
+// The limb-darkening role from the law's basis table (rr_ld_basis_table), k0 inside the
+// weight table: the basis means of the pv lerped in k, then for each of the gn passbands
+// ldm(g) = sum_b coef_b M_b(g) and I* likewise or analytic.  The other forms read two
+// table rows of nz nodes for each pv (64 KB at 40 nodes and 100 g), which bounded the
+// setup of large populations by L2 reads and of small ones by five dependent rounds of
+// loads; this one reads 2 nb nodes in one round.  Setup kernel, before and after: 1,500 pvs of
+// the nonlinear law 16.1 -> 7.7 us, 600 pvs in four passbands 22.3 -> 8.8 us, 64 pvs
+// 9.0 -> 7.0 us, where the orbits' chain is what is left.
+// sm: [gn][nb] coefficients, then [gn] disk integrals.
+template <int V>
+__device__ __forceinline__ void basis_table_means(const SetupArgs& s, const double* B, int nb, int gn, size_t j0, double ak,
+                                                  const double* s_coef) {
+    typedef double vec __attribute__((ext_vector_type(V)));
+    const int ng = s.ng;
+    for (int v = threadIdx.x; v < ng / V; v += 64) {
+        double m[kMaxBasis - 1][V];
+#pragma unroll
+        for (int b = 0; b < kMaxBasis - 1; ++b) {
+            if (b < nb) {
+                const vec w0 = *(const vec*)(B + b * ng + V * v), w1 = *(const vec*)(B + (nb + b) * ng + V * v);
+#pragma unroll
+                for (int e = 0; e < V; ++e) m[b][e] = (1.0 - ak) * w0[e] + ak * w1[e];
+            }
+        }
+        for (int q = 0; q < gn; ++q) {
+            const size_t o = (j0 + q) * ng + V * v;
+#pragma unroll
+            for (int e = 0; e < V; ++e) {
+                double val = 0.0;
+#pragma unroll
+                for (int b = 0; b < kMaxBasis - 1; ++b)
+                    if (b < nb) val += s_coef[q * nb + b] * m[b][e];
+                if (s.ldm32) s.ldm32[o + e] = (float)val;
+                else s.ldm64[o + e] = val;
+            }
+        }
+    }
+}
+
+__device__ __forceinline__ void ld_table_role(const SetupArgs& s, int pv, int pb0, int gn, size_t j0, int ik, double ak,
+                                              double* sm) {
+    const int lane = threadIdx.x, nb = ld_basis_count(s.law, s.nldc);
+    double* s_coef = sm;
+    double* s_ist = sm + gn * nb;
+    const double* B = s.ldp_in + (size_t)ik * nb * s.ng;
+    const double* T = s.ldp_in + (size_t)s.nk * nb * s.ng;
+    for (int i = lane; i < gn * nb; i += 64) {
+        const int q = i / nb;
+        s_coef[i] = ld_basis_coef(s.law, i - q * nb, s.ldc + (j0 + q) * s.nldc);
+    }
+    if (lane == 0 && pb0 == 0)
+        s.rec[pv].ldok = isnan(ld_law(s.law, s.mu[0], s.ldc + j0 * s.nldc, s.nldc)) ? 0 : 1;
+    __syncthreads();
+    for (int q = lane; q < gn; q += 64) {
+        double ist;
+        if (!ld_integral(s.law, s.ldc + (j0 + q) * s.nldc, ist)) {
+            ist = 0.0;
+            for (int b = 0; b < nb; ++b) ist += s_coef[q * nb + b] * T[b];
+        }
+        s_ist[q] = ist;
+        s.istar[j0 + q] = ist;
+    }
+    if (s.ng % 2 == 0 && ((uintptr_t)s.ldp_in & 15) == 0) basis_table_means<2>(s, B, nb, gn, j0, ak, s_coef);
+    else basis_table_means<1>(s, B, nb, gn, j0, ak, s_coef);
+    __syncthreads();
+    const int q0 = lc0_pb(s.pbids, s.npb) - pb0;
+    if (lane == 0 && q0 >= 0 && q0 < gn) s.rec[pv].ist_lc0 = s_ist[q0];
+}
+
 // kMulti = false serves launches whose requests all have one passband (every group
 // holds one); it leaves out the group and basis forms, whose registers would make
 // the one-passband blocks spill to scratch.
@@ -699,6 +800,10 @@ __device__ __forceinline__ void setup_ld_role(const SetupArgs& s, int pv, int gr
         return in;
     };
     const size_t j0 = (size_t)pv * s.npb + pb0;
+    if (s.law != RR_LD_TABULATED && s.ldp_in && table_pos()) {
+        ld_table_role(s, pv, pb0, gn, j0, ik, ak, sm);
+        return;
+    }
     if (kMulti && ld_basis_group(nz, s.law, s.nldc, s.npb) > 0) {
         const bool in_table = table_pos();
         ld_basis_role(s, pv, pb0, gn, gs, j0, in_table, ik, ak, k0, sm);
@@ -1891,6 +1996,22 @@ int rr_weights_3d(int nk, double kmin, double kmax, const double* ze, int nz, in
 
 static const int kMinCoeffs[] = {0, 1, 2, 2, 4, 0, 2, 2, 2, 2, 2};
 
+int rr_ld_basis_count(int law) {
+    return law == RR_LD_GENERAL ? 0 : ld_basis_count(law, 0);
+}
+
+int rr_ld_basis_table(int law, const rr_table* tab, double* out, void* stream) {
+    const int nb = rr_ld_basis_count(law);
+    if (nb == 0) return set_error(RR_EINVAL, "rr_ld_basis_table: law %d has no basis", law);
+    if (!tab || !out || !tab->weights || !tab->mu || tab->nk < 2 || tab->ng < 2 || tab->nz < 1)
+        return set_error(RR_EINVAL, "rr_ld_basis_table: bad table or null output");
+    const long long blocks = (long long)tab->nk * ((tab->ng + 63) / 64) + 1;
+    if (blocks > 0x7fffffffLL) return set_error(RR_ERANGE, "rr_ld_basis_table: table too large");
+    hipLaunchKernelGGL(ld_basis_table_kernel, dim3((unsigned)blocks), dim3(64), 0, (hipStream_t)stream, law, nb,
+                       tab->nk, tab->nz, tab->ng, tab->weights, tab->mu, out);
+    return check_launch("ld_basis_table_kernel");
+}
+
 int rr_ld_profiles(int law, const double* ldc, int npv, int npb, int nldc, const double* mu, int nmu, double* ldp,
                    double* istar, void* stream) {
     if (law < RR_LD_UNIFORM || law > RR_LD_POWER_2_PM) return set_error(RR_EINVAL, "rr_ld_profiles: unknown law %d", law);
@@ -2024,15 +2145,18 @@ static int prepare_setup(const char* who, int precision, const rr_table* tab, co
     const int npv = pv->npv, npb = lc->npb;
     if (npv == 0 || lc->npt == 0) return RR_OK;
     if (!ld) return set_error(RR_EINVAL, "%s: null limb-darkening descriptor", who);
-    if (ld->law == RR_LD_TABULATED) {
+    const bool basis = ld->law >= RR_LD_BASIS;
+    const int law = basis ? ld->law - RR_LD_BASIS : ld->law;
+    if (law == RR_LD_TABULATED && !basis) {
         if (!ld->ldp || !ld->istar) return set_error(RR_EINVAL, "%s: tabulated LD needs ldp and istar", who);
     } else {
-        if (ld->law < RR_LD_UNIFORM || ld->law > RR_LD_POWER_2_PM)
+        if (law < RR_LD_UNIFORM || law > RR_LD_POWER_2_PM || (basis && rr_ld_basis_count(law) == 0))
             return set_error(RR_EINVAL, "%s: unknown limb-darkening law %d", who, ld->law);
-        if (ld->nldc < kMinCoeffs[ld->law])
-            return set_error(RR_EINVAL, "%s: law %d needs %d coefficients, got %d", who, ld->law,
-                             kMinCoeffs[ld->law], ld->nldc);
+        if (ld->nldc < kMinCoeffs[law])
+            return set_error(RR_EINVAL, "%s: law %d needs %d coefficients, got %d", who, law,
+                             kMinCoeffs[law], ld->nldc);
         if (ld->nldc > 0 && !ld->ldc) return set_error(RR_EINVAL, "%s: null ldc", who);
+        if (basis && (!ld->ldp || !tab->weights)) return set_error(RR_EINVAL, "%s: null basis or weight table", who);
     }
     if (!pv->k || !pv->p || !pv->a || !pv->inc || !pv->e || !pv->w || !pv->t0)
         return set_error(RR_EINVAL, "%s: null parameter array", who);
@@ -2040,7 +2164,8 @@ static int prepare_setup(const char* who, int precision, const rr_table* tab, co
     WsView v = carve(workspace, npv, lc->npt, npb, tab->ng);
     sa.t0 = pv->t0; sa.pbids = lc->pbids; sa.epids = lc->epids; sa.t0cols = pv->t0cols;
     sa.k = pv->k; sa.p = pv->p; sa.a = pv->a; sa.inc = pv->inc; sa.e = pv->e; sa.w = pv->w;
-    sa.law = ld->law; sa.nldc = ld->nldc; sa.ldc = ld->ldc; sa.ldp_in = ld->ldp; sa.istar_in = ld->istar;
+    sa.law = law; sa.nldc = ld->nldc; sa.ldc = ld->ldc; sa.istar_in = ld->istar;
+    sa.ldp_in = basis || law == RR_LD_TABULATED ? ld->ldp : nullptr;
     sa.W = tab->weights; sa.W32 = tab->weights32; sa.ze = tab->ze; sa.mu = tab->mu;
     sa.rec = v.rec; sa.istar = v.istar;
     sa.ldm64 = precision == RR_FP64 ? v.ldm64 : nullptr;
@@ -2048,8 +2173,8 @@ static int prepare_setup(const char* who, int precision, const rr_table* tab, co
     sa.npv = npv; sa.npb = npb; sa.kcols = pv->kcols; sa.nk = tab->nk; sa.ng = tab->ng; sa.nz = tab->nz;
     sa.kmin = tab->kmin; sa.kmax = tab->kmax; sa.dk = tab->dk;
     sa.n_orbit_blocks = (npv + kOrbitGroup - 1) / kOrbitGroup;
-    sa.ld_lds = ld_lds_doubles(tab->nz, tab->ng, ld->law, ld->nldc, npb);
-    const int gs = ld_group_size(tab->nz, ld->law, ld->nldc, npb);
+    sa.ld_lds = ld_lds_doubles(tab->nz, tab->ng, law, ld->nldc, npb);
+    const int gs = ld_group_size(tab->nz, law, ld->nldc, npb);
     const long long nb = (long long)sa.n_orbit_blocks + (long long)npv * ((npb + gs - 1) / gs);
     if (nb > 0x7fffffffLL) return set_error(RR_ERANGE, "%s: setup grid too large", who);
     nblocks = (int)nb;

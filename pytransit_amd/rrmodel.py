@@ -206,8 +206,22 @@ class RoadRunnerModel(TransitModel):
                           kmax=float(self.klims[1]), dk=self.dk, dg=self.dg, weights=ptr(W), weights32=ptr(W32),
                           ze=ptr(ze), mu=ptr(mu))
             t = (tab, dict(ze=ze, mu=mu, W=W, W32=W32))
+            if self.ldname is not None and device.type == 'cuda':
+                t[1]['basis'] = self._basis_table(LD_LAW_IDS[self.ldname][0], tab, device)
             self._tables[device] = t
         return t
+
+    @staticmethod
+    def _basis_table(law, tab, device):
+        """The basis means of a law linear in its coefficients over the weight table,
+        on the device; None for the other laws."""
+        lib = _lib.load()
+        nb = lib.rr_ld_basis_count(law)
+        if nb == 0:
+            return None
+        out = torch.empty((tab.nk * tab.ng + 1) * nb, dtype=torch.float64, device=device)
+        check(lib.rr_ld_basis_table(law, _lib.ctypes.byref(tab), ptr(out), stream_handle(device)))
+        return out
 
     @property
     def weights(self) -> ndarray:
@@ -359,6 +373,10 @@ class RoadRunnerModel(TransitModel):
             ldc = np.atleast_1d(ldc)
         ld, _ld_keep = self._ld_descriptor(ldc, npv, npb, device)
         tab, _keep = self._table(device)
+        basis = _keep.get('basis')
+        if basis is not None:
+            ld.law += _lib.RR_LD_BASIS
+            ld.ldp = ptr(basis)
         lc = self._lc_descriptor(device, npb, t0.shape[1])
         prm = RRParams(npv, k.shape[1], t0.shape[1], 0, ptr(k), ptr(t0), ptr(p), ptr(a), ptr(inc), ptr(e), ptr(w))
         return npv, tab, lc, prm, ld, (k, t0, p, a, inc, e, w, _ld_keep, _keep)

@@ -439,6 +439,8 @@ class _HipExecutor:
         self.max_batch = min(max_batch, self.lib.rr_max_batch())
         self.model = RoadRunnerModel('quadratic', precision=precision, device=self.device, **table_kw)
         self.table, self._table_keep = self.model._table(self.device)
+        self.basis = {law: self.model._basis_table(law, self.table, self.device) for law, _ in LD_LAW_IDS.values()}
+        torch.cuda.current_stream(self.device).synchronize()   # the slots' streams read the tables
         self.arena = torch.empty(server._arena.capacity, dtype=torch.uint8, device=self.device)
         self.arena_out = self.arena.view(torch.float32 if precision == 'mixed' else torch.float64)
         self.base = self.arena.data_ptr()
@@ -510,14 +512,15 @@ class _HipExecutor:
                                         ('times', 'lcids', 'pbids', 'epids', 'nsamples', 'exptimes')]
             base = self.base + r.offset
             pieces[j] = RRPiece(r.block.ctypes.data, base, r.params.nbytes)
-            o = r.params.off
+            o, basis = r.params.off, self.basis[r.law]
             f0 = r.flux_offset // out.element_size()
             r.flux = out[f0:f0 + r.points].view(r.npv, ds.npt)
             descs[j] = RRRequest(
                 RRLcData(ds.npt, ds.nlc, ds.npb, r.t0cols, int(ds.sorted), ds.uniform_ns, *dptr),
                 RRParams(r.npv, r.kcols, r.t0cols, 0, base + o['k'], base + o['t0'], base + o['p'], base + o['a'],
                          base + o['inc'], base + o['e'], base + o['w']),
-                RRLd(r.law, r.nldc, base + o['ldc'], 0, 0),
+                RRLd(r.law, r.nldc, base + o['ldc'], 0, 0) if basis is None else
+                RRLd(r.law + _lib.RR_LD_BASIS, r.nldc, base + o['ldc'], basis.data_ptr(), 0),
                 base + r.params.nbytes, r.ws_bytes, self.base + r.flux_offset)
         check(lib.rr_upload(len(reqs), pieces, staging.data_ptr(), self.staging_bytes, stream.cuda_stream))
         if self.graphs:
