@@ -987,6 +987,7 @@ struct FluxArgs {
     const double* k; const double* t0; const double* istar;
     const double* ldm64; const float* ldm32;
     int npt, nlc, npb, kcols, t0cols, ng, ntiles;
+    int tile;                         // times per tile, at most kTile
     int uniform_ns;                   // the common nsamples of all light curves, or 0
     int chunk_pts;                    // points per phase-B chunk (uniform_ns > 0)
     int row_lds;                      // stage the limb-darkening row in LDS (one light curve)
@@ -1001,7 +1002,7 @@ struct FluxArgs {
 constexpr int kThreads = 64;
 constexpr int kRun = 8;
 constexpr int kRuns = 2;
-constexpr int kTile = kThreads * kRun * kRuns;       // 1024 times per workgroup
+constexpr int kTile = kThreads * kRun * kRuns;       // most times of a workgroup: 1024
 constexpr int kMaxItems = 1024;                       // (point, sample) items per LDS chunk
 constexpr int kMaxChunk = 64;
 constexpr int kPartQ = 2 * kThreads;                  // queued partial-overlap samples
@@ -1408,12 +1409,12 @@ __device__ __forceinline__ void flux_body(const FluxArgs& f, int pv, int tile) {
     Real* s_row = s_dep + (f.uniform_ns > 0 ? f.chunk_pts * f.uniform_ns : 0);
 
     const int wl = threadIdx.x;
-    const int tbase = tile * kTile;
+    const int tbase = tile * f.tile, tend = min(tbase + f.tile, f.npt);
     int its[kRuns], nrun[kRuns];
 #pragma unroll
     for (int m = 0; m < kRuns; ++m) {
         its[m] = tbase + (m * kThreads + wl) * kRun;
-        nrun[m] = min(kRun, f.npt - its[m]);  // <= 0 past the end
+        nrun[m] = min(kRun, tend - its[m]);  // <= 0 past the end
     }
     const PvRec& r = f.rec[pv];
     Real* out = (Real*)f.flux + (size_t)pv * f.npt;
@@ -1421,7 +1422,7 @@ __device__ __forceinline__ void flux_body(const FluxArgs& f, int pv, int tile) {
     // window shared by all), computed ahead of any branch so that its loads (the
     // record, light curve 0's context, the tile's first and last times) are all in
     // flight together; a pv without a valid record gets NaN.
-    const int tlast = min(tbase + kTile, f.npt) - 1;
+    const int tlast = tend - 1;
     const double t_first = f.times[tbase], t_last = f.times[tlast];
     const bool rec_ok = (r.good != 0) & (r.ldok != 0);
     const PointCtx ctx0 = point_ctx0(f, r);
@@ -1444,7 +1445,7 @@ __device__ __forceinline__ void flux_body(const FluxArgs& f, int pv, int tile) {
     auto stage_lcs = [&]() {
         if (!(kFast && f.nlc > 1)) return;
         la0 = min(max(f.lcids[tbase], 0), f.nlc - 1);
-        const int lb0 = min(max(f.lcids[min(tbase + kTile, f.npt) - 1], 0), f.nlc - 1);
+        const int lb0 = min(max(f.lcids[tlast], 0), f.nlc - 1);
         lc_lds = lb0 != la0 && lb0 - la0 < kTileLcs;
         if (lc_lds) {
             if (wl <= lb0 - la0) s_lc[wl] = point_ctx(f, r, pv, la0 + wl);
@@ -1553,7 +1554,7 @@ __device__ __forceinline__ void flux_body(const FluxArgs& f, int pv, int tile) {
             }
             const int step0 = tbase + m * kThreads * kRun;
             if (__ballot(!all_out) == 0ull) {  // the wave's whole run step is outside the window
-                wave_fill<Real>(out, step0, min(kThreads * kRun, f.npt - step0), Real(1), wl);
+                wave_fill<Real>(out, step0, min(kThreads * kRun, tend - step0), Real(1), wl);
                 continue;
             }
             if (all_out && nrun[m] > 0)
@@ -2181,11 +2182,24 @@ static int prepare_setup(const char* who, int precision, const rr_table* tab, co
     return RR_OK;
 }
 
+// Times per tile.  A tile's samples are one wave's serial chain, so a problem of few
+// tiles takes the smallest that leaves the launch at up to 40 waves per CU; beyond that
+// the cost of a tile itself (its record, window test and row) shows.  64 pvs x 20,000
+// times x 10 samples FP64 at 1024 / 512 / 256 / 128 times: 31.8 / 29.4 / 29.4 / 28.3 us;
+// 250 x 18,000 x 5: 29.6 / 29.5 / 31.0 / 34.4 us; 1,000 x 2,000: 22.9 / 21.5 / 21.4 / 24.8.
+// The requests of a batch fill the chip together and keep 1024 (sixteen requests: 505 us,
+// 545 with their own lengths).
+static int flux_tile(int npv, int npt) {
+    int tile = 128;
+    while (tile < kTile && (long long)npv * (((long long)npt + tile - 1) / tile) > 40 * 256) tile *= 2;
+    return tile;
+}
+
 // Validates one request and fills the flux kernel's arguments, its dynamic LDS
 // bytes and its variant (light curves contiguous and sorted, or general).
 static int prepare_flux(const char* who, int precision, const rr_table* tab, const rr_lcdata* lc,
                         const rr_params* pv, void* workspace, size_t workspace_bytes, void* flux, FluxArgs& fa,
-                        long long& nblocks, size_t& lds, bool& fast) {
+                        long long& nblocks, size_t& lds, bool& fast, bool batch) {
     nblocks = 0;
     int rc = validate(who, precision, tab, lc, pv, workspace_bytes, workspace);
     if (rc) return rc;
@@ -2206,7 +2220,8 @@ static int prepare_flux(const char* who, int precision, const rr_table* tab, con
     fa.uniform_ns = (uns > 0 && uns <= kMaxItems) ? uns : 0;
     fa.chunk_pts = fa.uniform_ns > 0 ? (kMaxItems / fa.uniform_ns < kMaxChunk ? kMaxItems / fa.uniform_ns : kMaxChunk) : 0;
     fa.row_lds = (nlc == 1 && tab->ng <= 2048) ? 1 : 0;
-    fa.ntiles = (npt + kTile - 1) / kTile;
+    fa.tile = batch ? kTile : flux_tile(npv, npt);
+    fa.ntiles = (npt + fa.tile - 1) / fa.tile;
     nblocks = (long long)fa.ntiles * npv;
     if (nblocks > 0x7fffffffLL) return set_error(RR_ERANGE, "%s: grid too large", who);
     fa.npv = npv;
@@ -2238,7 +2253,7 @@ int rr_flux(int precision, const rr_table* tab, const rr_lcdata* lc, const rr_pa
     long long nblocks = 0;
     size_t lds = 0;
     bool fast = false;
-    int rc = prepare_flux("rr_flux", precision, tab, lc, pv, workspace, workspace_bytes, flux, fa, nblocks, lds, fast);
+    int rc = prepare_flux("rr_flux", precision, tab, lc, pv, workspace, workspace_bytes, flux, fa, nblocks, lds, fast, false);
     if (rc || nblocks == 0) return rc;
     hipStream_t s = (hipStream_t)stream;
     // several light curves whose samples the tile kernel's item loops do not take (FP64,
@@ -2295,7 +2310,7 @@ static int plan_batch(const char* who0, int precision, const rr_table* tab, int 
         long long nf = 0;
         size_t l = 0;
         bool fast = false;
-        rc = prepare_flux(who, precision, tab, &q.lc, &q.pv, q.workspace, q.workspace_bytes, q.flux, fa, nf, l, fast);
+        rc = prepare_flux(who, precision, tab, &q.lc, &q.pv, q.workspace, q.workspace_bytes, q.flux, fa, nf, l, fast, true);
         if (rc) return rc;
         if (nb == 0) continue;
         sb.start[sb.n] = (int)sblocks;
