@@ -1373,7 +1373,8 @@ int ts_evaluate(int precision, const rr_table* tab, const rr_lcdata* lc, const r
     const int want = (1024 + npv - 1) / npv, min_rows = 320000 / npt > 64 ? 320000 / npt : 64, most_rows = npb / min_rows;
     a.row_split = want < most_rows ? want : (most_rows > 1 ? most_rows : 1);
     if (uns == 1 && ((uintptr_t)flux % 16) == 0 && (long long)npv * a.row_split >= 256) {
-        if (mixed && npt % 4 == 0 && npt <= ts_row_max_npt<float>() && kTsRowPc * a.ng <= kTsStageRegs * kTsRowThreads &&
+        // (a row of at least one 128-byte line: the rotated slots wrap once)
+        if (mixed && npt % 4 == 0 && npt >= kTsLine && npt <= ts_row_max_npt<float>() && kTsRowPc * a.ng <= kTsStageRegs * kTsRowThreads &&
             ts_rows_aligned_lds(a.ng, npt) <= kTsRowsAlignedMaxLds) {
             hipLaunchKernelGGL(ts_flux_rows_aligned_kernel, dim3((unsigned)npv * a.row_split), dim3(kTsRowThreads),
                                ts_rows_aligned_lds(a.ng, npt), st, a, (float*)flux);

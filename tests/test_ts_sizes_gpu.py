@@ -33,3 +33,18 @@ def test_ts_sizes(gpu, oracle, npv, npb, npt, nss, precision):
                                 wl.ldp[r], wl.istar[r], None, 0, 0, 0, 100, 0, ze)
     assert np.array_equal(np.isnan(f[r]), np.isnan(ref)) and np.nanmin(ref) < 1
     assert np.nanmax(np.abs(f[r] - ref)) <= (1e-9 if precision == 'fp64' else 1e-6)
+
+
+# rows shorter than a cache line, and just as long, with enough pvs for the row forms: every
+# value, and nothing written behind the last row
+@pytest.mark.parametrize('npv,npb,npt', [(257, 3, 4), (300, 5, 8), (256, 9, 20), (256, 6, 28), (256, 6, 32), (260, 3, 36)])
+def test_ts_short_rows(gpu, oracle, npv, npb, npt):
+    wl = workloads.ts_many_pb(npv=npv, npt=npt, npb=npb, seed=npt, mu=TSModel('quadratic', nzin=24, nzlimb=24).mu)
+    tm = TSModel(TabulatedLDModel(wl.ldp, wl.istar), nzin=24, nzlimb=24, precision='mixed')
+    tm.set_data(wl.times)
+    f = tm.evaluate(wl.k, None, wl.t0, wl.p, wl.a, wl.i)
+    ze, _ = oracle.create_z_grid(0.7, 24, 24)
+    ref = oracle.tsmodel_serial(wl.times, wl.k, wl.t0, wl.p, wl.a, wl.i, wl.e, wl.w, 1, 0.0, wl.ldp, wl.istar, None, 0, 0,
+                                0, 100, 0, ze)
+    assert np.nanmin(ref) < 1
+    assert np.nanmax(np.abs(f - ref)) <= 1e-6
