@@ -787,39 +787,96 @@ __global__ void __launch_bounds__(kTsRowThreads) ts_flux_rows_kernel(TsArgs s, R
 // kilobyte.  Rows P = 32 / gcd(npt, 32) apart have the same head and share one
 // load of the coefficients from the table into registers; the per-value
 // arithmetic is the row form's.
+//
+// Bound by HBM's writes, whose rate falls with the span that is being written: a
+// workgroup takes 32 rows of one segment of at most 512 slots, and neighbouring
+// workgroups the segments of the same rows.  1024 pv x 512 x 5,000 (10.5 GB), whole
+// call, against one workgroup of 1024 lanes per pv (2410 us): 64 rows 2357, 32 rows
+// 2286, 16 rows 3363 (too few rows to a load of the coefficients); 300 x 512 x 5,000
+// 746 -> 697 us, 500 x 200 x 1,236 262 -> 225.  Its table is computed by each workgroup
+// (the cores are idle three quarters of the time): one made once per pv and read from
+// memory was slower, 2405 us.
 constexpr int kTsLine = 32;   // FP32 values per 128-byte cache line
-constexpr int kTsStageRegs = 8;   // LD values per thread of a staged chunk: kTsRowPc x ng <= 8 x 1024
+constexpr int kTsAlThreads = 512;
+constexpr int kTsAlPc = 32;        // passbands per staged chunk
+constexpr int kTsAlLd = kTsAlPc + 1;   // LDS stride of one g
+constexpr int kTsStageRegs = 8;    // LD values per thread of a staged chunk: kTsAlPc x ng <= 8 x 512
 constexpr size_t kTsRowsAlignedMaxLds = 160 * 1024;
 
-__host__ __device__ inline size_t ts_rows_table_offset(int ng) { return (ts_rows_lds(ng, 4) + 15) / 16 * 16; }
-__host__ __device__ inline size_t ts_rows_aligned_lds(int ng, int npt) { return ts_rows_table_offset(ng) + (size_t)npt * 5 * 4; }
+__host__ __device__ inline size_t ts_rows_table_offset(int ng) {
+    return (((size_t)kTsAlLd * ng + 3 * kTsAlPc) * 4 + 15) / 16 * 16;
+}
+// Vector slots of a segment of a row of nv, a multiple of a wave, and the segments of the row.
+__host__ __device__ inline int ts_segments(int nv) { return (nv + kTsAlThreads - 1) / kTsAlThreads; }
+__host__ __device__ inline int ts_segment_slots(int nv) {
+    const int n = ts_segments(nv);
+    return ((nv + n - 1) / n + 63) / 64 * 64;
+}
+// Values of a segment's table: its slots' vectors under every rotation (0 to 7 vectors).
+__host__ __device__ inline int ts_segment_values(int nv) { return 4 * (ts_segment_slots(nv) + 8); }
+__host__ __device__ inline size_t ts_rows_aligned_lds(int ng, int npt) {
+    return ts_rows_table_offset(ng) + (size_t)ts_segment_values(npt / 4) * 5 * 4;
+}
 
-__global__ void __launch_bounds__(kTsRowThreads) ts_flux_rows_aligned_kernel(TsArgs s, float* flux) {
+// The row coefficients of time `it` of a pv: LDS offset << 2 | inside << 1 | use, the lerp
+// weights, the area at k_mean and its k-derivative.
+__device__ __forceinline__ void ts_row_coefficients(const TsArgs& s, const TsRec& r, double t0v, double ext, double inv_1pk,
+                                                    double inv_dg, int it, int& pk, float& ra, float& rb, float& a0,
+                                                    float& dk) {
+    using Real = float;
+        double tc;
+        {
+#pragma clang fp contract(off)
+            const double tt = s.times[it];
+            const double epoch = floor((tt - t0v + 0.5 * r.p) * r.inv_p);
+            const double uu = tt - t0v + 0.5 * r.p;
+            const double rem = uu - epoch * r.p;
+            const double ep = epoch + ((rem < 0.0) ? -1.0 : ((rem >= r.p) ? 1.0 : 0.0));
+            tc = tt - (t0v + ep * r.p);
+        }
+        pk = 0;
+        ra = rb = a0 = dk = Real(0);
+        if ((r.bt1 <= tc) && (tc <= r.bt4)) {
+            const TsGeo<Real> g = ts_geometry<Real>(r, tc, ext, 1.0, 0, inv_1pk, inv_dg, s.ng);
+            if (!g.gz) {
+                pk = ((g.ig * kTsAlLd) << 2) | (g.inside ? 2 : 0) | 1;
+                ra = g.ra;
+                rb = g.rb;
+                a0 = g.ap0;
+                dk = g.dadk;
+            }
+        }
+}
+
+__global__ void __launch_bounds__(kTsAlThreads, 4) ts_flux_rows_aligned_kernel(TsArgs s, float* flux) {
     using Real = float;
     constexpr int TPL = ts_tpl<float>();
-    constexpr int NV = ts_row_vec<float>();
     extern __shared__ __align__(16) unsigned char lds[];
-    Real* s_ldm = (Real*)lds;                        // [ng][kTsRowLd]
-    Real* s_afac = s_ldm + (size_t)kTsRowLd * s.ng;
-    Real* s_kd = s_afac + kTsRowPc;
-    Real* s_iist = s_kd + kTsRowPc;
-    const int npt = s.npt, nv = npt / TPL;
+    Real* s_ldm = (Real*)lds;                        // [ng][kTsAlLd]
+    Real* s_afac = s_ldm + (size_t)kTsAlLd * s.ng;
+    Real* s_kd = s_afac + kTsAlPc;
+    Real* s_iist = s_kd + kTsAlPc;
+    const int npt = s.npt, nv = npt / TPL, ntab = ts_segment_values(nv);
     // the row coefficients of every time: LDS offset << 2 | inside << 1 | use, and
     // the lerp weights, the area at k_mean and its k-derivative
     int* t_pk = (int*)(lds + ts_rows_table_offset(s.ng));
-    Real* t_ra = (Real*)(t_pk + npt);
-    Real* t_rb = t_ra + npt;
-    Real* t_a0 = t_rb + npt;
-    Real* t_dk = t_a0 + npt;
+    Real* t_ra = (Real*)(t_pk + ntab);
+    Real* t_rb = t_ra + ntab;
+    Real* t_a0 = t_rb + ntab;
+    Real* t_dk = t_a0 + ntab;
 
-    int pv, qa, qb;      // this workgroup's pv and passbands
-    ts_row_range(s, xcd_remap(blockIdx.x, gridDim.x), pv, qa, qb);
+    // this workgroup's pv, passbands and segment of the rows: slots v0 .. v0 + nslots
+    int pv, qa, qb;
+    const int bid = xcd_remap(blockIdx.x, gridDim.x), nseg = ts_segments(nv), seg = bid % nseg;
+    ts_row_range(s, bid / nseg, pv, qa, qb);
+    const int v0 = seg * ts_segment_slots(nv), nslots = min(ts_segment_slots(nv), nv - v0);
+    const int tid = threadIdx.x;
     const TsRec& r = s.rec[pv];
     float* out = flux + (size_t)pv * s.npb * npt;
     if (!r.good) {
         const f32x4_t vnan = {NAN, NAN, NAN, NAN};
-        for (size_t i = (size_t)qa * nv + threadIdx.x; i < (size_t)qb * nv; i += kTsRowThreads)
-            __builtin_nontemporal_store(vnan, (f32x4_t*)(out + i * TPL));
+        for (int q = qa; q < qb; ++q)
+            if (tid < nslots) __builtin_nontemporal_store(vnan, (f32x4_t*)(out + ((size_t)q * nv + v0 + tid) * TPL));
         return;
     }
     // a chunk's LD rows and per-passband k and disk integral, loaded into registers
@@ -828,58 +885,40 @@ __global__ void __launch_bounds__(kTsRowThreads) ts_flux_rows_aligned_kernel(TsA
     float st[kTsStageRegs];
     double kq = 0.0, isq = 1.0;
     auto stage_load = [&](int pb0) {
-        const int npc = min(kTsRowPc, qb - pb0);
+        const int npc = min(kTsAlPc, qb - pb0);
 #pragma unroll
         for (int m = 0; m < kTsStageRegs; ++m) {
-            const int i = threadIdx.x + m * kTsRowThreads;
+            const int i = tid + m * kTsAlThreads;
             const int q = i / s.ng, g = i - q * s.ng;
-            st[m] = (i < kTsRowPc * s.ng && q < npc) ? s.ldm32[((size_t)pv * s.npb + pb0 + q) * s.ng + g] : 0.0f;
+            st[m] = (i < kTsAlPc * s.ng && q < npc) ? s.ldm32[((size_t)pv * s.npb + pb0 + q) * s.ng + g] : 0.0f;
         }
-        if ((int)threadIdx.x < npc) {
-            kq = s.k[(size_t)pv * s.npb + pb0 + threadIdx.x];
-            isq = s.istar[(size_t)pv * s.npb + pb0 + threadIdx.x];
+        if (tid < npc) {
+            kq = s.k[(size_t)pv * s.npb + pb0 + tid];
+            isq = s.istar[(size_t)pv * s.npb + pb0 + tid];
         }
     };
     auto stage_store = [&](int pb0) {
-        const int npc = min(kTsRowPc, qb - pb0);
+        const int npc = min(kTsAlPc, qb - pb0);
 #pragma unroll
         for (int m = 0; m < kTsStageRegs; ++m) {
-            const int i = threadIdx.x + m * kTsRowThreads;
+            const int i = tid + m * kTsAlThreads;
             const int q = i / s.ng, g = i - q * s.ng;
-            if (i < kTsRowPc * s.ng) s_ldm[g * kTsRowLd + q] = st[m];
+            if (i < kTsAlPc * s.ng) s_ldm[g * kTsAlLd + q] = st[m];
         }
-        if ((int)threadIdx.x < npc) {
-            s_afac[threadIdx.x] = (Real)(kq * kq / (r.kmean * r.kmean));
-            s_kd[threadIdx.x] = (Real)(kq - r.kmean);
-            s_iist[threadIdx.x] = (Real)(1.0 / isq);
+        if (tid < npc) {
+            s_afac[tid] = (Real)(kq * kq / (r.kmean * r.kmean));
+            s_kd[tid] = (Real)(kq - r.kmean);
+            s_iist[tid] = (Real)(1.0 / isq);
         }
     };
     const double ext = s.exptimes[0];
     const double inv_1pk = 1.0 / (1.0 + r.kmean), inv_dg = 1.0 / s.dg;
     const double t0v = s.t0[pv];
-    for (int t = threadIdx.x; t < npt; t += kTsRowThreads) {
-        double tc;
-        {
-#pragma clang fp contract(off)
-            const double tt = s.times[t];
-            const double epoch = floor((tt - t0v + 0.5 * r.p) * r.inv_p);
-            const double uu = tt - t0v + 0.5 * r.p;
-            const double rem = uu - epoch * r.p;
-            const double ep = epoch + ((rem < 0.0) ? -1.0 : ((rem >= r.p) ? 1.0 : 0.0));
-            tc = tt - (t0v + ep * r.p);
-        }
-        int pk = 0;
-        Real ra = Real(0), rb = Real(0), a0 = Real(0), dk = Real(0);
-        if ((r.bt1 <= tc) && (tc <= r.bt4)) {
-            const TsGeo<Real> g = ts_geometry<Real>(r, tc, ext, 1.0, 0, inv_1pk, inv_dg, s.ng);
-            if (!g.gz) {
-                pk = ((g.ig * kTsRowLd) << 2) | (g.inside ? 2 : 0) | 1;
-                ra = g.ra;
-                rb = g.rb;
-                a0 = g.ap0;
-                dk = g.dadk;
-            }
-        }
+    for (int t = tid; t < 4 * (nslots + 8); t += kTsAlThreads) {
+        const int tv = 4 * v0 + t;      // the row's values go round
+        int pk;
+        Real ra, rb, a0, dk;
+        ts_row_coefficients(s, r, t0v, ext, inv_1pk, inv_dg, tv < npt ? tv : tv - npt, pk, ra, rb, a0, dk);
         t_pk[t] = pk;
         t_ra[t] = ra;
         t_rb[t] = rb;
@@ -890,12 +929,12 @@ __global__ void __launch_bounds__(kTsRowThreads) ts_flux_rows_aligned_kernel(TsA
     // rows P apart start equally far past a 128-byte boundary
     const int gl = npt & -npt;   // lowest set bit of npt
     const int P = kTsLine / (gl < kTsLine ? gl : kTsLine);
-    for (int pb0 = qa; pb0 < qb; pb0 += kTsRowPc) {
-        const int npc = min(kTsRowPc, qb - pb0);
+    for (int pb0 = qa; pb0 < qb; pb0 += kTsAlPc) {
+        const int npc = min(kTsAlPc, qb - pb0);
         __syncthreads();  // the previous chunk's rows are no longer read (and the table is written)
         stage_store(pb0);
         __syncthreads();
-        if (pb0 + kTsRowPc < qb) stage_load(pb0 + kTsRowPc);
+        if (pb0 + kTsAlPc < qb) stage_load(pb0 + kTsAlPc);
         for (int q0 = pb0; q0 < pb0 + min(P, npc); ++q0) {
             // this class's head, and each slot's coefficients from the table
             const int mis = (int)(((uintptr_t)(out + (size_t)q0 * npt) >> 2) & (kTsLine - 1));
@@ -904,65 +943,54 @@ __global__ void __launch_bounds__(kTsRowThreads) ts_flux_rows_aligned_kernel(TsA
             // the planet is inside the disk, where it scales by afac) and its
             // k-derivative (0 inside); bit u * TPL + j of `use` marks a value in the
             // window with g <= 1
-            int vi[NV], off[NV][TPL];
-            Real rb[NV][TPL], ra[NV][TPL], as[NV][TPL], dk[NV][TPL];
+            const int lv = tid + head, vi = v0 + lv < nv ? v0 + lv : v0 + lv - nv;
+            int off[TPL];
+            Real rb[TPL], ra[TPL], as[TPL], dk[TPL];
             unsigned use = 0u;
-            bool act[NV];
 #pragma unroll
-            for (int u = 0; u < NV; ++u) {
-                const int slot = threadIdx.x + u * kTsRowThreads;
-                vi[u] = slot + head < nv ? slot + head : slot + head - nv;
-                bool any = false;
+            for (int j = 0; j < TPL; ++j) {
+                off[j] = 0;
+                ra[j] = rb[j] = as[j] = dk[j] = Real(0);
+            }
+            if (tid < nslots) {
+                const int4 pk4 = *(const int4*)(t_pk + TPL * lv);
+                const f32x4_t ra4 = *(const f32x4_t*)(t_ra + TPL * lv);
+                const f32x4_t rb4 = *(const f32x4_t*)(t_rb + TPL * lv);
+                const f32x4_t a04 = *(const f32x4_t*)(t_a0 + TPL * lv);
+                const f32x4_t dk4 = *(const f32x4_t*)(t_dk + TPL * lv);
+                const int pk[TPL] = {pk4.x, pk4.y, pk4.z, pk4.w};
 #pragma unroll
                 for (int j = 0; j < TPL; ++j) {
-                    off[u][j] = 0;
-                    ra[u][j] = rb[u][j] = as[u][j] = dk[u][j] = Real(0);
+                    const bool inside = (pk[j] & 2) != 0;
+                    if (pk[j] & 1) use |= 1u << j;
+                    off[j] = pk[j] >> 2;
+                    ra[j] = ra4[j];
+                    rb[j] = rb4[j];
+                    as[j] = inside ? -a04[j] : a04[j];
+                    dk[j] = inside ? Real(0) : dk4[j];
                 }
-                if (slot < nv) {
-                    const int4 pk4 = *(const int4*)(t_pk + TPL * vi[u]);
-                    const f32x4_t ra4 = *(const f32x4_t*)(t_ra + TPL * vi[u]);
-                    const f32x4_t rb4 = *(const f32x4_t*)(t_rb + TPL * vi[u]);
-                    const f32x4_t a04 = *(const f32x4_t*)(t_a0 + TPL * vi[u]);
-                    const f32x4_t dk4 = *(const f32x4_t*)(t_dk + TPL * vi[u]);
-                    const int pk[TPL] = {pk4.x, pk4.y, pk4.z, pk4.w};
-#pragma unroll
-                    for (int j = 0; j < TPL; ++j) {
-                        const bool inside = (pk[j] & 2) != 0;
-                        if (pk[j] & 1) use |= 1u << (u * TPL + j);
-                        any = any || (pk[j] & 1) != 0;
-                        off[u][j] = pk[j] >> 2;
-                        ra[u][j] = ra4[j];
-                        rb[u][j] = rb4[j];
-                        as[u][j] = inside ? -a04[j] : a04[j];
-                        dk[u][j] = inside ? Real(0) : dk4[j];
-                    }
-                }
-                act[u] = __ballot(any) != 0ull;
             }
+            const bool act = __ballot(use != 0u) != 0ull;
 #pragma unroll 1
             for (int q = q0; q < pb0 + npc; q += P) {
                 const int ql = q - pb0;
                 const Real f = s_iist[ql], afac = s_afac[ql], kd = s_kd[ql];
                 const Real* lq = s_ldm + ql;
                 float* o = out + (size_t)q * npt;
+                if (tid < nslots) {
+                    f32x4_t w = {1.0f, 1.0f, 1.0f, 1.0f};
+                    if (act) {
 #pragma unroll
-                for (int u = 0; u < NV; ++u) {
-                    const int slot = threadIdx.x + u * kTsRowThreads;
-                    if (slot < nv) {
-                        f32x4_t w = {1.0f, 1.0f, 1.0f, 1.0f};
-                        if (act[u]) {
-#pragma unroll
-                            for (int j = 0; j < TPL; ++j) {
-                                const Real* l = lq + off[u][j];
-                                const Real ip = rb[u][j] * l[0] + ra[u][j] * l[kTsRowLd];
-                                // the row form's c1 afac + (c2 + c3 (k - k_mean)), with c1 = A0
-                                // inside and c2 = A0, c3 = 2 k_mean kappa_0 otherwise
-                                const Real area = as[u][j] < Real(0) ? (-as[u][j]) * afac : dk[u][j] * kd + as[u][j];
-                                w[j] = ((use >> (u * TPL + j)) & 1u) ? Real(1) - (ip * area) * f : Real(1);
-                            }
+                        for (int j = 0; j < TPL; ++j) {
+                            const Real* l = lq + off[j];
+                            const Real ip = rb[j] * l[0] + ra[j] * l[kTsAlLd];
+                            // the row form's c1 afac + (c2 + c3 (k - k_mean)), with c1 = A0
+                            // inside and c2 = A0, c3 = 2 k_mean kappa_0 otherwise
+                            const Real area = as[j] < Real(0) ? (-as[j]) * afac : dk[j] * kd + as[j];
+                            w[j] = ((use >> j) & 1u) ? Real(1) - (ip * area) * f : Real(1);
                         }
-                        __builtin_nontemporal_store(w, (f32x4_t*)(o + (size_t)vi[u] * TPL));
                     }
+                    __builtin_nontemporal_store(w, (f32x4_t*)(o + (size_t)vi * TPL));
                 }
             }
         }
@@ -1366,20 +1394,25 @@ int ts_evaluate(int precision, const rr_table* tab, const rr_lcdata* lc, const r
     const int uns = lc->uniform_nsamples;
     // one sample, rows of whole 16-byte vectors: the row form, where it gives every CU a
     // workgroup.  A pv's passbands go to several workgroups (1024 in all) if each keeps
-    // 64 rows and 320,000 values to pay for its geometry: 300 pv x 512 x 5,000 mixed 798
-    // -> 724 us with 4; 500 x 200 x 1,236 would go from 221 to 245.  With fewer
-    // workgroups than CUs the tiles below are faster (8 x 200 x 1,236: 95 -> 39 us, 128:
-    // 104 -> 72 us; at 256 125 against 130).
+    // 64 rows and 320,000 values to pay for its geometry.  With fewer workgroups than CUs
+    // the tiles below are faster (8 x 200 x 1,236 mixed: 95 -> 39 us).
     const int want = (1024 + npv - 1) / npv, min_rows = 320000 / npt > 64 ? 320000 / npt : 64, most_rows = npb / min_rows;
     a.row_split = want < most_rows ? want : (most_rows > 1 ? most_rows : 1);
-    if (uns == 1 && ((uintptr_t)flux % 16) == 0 && (long long)npv * a.row_split >= 256) {
-        // (a row of at least one 128-byte line: the rotated slots wrap once)
-        if (mixed && npt % 4 == 0 && npt >= kTsLine && npt <= ts_row_max_npt<float>() && kTsRowPc * a.ng <= kTsStageRegs * kTsRowThreads &&
-            ts_rows_aligned_lds(a.ng, npt) <= kTsRowsAlignedMaxLds) {
-            hipLaunchKernelGGL(ts_flux_rows_aligned_kernel, dim3((unsigned)npv * a.row_split), dim3(kTsRowThreads),
+    // FP32 rows in whole cache lines (of at least one: the rotated slots wrap once), where
+    // that gives every CU a workgroup (aligned against the forms below, us: 8 x 200 x 1,236
+    // 47.7 / 45.5, 64 x 200 x 1,236 59.5 / 61.8, 32 x 512 x 5,000 111 / 139)
+    if (mixed && uns == 1 && ((uintptr_t)flux % 16) == 0 && npt % 4 == 0 && npt >= kTsLine && npt <= ts_row_max_npt<float>() &&
+        kTsAlPc * a.ng <= kTsStageRegs * kTsAlThreads && ts_rows_aligned_lds(a.ng, npt) <= kTsRowsAlignedMaxLds) {
+        const int split = (npb + kTsAlPc - 1) / kTsAlPc;
+        const long long nwg = (long long)npv * split * ts_segments(npt / 4);
+        if (nwg >= 256 && nwg <= 0x7fffffffLL) {
+            a.row_split = split;
+            hipLaunchKernelGGL(ts_flux_rows_aligned_kernel, dim3((unsigned)nwg), dim3(kTsAlThreads),
                                ts_rows_aligned_lds(a.ng, npt), st, a, (float*)flux);
             return check_launch("ts_flux_rows_aligned_kernel");
         }
+    }
+    if (uns == 1 && ((uintptr_t)flux % 16) == 0 && (long long)npv * a.row_split >= 256) {
         if (mixed && npt % 4 == 0 && npt <= ts_row_max_npt<float>() && ts_rows_lds(a.ng, 4) <= 64 * 1024) {
             hipLaunchKernelGGL(ts_flux_rows_kernel<float>, dim3((unsigned)npv * a.row_split), dim3(kTsRowThreads),
                                ts_rows_lds(a.ng, 4), st, a, (float*)flux);
