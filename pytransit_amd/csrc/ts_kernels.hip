@@ -543,6 +543,71 @@ __global__ void __launch_bounds__(256) ts_ldm_f32_kernel(TsArgs s) {
     s.ldm32[idx] = (float)d;
 }
 
+// ---- a law linear in its coefficients ----------------------------------------------
+//
+// Its basis functions are the same for every passband: a workgroup contracts the nb of
+// them with the pv's weights into M_b(g) in LDS and writes ldm = sum_b coef_b M_b(g) of
+// its passbands in order, in place of npb contractions of nz nodes.  FP64 sums, FP32
+// means.  Quadratic law, mixed, whole call against the MFMA contraction: 300 x 512 x
+// 1,000 230 -> 186 us, 1,024 x 512 x 1,000 645 -> 584, 8 x 200 x 1,237 39.7 -> 37.6.  FP64
+// stays on MFMA: 100 x 203 x 1,237 x 3 96.6 us, 100.6 in this form.
+// The nodes are split over the parts of a workgroup that its lanes over g leave.
+__host__ __device__ inline int ts_basis_parts(int ng) {
+    const int gw = (ng + 63) / 64 * 64;
+    return gw >= 256 ? 1 : 256 / gw;
+}
+__host__ __device__ inline size_t ts_basis_lds(int nb, int nz, int ng, int pbs) {
+    return (size_t)nb * (nz + ts_basis_parts(ng) * ng + pbs) * sizeof(double);
+}
+
+__global__ void __launch_bounds__(256) ts_ldm_basis_kernel(TsArgs s, int nb) {
+    extern __shared__ double lds_basis[];
+    const int pv = blockIdx.x / s.ldm_split, part = blockIdx.x - pv * s.ldm_split, tid = threadIdx.x;
+    const int per = (s.npb + s.ldm_split - 1) / s.ldm_split, pa = min(part * per, s.npb), np = min(per, s.npb - pa);
+    const int nz = s.nz, ng = s.ng, parts = ts_basis_parts(ng);
+    double* s_B = lds_basis;                     // [nb][nz]
+    double* s_M = s_B + nb * nz;                 // [parts][nb][ng]
+    double* s_c = s_M + parts * nb * ng;         // [np][nb]
+    const size_t j0 = (size_t)pv * s.npb + pa;
+    for (int i = tid; i < nb * nz; i += 256) s_B[i] = ld_basis(s.law, i / nz, s.mu[i % nz]);
+    for (int i = tid; i < np * nb; i += 256) s_c[i] = ld_basis_coef(s.law, i % nb, s.ldc + (j0 + i / nb) * s.nldc);
+    __syncthreads();
+    const float* w = s.w2_32 + (size_t)pv * s.nzp * s.ngp;
+    const int gw = 256 / parts, zp = tid / gw, zn = (nz + parts - 1) / parts, za = zp * zn, ze = min(za + zn, nz);
+    for (int g = tid - zp * gw; g < ng; g += gw) {
+        double m[kMaxBasis];
+#pragma unroll
+        for (int b = 0; b < kMaxBasis; ++b) m[b] = 0.0;
+        constexpr int kB = 20;                   // loads in flight
+        for (int z0 = za; z0 < ze; z0 += kB) {
+            float v[kB];
+#pragma unroll
+            for (int u = 0; u < kB; ++u) v[u] = w[(size_t)min(z0 + u, ze - 1) * s.ngp + g];
+#pragma unroll
+            for (int u = 0; u < kB; ++u) {
+                if (z0 + u < ze) {
+#pragma unroll
+                    for (int b = 0; b < kMaxBasis; ++b)
+                        if (b < nb) m[b] += (double)v[u] * s_B[b * nz + z0 + u];
+                }
+            }
+        }
+#pragma unroll
+        for (int b = 0; b < kMaxBasis; ++b)
+            if (b < nb) s_M[(zp * nb + b) * ng + g] = m[b];
+    }
+    __syncthreads();
+    for (int i = tid; i < nb * ng; i += 256)
+        for (int p = 1; p < parts; ++p) s_M[i] += s_M[p * nb * ng + i];
+    __syncthreads();
+    for (int i = tid; i < np * ng; i += 256) {
+        const int q = i / ng, g = i - q * ng;
+        double v = 0.0;
+        for (int b = 0; b < nb; ++b) v += s_c[q * nb + b] * s_M[b * ng + g];
+        s.ldm32[j0 * ng + i] = (float)v;
+    }
+}
+
 // ---- flux --------------------------------------------------------------------------
 constexpr int kTsThreads = 256;
 
@@ -1343,7 +1408,17 @@ int ts_evaluate(int precision, const rr_table* tab, const rr_lcdata* lc, const r
     };
     const bool tab_rows = mixed && tab_ld && a.nz % 4 == 0 && a.nz <= 16 * kTabMfmaMaxJ && nct <= kTabMfmaMaxCt &&
                           ((uintptr_t)ld->ldp & 15) == 0;
-    if (tab_rows) {
+    const int nbasis = !mixed || tab_ld ? 0 : ld_basis_count(ld->law, ld->nldc);
+    if (nbasis > 0) {
+        // workgroups for every CU four times, of at least 8 passbands each and at most 128
+        const int want = (1024 + npv - 1) / npv, most = (npb + 7) / 8, least = (npb + 127) / 128;
+        a.ldm_split = want < least ? least : (want < most ? want : most);
+        const size_t lds = ts_basis_lds(nbasis, a.nz, a.ng, (npb + a.ldm_split - 1) / a.ldm_split);
+        if ((long long)npv * a.ldm_split > 0x7fffffffLL) return set_error(RR_ERANGE, "ts_evaluate: grid too large");
+        const dim3 g((unsigned)npv * a.ldm_split);
+        hipLaunchKernelGGL(ts_ldm_basis_kernel, g, dim3(256), lds, st, a, nbasis);
+        if ((rc = check_launch("ts_ldm_basis_kernel"))) return rc;
+    } else if (tab_rows) {
         const size_t lds = (size_t)((a.nz + 15) / 16 * 16) * ts_tab_ldb(a.ngp) * sizeof(float);
         a.ldm_split = ldm_split(kTabMfmaThreads / 64);
         const dim3 g((unsigned)npv * a.ldm_split), b(kTabMfmaThreads);

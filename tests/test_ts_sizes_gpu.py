@@ -66,3 +66,23 @@ def test_ts_row_segments(gpu, oracle, npv, npb, npt):
                                 wl.istar[r], None, 0, 0, 0, 100, 0, ze)
     assert np.nanmin(ref) < 1
     assert np.nanmax(np.abs(f[r] - ref)) <= 1e-6
+
+
+# named laws: those linear in their coefficients through their basis (mixed), against the
+# oracle's profiles; one and several workgroups of passbands, even and odd numbers of g
+@pytest.mark.parametrize('law,nc', [('linear', 1), ('quadratic', 2), ('quadratic-tri', 2), ('nonlinear', 4), ('general', 3),
+                                    ('square_root', 2), ('power-2', 2)])
+@pytest.mark.parametrize('npb,ng', [(1, 100), (9, 51), (150, 64), (40, 300)])
+def test_ts_named_laws(gpu, oracle, law, nc, npb, ng):
+    rng = np.random.default_rng(npb + nc)
+    tm = TSModel(law, nzin=24, nzlimb=24, ng=ng, precision='mixed')
+    wl = workloads.ts_many_pb(npv=3, npt=300, npb=npb, seed=nc, mu=tm.mu)
+    ldc = rng.uniform(0.1, 0.4, (3, npb, nc))
+    tm.set_data(wl.times)
+    f = tm.evaluate(wl.k, ldc, wl.t0, wl.p, wl.a, wl.i)
+    ze, _ = oracle.create_z_grid(0.7, 24, 24)
+    ldp, istar = oracle.evaluate_ld(law, tm.mu, ldc)
+    ref = oracle.tsmodel_serial(wl.times, wl.k, wl.t0, wl.p, wl.a, wl.i, wl.e, wl.w, 1, 0.0, ldp, istar, None, 0, 0, 0, ng, 0,
+                                ze)
+    assert np.nanmin(ref) < 1
+    assert np.nanmax(np.abs(f - ref)) <= 1e-6
