@@ -439,8 +439,7 @@ class _HipExecutor:
         self.max_batch = min(max_batch, self.lib.rr_max_batch())
         self.model = RoadRunnerModel('quadratic', precision=precision, device=self.device, **table_kw)
         self.table, self._table_keep = self.model._table(self.device)
-        self.basis = {law: self.model._basis_table(law, self.table, self.device) for law, _ in LD_LAW_IDS.values()}
-        torch.cuda.current_stream(self.device).synchronize()   # the slots' streams read the tables
+        self.basis = {}     # law -> its basis table or None
         self.arena = torch.empty(server._arena.capacity, dtype=torch.uint8, device=self.device)
         self.arena_out = self.arena.view(torch.float32 if precision == 'mixed' else torch.float64)
         self.base = self.arena.data_ptr()
@@ -495,6 +494,14 @@ class _HipExecutor:
             ds.ready.synchronize()
         ds._staging = None
 
+    def _law_basis(self, law: int):
+        """The basis table of a law, made at its first request; the slots' streams read
+        it from then on, so its kernel is waited for."""
+        if law not in self.basis:
+            self.basis[law] = self.model._basis_table(law, self.table, self.device)
+            torch.cuda.current_stream(self.device).synchronize()
+        return self.basis[law]
+
     def launch(self, slot: int, reqs: List[Request]):
         stream, staging = self.streams[slot], self.staging[slot]
         lib = self.lib
@@ -512,7 +519,7 @@ class _HipExecutor:
                                         ('times', 'lcids', 'pbids', 'epids', 'nsamples', 'exptimes')]
             base = self.base + r.offset
             pieces[j] = RRPiece(r.block.ctypes.data, base, r.params.nbytes)
-            o, basis = r.params.off, self.basis[r.law]
+            o, basis = r.params.off, self._law_basis(r.law)
             f0 = r.flux_offset // out.element_size()
             r.flux = out[f0:f0 + r.points].view(r.npv, ds.npt)
             descs[j] = RRRequest(
