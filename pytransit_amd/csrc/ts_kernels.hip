@@ -704,6 +704,7 @@ constexpr int kTsRowThreads = 1024;
 constexpr int kTsRowPc = 64;      // passbands per staged chunk
 constexpr int kTsRowLd = kTsRowPc + 1;   // LDS stride of one g
 constexpr int kTsRowQ = 16;       // passbands per unrolled group
+constexpr int kTsRowSplit = 32;   // passbands of a workgroup
 // time vectors (16 bytes: 4 FP32 or 2 FP64 times) per thread; npt <= 8192 (FP32), 6144 (FP64)
 template <typename Real> constexpr int ts_row_vec() { return sizeof(Real) == 4 ? 2 : 3; }
 template <typename Real> constexpr int ts_row_max_npt() { return kTsRowThreads * ts_row_vec<Real>() * ts_tpl<Real>(); }
@@ -1467,34 +1468,36 @@ int ts_evaluate(int precision, const rr_table* tab, const rr_lcdata* lc, const r
     const dim3 block(kTsThreads);
     // nsamples[0] as given by the host (0: unknown)
     const int uns = lc->uniform_nsamples;
-    // one sample, rows of whole 16-byte vectors: the row form, where it gives every CU a
-    // workgroup.  A pv's passbands go to several workgroups (1024 in all) if each keeps
-    // 64 rows and 320,000 values to pay for its geometry.  With fewer workgroups than CUs
-    // the tiles below are faster (8 x 200 x 1,236 mixed: 95 -> 39 us).
-    const int want = (1024 + npv - 1) / npv, min_rows = 320000 / npt > 64 ? 320000 / npt : 64, most_rows = npb / min_rows;
-    a.row_split = want < most_rows ? want : (most_rows > 1 ? most_rows : 1);
     // FP32 rows in whole cache lines (of at least one: the rotated slots wrap once), where
     // that gives every CU a workgroup (aligned against the forms below, us: 8 x 200 x 1,236
     // 47.7 / 45.5, 64 x 200 x 1,236 59.5 / 61.8, 32 x 512 x 5,000 111 / 139)
     if (mixed && uns == 1 && ((uintptr_t)flux % 16) == 0 && npt % 4 == 0 && npt >= kTsLine && npt <= ts_row_max_npt<float>() &&
         kTsAlPc * a.ng <= kTsStageRegs * kTsAlThreads && ts_rows_aligned_lds(a.ng, npt) <= kTsRowsAlignedMaxLds) {
-        const int split = (npb + kTsAlPc - 1) / kTsAlPc;
-        const long long nwg = (long long)npv * split * ts_segments(npt / 4);
+        a.row_split = (npb + kTsAlPc - 1) / kTsAlPc;
+        const long long nwg = (long long)npv * a.row_split * ts_segments(npt / 4);
         if (nwg >= 256 && nwg <= 0x7fffffffLL) {
-            a.row_split = split;
             hipLaunchKernelGGL(ts_flux_rows_aligned_kernel, dim3((unsigned)nwg), dim3(kTsAlThreads),
                                ts_rows_aligned_lds(a.ng, npt), st, a, (float*)flux);
             return check_launch("ts_flux_rows_aligned_kernel");
         }
     }
-    if (uns == 1 && ((uintptr_t)flux % 16) == 0 && (long long)npv * a.row_split >= 256) {
+    // one sample, rows of whole 16-byte vectors: 32 rows a workgroup, which computes its
+    // geometry in registers (FP64 against one workgroup or few per pv: 1,024 x 256 x 5,000
+    // 2187 -> 2135 us, 300 x 200 x 2,000 283 -> 245, 260 x 512 x 3,000 757 -> 717), where that
+    // is a workgroup for every CU and 24 million values (rows against the tiles below, FP64,
+    // us: 64 x 200 x 1,236 67.9 / 63.0, 128 x 200 x 1,236 101 / 109, 20 x 512 x 5,000 127 / 146,
+    // 8 x 512 x 5,000 71.7 / 64.3)
+    a.row_split = (npb + kTsRowSplit - 1) / kTsRowSplit;
+    const long long nrow = (long long)npv * a.row_split;
+    if (uns == 1 && ((uintptr_t)flux % 16) == 0 && nrow >= 256 && nrow <= 0x7fffffffLL &&
+        (long long)npv * npb * npt >= 24000000LL) {
         if (mixed && npt % 4 == 0 && npt <= ts_row_max_npt<float>() && ts_rows_lds(a.ng, 4) <= 64 * 1024) {
-            hipLaunchKernelGGL(ts_flux_rows_kernel<float>, dim3((unsigned)npv * a.row_split), dim3(kTsRowThreads),
+            hipLaunchKernelGGL(ts_flux_rows_kernel<float>, dim3((unsigned)nrow), dim3(kTsRowThreads),
                                ts_rows_lds(a.ng, 4), st, a, (float*)flux);
             return check_launch("ts_flux_rows_kernel");
         }
         if (!mixed && npt % 2 == 0 && npt <= ts_row_max_npt<double>() && ts_rows_lds(a.ng, 8) <= 64 * 1024) {
-            hipLaunchKernelGGL(ts_flux_rows_kernel<double>, dim3((unsigned)npv * a.row_split), dim3(kTsRowThreads),
+            hipLaunchKernelGGL(ts_flux_rows_kernel<double>, dim3((unsigned)nrow), dim3(kTsRowThreads),
                                ts_rows_lds(a.ng, 8), st, a, (double*)flux);
             return check_launch("ts_flux_rows_kernel");
         }

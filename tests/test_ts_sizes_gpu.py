@@ -86,3 +86,20 @@ def test_ts_named_laws(gpu, oracle, law, nc, npb, ng):
                                 ze)
     assert np.nanmin(ref) < 1
     assert np.nanmax(np.abs(f - ref)) <= 1e-6
+
+
+# FP64 rows, 32 passbands a workgroup: one past a workgroup's rows and one short, the longest row
+@pytest.mark.parametrize('npv,npb,npt', [(260, 33, 3000), (300, 31, 2600), (90, 97, 3072)])
+def test_ts_fp64_rows(gpu, oracle, npv, npb, npt):
+    wl = workloads.ts_many_pb(npv=npv, npt=npt, npb=npb, seed=npt, mu=TSModel('quadratic', nzin=24, nzlimb=24).mu)
+    wl.a[1] = 0.5                           # an invalid vector
+    tm = TSModel(TabulatedLDModel(wl.ldp, wl.istar), nzin=24, nzlimb=24)
+    tm.set_data(wl.times)
+    f = tm.evaluate(wl.k, None, wl.t0, wl.p, wl.a, wl.i)
+    assert np.isnan(f[1]).all() and not np.isnan(np.delete(f, 1, 0)).any()
+    r = np.array([0, 1, npv - 1])
+    ze, _ = oracle.create_z_grid(0.7, 24, 24)
+    ref = oracle.tsmodel_serial(wl.times, wl.k[r], wl.t0[r], wl.p[r], wl.a[r], wl.i[r], wl.e[r], wl.w[r], 1, 0.0, wl.ldp[r],
+                                wl.istar[r], None, 0, 0, 0, 100, 0, ze)
+    assert np.nanmin(ref) < 1
+    assert np.nanmax(np.abs(f[r] - ref)) <= 1e-9
