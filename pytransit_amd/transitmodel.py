@@ -12,7 +12,7 @@ import numpy as np
 import torch
 from numpy import asarray, atleast_1d, float64, integer, issubdtype, ndarray, ones, unique, zeros
 
-from ._lib import RRLcData, ptr
+from ._lib import RRLcData
 
 
 def runs_sorted(time: ndarray, lcids: ndarray) -> bool:
@@ -138,7 +138,7 @@ class TransitModel:
             if (nsamples < 1).any():
                 raise ValueError('nsamples must be >= 1')
             d = dict(
-                sorted=layout_flags(self.time, self.lcids, self.epids, self._per_lc(self.exptimes, np.float64)),
+                sorted=int(layout_flags(self.time, self.lcids, self.epids, self._per_lc(self.exptimes, np.float64))),
                 uniform_ns=int(nsamples[0]) if (nsamples == nsamples[0]).all() else 0,
                 times=torch.as_tensor(np.ascontiguousarray(self.time), device=device),
                 lcids=torch.as_tensor(self.lcids.astype(np.int32), device=device),
@@ -152,16 +152,12 @@ class TransitModel:
 
     def _lc_descriptor(self, device, npb: int, nep: int, epids: str = 'epids', uniform_ns=None) -> RRLcData:
         """The C-ABI view of the device copies; ``epids`` names the array passed as
-        epoch indices.  Only the pointers and flags of a set_data are laid out once
-        (12 us of ctypes each call): the sizes are the call's."""
+        epoch indices.  The addresses are read from the tensors at each call: a copied
+        or unpickled model has arrays of its own."""
         d = self._device_data(device)
-        a = d.get('c')
-        if a is None:
-            a = d['c'] = ((int(d['sorted']), d['uniform_ns'], ptr(d['times']), ptr(d['lcids']), ptr(d['pbids'])),
-                          {x: ptr(d[x]) for x in ('epids', 'pbids')}, (ptr(d['nsamples']), ptr(d['exptimes'])))
-        (srt, uns, *arrays), ids, tail = a
-        return RRLcData(self.npt, self.nlc, npb, nep, srt, uns if uniform_ns is None else uniform_ns, *arrays,
-                        ids[epids], *tail)
+        return RRLcData(self.npt, self.nlc, npb, nep, d['sorted'], d['uniform_ns'] if uniform_ns is None else uniform_ns,
+                        d['times'].data_ptr(), d['lcids'].data_ptr(), d['pbids'].data_ptr(), d[epids].data_ptr(),
+                        d['nsamples'].data_ptr(), d['exptimes'].data_ptr())
 
     def __call__(self, *nargs, **kwargs):
         raise NotImplementedError
