@@ -203,6 +203,13 @@ def stream_handle(device) -> int:
     return torch.cuda.current_stream(device).cuda_stream
 
 
+def synchronize_stream(device) -> None:
+    """Waits for torch's current stream on ``device``: what was launched there may be
+    read on any stream afterwards."""
+    if device.type == 'cuda':
+        torch.cuda.current_stream(device).synchronize()
+
+
 def z_grid(zcut: float, nin: int, nedge: int):
     """Host call of rr_z_grid; returns (ze, zm, mu) as float64 numpy arrays."""
     import numpy as np

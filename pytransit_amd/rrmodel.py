@@ -187,7 +187,8 @@ class RoadRunnerModel(TransitModel):
 
     def _table(self, device):
         """Device-resident z grid, mu nodes and weight table (FP64 and FP32 copies, in
-        the device layout [nk, nz, ng]); returns (RRTable, keep-alive dict)."""
+        the device layout [nk, nz, ng]); returns (RRTable, keep-alive dict).  Complete
+        when it is kept, so calls on any stream may read it."""
         t = self._tables.get(device)
         if t is None:
             lib = _lib.load()
@@ -208,19 +209,21 @@ class RoadRunnerModel(TransitModel):
             t = (tab, dict(ze=ze, mu=mu, W=W, W32=W32))
             if self.ldname is not None and device.type == 'cuda':
                 t[1]['basis'] = self._basis_table(LD_LAW_IDS[self.ldname][0], tab, device)
+            _lib.synchronize_stream(device)
             self._tables[device] = t
         return t
 
     @staticmethod
     def _basis_table(law, tab, device):
         """The basis means of a law linear in its coefficients over the weight table,
-        on the device; None for the other laws."""
+        on the device, complete for every stream; None for the other laws."""
         lib = _lib.load()
         nb = lib.rr_ld_basis_count(law)
         if nb == 0:
             return None
         out = torch.empty((tab.nk * tab.ng + 1) * nb, dtype=torch.float64, device=device)
         check(lib.rr_ld_basis_table(law, _lib.ctypes.byref(tab), ptr(out), stream_handle(device)))
+        _lib.synchronize_stream(device)
         return out
 
     @property

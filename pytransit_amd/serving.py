@@ -495,11 +495,9 @@ class _HipExecutor:
         ds._staging = None
 
     def _law_basis(self, law: int):
-        """The basis table of a law, made at its first request; the slots' streams read
-        it from then on, so its kernel is waited for."""
+        """The basis table of a law, made at its first request."""
         if law not in self.basis:
             self.basis[law] = self.model._basis_table(law, self.table, self.device)
-            torch.cuda.current_stream(self.device).synchronize()
         return self.basis[law]
 
     def launch(self, slot: int, reqs: List[Request]):
