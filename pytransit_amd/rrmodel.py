@@ -185,11 +185,15 @@ class RoadRunnerModel(TransitModel):
             self._device = torch.device('cuda', torch.cuda.current_device())
         return self._device
 
-    def _table(self, device):
+    def _table(self, device, basis: bool = False):
         """Device-resident z grid, mu nodes and weight table (FP64 and FP32 copies, in
-        the device layout [nk, nz, ng]); returns (RRTable, keep-alive dict).  Complete
-        when it is kept, so calls on any stream may read it."""
+        the device layout [nk, nz, ng]); returns (RRTable, keep-alive dict).  With
+        ``basis`` the law's basis table too, under 'basis' (None for a law without): only
+        evaluate reads it, not lnlike or TSModel.  Complete when they are kept, so calls
+        on any stream may read them."""
         t = self._tables.get(device)
+        if t is not None and (not basis or 'basis' in t[1]):
+            return t
         if t is None:
             lib = _lib.load()
             ze = torch.as_tensor(self.ze, device=device)
@@ -207,10 +211,16 @@ class RoadRunnerModel(TransitModel):
                           kmax=float(self.klims[1]), dk=self.dk, dg=self.dg, weights=ptr(W), weights32=ptr(W32),
                           ze=ptr(ze), mu=ptr(mu))
             t = (tab, dict(ze=ze, mu=mu, W=W, W32=W32))
-            if self.ldname is not None and device.type == 'cuda':
-                t[1]['basis'] = self._basis_table(LD_LAW_IDS[self.ldname][0], tab, device)
+        elif torch.cuda.is_current_stream_capturing():
+            # neither the wait nor memory that outlives the capture; without the basis the
+            # setup reads the weight table, as it does for the laws that have none
+            return t
+        if basis:
+            t = (t[0], dict(t[1], basis=self._basis_table(LD_LAW_IDS[self.ldname][0], t[0], device)
+                            if self.ldname is not None and device.type == 'cuda' else None))
+        if t[1].get('basis') is None:
             _lib.synchronize_stream(device)
-            self._tables[device] = t
+        self._tables[device] = t
         return t
 
     @staticmethod
@@ -375,7 +385,7 @@ class RoadRunnerModel(TransitModel):
         if not isscalar(ldc) and not isinstance(ldc, torch.Tensor):
             ldc = np.atleast_1d(ldc)
         ld, _ld_keep = self._ld_descriptor(ldc, npv, npb, device)
-        tab, _keep = self._table(device)
+        tab, _keep = self._table(device, basis=True)
         basis = _keep.get('basis')
         if basis is not None:
             ld.law += _lib.RR_LD_BASIS

@@ -76,3 +76,32 @@ def test_first_calls_on_two_streams(gpu, law, nc):
     assert ref.min() < 0.995
     for f in out:
         assert np.array_equal(f.cpu().numpy(), ref)
+
+
+def test_only_evaluate_makes_the_basis_table(monkeypatch):
+    """lnlike, the weights property, TSModel and the server's model do without; the first
+    evaluate makes it once."""
+    made = []
+    lib = types.SimpleNamespace(rr_weights_3d=lambda *a: 0)
+    monkeypatch.setattr(_lib, 'load', lambda require_gpu=True: lib)
+    monkeypatch.setattr(rrmod, 'stream_handle', lambda device: 0)
+    monkeypatch.setattr(RoadRunnerModel, '_basis_table', staticmethod(lambda law, tab, device: made.append(law) or 'basis'))
+    # a device that says it is a GPU, with tensors on the CPU
+    class Device:
+        type = 'cuda'
+    for f in ('as_tensor', 'empty'):
+        real = getattr(torch, f)
+        monkeypatch.setattr(torch, f, lambda *a, real=real, device=None, **k: real(*a, **k))
+    monkeypatch.setattr(_lib, 'synchronize_stream', lambda device: None)
+    capturing = []
+    monkeypatch.setattr(torch.cuda, 'is_current_stream_capturing', lambda: bool(capturing))
+    m = RoadRunnerModel.__new__(RoadRunnerModel)
+    m.klims, m.nk, m.ng, m.ze, m.mu, m.ldname = (0.01, 0.2), 4, 6, np.zeros(5), np.zeros(5), 'quadratic'
+    m._tables = {}
+    dev = Device()
+    assert 'basis' not in m._table(dev)[1] and made == []
+    capturing.append(True)
+    assert 'basis' not in m._table(dev, basis=True)[1] and made == []
+    capturing.clear()
+    tab = m._table(dev)[0]
+    assert m._table(dev, basis=True)[1]['basis'] == 'basis' and m._table(dev, basis=True)[0] is tab and len(made) == 1
