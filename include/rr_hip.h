@@ -289,7 +289,10 @@ typedef struct rr_vec {
  * ldc[2] = (c0, c1), sigma.  t0 with several epochs has t0cols consecutive columns at
  * ptr + i * stride.  The setup runs in its own kernel and a light curve is split over
  * several workgroups when npv is small, with the state in between in the caller's
- * workspace; with RR_SORTED_RUNS times outside the transit window are not read per pv. */
+ * workspace; with RR_SORTED_RUNS times outside the transit window are not read per pv.
+ * More than 32,768 parameter vectors take several launches, which share the workspace.
+ * Its size: for a precision and with or without a gradient, or enough for any of them. */
+size_t rr_lnlike_vec_workspace_bytes(int precision, int grad, int npv, int npt, int ng);
 size_t rr_lnlike_workspace_bytes(int npv, int npt, int ng);
 int rr_lnlike_vec(int precision, const rr_table* tab, const rr_lcdata* lc, int npv, int t0cols,
                   const rr_vec* par, int law, const rr_vec* ldc, const double* obs, const rr_vec* sigma,

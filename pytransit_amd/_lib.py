@@ -96,6 +96,7 @@ _SIGNATURES = {
     'rr_lnlike': (c_int, [c_int, POINTER(RRTable), POINTER(RRLcData), POINTER(RRParams), POINTER(RRLd), c_void_p,
                           c_void_p, c_void_p, c_void_p, c_void_p]),
     'rr_lnlike_workspace_bytes': (c_size_t, [c_int, c_int, c_int]),
+    'rr_lnlike_vec_workspace_bytes': (c_size_t, [c_int, c_int, c_int, c_int, c_int]),
     'rr_lnlike_vec': (c_int, [c_int, POINTER(RRTable), POINTER(RRLcData), c_int, c_int, POINTER(RRVec), c_int,
                               POINTER(RRVec), c_void_p, POINTER(RRVec), c_void_p, c_size_t, c_void_p, c_void_p,
                               c_void_p]),

@@ -749,6 +749,19 @@ static int lnl_split(int npv, int npt) {
     return n < 1 ? 1 : n;
 }
 
+// Parameter vectors of a launch: the state between its kernels, up to 6.7 KB a vector
+// at 100 g (FP64 with the gradient; 0.4 KB as FP32 values only), stays below a quarter
+// of a GB however many vectors a call has.  Equal parts, the last one shorter.
+constexpr int kLnlMaxPvs = 32768;
+static int lnl_chunk(int npv) {
+    const int n = (int)(((long long)npv + kLnlMaxPvs - 1) / kLnlMaxPvs);
+    return n < 2 ? npv : (int)(((long long)npv + n - 1) / n);
+}
+static size_t lnl_rows_bytes(int precision, bool grad, int ng) {
+    if (precision == RR_MIXED) return grad ? lnl_rows_bytes<float, true>(ng) : lnl_rows_bytes<float, false>(ng);
+    return grad ? lnl_rows_bytes<double, true>(ng) : lnl_rows_bytes<double, false>(ng);
+}
+
 }  // namespace rr
 
 using namespace rr;
@@ -777,13 +790,17 @@ int rr_lnlike(int precision, const rr_table* tab, const rr_lcdata* lc, const rr_
     return lnl_dispatch(precision, s, true, (hipStream_t)stream);
 }
 
-size_t rr_lnlike_workspace_bytes(int npv, int npt, int ng) {
+size_t rr_lnlike_vec_workspace_bytes(int precision, int grad, int npv, int npt, int ng) {
     if (npv < 0 || npt < 0 || ng < 2) return 0;
-    const size_t ntile = ((size_t)npt + kLnlTile - 1) / kLnlTile;
-    size_t b = align_up((size_t)npv * sizeof(LnlRec), 256);
-    b += align_up((size_t)npv * lnl_rows_bytes<double, true>(ng), 256);
+    const size_t n = lnl_chunk(npv), ntile = ((size_t)npt + kLnlTile - 1) / kLnlTile;
+    size_t b = align_up(n * sizeof(LnlRec), 256);
+    b += align_up(n * lnl_rows_bytes(precision, grad != 0, ng), 256);
     b += align_up(ntile * sizeof(double), 256);
-    return b + align_up((size_t)npv * lnl_split(npv, npt) * 8 * sizeof(double), 256);
+    return b + align_up(n * lnl_split((int)n, npt) * 8 * sizeof(double), 256);
+}
+
+size_t rr_lnlike_workspace_bytes(int npv, int npt, int ng) {
+    return rr_lnlike_vec_workspace_bytes(RR_FP64, 1, npv, npt, ng);
 }
 
 int rr_lnlike_vec(int precision, const rr_table* tab, const rr_lcdata* lc, int npv, int t0cols, const rr_vec* par,
@@ -793,24 +810,33 @@ int rr_lnlike_vec(int precision, const rr_table* tab, const rr_lcdata* lc, int n
     LnlArgs s;
     int rc = lnl_prepare("rr_lnlike_vec", precision, tab, lc, npv, t0cols, law, obs, lnl, grad, s);
     if (rc || npv == 0) return rc;
-    const size_t need = rr_lnlike_workspace_bytes(npv, lc->npt, tab->ng);
+    const size_t need = rr_lnlike_vec_workspace_bytes(precision, grad != nullptr, npv, lc->npt, tab->ng);
     if (!workspace || workspace_bytes < need)
         return set_error(RR_EINVAL, "rr_lnlike_vec: workspace of %zu bytes needed, got %zu", need, workspace_bytes);
-    auto vec = [](const rr_vec& v) { return LnlVec{v.ptr, (long long)v.stride, v.value}; };
-    s.k = vec(par[0]); s.t0 = vec(par[1]); s.p = vec(par[2]); s.a = vec(par[3]); s.inc = vec(par[4]);
-    s.e = vec(par[5]); s.w = vec(par[6]); s.c0 = vec(ldc[0]); s.c1 = vec(ldc[1]); s.sigma = vec(*sigma);
+    const int chunk = lnl_chunk(npv);
     s.sorted = (lc->sorted & RR_SORTED_RUNS) != 0;
-    s.nsplit = lnl_split(npv, lc->npt);
+    s.nsplit = lnl_split(chunk, lc->npt);
     s.per = (s.ntile + s.nsplit - 1) / s.nsplit;
     char* ws = (char*)workspace;
     s.rec = (LnlRec*)ws;
-    ws += align_up((size_t)npv * sizeof(LnlRec), 256);
+    ws += align_up((size_t)chunk * sizeof(LnlRec), 256);
     s.rows = ws;
-    ws += align_up((size_t)npv * lnl_rows_bytes<double, true>(tab->ng), 256);
+    ws += align_up((size_t)chunk * lnl_rows_bytes(precision, grad != nullptr, tab->ng), 256);
     s.tsum = (double*)ws;
     ws += align_up((size_t)s.ntile * sizeof(double), 256);
     s.part = (double*)ws;
-    return lnl_dispatch(precision, s, false, (hipStream_t)stream);
+    for (long long pv0 = 0; pv0 < npv && rc == RR_OK; pv0 += chunk) {
+        auto vec = [pv0](const rr_vec& v) {
+            return LnlVec{v.ptr ? v.ptr + v.stride * pv0 : nullptr, (long long)v.stride, v.value};
+        };
+        s.k = vec(par[0]); s.t0 = vec(par[1]); s.p = vec(par[2]); s.a = vec(par[3]); s.inc = vec(par[4]);
+        s.e = vec(par[5]); s.w = vec(par[6]); s.c0 = vec(ldc[0]); s.c1 = vec(ldc[1]); s.sigma = vec(*sigma);
+        s.npv = (int)(npv - pv0 < chunk ? npv - pv0 : chunk);
+        s.lnl = lnl + pv0;
+        s.grad = grad ? grad + 7 * pv0 : nullptr;
+        rc = lnl_dispatch(precision, s, false, (hipStream_t)stream);
+    }
+    return rc;
 }
 
 }  // extern "C"

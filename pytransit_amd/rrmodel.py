@@ -489,13 +489,14 @@ class RoadRunnerModel(TransitModel):
         lc = self._lc_descriptor(device, 1, t0cols)
         lnl = torch.empty(npv, dtype=torch.float64, device=device)
         g = torch.empty((npv, 7), dtype=torch.float64, device=device) if grad else None
-        nbytes = lib.rr_lnlike_workspace_bytes(npv, self.npt, self.ng)
+        prec = _PRECISIONS[self.precision]
+        nbytes = lib.rr_lnlike_vec_workspace_bytes(prec, int(grad), npv, self.npt, self.ng)
         ws = torch.empty(nbytes, dtype=torch.uint8, device=device)
         byref = _lib.ctypes.byref
         law = LD_LAW_IDS[self.ldname][0]
         cv = (RRVec * 2)(RRVec(c.data_ptr(), cs, 0.0), RRVec(c.data_ptr() + 8 * cc, cs, 0.0))
-        check(lib.rr_lnlike_vec(_PRECISIONS[self.precision], byref(tab), byref(lc), npv, t0cols, (RRVec * 7)(*vecs), law,
-                                cv, ptr(obs), byref(sv), ptr(ws), nbytes, ptr(lnl), ptr(g), stream_handle(device)))
+        check(lib.rr_lnlike_vec(prec, byref(tab), byref(lc), npv, t0cols, (RRVec * 7)(*vecs), law, cv, ptr(obs), byref(sv),
+                                ptr(ws), nbytes, ptr(lnl), ptr(g), stream_handle(device)))
         return lnl, g
 
 
