@@ -50,7 +50,7 @@ struct LnlVec {
 
 // Per-pv state between the setup and the main kernel.
 struct alignas(16) LnlRec {
-    double c[10], dc[10];          // orbit coefficients and their period derivatives
+    double c[20];                  // orbit coefficients, then their period derivatives
     double lo, hi;                 // the window
     double k, t0, p, inv_p, inv_a, tan_i;
     double ist, dist0, dist1;      // disk integral and its coefficient derivatives
@@ -204,7 +204,7 @@ __device__ __forceinline__ void lnl_orbit(const LnlArgs& s, int pv, bool active,
     __syncthreads();
     if (!active) return;
     if (valid)
-        for (int m = j; m < (kGrad ? 20 : 10); m += 8) rec->c[m] = s_c[m];   // c, then dc
+        for (int m = j; m < (kGrad ? 20 : 10); m += 8) rec->c[m] = s_c[m];
     if (j == 0) {
         const double ext = s.exptimes[0];
         // the light curve's epoch column, clamped as the evaluate path does
@@ -538,8 +538,8 @@ __global__ void __launch_bounds__(kLnlThreads) rr_lnlike_kernel(LnlArgs s) {
         for (int i = 0; i < 5; ++i) {
             v.cx[i] = (Real)r.c[i];
             v.cy[i] = (Real)r.c[5 + i];
-            v.dcx[i] = kGrad ? (Real)r.dc[i] : Real(0);
-            v.dcy[i] = kGrad ? (Real)r.dc[5 + i] : Real(0);
+            v.dcx[i] = kGrad ? (Real)r.c[10 + i] : Real(0);
+            v.dcy[i] = kGrad ? (Real)r.c[15 + i] : Real(0);
         }
         v.c0 = r.c[0]; v.c1 = r.c[1]; v.c5 = r.c[5]; v.c6 = r.c[6];
         v.k = (Real)r.k;
