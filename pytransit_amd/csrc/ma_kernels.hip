@@ -61,6 +61,7 @@ __device__ __forceinline__ double ma_quad_z(double z, double k, double u1, doubl
     }
     if (z > 1.0 + k) return 1.0;
     if (k >= 1.0 && z <= k - 1.0) return 0.0;
+    if (k < 0.0) return NAN;                                 // the modulus' square is negative
     const double k2 = k * k, z2 = z * z;
     const double dm = k - z, sp = k + z;
     const double x1 = dm * dm, x2 = sp * sp, x3 = dm * sp;
@@ -124,7 +125,8 @@ __device__ __forceinline__ double ma_quad_z(double z, double k, double u1, doubl
             ed = 0.5 * inv_pi * (kap1 + k2 * (k2 + 2.0 * z2) * kap0 - 0.25 * (1.0 + 5.0 * k2 + z2) * lune);
     }
     if (edge && k == 0.5) ed = 3.0 / 32.0;
-    return 1.0 - f64_div((1.0 - u1 - 2.0 * u2) * le + (u1 + 2.0 * u2) * ld + u2 * ed, 1.0 - u1 / 3.0 - u2 / 6.0);
+    // (an IEEE quotient: coefficients whose disk integral is 0 give an infinity)
+    return 1.0 - ((1.0 - u1 - 2.0 * u2) * le + (u1 + 2.0 * u2) * ld + u2 * ed) / (1.0 - u1 / 3.0 - u2 / 6.0);
 }
 
 struct MaArgs {
