@@ -477,15 +477,18 @@ __device__ __forceinline__ double find_contact_point(double k, int point, const 
 
 // Division-free form of epoch = floor((t - t0 + p/2) / p), tc = t - (t0 + epoch*p): the
 // epoch from a multiply by 1/p, then one correction step so that
-// r = (t - t0 + p/2) - epoch*p lies in [0, p), with no contraction so each step rounds
-// as in numpy.  It can differ from the division only where the quotient is within
-// rounding of an integer, i.e. at tc = +-p/2, far outside any transit window.
+// r = (t - t0 + p/2) - epoch*p lies in [0, p), or in (p, 0] for a negative period, with no
+// contraction so each step rounds as in numpy.  It can differ from the division only
+// where the quotient is within rounding of an integer, i.e. at tc = +-p/2, far outside
+// any transit window.
 __device__ __forceinline__ double epoch_phase(double t, double t0, double p, double inv_p, double& epoch) {
 #pragma clang fp contract(off)
     const double u = t - t0 + 0.5 * p;
     double ep = floor(u * inv_p);
     const double r = u - ep * p;
-    ep += (r < 0.0) ? -1.0 : ((r >= p) ? 1.0 : 0.0);
+    // r / p has the sign of r with p's sign taken off
+    const double rs = __hiloint2double(__double2hiint(r) ^ (__double2hiint(p) & (int)0x80000000), __double2loint(r));
+    ep += (rs < 0.0) ? -1.0 : ((rs >= fabs(p)) ? 1.0 : 0.0);
     epoch = ep;
     return t - (t0 + ep * p);
 }
