@@ -333,7 +333,10 @@ struct OblateFlux {
                 const double left = east ? x0 : fmax(x0, -half - cx);
                 const double right = west ? x1 : fmin(x1, half - cx);
                 const double w = right - left;
-                acc += west || east ? fmax(w, 0.0) : w;
+                // a chord cut by the disk's edge on its side may leave nothing; an uncut
+                // one counts as it is, also with its ends swapped (f > 1)
+                const bool cut = west ? left > x0 : east && right < x1;
+                acc += cut ? fmax(w, 0.0) : w;
             }
         }
 #pragma unroll
