@@ -45,7 +45,7 @@ __device__ __forceinline__ double f64_sqrt(double x) {
     g = fma(g, e, g);
     h = fma(h, e, h);
     g = fma(fma(-g, g, x), h, g);
-    return x == 0.0 ? x : g;
+    return __builtin_amdgcn_class(x, 0x260) ? x : g;   // +-0 and +inf are their own roots
 }
 
 // Coefficient tables in constant memory, read inside loops through a pointer the
