@@ -662,30 +662,25 @@ __device__ __forceinline__ TsGeo<Real> ts_geometry(const TsRec& r, double tc, do
 template <typename Real> constexpr int ts_tpl() { return 16 / (int)sizeof(Real); }
 
 template <typename Real>
-__device__ __forceinline__ void ts_store(Real* o, const Real* v, int n, bool vec) {
-    if (vec && n == ts_tpl<Real>()) {
-        if constexpr (std::is_same<Real, float>::value) {
-            const f32x4_t w = {v[0], v[1], v[2], v[3]};
-            __builtin_nontemporal_store(w, (f32x4_t*)o);
-        } else {
-            typedef double f64x2_t __attribute__((ext_vector_type(2)));
-            const f64x2_t w = {v[0], v[1]};
-            __builtin_nontemporal_store(w, (f64x2_t*)o);
-        }
+__device__ __forceinline__ void ts_store(Real* o, const Real* v) {
+    if constexpr (std::is_same<Real, float>::value) {
+        const f32x4_t w = {v[0], v[1], v[2], v[3]};
+        __builtin_nontemporal_store(w, (f32x4_t*)o);
     } else {
-        for (int j = 0; j < n; ++j) o[j] = v[j];
+        const f64x2_t w = {v[0], v[1]};
+        __builtin_nontemporal_store(w, (f64x2_t*)o);
     }
 }
 
-// ---- FP32 flux, one workgroup per pv, rows written in order ----------------------------
+// ---- one sample, 32 whole rows a workgroup, written in order ----------------------------
 //
-// The tile form above has each workgroup write a 4 KB piece of every passband row
-// (rows npt apart), and HBM takes such strided pieces at ~4.3 TB/s where it takes
-// the same bytes written in address order at ~5.3 TB/s.  With one sample and
-// npt <= 8192 (the usual transmission-spectroscopy shape: a few thousand times,
-// hundreds of passbands), one 1024-thread workgroup per pv writes the pv's
-// [npb][npt] block front to back: thread i owns the 16-byte time vectors i and
-// i + 1024 of every row, and each step writes one whole row.
+// The tile form below has each workgroup write a piece of every passband row (rows npt
+// apart), and HBM takes such strided pieces at ~4.3 TB/s where it takes the same bytes
+// written in address order at ~5.3 TB/s.  With one sample and npt <= 8192 (FP64 6144;
+// the usual transmission-spectroscopy shape: a few thousand times, hundreds of
+// passbands) a workgroup of 1024 threads writes up to 32 rows of a pv front to back:
+// thread i owns the 16-byte time vectors i, i + 1024 and so on of every row, and each
+// step writes one whole row.
 //
 // A row costs few operations per value: the geometry of each time is reduced once
 // to the LDS offset of its limb-darkening interval and five coefficients, with
@@ -694,20 +689,22 @@ __device__ __forceinline__ void ts_store(Real* o, const Real* v, int n, bool vec
 // (c1 = A0 inside z <= 1 - k_max, else c2 = A0 and c3 = 2 k_mean kappa0, the
 // serial model's two branches); outside the window, and for g > 1 where both the
 // mean and the area vanish, F = 1 is selected, so a NaN row of limb-darkening
-// means reaches only the in-window values, as in the reference.  The LD rows of a
-// chunk of passbands sit in LDS transposed, passband fastest, so the rows of a
-// 16-passband group are read with immediate offsets from one address; the row
-// stride is 65 values, so lanes reading different g hit different banks (a stride
-// of 64 would put every lane of a row read in one bank).  A wave none of whose
-// times is in the window stores ones without arithmetic.
+// means reaches only the in-window values, as in the reference.  The passbands' LD
+// rows sit in LDS transposed, passband fastest, so the rows of a 16-passband group
+// are read with immediate offsets from one address; the row stride is 33 values, so
+// lanes reading different g hit different banks (a stride of 32 would put every lane
+// of a row read in one bank).  A wave none of whose times is in the window stores
+// ones without arithmetic.
 constexpr int kTsRowThreads = 1024;
-constexpr int kTsRowPc = 64;      // passbands per staged chunk
+constexpr int kTsRowPc = 32;      // passbands of a workgroup
 constexpr int kTsRowLd = kTsRowPc + 1;   // LDS stride of one g
 constexpr int kTsRowQ = 16;       // passbands per unrolled group
-constexpr int kTsRowSplit = 32;   // passbands of a workgroup
 // time vectors (16 bytes: 4 FP32 or 2 FP64 times) per thread; npt <= 8192 (FP32), 6144 (FP64)
 template <typename Real> constexpr int ts_row_vec() { return sizeof(Real) == 4 ? 2 : 3; }
 template <typename Real> constexpr int ts_row_max_npt() { return kTsRowThreads * ts_row_vec<Real>() * ts_tpl<Real>(); }
+// finer g grids go to the tiles: the line of a workgroup that held 64 passbands' rows in
+// 64 KB, not moved since
+template <typename Real> constexpr int ts_row_max_ng() { return sizeof(Real) == 4 ? 249 : 123; }
 
 __host__ __device__ inline size_t ts_rows_lds(int ng, size_t real) { return ((size_t)kTsRowLd * ng + 3 * kTsRowPc) * real; }
 
@@ -742,7 +739,7 @@ __global__ void __launch_bounds__(kTsRowThreads) ts_flux_rows_kernel(TsArgs s, R
     }
     if (!r.good) {
         for (size_t i = (size_t)qa * nv + threadIdx.x; i < (size_t)qb * nv; i += kTsRowThreads)
-            ts_store(out + i * TPL, vnan, TPL, true);
+            ts_store(out + i * TPL, vnan);
         return;
     }
     // the geometry of the thread's times, once, as row coefficients
@@ -762,17 +759,8 @@ __global__ void __launch_bounds__(kTsRowThreads) ts_flux_rows_kernel(TsArgs s, R
             rb[u][j] = ra[u][j] = c1[u][j] = c2[u][j] = c3[u][j] = Real(0);
             use[u][j] = false;
             if (v < nv) {
-                double tc;
-                {
-#pragma clang fp contract(off)
-                    const double t = s.times[TPL * v + j];
-                    const double t0v = s.t0[pv];
-                    const double epoch = floor((t - t0v + 0.5 * r.p) * r.inv_p);
-                    const double uu = t - t0v + 0.5 * r.p;
-                    const double rem = uu - epoch * r.p;
-                    const double ep = epoch + ((rem < 0.0) ? -1.0 : ((rem >= r.p) ? 1.0 : 0.0));
-                    tc = t - (t0v + ep * r.p);
-                }
+                double ep;
+                const double tc = epoch_phase(s.times[TPL * v + j], s.t0[pv], r.p, r.inv_p, ep);
                 if ((r.bt1 <= tc) && (tc <= r.bt4)) {
                     const TsGeo<Real> g = ts_geometry<Real>(r, tc, ext, 1.0, 0, inv_1pk, inv_dg, s.ng);
                     any = true;
@@ -790,47 +778,44 @@ __global__ void __launch_bounds__(kTsRowThreads) ts_flux_rows_kernel(TsArgs s, R
         }
         act[u] = __ballot(any) != 0ull;
     }
-    for (int pb0 = qa; pb0 < qb; pb0 += kTsRowPc) {
-        const int npc = min(kTsRowPc, qb - pb0);
-        __syncthreads();  // the previous chunk's rows are no longer read
-        for (int i = threadIdx.x; i < kTsRowPc * s.ng; i += kTsRowThreads) {
-            const int q = i / s.ng, g = i - q * s.ng;   // coalesced global reads along g
-            const size_t src = ((size_t)pv * s.npb + pb0 + q) * s.ng + g;
-            s_ldm[g * kTsRowLd + q] = q < npc ? (sizeof(Real) == 4 ? (Real)s.ldm32[src] : (Real)s.ldm64[src]) : Real(0);
-        }
-        for (int q = threadIdx.x; q < npc; q += kTsRowThreads) {
-            const double kq = s.k[(size_t)pv * s.npb + pb0 + q];
-            s_afac[q] = (Real)(kq * kq / (r.kmean * r.kmean));
-            s_kd[q] = (Real)(kq - r.kmean);
-            s_iist[q] = (Real)(1.0 / s.istar[(size_t)pv * s.npb + pb0 + q]);
-        }
-        __syncthreads();
+    const int npc = qb - qa;     // at most kTsRowPc
+    for (int i = threadIdx.x; i < npc * s.ng; i += kTsRowThreads) {
+        const int q = i / s.ng, g = i - q * s.ng;   // coalesced global reads along g
+        const size_t src = ((size_t)pv * s.npb + qa + q) * s.ng + g;
+        s_ldm[g * kTsRowLd + q] = sizeof(Real) == 4 ? (Real)s.ldm32[src] : (Real)s.ldm64[src];
+    }
+    for (int q = threadIdx.x; q < npc; q += kTsRowThreads) {
+        const double kq = s.k[(size_t)pv * s.npb + qa + q];
+        s_afac[q] = (Real)(kq * kq / (r.kmean * r.kmean));
+        s_kd[q] = (Real)(kq - r.kmean);
+        s_iist[q] = (Real)(1.0 / s.istar[(size_t)pv * s.npb + qa + q]);
+    }
+    __syncthreads();
 #pragma unroll 1
-        for (int q0 = 0; q0 < npc; q0 += kTsRowQ) {
-            const Real* lq = s_ldm + q0;
+    for (int q0 = 0; q0 < npc; q0 += kTsRowQ) {
+        const Real* lq = s_ldm + q0;
 #pragma unroll
-            for (int qq = 0; qq < kTsRowQ; ++qq) {
-                const int q = q0 + qq;
-                if (q < npc) {
-                    const Real f = s_iist[q], afac = s_afac[q], kd = s_kd[q];
-                    Real* o = out + (size_t)(pb0 + q) * npt;
+        for (int qq = 0; qq < kTsRowQ; ++qq) {
+            const int q = q0 + qq;
+            if (q < npc) {
+                const Real f = s_iist[q], afac = s_afac[q], kd = s_kd[q];
+                Real* o = out + (size_t)(qa + q) * npt;
 #pragma unroll
-                    for (int u = 0; u < NV; ++u) {
-                        const int v = threadIdx.x + u * kTsRowThreads;
-                        if (v < nv) {
-                            if (act[u]) {
-                                Real w[TPL];
+                for (int u = 0; u < NV; ++u) {
+                    const int v = threadIdx.x + u * kTsRowThreads;
+                    if (v < nv) {
+                        if (act[u]) {
+                            Real w[TPL];
 #pragma unroll
-                                for (int j = 0; j < TPL; ++j) {
-                                    const Real* l = lq + off[u][j] + qq;
-                                    const Real ip = rb[u][j] * l[0] + ra[u][j] * l[kTsRowLd];
-                                    const Real area = c1[u][j] * afac + (c2[u][j] + c3[u][j] * kd);
-                                    w[j] = use[u][j] ? Real(1) - (ip * area) * f : Real(1);
-                                }
-                                ts_store(o + (size_t)v * TPL, w, TPL, true);
-                            } else {
-                                ts_store(o + (size_t)v * TPL, vone, TPL, true);
+                            for (int j = 0; j < TPL; ++j) {
+                                const Real* l = lq + off[u][j] + qq;
+                                const Real ip = rb[u][j] * l[0] + ra[u][j] * l[kTsRowLd];
+                                const Real area = c1[u][j] * afac + (c2[u][j] + c3[u][j] * kd);
+                                w[j] = use[u][j] ? Real(1) - (ip * area) * f : Real(1);
                             }
+                            ts_store(o + (size_t)v * TPL, w);
+                        } else {
+                            ts_store(o + (size_t)v * TPL, vone);
                         }
                     }
                 }
@@ -864,9 +849,9 @@ __global__ void __launch_bounds__(kTsRowThreads) ts_flux_rows_kernel(TsArgs s, R
 // memory was slower, 2405 us.
 constexpr int kTsLine = 32;   // FP32 values per 128-byte cache line
 constexpr int kTsAlThreads = 512;
-constexpr int kTsAlPc = 32;        // passbands per staged chunk
+constexpr int kTsAlPc = 32;        // passbands of a workgroup
 constexpr int kTsAlLd = kTsAlPc + 1;   // LDS stride of one g
-constexpr int kTsStageRegs = 8;    // LD values per thread of a staged chunk: kTsAlPc x ng <= 8 x 512
+constexpr int kTsStageRegs = 8;    // LD values per thread: kTsAlPc x ng <= 8 x 512
 constexpr size_t kTsRowsAlignedMaxLds = 160 * 1024;
 
 __host__ __device__ inline size_t ts_rows_table_offset(int ng) {
@@ -889,32 +874,26 @@ __host__ __device__ inline size_t ts_rows_aligned_lds(int ng, int npt) {
 __device__ __forceinline__ void ts_row_coefficients(const TsArgs& s, const TsRec& r, double t0v, double ext, double inv_1pk,
                                                     double inv_dg, int it, int& pk, float& ra, float& rb, float& a0,
                                                     float& dk) {
-    using Real = float;
-        double tc;
-        {
-#pragma clang fp contract(off)
-            const double tt = s.times[it];
-            const double epoch = floor((tt - t0v + 0.5 * r.p) * r.inv_p);
-            const double uu = tt - t0v + 0.5 * r.p;
-            const double rem = uu - epoch * r.p;
-            const double ep = epoch + ((rem < 0.0) ? -1.0 : ((rem >= r.p) ? 1.0 : 0.0));
-            tc = tt - (t0v + ep * r.p);
+    double ep;
+    const double tc = epoch_phase(s.times[it], t0v, r.p, r.inv_p, ep);
+    pk = 0;
+    ra = rb = a0 = dk = 0.0f;
+    if ((r.bt1 <= tc) && (tc <= r.bt4)) {
+        const TsGeo<float> g = ts_geometry<float>(r, tc, ext, 1.0, 0, inv_1pk, inv_dg, s.ng);
+        if (!g.gz) {
+            pk = ((g.ig * kTsAlLd) << 2) | (g.inside ? 2 : 0) | 1;
+            ra = g.ra;
+            rb = g.rb;
+            a0 = g.ap0;
+            dk = g.dadk;
         }
-        pk = 0;
-        ra = rb = a0 = dk = Real(0);
-        if ((r.bt1 <= tc) && (tc <= r.bt4)) {
-            const TsGeo<Real> g = ts_geometry<Real>(r, tc, ext, 1.0, 0, inv_1pk, inv_dg, s.ng);
-            if (!g.gz) {
-                pk = ((g.ig * kTsAlLd) << 2) | (g.inside ? 2 : 0) | 1;
-                ra = g.ra;
-                rb = g.rb;
-                a0 = g.ap0;
-                dk = g.dadk;
-            }
-        }
+    }
 }
 
-__global__ void __launch_bounds__(kTsAlThreads, 4) ts_flux_rows_aligned_kernel(TsArgs s, float* flux) {
+// Four waves a SIMD: two workgroups a CU, though the registers would let three or four
+// in, which widens the span being written (1024 pv x 512 x 1,000: 553 us, 561 with 7).
+__global__ void __launch_bounds__(kTsAlThreads) __attribute__((amdgpu_waves_per_eu(4, 4)))
+ts_flux_rows_aligned_kernel(TsArgs s, float* flux) {
     using Real = float;
     constexpr int TPL = ts_tpl<float>();
     extern __shared__ __align__(16) unsigned char lds[];
@@ -945,38 +924,7 @@ __global__ void __launch_bounds__(kTsAlThreads, 4) ts_flux_rows_aligned_kernel(T
             if (tid < nslots) __builtin_nontemporal_store(vnan, (f32x4_t*)(out + ((size_t)q * nv + v0 + tid) * TPL));
         return;
     }
-    // a chunk's LD rows and per-passband k and disk integral, loaded into registers
-    // one chunk ahead (every load of a chunk in flight at once, the wait for them
-    // after the previous chunk's rows) and stored to LDS after the chunk barrier
-    float st[kTsStageRegs];
-    double kq = 0.0, isq = 1.0;
-    auto stage_load = [&](int pb0) {
-        const int npc = min(kTsAlPc, qb - pb0);
-#pragma unroll
-        for (int m = 0; m < kTsStageRegs; ++m) {
-            const int i = tid + m * kTsAlThreads;
-            const int q = i / s.ng, g = i - q * s.ng;
-            st[m] = (i < kTsAlPc * s.ng && q < npc) ? s.ldm32[((size_t)pv * s.npb + pb0 + q) * s.ng + g] : 0.0f;
-        }
-        if (tid < npc) {
-            kq = s.k[(size_t)pv * s.npb + pb0 + tid];
-            isq = s.istar[(size_t)pv * s.npb + pb0 + tid];
-        }
-    };
-    auto stage_store = [&](int pb0) {
-        const int npc = min(kTsAlPc, qb - pb0);
-#pragma unroll
-        for (int m = 0; m < kTsStageRegs; ++m) {
-            const int i = tid + m * kTsAlThreads;
-            const int q = i / s.ng, g = i - q * s.ng;
-            if (i < kTsAlPc * s.ng) s_ldm[g * kTsAlLd + q] = st[m];
-        }
-        if (tid < npc) {
-            s_afac[tid] = (Real)(kq * kq / (r.kmean * r.kmean));
-            s_kd[tid] = (Real)(kq - r.kmean);
-            s_iist[tid] = (Real)(1.0 / isq);
-        }
-    };
+    const int npc = qb - qa;         // at most kTsAlPc
     const double ext = s.exptimes[0];
     const double inv_1pk = 1.0 / (1.0 + r.kmean), inv_dg = 1.0 / s.dg;
     const double t0v = s.t0[pv];
@@ -991,73 +939,88 @@ __global__ void __launch_bounds__(kTsAlThreads, 4) ts_flux_rows_aligned_kernel(T
         t_a0[t] = a0;
         t_dk[t] = dk;
     }
-    stage_load(qa);
+    // the LD rows and the passbands' k and disk integrals: all loads in flight together
+    float st[kTsStageRegs];
+#pragma unroll
+    for (int m = 0; m < kTsStageRegs; ++m) {
+        const int i = tid + m * kTsAlThreads;
+        st[m] = i < npc * s.ng ? s.ldm32[((size_t)pv * s.npb + qa) * s.ng + i] : 0.0f;
+    }
+    double kq = 0.0, isq = 1.0;
+    if (tid < npc) {
+        kq = s.k[(size_t)pv * s.npb + qa + tid];
+        isq = s.istar[(size_t)pv * s.npb + qa + tid];
+    }
+#pragma unroll
+    for (int m = 0; m < kTsStageRegs; ++m) {
+        const int i = tid + m * kTsAlThreads;
+        const int q = i / s.ng, g = i - q * s.ng;
+        if (i < npc * s.ng) s_ldm[g * kTsAlLd + q] = st[m];
+    }
+    if (tid < npc) {
+        s_afac[tid] = (Real)(kq * kq / (r.kmean * r.kmean));
+        s_kd[tid] = (Real)(kq - r.kmean);
+        s_iist[tid] = (Real)(1.0 / isq);
+    }
+    __syncthreads();
     // rows P apart start equally far past a 128-byte boundary
     const int gl = npt & -npt;   // lowest set bit of npt
     const int P = kTsLine / (gl < kTsLine ? gl : kTsLine);
-    for (int pb0 = qa; pb0 < qb; pb0 += kTsAlPc) {
-        const int npc = min(kTsAlPc, qb - pb0);
-        __syncthreads();  // the previous chunk's rows are no longer read (and the table is written)
-        stage_store(pb0);
-        __syncthreads();
-        if (pb0 + kTsAlPc < qb) stage_load(pb0 + kTsAlPc);
-        for (int q0 = pb0; q0 < pb0 + min(P, npc); ++q0) {
-            // this class's head, and each slot's coefficients from the table
-            const int mis = (int)(((uintptr_t)(out + (size_t)q0 * npt) >> 2) & (kTsLine - 1));
-            const int head = ((kTsLine - mis) & (kTsLine - 1)) / TPL;
-            // per value: LDS offset, lerp weights, the area at k_mean (negated when
-            // the planet is inside the disk, where it scales by afac) and its
-            // k-derivative (0 inside); bit u * TPL + j of `use` marks a value in the
-            // window with g <= 1
-            const int lv = tid + head, vi = v0 + lv < nv ? v0 + lv : v0 + lv - nv;
-            int off[TPL];
-            Real rb[TPL], ra[TPL], as[TPL], dk[TPL];
-            unsigned use = 0u;
+    for (int q0 = 0; q0 < min(P, npc); ++q0) {
+        // this class's head, and each slot's coefficients from the table
+        const int mis = (int)(((uintptr_t)(out + (size_t)(qa + q0) * npt) >> 2) & (kTsLine - 1));
+        const int head = ((kTsLine - mis) & (kTsLine - 1)) / TPL;
+        // per value: LDS offset, lerp weights, the area at k_mean (negated when
+        // the planet is inside the disk, where it scales by afac) and its
+        // k-derivative (0 inside); bit j of `use` marks a value in the
+        // window with g <= 1
+        const int lv = tid + head, vi = v0 + lv < nv ? v0 + lv : v0 + lv - nv;
+        int off[TPL];
+        Real rb[TPL], ra[TPL], as[TPL], dk[TPL];
+        unsigned use = 0u;
+#pragma unroll
+        for (int j = 0; j < TPL; ++j) {
+            off[j] = 0;
+            ra[j] = rb[j] = as[j] = dk[j] = Real(0);
+        }
+        if (tid < nslots) {
+            const int4 pk4 = *(const int4*)(t_pk + TPL * lv);
+            const f32x4_t ra4 = *(const f32x4_t*)(t_ra + TPL * lv);
+            const f32x4_t rb4 = *(const f32x4_t*)(t_rb + TPL * lv);
+            const f32x4_t a04 = *(const f32x4_t*)(t_a0 + TPL * lv);
+            const f32x4_t dk4 = *(const f32x4_t*)(t_dk + TPL * lv);
+            const int pk[TPL] = {pk4.x, pk4.y, pk4.z, pk4.w};
 #pragma unroll
             for (int j = 0; j < TPL; ++j) {
-                off[j] = 0;
-                ra[j] = rb[j] = as[j] = dk[j] = Real(0);
+                const bool inside = (pk[j] & 2) != 0;
+                if (pk[j] & 1) use |= 1u << j;
+                off[j] = pk[j] >> 2;
+                ra[j] = ra4[j];
+                rb[j] = rb4[j];
+                as[j] = inside ? -a04[j] : a04[j];
+                dk[j] = inside ? Real(0) : dk4[j];
             }
-            if (tid < nslots) {
-                const int4 pk4 = *(const int4*)(t_pk + TPL * lv);
-                const f32x4_t ra4 = *(const f32x4_t*)(t_ra + TPL * lv);
-                const f32x4_t rb4 = *(const f32x4_t*)(t_rb + TPL * lv);
-                const f32x4_t a04 = *(const f32x4_t*)(t_a0 + TPL * lv);
-                const f32x4_t dk4 = *(const f32x4_t*)(t_dk + TPL * lv);
-                const int pk[TPL] = {pk4.x, pk4.y, pk4.z, pk4.w};
-#pragma unroll
-                for (int j = 0; j < TPL; ++j) {
-                    const bool inside = (pk[j] & 2) != 0;
-                    if (pk[j] & 1) use |= 1u << j;
-                    off[j] = pk[j] >> 2;
-                    ra[j] = ra4[j];
-                    rb[j] = rb4[j];
-                    as[j] = inside ? -a04[j] : a04[j];
-                    dk[j] = inside ? Real(0) : dk4[j];
-                }
-            }
-            const bool act = __ballot(use != 0u) != 0ull;
+        }
+        const bool act = __ballot(use != 0u) != 0ull;
 #pragma unroll 1
-            for (int q = q0; q < pb0 + npc; q += P) {
-                const int ql = q - pb0;
-                const Real f = s_iist[ql], afac = s_afac[ql], kd = s_kd[ql];
-                const Real* lq = s_ldm + ql;
-                float* o = out + (size_t)q * npt;
-                if (tid < nslots) {
-                    f32x4_t w = {1.0f, 1.0f, 1.0f, 1.0f};
-                    if (act) {
+        for (int q = q0; q < npc; q += P) {
+            const Real f = s_iist[q], afac = s_afac[q], kd = s_kd[q];
+            const Real* lq = s_ldm + q;
+            float* o = out + (size_t)(qa + q) * npt;
+            if (tid < nslots) {
+                f32x4_t w = {1.0f, 1.0f, 1.0f, 1.0f};
+                if (act) {
 #pragma unroll
-                        for (int j = 0; j < TPL; ++j) {
-                            const Real* l = lq + off[j];
-                            const Real ip = rb[j] * l[0] + ra[j] * l[kTsAlLd];
-                            // the row form's c1 afac + (c2 + c3 (k - k_mean)), with c1 = A0
-                            // inside and c2 = A0, c3 = 2 k_mean kappa_0 otherwise
-                            const Real area = as[j] < Real(0) ? (-as[j]) * afac : dk[j] * kd + as[j];
-                            w[j] = ((use >> j) & 1u) ? Real(1) - (ip * area) * f : Real(1);
-                        }
+                    for (int j = 0; j < TPL; ++j) {
+                        const Real* l = lq + off[j];
+                        const Real ip = rb[j] * l[0] + ra[j] * l[kTsAlLd];
+                        // the row form's c1 afac + (c2 + c3 (k - k_mean)), with c1 = A0
+                        // inside and c2 = A0, c3 = 2 k_mean kappa_0 otherwise
+                        const Real area = as[j] < Real(0) ? (-as[j]) * afac : dk[j] * kd + as[j];
+                        w[j] = ((use >> j) & 1u) ? Real(1) - (ip * area) * f : Real(1);
                     }
-                    __builtin_nontemporal_store(w, (f32x4_t*)(o + (size_t)vi * TPL));
                 }
+                __builtin_nontemporal_store(w, (f32x4_t*)(o + (size_t)vi * TPL));
             }
         }
     }
@@ -1067,9 +1030,9 @@ __global__ void __launch_bounds__(kTsAlThreads, 4) ts_flux_rows_aligned_kernel(T
 //
 // A workgroup of 4 waves takes a tile of T = 64, 128 or 256 times of one pv and a range
 // of passbands.  The geometry of every (time, sample) of the tile goes to LDS once, and
-// the passbands' LD rows pass through LDS in chunks; a wave takes 64 times, one a lane
-// (so its stores are contiguous), and every (4 / (T / 64))-th passband of a chunk.  The
-// form that recomputed the geometry for each chunk of 16 passbands spent most of its
+// the passbands' LD rows pass through LDS in chunks; a wave takes every fourth group of
+// four passbands of a chunk and all T times of the tile, 64 at a time, one a lane (so its
+// stores are contiguous).  The form that recomputed the geometry for each chunk of 16 passbands spent most of its
 // time on FP64 arctangents: 100 pv x 203 passbands x 1,237 t, 3 samples, FP64: 172 -> 65
 // us (201 MB written: 29 us at the rate of a fill, 45 as rows of odd length).
 constexpr int kTsTabSamples = 32;
@@ -1487,16 +1450,16 @@ int ts_evaluate(int precision, const rr_table* tab, const rr_lcdata* lc, const r
     // is a workgroup for every CU and 24 million values (rows against the tiles below, FP64,
     // us: 64 x 200 x 1,236 67.9 / 63.0, 128 x 200 x 1,236 101 / 109, 20 x 512 x 5,000 127 / 146,
     // 8 x 512 x 5,000 71.7 / 64.3)
-    a.row_split = (npb + kTsRowSplit - 1) / kTsRowSplit;
+    a.row_split = (npb + kTsRowPc - 1) / kTsRowPc;
     const long long nrow = (long long)npv * a.row_split;
     if (uns == 1 && ((uintptr_t)flux % 16) == 0 && nrow >= 256 && nrow <= 0x7fffffffLL &&
         (long long)npv * npb * npt >= 24000000LL) {
-        if (mixed && npt % 4 == 0 && npt <= ts_row_max_npt<float>() && ts_rows_lds(a.ng, 4) <= 64 * 1024) {
+        if (mixed && npt % 4 == 0 && npt <= ts_row_max_npt<float>() && a.ng <= ts_row_max_ng<float>()) {
             hipLaunchKernelGGL(ts_flux_rows_kernel<float>, dim3((unsigned)nrow), dim3(kTsRowThreads),
                                ts_rows_lds(a.ng, 4), st, a, (float*)flux);
             return check_launch("ts_flux_rows_kernel");
         }
-        if (!mixed && npt % 2 == 0 && npt <= ts_row_max_npt<double>() && ts_rows_lds(a.ng, 8) <= 64 * 1024) {
+        if (!mixed && npt % 2 == 0 && npt <= ts_row_max_npt<double>() && a.ng <= ts_row_max_ng<double>()) {
             hipLaunchKernelGGL(ts_flux_rows_kernel<double>, dim3((unsigned)nrow), dim3(kTsRowThreads),
                                ts_rows_lds(a.ng, 8), st, a, (double*)flux);
             return check_launch("ts_flux_rows_kernel");
