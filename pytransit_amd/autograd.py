@@ -13,7 +13,7 @@ __all__ = ['RRLogLikelihood', 'rr_lnlike']
 class RRLogLikelihood(torch.autograd.Function):
     @staticmethod
     def forward(ctx, theta, model, obs, sigma, e=0.0, w=0.0):
-        th = theta.detach()
+        th = theta.detach().resolve_neg()
         if th.dtype is not torch.float64 or th.device != model.device:
             th = th.to(device=model.device, dtype=torch.float64)
         if th.dim() == 2 and th.shape[1] >= 7:

@@ -71,16 +71,17 @@ def _per_pv(name, x, npv, device) -> torch.Tensor:
 
 def _vec_in_place(x, npv, device):
     """The RRVec of one value per pv that can be read where it is: a number, or a
-    float64 tensor on ``device`` with one value or one per pv (any stride).  None for
-    everything else."""
+    float64 tensor on ``device`` with one value or one per pv (any stride, up to two
+    dimensions).  None for everything else, also for a view whose values are stored
+    with the other sign (the imaginary part of a conjugate)."""
     if isinstance(x, (int, float)):
         return RRVec(0, 0, float(x))
-    if not (isinstance(x, torch.Tensor) and x.dtype == torch.float64 and x.device == device):
+    if not (isinstance(x, torch.Tensor) and x.dtype == torch.float64 and x.device == device) or x.is_neg():
         return None
-    n = x.numel()
-    if n == 1:
+    n, dim = x.numel(), x.dim()
+    if n == 1 and dim <= 2:
         return RRVec(x.data_ptr(), 0, 0.0)
-    if n == npv and (x.dim() == 1 or (x.dim() == 2 and x.shape[1] == 1)):
+    if n == npv and (dim == 1 or (dim == 2 and x.shape[1] == 1)):
         return RRVec(x.data_ptr(), x.stride(0), 0.0)
     return None
 
@@ -471,7 +472,7 @@ class RoadRunnerModel(TransitModel):
         if _max_id(self.epids) >= t0cols:
             raise ValueError(f"t0 has {t0cols} columns but the epoch indices go up to {self.epids.max()}")
         if (isinstance(ldc, torch.Tensor) and ldc.device == device and ldc.dtype == torch.float64 and ldc.dim() == 3
-                and ldc.shape[0] in (1, npv) and ldc.shape[1] == 1 and ldc.shape[2] >= 2):
+                and not ldc.is_neg() and ldc.shape[0] in (1, npv) and ldc.shape[1] == 1 and ldc.shape[2] >= 2):
             c, cs, cc = ldc, (ldc.stride(0) if ldc.shape[0] > 1 else 0), ldc.stride(2)
         else:
             ld, _keep = self._ld_descriptor(ldc, npv, 1, device)
