@@ -322,7 +322,7 @@ struct OblateFlux {
         const double* xl = ys + f.nlines;
         const double* xr = xl + f.nlines;
         const double cx = centre(c.c, t), cy = centre(c.c + 5, t), k = I.k;
-        const bool west = cx < -k, east = cx > k;
+        const bool west = cx < -k, east = cx > k, swapped = c.fl > 1.0;
         double acc = 0.0;
         for (int j = sub; j < f.nlines; j += kGroup) {
             const double x0 = xl[j], x1 = xr[j], v = ys[j] + cy;
@@ -333,10 +333,10 @@ struct OblateFlux {
                 const double left = east ? x0 : fmax(x0, -half - cx);
                 const double right = west ? x1 : fmin(x1, half - cx);
                 const double w = right - left;
-                // a chord cut by the disk's edge on its side may leave nothing; an uncut
-                // one counts as it is, also with its ends swapped (f > 1)
-                const bool cut = west ? left > x0 : east && right < x1;
-                acc += cut ? fmax(w, 0.0) : w;
+                // a chord that the disk's edge cuts on its side may leave nothing; with its
+                // ends swapped (f > 1) an uncut one counts as it is, less than nothing
+                if (!swapped) acc += west || east ? fmax(w, 0.0) : w;
+                else acc += (west ? left > x0 : east && right < x1) ? 0.0 : w;
             }
         }
 #pragma unroll
