@@ -24,7 +24,8 @@ __device__ __forceinline__ double d_sqrt(double x) { return sqrt(x); }
 __device__ __forceinline__ float d_sqrt(float x) { return __builtin_amdgcn_sqrtf(x); }
 
 // FP64 reciprocal, quotient and square root of ordinary magnitudes (no denormal or
-// overflow rescaling): the hardware's seed refined by Newton steps, to an ulp or so.
+// overflow rescaling): the hardware's seed refined by Newton steps, for the root in
+// Goldschmidt's coupled form of sqrt(x) and 1 / (2 sqrt(x)), to an ulp or so.
 // The compiler's forms add the scaling and fix-up steps that only extreme exponents
 // need, twice the instructions.
 __device__ __forceinline__ double f64_rcp(double x) {
@@ -89,7 +90,7 @@ __device__ __forceinline__ void f64_sqrt_rsqrt(double x, double& s, double& r) {
 
 // log(x) in FP64: x = m 2^e with m in [sqrt(1/2), sqrt 2), log m = 2 atanh(s) with
 // s = (m - 1) / (m + 1), atanh(s) / s an interpolating polynomial in s^2 at Chebyshev
-// nodes (relative error 1.5e-18).
+// nodes (relative error 2.1e-18 with the coefficients as stored).
 __device__ __forceinline__ double f64_log(double x) {
     double m = __builtin_amdgcn_frexp_mant(x);
     int e = __builtin_amdgcn_frexp_exp(x);
@@ -105,8 +106,9 @@ __device__ __forceinline__ double f64_log(double x) {
 
 // atan2(y, x) in FP64 for y >= 0, not both 0: the quotient of the smaller by the larger
 // side, taken about tan(pi/4) above tan(pi/8), then atan(t) / t on |t| <= tan(pi/8) as
-// an interpolating polynomial in t^2 at Chebyshev nodes (relative error 1.4e-18).  One
-// division; libm's form handles signs, zeros and infinities that the kite never gives.
+// an interpolating polynomial in t^2 at Chebyshev nodes (relative error 4.6e-18 with
+// the coefficients as stored).  One division; libm's form handles signs, zeros and
+// infinities that the kite never gives.
 __device__ __forceinline__ double f64_atan2_ypos(double y, double x) {
     const double ax = fabs(x);
     const bool steep = y > ax;

@@ -14,9 +14,9 @@
 // integrals, and the table-lerp contraction with lanes over g reading the table
 // coalesced, each table value serving the whole group).
 //
-// The flux kernel runs one wavefront per workgroup over a tile of 1024 times of
-// one pv; each lane owns two runs of 8 consecutive times and issues all its time
-// loads up front.  With contiguous light curves sorted in time, a lane classifies
+// The flux kernel runs one wavefront per workgroup over a tile of 128 to 1024 times
+// (flux_tile) of one pv; each lane owns up to two runs of 8 consecutive times and issues
+// all its time loads up front.  With contiguous light curves sorted in time, a lane classifies
 // each run from the phases of its first and last time: runs entirely outside the
 // transit window store 1.0 as vectors.  In-window points are compacted into a
 // per-wave LDS queue (ballot + popcount, count kept in a register), and all 64

@@ -105,3 +105,32 @@ def test_only_evaluate_makes_the_basis_table(monkeypatch):
     capturing.clear()
     tab = m._table(dev)[0]
     assert m._table(dev, basis=True)[1]['basis'] == 'basis' and m._table(dev, basis=True)[0] is tab and len(made) == 1
+
+
+@pytest.mark.gpu
+def test_first_evaluate_under_capture(gpu):
+    """A model whose weight table exists but not its basis table: the captured setup reads the
+    weights, and every replay gives the eager flux to rounding (FP64, 1e-12)."""
+    t = np.linspace(-0.1, 0.1, 700)
+    m, ref = RoadRunnerModel('quadratic', device=gpu), RoadRunnerModel('quadratic', device=gpu)
+    for x in (m, ref):
+        x.set_data(t, nsamples=3, exptimes=0.01)
+    col = lambda *v: torch.as_tensor(v, dtype=torch.float64, device=gpu)
+    k, ldc, t0 = col(0.1, 0.05)[:, None], col(0.4, 0.2, 0.3, 0.1).reshape(2, 1, 2), col(0.001, 0.0)[:, None]
+    orbit = (col(3.0, 2.5), col(9.0, 8.0), col(1.55, 1.53), col(0.0, 0.1), col(0.0, 0.4))
+    m.lnlike(k, ldc, t0, *orbit[:3], np.ones(700), 1e-3)     # uploads the data and makes the weight table
+    assert 'basis' not in m._table(gpu)[1]
+    stream = torch.cuda.Stream(gpu)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=stream):
+        out = m.evaluate(k, ldc, t0, *orbit, copy=False)
+    assert 'basis' not in m._table(gpu)[1]
+    for replay in range(3):
+        k.copy_(col(0.1 + 0.01 * replay, 0.05)[:, None])
+        g.replay()
+        torch.cuda.synchronize()
+        f = ref.evaluate(k, ldc, t0, *orbit)
+        assert f.min() < 0.995 and np.abs(out.cpu().numpy() - f).max() <= 1e-12
+    again = m.evaluate(k, ldc, t0, *orbit)
+    assert 'basis' in m._table(gpu)[1] and np.array_equal(again, f)
