@@ -1067,7 +1067,8 @@ __global__ void __launch_bounds__(kTsThreads) ts_flux_table_kernel(TsArgs s, Rea
     Real* t_dk = t_a0 + n;
     int* t_pk = (int*)(t_dk + n);               // interval << 3 | in the window << 2 | inside << 1 | g <= 1
     constexpr int kLd = ts_tab_ld<Real>(), kPc = ts_tab_pc<Real>();
-    Real* s_l = (Real*)(((uintptr_t)(t_pk + n) + 15) & ~(uintptr_t)15);   // [ng][kLd]
+    // [ng][kLd], by its offset: through a rounded address its reads become flat loads
+    Real* s_l = (Real*)(lds + (n * TsTab<Real>::kBytes + 15) / 16 * 16);
     Real* s_afac = s_l + (size_t)kLd * s.ng;
     Real* s_kd = s_afac + kPc;
     Real* s_f = s_kd + kPc;

@@ -102,8 +102,10 @@ __device__ __forceinline__ void window_flux_body(const typename M::Args& f) {
     uint16_t* s_list = s_it + kSub * d.nsub;                       // [kWfCap] heavy items, kind 1 from the front, 2 from the back
     uint16_t* s_map = s_list + kWfCap;                             // [kWfCap] item -> point (several light curves)
     uint16_t* s_beg = s_map + kWfCap;                              // [kWfThreads] point -> first item
-    const uintptr_t end = (uintptr_t)(kMulti ? s_beg + kWfThreads : s_map);
-    unsigned char* shared = (unsigned char*)((end + 15) & ~(uintptr_t)15);
+    // (an offset from lds, not a rounded address: the compiler loses sight of LDS through a
+    // cast to an integer and reads it with flat loads)
+    const int end = (int)((kMulti ? (unsigned char*)(s_beg + kWfThreads) : (unsigned char*)s_map) - lds);
+    unsigned char* shared = lds + (end + 15) / 16 * 16;
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int bid = xcd_remap(blockIdx.x, gridDim.x);
