@@ -183,7 +183,6 @@ struct EclipseFlux {
     using Real = double;
     using Args = EclArgs;
     static constexpr int kKinds = 1;    // the planet's limb crosses the star's
-    static constexpr int kGroup = 1;
     static constexpr int kBlocks = 6;
     struct Pv {
         double c[10], bt1, bt4, p, inv_p, shift, k, k2;
@@ -229,10 +228,11 @@ struct EclipseFlux {
         else v = NAN;
         return 0;
     }
-    static __device__ __forceinline__ double heavy(const EclArgs&, const Pv& c, const Item&, double, double z, int, int,
+    static __device__ __forceinline__ double heavy(const EclArgs&, const Pv& c, const Item&, double, double z, int, int, int,
                                                    unsigned char*) {
         return c.k2 - lens_area_f64(c.k, z);
     }
+    static __device__ __forceinline__ int group(const EclArgs&) { return 1; }
     static __device__ __forceinline__ double finish(const Pv&, double acc, int ns, const Item&) { return acc / ns; }
     static __device__ __forceinline__ void stage(const EclArgs&, const Pv&, int, unsigned char*) {}
 };
@@ -267,7 +267,6 @@ struct OblateFlux {
     using Real = double;
     using Args = OpArgs;
     static constexpr int kKinds = 1;
-    static constexpr int kGroup = 8;    // 400 pv x 10,000 t, nss 5: 8 lanes 81, 16 lanes 90, 32 lanes 109 us
     static constexpr int kBlocks = 4;
     struct Pv {
         double c[10], bt1, bt4, p, inv_p, fl;
@@ -317,14 +316,14 @@ struct OblateFlux {
         return 0;
     }
     static __device__ __forceinline__ double heavy(const OpArgs& f, const Pv& c, const Item& I, double t, double z, int,
-                                                   int sub, unsigned char* sh) {
+                                                   int sub, int G, unsigned char* sh) {
         const double* ys = (const double*)sh;
         const double* xl = ys + f.nlines;
         const double* xr = xl + f.nlines;
         const double cx = centre(c.c, t), cy = centre(c.c + 5, t), k = I.k;
         const bool west = cx < -k, east = cx > k, swapped = c.fl > 1.0;
         double acc = 0.0;
-        for (int j = sub; j < f.nlines; j += kGroup) {
+        for (int j = sub; j < f.nlines; j += G) {
             const double x0 = xl[j], x1 = xr[j], v = ys[j] + cy;
             const double h2 = 1.0 - v * v;
             // a row without a chord or off the disk adds nothing
@@ -339,11 +338,19 @@ struct OblateFlux {
                 else acc += (west ? left > x0 : east && right < x1) ? 0.0 : w;
             }
         }
-#pragma unroll
-        for (int o = kGroup / 2; o > 0; o >>= 1) acc += __shfl_xor(acc, o, kGroup);
+        for (int o = G / 2; o > 0; o >>= 1) acc += __shfl_xor(acc, o, 64);
         return flux_of(f, I, z, acc * (ys[1] - ys[0]));
     }
     static __device__ __forceinline__ double finish(const Pv&, double acc, int ns, const Item&) { return acc / ns; }
+    // Lanes of a listed sample.  Its own work is some 25 lines', so few lines take few lanes;
+    // with fewer samples a point, lists are short and the sample's latency counts
+    // (400 pv x 20,000 t over 36 d / 1.3 d, us with 8, 4 and 1 lanes: nss 5, 10 lines
+    // 73, 64, 61 / 165, 126, 107, 100 lines 142, 137, 153 / 360, 328, 323; nss 1, 10 lines
+    // 48, 49, 51 / 68, 55, 49, 100 lines 64, 70, 114 / 147, 132, 137).
+    static __device__ __forceinline__ int group(const OpArgs& f) {
+        const bool few = f.d.uniform_ns > 0 && f.d.uniform_ns < 4;
+        return few ? (f.nlines >= 48 ? 8 : 4) : (f.nlines >= 16 ? 4 : 1);
+    }
     static size_t shared_bytes(int nlines) { return 3 * (size_t)nlines * sizeof(double); }
     static __device__ __forceinline__ void stage(const OpArgs& f, const Pv& c, int pv, unsigned char* sh) {
         double* ys = (double*)sh;

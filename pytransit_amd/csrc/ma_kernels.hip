@@ -167,7 +167,6 @@ struct MaModel {
     using Real = double;
     using Args = MaArgs;
     static constexpr int kKinds = 2;    // 1 inside the disk, 2 on the limb
-    static constexpr int kGroup = 1;
     static constexpr int kBlocks = 4;   // workgroups per CU: 128 registers (3: 87, 4: 80, 5 with spills: 84 us)
     struct Pv {
         double c[10], lo, hi, p, inv_p;
@@ -209,9 +208,10 @@ struct MaModel {
         return z < 1.0 - I.k ? 1 : 2;
     }
     static __device__ __forceinline__ double heavy(const MaArgs&, const Pv&, const Item& I, double, double z, int kind,
-                                                   int, unsigned char*) {
+                                                   int, int, unsigned char*) {
         return ma_quad_z(z, I.k, I.u1, I.u2, kind == 1);
     }
+    static __device__ __forceinline__ int group(const MaArgs&) { return 1; }
     static __device__ __forceinline__ double finish(const Pv&, double acc, int ns, const Item&) { return acc / ns; }
     static __device__ __forceinline__ void stage(const MaArgs&, const Pv&, int, unsigned char*) {}
 };

@@ -1370,7 +1370,6 @@ struct RrWindow {
     using Args = RrWindowArgs<kMixed>;
     using Item = RrItem<Real>;
     static constexpr int kKinds = 1;
-    static constexpr int kGroup = 1;
     static constexpr int kBlocks = kMixed ? 6 : 5;
     struct Pv {
         Real c[10];
@@ -1404,10 +1403,11 @@ struct RrWindow {
     static __device__ __forceinline__ int classify(const Args& f, const Pv& c, const Item& I, double t, Real& v) {
         return rr_light<Real>(I, c.c, (Real)f.inv_dg, f.ng, t, v) ? 1 : 0;
     }
-    static __device__ __forceinline__ Real heavy(const Args& f, const Pv&, const Item& I, double, Real z, int, int,
+    static __device__ __forceinline__ Real heavy(const Args& f, const Pv&, const Item& I, double, Real z, int, int, int,
                                                  unsigned char*) {
         return rr_limb<Real>(I, (Real)f.inv_dg, f.ng, z);
     }
+    static __device__ __forceinline__ int group(const Args&) { return 1; }
     static __device__ __forceinline__ Real finish(const Pv&, Real acc, int ns, const Item& I) {
         return rr_point<Real>(I, acc, ns);
     }

@@ -9,7 +9,7 @@
 //   2. The queue is worked through in chunks of up to 256 points and kWfCap (point,
 //      sample) items, one item a lane: a first pass settles the cheap samples (planet
 //      off the disk, wholly inside it) and lists the others, which a second pass
-//      evaluates on full waves, M::kGroup lanes to a sample.
+//      evaluates on full waves, M::group lanes to a sample.
 //   3. A lane sums the samples of a point in order and stores the point.
 //   4. The sub-tiles outside are filled with the constant (16-byte stores), last: loads
 //      after them would wait for them.
@@ -31,8 +31,9 @@
 //   classify(f, P, I, t, v)   the sample at time t from conjunction: 0 when v is its
 //                             value, 1 or 2 when a heavy evaluation has to follow,
 //                             with v the separation
-//   heavy(f, P, I, t, z, kind, sub, sh)   that evaluation by kGroup lanes, this one the
-//                             sub-th; lane 0 of the group returns the value
+//   heavy(f, P, I, t, z, kind, sub, G, sh)   that evaluation by G = group(f) lanes, a power
+//                             of two up to 64, this one the sub-th; lane 0 of the group
+//                             returns the value
 //   stage(f, P, pv, sh), shared_bytes(f)     block-wide tables in LDS
 #pragma once
 
@@ -260,8 +261,7 @@ __device__ __forceinline__ void window_flux_body(const typename M::Args& f) {
             }
         }
         __syncthreads();
-        constexpr int G = M::kGroup;
-        const int na = s_na, nh = na + s_nb;
+        const int na = s_na, nh = na + s_nb, G = M::group(f);
 #pragma unroll 1
         for (int j = tid / G; j < nh; j += kWfThreads / G) {
             const int kind = j < na ? 1 : 2;
@@ -269,7 +269,7 @@ __device__ __forceinline__ void window_flux_body(const typename M::Args& f) {
             const int q = point_of(i);
             const Item I = kMulti ? s_ctx[q] : ctx0;
             const double t = sample_time(s_tc[q], I.ext, I.inv_ns, s0 + i - first_of(q));
-            const Real v = M::heavy(f, c, I, t, s_val[i], kind, tid % G, shared);
+            const Real v = M::heavy(f, c, I, t, s_val[i], kind, tid % G, G, shared);
             if (tid % G == 0) s_val[i] = v;
         }
         __syncthreads();

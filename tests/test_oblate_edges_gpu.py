@@ -58,3 +58,16 @@ def test_too_many_scanlines_are_refused(gpu):
     m.set_data(np.linspace(-0.1, 0.1, 11))
     with pytest.raises(Exception, match='nlines'):
         m.evaluate(0.1, 0.1, 0.0, [0.4, 0.2], 0.0, 3.0, 9.0, 1.55)
+
+
+# the number of lanes that share a sample's scanlines changes at 16 and 48 lines, and at
+# four samples a point
+@pytest.mark.parametrize('nlines', [2, 15, 16, 47, 48, 65])
+@pytest.mark.parametrize('ns', [1, 3, 4, (1, 6)])
+def test_lanes_of_a_sample(gpu, oracle, nlines, ns):
+    t = np.linspace(-0.12, 0.12, 301)
+    kw = dict(lcids=np.repeat([0, 1], [130, 171]), nsamples=ns, exptimes=(0.0, 0.01)) if ns == (1, 6) else \
+        dict(nsamples=(ns,), exptimes=(0.01,))
+    got, ref = both(oracle, t, np.array([0.0, 0.2, 1.3]), np.array([0.1, -1.0, 2.0]), nlines, **kw)
+    assert ref.min() < 0.995
+    assert np.abs(got - ref).max() <= 1e-9
