@@ -88,11 +88,17 @@ typedef struct rr_ld {
 #define RR_SORTED_RUNS 1
 #define RR_SORTED_TIMES 2
 #define RR_ONE_WINDOW 4
+/* Bits 8 to 12 may hold c > 0 where a tenth of a day holds at least 2^c times (0: not
+ * known, or few), and with them bits 13 to 17 hold s where a point has 2^s samples or
+ * more on average: launches share out the points of a transit by them.  They never change
+ * a result. */
+#define RR_DENSITY_SHIFT 8
+#define RR_SAMPLES_SHIFT 13
 
 /* Light-curve data set by set_data() (transitmodel.py:56-125), device-resident. */
 typedef struct rr_lcdata {
     int32_t npt, nlc, npb, nep;
-    int32_t sorted;           /* layout bits, RR_SORTED_*: see below                  */
+    int32_t sorted;           /* layout bits, RR_SORTED_* and the density: see above  */
     int32_t uniform_nsamples; /* the common nsamples of all light curves, or 0         */
     const double* times;      /* [npt]                                               */
     const int32_t* lcids;     /* [npt], values in [0, nlc)                           */

@@ -183,6 +183,7 @@ struct EclipseFlux {
     using Real = double;
     using Args = EclArgs;
     static constexpr int kKinds = 1;    // the planet's limb crosses the star's
+    static constexpr int kDense = 4096, kDenseNs = 16;
     static constexpr int kBlocks = 6;
     struct Pv {
         double c[10], bt1, bt4, p, inv_p, shift, k, k2;
@@ -267,6 +268,7 @@ struct OblateFlux {
     using Real = double;
     using Args = OpArgs;
     static constexpr int kKinds = 1;
+    static constexpr int kDense = 1024, kDenseNs = 4;
     static constexpr int kBlocks = 4;
     struct Pv {
         double c[10], bt1, bt4, p, inv_p, fl;

@@ -167,6 +167,7 @@ struct MaModel {
     using Real = double;
     using Args = MaArgs;
     static constexpr int kKinds = 2;    // 1 inside the disk, 2 on the limb
+    static constexpr int kDense = 4096, kDenseNs = 16;
     static constexpr int kBlocks = 4;   // workgroups per CU: 128 registers (3: 87, 4: 80, 5 with spills: 84 us)
     struct Pv {
         double c[10], lo, hi, p, inv_p;

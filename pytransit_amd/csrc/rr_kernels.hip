@@ -1370,6 +1370,7 @@ struct RrWindow {
     using Args = RrWindowArgs<kMixed>;
     using Item = RrItem<Real>;
     static constexpr int kKinds = 1;
+    static constexpr int kDense = 4096, kDenseNs = 16;
     static constexpr int kBlocks = kMixed ? 6 : 5;
     struct Pv {
         Real c[10];

@@ -28,6 +28,7 @@
 //   fill(P), bad()            the values outside the window and of an invalid pv
 //   window(f, P, pv, ilc)     -> WfWindow
 //   item(f, P, pv, ilc)       -> Item
+//   kDense, kDenseNs          when a launch takes small workgroups (wf_launch)
 //   classify(f, P, I, t, v)   the sample at time t from conjunction: 0 when v is its
 //                             value, 1 or 2 when a heavy evaluation has to follow,
 //                             with v the separation
@@ -51,6 +52,8 @@ struct WfData {
     int sorted;       // contiguous light curves, each sorted in time
     int one_window;   // with `sorted`: times sorted throughout, one window for all
     int uniform_ns;   // the common nsamples, or 0
+    int density;      // times in a tenth of a day, a power of two at most that, or 0: unknown
+    int samples;      // with it: samples a point
 };
 
 struct WfWindow {
@@ -296,7 +299,23 @@ __device__ __forceinline__ void window_flux_body(const typename M::Args& f) {
 // and 92 us with 2000, 3000, 5000 and 10,000 workgroups; at 2000 x 20,000, nss 1: 119
 // and 160 us with 6000 and 20,000); one time a lane where single sub-tiles of four
 // leave CUs short of work.
+//
+// That suits long light curves, whose windows are a few points of each workgroup.  Where
+// the times lie so close that a transit fills whole workgroups, these are the launch's
+// length, and small ones even it out: from M::kDense samples in a tenth of a day single
+// sub-tiles, and from M::kDenseNs samples a point one time a lane (1000 pv x 20,000 t with
+// 1500 times in a tenth of a day, us by the first rule, with single sub-tiles of four, with
+// one time a lane: MA nss 5 428, 381, 416, nss 20 1593, 1314, 1161, oblate 100 lines nss 5
+// 1478, 914, 703, nss 20 5766, 3469, 2420; with 50 times, nss 5: MA 139, 201, 258, EC 62,
+// 85, 128).  With the density known a pv also keeps four tiles (3000 x 3000, 225 times, nss
+// 1, without and with: MA 129, 92, EC 60, 49, oblate 170, 122).
 constexpr int kWfBlocks = 4096;
+static inline long long wf_density(const rr_lcdata* lc) {
+    const int c = (lc->sorted >> RR_DENSITY_SHIFT) & 31;
+    return c ? 1ll << c : 0;
+}
+// Samples a point, known with the density
+static inline long long wf_samples(const rr_lcdata* lc) { return 1ll << ((lc->sorted >> RR_SAMPLES_SHIFT) & 31); }
 template <class M>
 struct WfKernels {
     typedef void (*Fn)(typename M::Args);
@@ -308,10 +327,15 @@ static inline int wf_launch(const char* who, const WfKernels<M>& kn, typename M:
                             hipStream_t s) {
     const int npt = f.d.npt;
     const long long sub4 = ((long long)npt + 4 * kWfThreads - 1) / (4 * kWfThreads);
-    const int P = sub4 * npv < 2048 ? 1 : 4;
+    const int ns = f.d.samples;
+    const bool known = f.d.density >= 64, dense = known && (long long)f.d.density * ns >= M::kDense;
+    const int P = sub4 * npv < 2048 || (dense && ns >= M::kDenseNs) ? 1 : 4;
     const long long nsubs = P == 4 ? sub4 : ((long long)npt + kWfThreads - 1) / kWfThreads;
     int per = 1;
-    while (per < kWfMaxSub && (nsubs + 2 * per - 1) / (2 * per) * npv >= kWfBlocks) per *= 2;
+    const int least = known ? 4 : 1;      // tiles of a pv
+    while (!dense && per < kWfMaxSub && (nsubs + 2 * per - 1) / (2 * per) >= least &&
+           (nsubs + 2 * per - 1) / (2 * per) * npv >= kWfBlocks)
+        per *= 2;
     const long long ntiles = (nsubs + per - 1) / per;
     if (ntiles * npv > 0x7fffffffLL) return set_error(RR_ERANGE, "%s: grid too large", who);
     f.d.ntiles = (int)ntiles;
@@ -338,6 +362,8 @@ static inline WfData wf_data(const rr_lcdata* lc, bool shared_epochs) {
     const int one = RR_SORTED_RUNS | RR_SORTED_TIMES | RR_ONE_WINDOW;
     d.one_window = shared_epochs && (lc->sorted & one) == one;
     d.uniform_ns = lc->uniform_nsamples > 0 ? lc->uniform_nsamples : 0;
+    d.density = (int)(wf_density(lc) < 0x40000000 ? wf_density(lc) : 0x40000000);
+    d.samples = d.uniform_ns > 0 ? d.uniform_ns : (int)(wf_samples(lc) < 0x40000000 ? wf_samples(lc) : 0x40000000);
     return d;
 }
 

@@ -39,6 +39,24 @@ def layout_flags(time: ndarray, lcids: ndarray, epids: ndarray, exptimes: ndarra
     return flags
 
 
+def density_bits(time: ndarray, nsamples: ndarray) -> int:
+    """Bits 8 to 17 of rr_lcdata.sorted (include/rr_hip.h), for the points' times and
+    numbers of samples: set where a tenth of a day holds 16 times or more, by the median
+    step of a thousand neighbouring pairs."""
+    if time.size < 65:
+        return 0
+    at = np.arange(0, time.size - 1, max(1, (time.size - 1) // 1024))
+    with np.errstate(invalid='ignore'):
+        dt = np.abs(time[at + 1] - time[at])
+    dt = dt[dt > 0]             # (several light curves may share their times)
+    if dt.size < 16:
+        return 0
+    n = 0.1 / float(np.median(dt)) * at.size / dt.size
+    if not n >= 16:
+        return 0
+    return min(int(np.log2(n)), 30) << 8 | min(int(np.log2(nsamples.mean())), 30) << 13
+
+
 class TransitModel:
     """Exoplanet transit light curve model (transitmodel.py:36-54)."""
 
@@ -137,11 +155,13 @@ class TransitModel:
             nsamples = self._per_lc(self.nsamples, np.int64)
             if (nsamples < 1).any():
                 raise ValueError('nsamples must be >= 1')
+            lcids = self.lcids.astype(np.int32)
             d = dict(
-                sorted=int(layout_flags(self.time, self.lcids, self.epids, self._per_lc(self.exptimes, np.float64))),
+                sorted=int(layout_flags(self.time, self.lcids, self.epids, self._per_lc(self.exptimes, np.float64)))
+                | density_bits(self.time, nsamples[lcids]),
                 uniform_ns=int(nsamples[0]) if (nsamples == nsamples[0]).all() else 0,
                 times=torch.as_tensor(np.ascontiguousarray(self.time), device=device),
-                lcids=torch.as_tensor(self.lcids.astype(np.int32), device=device),
+                lcids=torch.as_tensor(lcids, device=device),
                 pbids=torch.as_tensor(self.pbids.astype(np.int32), device=device),
                 epids=torch.as_tensor(self.epids.astype(np.int32), device=device),
                 nsamples=torch.as_tensor(nsamples.astype(np.int32), device=device),
