@@ -2268,6 +2268,35 @@ int rr_setup(int precision, const rr_table* tab, const rr_lcdata* lc, const rr_p
     return check_launch("rr_setup_kernel");
 }
 
+// Several light curves whose samples the tile kernel's item loops do not take (FP64, or
+// uneven nsamples) may go to the window kernel; both give the same bits.  The tile kernel
+// looks at every tile, skips those without a transit, and in the others a lane works
+// through all samples of a point; the window kernel shares samples out evenly, at a cost
+// per workgroup.  Times below are us of the window / the tile kernel, with the number of
+// times in a tenth of a day.
+static bool rr_takes_window(int precision, const rr_lcdata* lc, const FluxArgs& fa, int npv, bool fast) {
+    if (lc->nlc < 2 || (precision == RR_MIXED && fa.uniform_ns != 0)) return false;
+    const long long density = wf_density(lc), ns = wf_samples(lc), samples = density * ns;
+    const long long run = lc->npt / lc->nlc, sub4 = ((long long)lc->npt + 4 * kWfThreads - 1) / (4 * kWfThreads);
+    const bool big = sub4 * npv >= 2 * kWfBlocks;
+    if (precision == RR_FP64) {
+        // One sample a point leaves little to share out where tiles are skipped: 1000 pv x
+        // 20,000 t in 12 light curves: 78 / 52 (50 times), 61 / 50 (375), 97 / 94 (1500);
+        // without order 100 / 170.
+        if (fa.uniform_ns == 1)
+            return !((fa.one_window || (fast && run >= 768)) && density >= 16 && density < 512);
+        // Uneven samples that fill long stretches of a launch: 3000 x 3000, 12 light curves
+        // of 2 and 30 samples: 861 / 440 (750 times); 40 light curves: 565 / 594.
+        return !(fa.uniform_ns == 0 && big && fa.one_window && run >= 200 && ns >= 16 && samples >= 4096);
+    }
+    // FP32 samples are cheap, so the window kernel keeps small calls, and light curves of
+    // few tiles that it does not spread over a launch: light curves of 1 and 5 samples,
+    // 600 x 9000 in 12: 54 / 60 (169 times); 3000 x 3000 in 40: 61 / 77 (225); 1000 x 20,000
+    // in 12: 101 / 74 (375).
+    if (!big) return samples < 16384;
+    return fast && run < 768 && sub4 < 8 && (!fa.one_window || samples < 512);
+}
+
 int rr_flux(int precision, const rr_table* tab, const rr_lcdata* lc, const rr_params* pv, void* workspace,
             size_t workspace_bytes, void* flux, void* stream) {
     FluxArgs fa;
@@ -2277,9 +2306,7 @@ int rr_flux(int precision, const rr_table* tab, const rr_lcdata* lc, const rr_pa
     int rc = prepare_flux("rr_flux", precision, tab, lc, pv, workspace, workspace_bytes, flux, fa, nblocks, lds, fast, false);
     if (rc || nblocks == 0) return rc;
     hipStream_t s = (hipStream_t)stream;
-    // several light curves whose samples the tile kernel's item loops do not take (FP64,
-    // or uneven nsamples): the window kernel
-    if (lc->nlc > 1 && (precision == RR_FP64 || fa.uniform_ns == 0)) {
+    if (rr_takes_window(precision, lc, fa, pv->npv, fast)) {
         if (precision == RR_FP64) return rr_window_flux<false>(lc, pv, fa, s);
         return rr_window_flux<true>(lc, pv, fa, s);
     }

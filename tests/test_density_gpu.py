@@ -47,3 +47,25 @@ def test_window_models(gpu, npv, npt, span, ns, kind):
     got, plain = both(m, args)
     assert np.isfinite(got).all() and got.min() < 0.999
     assert np.array_equal(got, plain)
+
+
+# light curves one after another, and (apart) each with a transit of its own; the bits move
+# each of these calls between the window kernel and the tile kernel
+@pytest.mark.parametrize('precision,npv,npt,nlc,ns,span', [
+    ('fp64', 40, 2000, 3, (1,), 2.0), ('fp64', 700, 3073, 12, (1,), 4.0),    # one sample
+    ('fp64', 2100, 4097, 12, (2, 30), 0.5),                                  # uneven, many samples
+    ('mixed', 40, 3000, 3, (2, 30), 0.3),                                    # a small call that fills tiles
+    ('mixed', 2800, 3000, 12, (2, 30), 0.5), ('mixed', 2800, 3000, 12, (1, 5), 0.1)])
+@pytest.mark.parametrize('apart', [False, True])
+def test_roadrunner_routes(gpu, precision, npv, npt, nlc, ns, span, apart):
+    p, a, inc, k, t0, ldc, z = orbits(npv)
+    t = np.linspace(-span / 3, span, npt)
+    ids = np.arange(npt) * nlc // npt
+    if apart:
+        t += (p[0] * np.arange(nlc))[ids]
+    nss = [ns[i % len(ns)] for i in range(nlc)]
+    m = RoadRunnerModel('quadratic', precision=precision)
+    m.set_data(t, lcids=ids, pbids=[0] * nlc, epids=[0] * nlc, nsamples=nss, exptimes=[0.01] * nlc)
+    got, plain = both(m, (k[:, None], ldc[:, None], t0[:, None], p, a, inc, z, z))
+    assert np.isfinite(got).all() and got.min() < 0.999
+    assert np.array_equal(got, plain)
