@@ -348,10 +348,11 @@ struct OblateFlux {
     // with fewer samples a point, lists are short and the sample's latency counts
     // (400 pv x 20,000 t over 36 d / 1.3 d, us with 8, 4 and 1 lanes: nss 5, 10 lines
     // 73, 64, 61 / 165, 126, 107, 100 lines 142, 137, 153 / 360, 328, 323; nss 1, 10 lines
-    // 48, 49, 51 / 68, 55, 49, 100 lines 64, 70, 114 / 147, 132, 137).
+    // 48, 49, 51 / 68, 55, 49, 100 lines 64, 70, 114 / 147, 132, 137; at 200 lines 8 and 4
+    // are equal, and 8 answer a small call sooner).
     static __device__ __forceinline__ int group(const OpArgs& f) {
         const bool few = f.d.uniform_ns > 0 && f.d.uniform_ns < 4;
-        return few ? (f.nlines >= 48 ? 8 : 4) : (f.nlines >= 16 ? 4 : 1);
+        return f.nlines >= 128 || (few && f.nlines >= 48) ? 8 : (f.nlines >= 16 || few ? 4 : 1);
     }
     static size_t shared_bytes(int nlines) { return 3 * (size_t)nlines * sizeof(double); }
     static __device__ __forceinline__ void stage(const OpArgs& f, const Pv& c, int pv, unsigned char* sh) {

@@ -5,9 +5,14 @@ import warnings
 import numpy as np
 import pytest
 
-from pytransit_amd.transitmodel import density_bits
+from pytransit_amd import transitmodel
 
 one = lambda n: np.ones(n, int)
+
+
+def density_bits(t, ns):
+    """Every point in a light curve of its own."""
+    return transitmodel.density_bits(t, np.arange(t.size), ns)
 
 
 def parts(bits):
@@ -40,9 +45,12 @@ def test_unknown():
         warnings.simplefilter('error')
         for t in (np.full(500, np.nan), np.full(500, np.inf), np.zeros(500), np.zeros(0)):
             assert density_bits(t, one(t.size)) == 0
+    assert transitmodel.density_bits(np.arange(500) * 1e-3, np.zeros(500, int), np.array([6])) == 6 << 8 | 2 << 13
 
 
 def test_limits_of_the_fields():
+    t = np.arange(200) * 5e-324
+    assert parts(density_bits(t, one(200))) == (30, 0)
     t = np.arange(200) * 1e-300
     assert parts(density_bits(t, np.full(200, 2 ** 40))) == (30, 30)
     assert parts(density_bits(np.arange(200) * 1e-3, np.repeat([2, 30], 100)))[1] == 4

@@ -60,9 +60,9 @@ def test_too_many_scanlines_are_refused(gpu):
         m.evaluate(0.1, 0.1, 0.0, [0.4, 0.2], 0.0, 3.0, 9.0, 1.55)
 
 
-# the number of lanes that share a sample's scanlines changes at 16 and 48 lines, and at
-# four samples a point
-@pytest.mark.parametrize('nlines', [2, 15, 16, 47, 48, 65])
+# the number of lanes that share a sample's scanlines changes at 16, 48 and 128 lines, and
+# at four samples a point
+@pytest.mark.parametrize('nlines', [2, 15, 16, 47, 48, 65, 127, 128])
 @pytest.mark.parametrize('ns', [1, 3, 4, (1, 6)])
 def test_lanes_of_a_sample(gpu, oracle, nlines, ns):
     t = np.linspace(-0.12, 0.12, 301)
