@@ -25,8 +25,8 @@
 // One block per pv did all of it before: the setup idled three of its four waves for
 // 10-15 us, every pv read every time, a population of 250 left the chip two thirds
 // empty and the gradient was computed whether asked for or not.  250 pv x 18,000 t over
-// 24 d, nss 5, FP64, value only: 50 -> 11 + 13 + 4 us; 2048 pv x 10,000 t, 22 % in the
-// window, nss 5, mixed, with the gradient: 125 -> 16 + 74 us, VALU-bound (about 150
+// 24 d, nss 5, FP64, value only: 50 -> 8 + 13 + 4 us; 2048 pv x 10,000 t, 22 % in the
+// window, nss 5, mixed, with the gradient: 125 -> 14 + 72 us, VALU-bound (about 150
 // instructions a sample at 128 registers).
 #include <hip/hip_runtime.h>
 

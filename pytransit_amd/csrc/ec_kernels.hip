@@ -17,7 +17,7 @@
 //                     106-185), the light travel time and the contact window
 //   ec_flux_kernel    the planet disk area left visible by the star
 //                     over a tile of times of one pv (window_flux.hpp).  1000 pv x
-//                     20,001 t with 5 samples (160 MB written, 23 us): 45 us against
+//                     20,001 t with 5 samples (160 MB written, 23 us): 55 us against
 //                     147 us with one lane per (pv, time), whose samples ran in series
 //                     with two libm arctangents each
 //   es_flux_kernel    one lane per (pv, time): the mean lens area, fanned out over the
@@ -260,9 +260,9 @@ struct OpArgs {
 // opmodel_full.py:95-131 on the window kernel.  The planet's ellipse is a table of
 // scanlines (create_ellipse, ecintersection.py:93-134, at k[:, 0]) in LDS; a sample
 // whose planet crosses the limb sums the part of every scanline on the stellar disk
-// (ecintersection.py:137-207, the three branches by the centre's x).  Eight lanes
-// share a sample's scanlines: with one lane a sample the 100 square roots in a row
-// ran on the few lanes of a wave that held one (400 pv x 10,000 t, 5 samples, 100
+// (ecintersection.py:137-207, the three branches by the centre's x).  Several lanes
+// share a sample's scanlines (group): with one lane a sample the 100 square roots in a
+// row ran on the few lanes of a wave that held one (400 pv x 10,000 t, 5 samples, 100
 // lines: 744 us a call, now 81; floor 5 us of writes and 2 us of FP64).
 struct OblateFlux {
     using Real = double;

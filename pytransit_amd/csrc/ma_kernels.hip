@@ -13,7 +13,8 @@
 //                     flux [npv, npt] (window_flux.hpp)
 //
 // 1000 pv x 10,007 t with 5 samples (80 MB written, 2 % of the points in transit): the
-// flux kernel takes 60 us against 430 us with one lane per (pv, time), the orbits 10 us.
+// flux kernel takes 62 us (65-72 between other work) against 430 us with one lane per
+// (pv, time), the orbits 6 us.
 // The write alone is 12 us and the samples' FP64 arithmetic about as much again; the
 // rest is the latency of the workgroups that hold a window (about 10 us each, four
 // resident per CU).

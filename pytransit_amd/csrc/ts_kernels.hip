@@ -1032,9 +1032,9 @@ ts_flux_rows_aligned_kernel(TsArgs s, float* flux) {
 // of passbands.  The geometry of every (time, sample) of the tile goes to LDS once, and
 // the passbands' LD rows pass through LDS in chunks; a wave takes every fourth group of
 // four passbands of a chunk and all T times of the tile, 64 at a time, one a lane (so its
-// stores are contiguous).  The form that recomputed the geometry for each chunk of 16 passbands spent most of its
-// time on FP64 arctangents: 100 pv x 203 passbands x 1,237 t, 3 samples, FP64: 172 -> 65
-// us (201 MB written: 29 us at the rate of a fill, 45 as rows of odd length).
+// stores are contiguous).  The form that recomputed the geometry for each chunk of 16
+// passbands spent most of its time on FP64 arctangents: 100 pv x 203 passbands x 1,237 t, 3
+// samples, FP64: 172 -> 60 us (201 MB written: 29 us at the rate of a fill, 45 as rows of odd length).
 constexpr int kTsTabSamples = 32;
 // passbands of a chunk (FP64: 32 takes 105, 16 takes 100 us at the size above)
 template <typename Real> constexpr int ts_tab_pc() { return sizeof(Real) == 4 ? 32 : 16; }

@@ -18,7 +18,8 @@
 // left the rest of the chip waiting for those waves: only 2-10 % of the times of a
 // survey light curve are in a window.  A workgroup's entry (arguments, record, epoch,
 // boundary times: four dependent loads) is 2-3 us however few points it has, so it
-// takes several sub-tiles when that leaves enough workgroups.
+// takes several sub-tiles when that leaves enough workgroups, and few where a transit
+// fills them.
 //
 // A model M gives
 //   Args                      kernel arguments, with a WfData member `d`

@@ -42,7 +42,7 @@ def layout_flags(time: ndarray, lcids: ndarray, epids: ndarray, exptimes: ndarra
 
 def density_bits(time: ndarray, lcids: ndarray, nsamples: ndarray) -> int:
     """Bits 8 to 17 of rr_lcdata.sorted (include/rr_hip.h): set where a tenth of a day holds
-    16 times or more, by the median of 128 to 512 steps (15 us: part of a first evaluate)."""
+    16 times or more, by the median of 128 to 512 steps (12 us of a first evaluate)."""
     if time.size < 65:
         return 0
     every = max(1, (time.size - 1) // 256) | 1     # (odd: pairs of equal times)
