@@ -189,14 +189,16 @@ __global__ void __launch_bounds__(256) ts_weights_kernel(TsArgs s) {
     __shared__ double s_sum[kTwMaxRows];
     const int R = ts_weight_rows(s.nz), nz = s.nz;
     const int nchunk = (s.ngp + R - 1) / R;
-    // the launch's last blocks take the disk integrals
-    const int wb = s.npv * nchunk;
-    if ((int)blockIdx.x >= wb) {
-        ts_istar(s, (blockIdx.x - wb) * blockDim.x + threadIdx.x);
+    // the launch's first blocks take the disk integrals, a long chain for the laws without
+    // an analytic one: first, so that they spread over the CUs (340 x 82 of the power-2-pm
+    // law: 343 us so, 343-517 us behind the weights, several to a CU)
+    const int nint = (int)(gridDim.x - (unsigned)(s.npv * nchunk)), wb = (int)blockIdx.x - nint;
+    if (wb < 0) {
+        ts_istar(s, blockIdx.x * blockDim.x + threadIdx.x);
         return;
     }
-    const int pv = blockIdx.x / nchunk;
-    const int g0 = (blockIdx.x - pv * nchunk) * R;
+    const int pv = wb / nchunk;
+    const int g0 = (wb - pv * nchunk) * R;
     const int nr = min(R, s.ngp - g0);
     const int tid = threadIdx.x;
     const size_t base = (size_t)pv * s.nzp * s.ngp + g0;
