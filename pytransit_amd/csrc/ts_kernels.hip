@@ -1210,7 +1210,7 @@ __global__ void __launch_bounds__(kTsThreads) ts_flux_kernel(TsArgs s, void* flu
     Real* s_ldm = (Real*)lds;                       // [PC][ng]
     Real* s_afac = s_ldm + (size_t)PC * s.ng;       // k^2 / k_mean^2
     Real* s_kd = s_afac + PC;                       // k - k_mean
-    Real* s_iist = s_kd + PC;                       // 1 / istar
+    Real* s_f = s_kd + PC;                          // 1 / (ns istar)
     __shared__ int s_any;
 
     const int bid = xcd_remap(blockIdx.x, gridDim.x);
@@ -1243,8 +1243,7 @@ __global__ void __launch_bounds__(kTsThreads) ts_flux_kernel(TsArgs s, void* flu
     }
     const int ns = s.nsamples[0];
     const double ext = s.exptimes[0];
-    const Real inv_ns = Real(1) / Real(ns);
-    const double km = r.kmean, inv_1pk = 1.0 / (1.0 + km), inv_dg = 1.0 / s.dg;
+    const double km = r.kmean, inv_1pk = 1.0 / (1.0 + km), inv_dg = 1.0 / s.dg, inv_ns = 1.0 / ns;
     for (int pb0 = 0; pb0 < s.npb; pb0 += PC) {
         const int npc = min(PC, s.npb - pb0);
         __syncthreads();  // the previous chunk's rows are no longer read
@@ -1257,7 +1256,7 @@ __global__ void __launch_bounds__(kTsThreads) ts_flux_kernel(TsArgs s, void* flu
             const double kq = s.k[(size_t)pv * s.npb + pb0 + q];
             s_afac[q] = (Real)(kq * kq / (km * km));
             s_kd[q] = (Real)(kq - km);
-            s_iist[q] = (Real)(1.0 / s.istar[(size_t)pv * s.npb + pb0 + q]);
+            s_f[q] = (Real)(inv_ns / s.istar[(size_t)pv * s.npb + pb0 + q]);
         }
         __syncthreads();
         if (!in) continue;
@@ -1266,19 +1265,20 @@ __global__ void __launch_bounds__(kTsThreads) ts_flux_kernel(TsArgs s, void* flu
         for (int q = 0; q < PC; ++q) acc[q] = Real(0);
         if (inw) {
             for (int is = 0; is < ns; ++is) {
-                const TsGeo<Real> g = ts_geometry<Real>(r, tc, ext, 1.0 / ns, is, inv_1pk, inv_dg, s.ng);
+                const TsGeo<Real> g = ts_geometry<Real>(r, tc, ext, inv_ns, is, inv_1pk, inv_dg, s.ng);
 #pragma unroll
                 for (int q = 0; q < PC; ++q)
                     if (q < npc) {
                         const Real* l = s_ldm + (size_t)q * s.ng;
-                        const Real ip = g.gz ? Real(0) : (g.rb * l[g.ig] + g.ra * l[g.ig + 1]);
-                        acc[q] += ip * (g.inside ? g.ap0 * s_afac[q] : g.ap0 + s_kd[q] * g.dadk);
+                        const Real ip = g.rb * l[g.ig] + g.ra * l[g.ig + 1];
+                        const Real area = g.inside ? g.ap0 * s_afac[q] : g.ap0 + s_kd[q] * g.dadk;
+                        acc[q] += g.gz ? Real(0) : ip * area;
                     }
             }
         }
 #pragma unroll
         for (int q = 0; q < PC; ++q)
-            if (q < npc) out[(size_t)(pb0 + q) * s.npt] = inw ? Real(1) - acc[q] * (s_iist[q] * inv_ns) : Real(1);
+            if (q < npc) out[(size_t)(pb0 + q) * s.npt] = inw ? Real(1) - acc[q] * s_f[q] : Real(1);
     }
 }
 
@@ -1468,7 +1468,16 @@ int ts_evaluate(int precision, const rr_table* tab, const rr_lcdata* lc, const r
             return check_launch("ts_flux_rows_kernel");
         }
     }
-    if (uns >= 1 && uns <= kTsTabSamples) {
+    // Few passbands of many times leave the table kernel's waves without a group of four:
+    // they go to the kernel below, a lane a time with all passbands in its registers (us,
+    // table / a lane a time: 60 pv x 20,000 t, 10 samples, in 2, 8 and 16 passbands FP64
+    // 92 / 56, 96 / 67, 100 / 86, mixed 100 / 58, 106 / 66, 106 / 81; 1000 x 3000 mixed, 3
+    // samples, 16 passbands 195 / 241; 300 x 1237 mixed, 30 samples, 8 passbands 164 / 227).
+    const long long nlane = (long long)npv * ((npt + kTsThreads - 1) / kTsThreads);
+    const bool big = nlane >= 3072;
+    const bool few = nlane >= 1024 &&
+                     npb <= (mixed ? (uns > 16 && !big ? 0 : 8) : (uns >= 8 && big ? 16 : 12));
+    if (uns >= 1 && uns <= kTsTabSamples && !few) {
         const size_t lds = mixed ? ts_tab_lds<float>(uns, a.ng) : ts_tab_lds<double>(uns, a.ng);
         const int T = mixed ? ts_tab_times<float>(uns) : ts_tab_times<double>(uns);
         if (lds <= 160 * 1024) {

@@ -1,9 +1,10 @@
-"""TSModel: the disk integrals of a law without an analytic one, around a block of them,
-against the FP64 oracle (1e-9 in FP64, 1 ppm mixed)."""
+"""TSModel calls of few passbands around the sizes at which they leave the table kernel,
+and the disk integrals of a law without an analytic one around a block of them, against
+the FP64 oracle (1e-9 in FP64, 1 ppm mixed)."""
 import numpy as np
 import pytest
 
-from pytransit_amd import TSModel, workloads
+from pytransit_amd import TabulatedLDModel, TSModel, workloads
 
 pytestmark = pytest.mark.gpu
 MU = dict(nzin=24, nzlimb=24)
@@ -19,6 +20,21 @@ def check(oracle, tm, wl, ldc, ldp, istar, nss, ext, precision):
                                 ldp[r], istar[r], None, 0, 0, 0, 100, 0, ze)
     assert np.array_equal(np.isnan(f[r]), np.isnan(ref)) and np.nanmin(ref) < 1
     assert np.nanmax(np.abs(f[r] - ref)) <= (1e-9 if precision == 'fp64' else 1e-6)
+
+
+# 1024 and 3072 workgroups of 256 times, 8, 12 and 16 passbands, 8, 16 and 32 samples
+@pytest.mark.parametrize('npv,npb,npt,nss', [
+    (1024, 1, 70, 3), (512, 12, 257, 2), (512, 13, 257, 2), (1023, 2, 70, 5), (1024, 8, 70, 16), (1024, 9, 70, 16),
+    (1024, 8, 70, 17), (1536, 8, 300, 17), (3072, 16, 33, 8), (3072, 17, 33, 8), (3071, 16, 33, 8), (1024, 3, 40, 32),
+    (1024, 3, 1, 1), (1024, 2, 40, 33)])
+@pytest.mark.parametrize('precision', ['fp64', 'mixed'])
+def test_few_passbands(gpu, oracle, npv, npb, npt, nss, precision):
+    wl = workloads.ts_many_pb(npv=npv, npt=npt, npb=npb, seed=npv + npt, mu=TSModel('quadratic', **MU).mu)
+    if npt == 1:
+        wl.times = np.array([0.003])
+    wl.a[1] = 0.5                           # an invalid vector
+    tm = TSModel(TabulatedLDModel(wl.ldp, wl.istar), precision=precision, **MU)
+    check(oracle, tm, wl, None, wl.ldp, wl.istar, nss, 0.01 if nss > 1 else 0.0, precision)
 
 
 @pytest.mark.parametrize('npv,npb', [(1, 1), (5, 51), (4, 64), (1, 257), (9, 60)])
